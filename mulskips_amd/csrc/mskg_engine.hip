@@ -163,8 +163,31 @@ __device__ inline double read_lane(double v, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-__device__ inline void slot_add(RunState *st, int b, double r, unsigned long long n, unsigned long long nev,
-                                const unsigned long long *cnt) {
+// A pointer read from device memory (a replica's parameters, a descriptor) is
+// a generic pointer to the compiler, and every access through it a flat
+// instruction, which waits on both the vector-memory and the LDS counters.
+// Every pointer of a lattice is to global memory; the rate tables and the
+// geometry are constant while a kernel runs, so that reads of one value by
+// the whole wave are scalar loads.  A round trip through the address space
+// states that (through an integer: a direct cast there and back folds away).
+template <typename T>
+__device__ inline T *as_global(T *p) {
+  __attribute__((address_space(1))) T *g = (__attribute__((address_space(1))) T *)(uintptr_t)p;
+  return (T *)g;
+}
+template <typename T>
+__device__ inline const T *as_constant(const T *p) {
+  const __attribute__((address_space(4))) T *c = (const __attribute__((address_space(4))) T *)(uintptr_t)p;
+  return (const T *)c;
+}
+__device__ inline void to_global(Lattice &L) {
+  L.site = as_global(L.site); L.rate = as_global(L.rate); L.cls = as_global(L.cls);
+  L.inlist = as_global(L.inlist); L.tl_idx = as_global(L.tl_idx); L.tl_n = as_global(L.tl_n);
+  L.tl_own = as_global(L.tl_own); L.tile_r = as_global(L.tile_r); L.list_err = as_global(L.list_err);
+  L.win = as_global(L.win); L.geo = as_constant(L.geo); L.tab = as_constant(L.tab); L.key = as_global(L.key);
+  L.cl = as_global(L.cl);
+}
+__device__ inline void slot_add(RunState *st, int b, double r, unsigned long long n, unsigned long long nev) {
   Slot &sl = st->slot[b & (NSLOT - 1)];
   if (n) {
     const unsigned long long rb = (unsigned long long)__double_as_longlong(r);
@@ -172,12 +195,12 @@ __device__ inline void slot_add(RunState *st, int b, double r, unsigned long lon
     atomicAdd(&sl.n, n);
     atomicAdd(&sl.tiles, 1ull);
   }
-  if (nev) {
-    atomicAdd(&sl.events, nev);
-    if (cnt)
-      for (int q = 0; q < 8; q++)
-        if (cnt[q]) atomicAdd(&sl.counts[q], cnt[q]);
-  }
+  if (nev) atomicAdd(&sl.events, nev);
+}
+
+// The reference event's counter (RunState::counts).
+__device__ inline int count_slot(int itrans) {
+  return itrans <= 3 ? itrans - 1 : (itrans == 4 ? 3 : (itrans == 5 ? 4 : itrans - 1));
 }
 
 struct TileGeom {
@@ -231,111 +254,88 @@ __device__ inline int tile_local(const TileGeom &g, int T, const P3 &p) {
 // Each thread takes four consecutive points: four 16-byte record loads in
 // flight, one 16-byte store of the rates and one 4-byte store of the
 // classes.  Nearly every point is not an MC particle (a few per cent of the
-// stored points are), so the Get_Prob branch is rare and its registers
-// (spilled at four waves per SIMD) cost little.
-template <bool LA, bool COV>
-__device__ inline void sweep_point(const Lattice &L, double rtot, int64_t p, const Site &sp, int atoms_only,
-                                   int *err, float &r_out, uint8_t &c_out, bool &keep) {
-  const int kind = s_kind(sp), coor = s_coor(sp);
+// stored points are), so the Get_Prob branch is rare.
+// Whether a record is an MC particle's; keep: atoms_only leaves the point alone.
+__device__ inline bool sweep_mc(uint32_t w, int atoms_only, bool &keep) {
+  const int kind = w & 7, coor = (w >> 3) & 7;
   keep = atoms_only && !(kind_species(kind) && coor >= 1 && coor <= 3);
-  const bool mc = (kind == KIND_EMPTY && coor >= 1 && coor <= 3) || (kind >= KIND_COV0 && coor <= 3) ||
-                  (kind_species(kind) && coor <= 3);
-  int cls = 0, key = -1;
-  double r = 0.0;
-  if (mc && !keep) {
-    P3 pt;
-    pt.i = p;
-    pxyz(L.box, p, pt.x, pt.y, pt.z);
-    int e = ERR_NONE;
-    get_prob<LA, COV>(L, rtot, pt, sp, coor, list_of(L, pt, sp), cls, r, e, nullptr, &key);
-    if (e) atomicExch(err, e);
-  }
-  r_out = cls ? (float)r : 0.0f;
-  c_out = (uint8_t)cls;
-  if (L.key && !keep) L.key[p] = cls ? key : -1;
+  return !keep && ((kind == KIND_EMPTY && coor >= 1 && coor <= 3) || (kind >= KIND_COV0 && coor <= 3) ||
+                   (kind_species(kind) && coor <= 3));
 }
 
 // LA, COV: the rate model's laser-annealing and coverage branches are compiled in.
-// Four consecutive points from p0, or the points p0..n-1 at the end.
+// Four consecutive points from p0, or the points p0..n-1 at the end.  One
+// instance of Get_Prob: the group's MC particles are taken in turn and their
+// records read again (from the cache), so that the stream itself holds few
+// registers -- 62 with 8 waves per SIMD, against 128 and 4 with Get_Prob
+// inlined for each of the four records.
 template <bool LA, bool COV>
 __device__ inline void sweep_group(const Lattice &L, double rtot, int *err, int atoms_only, int64_t p0, int64_t n) {
-  if (p0 + 4 <= n) {
-    Site sp[4];
-    for (int k = 0; k < 4; k++) sp[k] = L.site[p0 + k];
-    float r[4];
-    uint8_t c[4];
-    bool keep[4];
-    for (int k = 0; k < 4; k++) sweep_point<LA, COV>(L, rtot, p0 + k, sp[k], atoms_only, err, r[k], c[k], keep[k]);
-    if (!(keep[0] || keep[1] || keep[2] || keep[3])) {
-      *(float4 *)(L.rate + p0) = make_float4(r[0], r[1], r[2], r[3]);
-      *(uchar4 *)(L.cls + p0) = make_uchar4(c[0], c[1], c[2], c[3]);
-    } else {
-      for (int k = 0; k < 4; k++)
-        if (!keep[k]) {
-          L.rate[p0 + k] = r[k];
-          L.cls[p0 + k] = c[k];
-        }
-    }
+  const int m = p0 + 4 <= n ? 4 : (int)(n - p0);
+  uint32_t w[4];
+  if (m == 4) {
+    Rec sp[4];
+    for (int k = 0; k < 4; k++) sp[k] = load_rec(L, p0 + k);
+    for (int k = 0; k < 4; k++) w[k] = sp[k].w;
   } else {
-    for (int64_t q = p0; q < n; q++) {
-      float r;
-      uint8_t c;
-      bool keep;
-      sweep_point<LA, COV>(L, rtot, q, L.site[q], atoms_only, err, r, c, keep);
-      if (!keep) {
-        L.rate[q] = r;
-        L.cls[q] = c;
+    for (int k = 0; k < 4; k++) w[k] = k < m ? load_rec(L, p0 + k).w : 0u;
+  }
+  float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  uint32_t c = 0;
+  unsigned mc = 0, kept = 0;
+  for (int k = 0; k < 4; k++) {
+    bool keep;
+    mc |= sweep_mc(w[k], atoms_only, keep) && k < m ? 1u << k : 0u;
+    kept |= keep ? 1u << k : 0u;
+    if (L.key && !keep && k < m) L.key[p0 + k] = -1;
+  }
+#pragma unroll 1
+  for (; mc; mc &= mc - 1u) {
+    const int k = __ffs((int)mc) - 1;
+    P3 pt;
+    pt.i = p0 + k;
+    pxyz(L.box, pt.i, pt.x, pt.y, pt.z);
+    int e = ERR_NONE, cls = 0, key = -1;
+    double rd = 0.0;
+    get_prob<LA, COV>(L, rtot, pt, load_rec(L, pt.i), cls, rd, e, key);
+    if (e) atomicExch(err, e);
+    const float rf = cls ? (float)rd : 0.0f;
+    if (k == 0) r.x = rf;
+    if (k == 1) r.y = rf;
+    if (k == 2) r.z = rf;
+    if (k == 3) r.w = rf;
+    c |= (uint32_t)cls << (8 * k);
+    if (L.key && cls) L.key[pt.i] = key;
+  }
+  if (m == 4 && !kept) {
+    *(float4 *)(L.rate + p0) = r;
+    *(uint32_t *)(L.cls + p0) = c;
+  } else {
+    for (int k = 0; k < 4; k++)
+      if (k < m && !((kept >> k) & 1u)) {
+        L.rate[p0 + k] = k == 0 ? r.x : (k == 1 ? r.y : (k == 2 ? r.z : r.w));
+        L.cls[p0 + k] = (uint8_t)(c >> (8 * k));
       }
-    }
   }
 }
 
-// LA, COV: the rate model's laser-annealing and coverage branches are compiled in.
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_rate_sweep(Lattice L, double rtot, int *err, int atoms_only) {
+  L.tab = as_constant(L.tab);
   const int64_t n = L.box.npts;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
-  for (int64_t p0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; p0 < n; p0 += stride) {
-    if (p0 + 4 <= n) {
-      Site sp[4];
-      for (int k = 0; k < 4; k++) sp[k] = L.site[p0 + k];
-      float r[4];
-      uint8_t c[4];
-      bool keep[4];
-      for (int k = 0; k < 4; k++) sweep_point<LA, COV>(L, rtot, p0 + k, sp[k], atoms_only, err, r[k], c[k], keep[k]);
-      if (!(keep[0] || keep[1] || keep[2] || keep[3])) {
-        *(float4 *)(L.rate + p0) = make_float4(r[0], r[1], r[2], r[3]);
-        *(uchar4 *)(L.cls + p0) = make_uchar4(c[0], c[1], c[2], c[3]);
-      } else {
-        for (int k = 0; k < 4; k++)
-          if (!keep[k]) {
-            L.rate[p0 + k] = r[k];
-            L.cls[p0 + k] = c[k];
-          }
-      }
-    } else {
-      for (int64_t q = p0; q < n; q++) {
-        float r;
-        uint8_t c;
-        bool keep;
-        sweep_point<LA, COV>(L, rtot, q, L.site[q], atoms_only, err, r, c, keep);
-        if (!keep) {
-          L.rate[q] = r;
-          L.cls[q] = c;
-        }
-      }
-    }
-  }
+  for (int64_t p0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; p0 < n; p0 += stride)
+    sweep_group<LA, COV>(L, rtot, err, atoms_only, p0, n);
 }
 
 // The same over the points [first, end) of the stored order (first a
 // multiple of 4), in groups of four counted in 32 bits (the largest lattice
-// holds fewer than 2^31 groups).  A kernel of its own: the whole-lattice
-// sweep keeps its registers without the range.
+// holds fewer than 2^31 groups).
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_rate_sweep_range(Lattice L, double rtot, int *err, int64_t first, int64_t end) {
+  L.tab = as_constant(L.tab);
   const int g_first = (int)(first >> 2), g_end = (int)((end + 3) >> 2);
   const int gstride = gridDim.x * blockDim.x;
   for (int g = g_first + blockIdx.x * blockDim.x + threadIdx.x; g < g_end; g += gstride)
@@ -346,51 +346,51 @@ k_rate_sweep_range(Lattice L, double rtot, int *err, int64_t first, int64_t end)
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) k_replay(Lattice L, const mskg_event *log, int64_t n, int clock_mode,
                                                  RunState *st) {
-  __shared__ EvScratch sc;
-  __shared__ int s_bad;
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
+  L.geo = as_constant(L.geo);
+  L.tab = as_constant(L.tab);
+  load_tables(*L.tab, tabs, lane);
+  __syncthreads();
   double clock = st->clock;
-  for (int64_t k = 0; k < n; k++) {
+  int bad = 0;
+  P3 s;
+  s.x = s.y = s.z = 0;
+  int64_t k = 0;
+  for (; k < n; k++) {
     const mskg_event ev = log[k];
-    const P3 s = at(L, ev.site[0], ev.site[1], ev.site[2]);
-    if (lane == 0) s_bad = (s.i < 0 || L.cls[s.i] == 0) ? 1 : 0;
-    __syncthreads();
-    if (s_bad) {
-      if (lane == 0) {
-        st->err = ERR_NOT_MC;
-        st->err_site[0] = s.x; st->err_site[1] = s.y; st->err_site[2] = s.z;
-        st->events = (unsigned long long)k;
-      }
-      return;
+    s = at(L, __builtin_amdgcn_readfirstlane(ev.site[0]), __builtin_amdgcn_readfirstlane(ev.site[1]),
+           __builtin_amdgcn_readfirstlane(ev.site[2]));
+    const int itrans = __builtin_amdgcn_readfirstlane(ev.itrans);
+    if (s.i < 0 || __builtin_amdgcn_readfirstlane((int)L.cls[s.i]) == 0) {
+      bad = ERR_NOT_MC;
+      break;
     }
     if (clock_mode == 0) clock = clock + 1.0 / ev.rtot;
     Choice ch;
-    ch.arm = ev.arm;
+    ch.arm = __builtin_amdgcn_readfirstlane(ev.arm);
     ch.u_arm = 0.0;
-    EvResult res;
-    execute<LA, COV>(L, ev.rtot, s, ev.itrans, ch, res, sc, lane);
-    if (lane == 0) s_bad = res.err;
-    __syncthreads();
-    if (s_bad) {
-      if (lane == 0) {
-        st->err = res.err;
-        st->err_site[0] = s.x; st->err_site[1] = s.y; st->err_site[2] = s.z;
-        st->events = (unsigned long long)k;
-      }
-      return;
-    }
+    EvOut o;
+    execute<LA, COV>(L, tabs, ev.rtot, s, uniform_rec(load_rec(L, s.i)), itrans, ch, o, lane);
+    bad = __builtin_amdgcn_readfirstlane(o.err);
+    if (bad) break;
     if (lane == 0) {
-      int slot = ev.itrans <= 3 ? ev.itrans - 1 : (ev.itrans == 4 ? 3 : (ev.itrans == 5 ? 4 : ev.itrans - 1));
+      const int slot = count_slot(itrans);
       if (slot >= 0 && slot < 8) st->counts[slot]++;
-      if (COV && ev.itrans == 5 && res.species) st->desorbed[res.species - 1]++;
-      if (LA && L.cl && res.species && ev.itrans <= 4) {  // CountCrystal, then the next iteration's CountLiquid
-        st->cc[res.species - 1] += ev.itrans <= 3 ? 1 : -1;
+      if (COV && itrans == 5 && o.species) st->desorbed[o.species - 1]++;
+      if (LA && L.cl && o.species && itrans <= 4) {  // CountCrystal, then the next iteration's CountLiquid
+        st->cc[o.species - 1] += itrans <= 3 ? 1 : -1;
         for (int q = 0; q < 3; q++) st->cl[q] = st->cinit[q] - st->cc[q];
       }
     }
-    __syncthreads();  // the next event's rates read the counts
+    __syncthreads();  // the next event reads this one's records, rates and counts
   }
-  if (lane == 0) {
+  if (lane != 0) return;
+  if (bad) {
+    st->err = bad;
+    st->err_site[0] = s.x; st->err_site[1] = s.y; st->err_site[2] = s.z;
+    st->events = (unsigned long long)k;
+  } else {
     st->events += (unsigned long long)n;
     st->clock = clock;
   }
@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(256) k_tile_rates(Lattice L, int ntiles, RunSt
   for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, WAVE);
   if (lane == 0) {
     L.tile_r[t] = cnt ? acc : 0.0;
-    if (cnt) slot_add(st, t, acc, (unsigned long long)cnt, 0, nullptr);
+    if (cnt) slot_add(st, t, acc, (unsigned long long)cnt, 0);
   }
 }
 
@@ -513,33 +513,31 @@ __device__ inline void sort_by_offset(int32_t *lk, float *lr, uint8_t *lc, int l
   }
 }
 
-// The LDS of one tile's pass besides its candidate list (which is dynamic).
-struct PassLds {
-  unsigned long long cnt[8];  // events by type (lane 0)
-  long long dcc[3];           // crystal count changes (laser-annealing build's form)
-  unsigned long long des[3];  // desorptions by coverage slot
-  EvScratch sc;
-};
-
 // One tile's share of a colour pass: its candidate list into LDS, rejection-
 // free KMC inside the tile for the window tau, the list back.  Returns the
-// error that ends the wave's work (0: none).
+// error that ends the wave's work (0: none).  The selected site, its record
+// and the event type are kept in scalar registers: the event's addresses and
+// branches are then scalar too.
 template <bool LA, bool COV>
 __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, const double tau, const int t,
-                                const int colour, PassLds &S, int32_t *lk, float *lr, uint8_t *lc, const int lane) {
+                                const int colour, const TabLds &tabs, int32_t *lk, float *lr, uint8_t *lc,
+                                const int lane) {
   const int cap = P.cap;
   // The tile's first loads leave together, in one round trip: its list
   // length and own count, the first WAVE list entries (read whatever the
   // length; a lane uses its entry only below it, and the index stays in the
   // tile's list storage), and the run state the window needs.
-  const int n_in = L.tl_n[t];
-  const int own = L.tl_own[t];
+  const int n_in = __builtin_amdgcn_readfirstlane(L.tl_n[t]);
+  const int own = __builtin_amdgcn_readfirstlane(L.tl_own[t]);
   const int k_first = L.tl_idx[(int64_t)t * L.capg + min(lane, L.capg - 1)];
   const double rtot = st->rtot;
   const unsigned long long sweeps = st->sweeps;
   if (n_in == 0) return 0;
-  L.cur_tile = t;
   TileGeom g = tile_geom(t, L.tile, L.ntx, L.nty, L.box.lz);
+  L.cur_tile = t;
+  L.cx = g.tx * L.tile;
+  L.cy = g.ty * L.tile;
+  L.cz = g.z0;
 
   // 1. the tile's candidate list -> LDS, dropping entries no longer active;
   // the entries other tiles appended since the tile's last pass (an order
@@ -582,21 +580,31 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
 
   // 2. rejection-free KMC inside the tile for the window tau
   double tloc = 0.0;
-  unsigned long long nev = 0;
-  if (lane < 8) S.cnt[lane] = 0;
-  if (lane < 3) S.dcc[lane] = 0;
-  if (COV && lane < 3) S.des[lane] = 0;
-  U4 ctr;
-  ctr.x = (uint32_t)t;
-  ctr.y = (uint32_t)sweeps;
-  ctr.z = (uint32_t)(sweeps >> 32) ^ ((uint32_t)colour << 29);
-  ctr.w = 0;
+  unsigned int nev = 0;
+  unsigned int my_cnt = 0, my_des = 0;  // lane l: events of counter l, desorptions of coverage slot l + 1
+  int my_dcc = 0;                       // lane l: change of CountCrystal(l + 1) (laser-annealing build's form)
+  U4 d;              // lane l: the Philox block of draw 64 b + l, b the current batch
+  double wait = 0.0;  // ... and -ln of its first uniform
   int err = 0;
   // every wave ends its pass: the window tau bounds the expected number of
   // events, and this cap bounds the worst case (a window cut short by it is
   // counted in RunState::guard_exits and reported by the run)
   int guard = 0;
   for (; guard < PASS_EVENT_CAP; guard++) {
+    // one Philox block per event: waiting time, selection, event type and
+    // stacking choice, 32 random bits each (the reference's ran3 has fewer).
+    // The block depends on the draw's number only, so the wave makes 64 of
+    // them, and their FP64 logarithms, at once.
+    const int dl = guard & (WAVE - 1);
+    if (dl == 0) {
+      U4 ctr;
+      ctr.x = (uint32_t)t;
+      ctr.y = (uint32_t)sweeps;
+      ctr.z = (uint32_t)(sweeps >> 32) ^ ((uint32_t)colour << 29);
+      ctr.w = (uint32_t)(guard + lane);
+      d = philox4x32_10(ctr, P.key0, P.key1);
+      wait = -log(u01_32(d.x));
+    }
     // lane-major order: lane l owns entries l, l + 64, ...; one wave scan of
     // the lanes' partial sums gives the total and the lane that holds the pick
     double part = 0.0;
@@ -604,107 +612,91 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
     const double inc = wave_incl_scan_dpp(part);
     const double R = read_lane(inc, WAVE - 1);
     if (!(R > 0.0)) break;
-    // one Philox block per event: waiting time, selection, event type and
-    // stacking choice, 32 random bits each (the reference's ran3 has fewer)
-    const U4 d = philox4x32_10(ctr, P.key0, P.key1);
-    ctr.w++;
-    const double dt = -log(u01_32(d.x)) / R;  // FP64 waiting time
+    const double dt = read_lane(wait, dl) / R;  // FP64 waiting time
     if (tloc + dt > tau) break;
     tloc += dt;
-    const double target = u01_32(d.y) * R;
+    const double target = u01_32((uint32_t)__builtin_amdgcn_readlane((int)d.y, dl)) * R;
     // the first lane whose inclusive prefix exceeds target (the last lane
     // with a rate when rounding leaves target at the top end), then the
     // first of its entries whose running prefix exceeds target
-    const unsigned long long hit = __ballot(part > 0.0 && inc > target);
     const unsigned long long nzl = __ballot(part > 0.0);
+    const unsigned long long hit = __ballot(part > 0.0 && inc > target);
     if (!nzl) break;
     const int owner = hit ? __ffsll((long long)hit) - 1 : 63 - __clzll((long long)nzl);
-    int sel = -1;
-    if (lane == owner) {
-      double acc = inc - part;
-      int last = -1;
-      for (int j = lane; j < n; j += WAVE) {
-        const double v = (double)lr[j];
-        if (v > 0.0) {
-          last = j;
-          acc += v;
-          if (acc > target) {
-            sel = j;
-            break;
+    int sel = owner;  // up to 64 entries: the lane's only one
+    if (n > WAVE) {
+      sel = -1;
+      if (lane == owner) {
+        double acc = inc - part;
+        int last = -1;
+        for (int j = lane; j < n; j += WAVE) {
+          const double v = (double)lr[j];
+          if (v > 0.0) {
+            last = j;
+            acc += v;
+            if (acc > target) {
+              sel = j;
+              break;
+            }
           }
         }
+        if (sel < 0) sel = last;
       }
-      if (sel < 0) sel = last;
+      sel = __builtin_amdgcn_readlane(sel, owner);
+      if (sel < 0) break;
     }
-    sel = __builtin_amdgcn_readlane(sel, owner);
-    if (sel < 0) break;
-    {
-      const P3 s = tile_point(L.box, g, L.tile, lk[sel]);
-      Choice ch;
-      ch.arm = -1;
-      ch.u_arm = u01_32(d.w);
-      const int itrans = la_swap<LA>(L, pick_itrans<LA, COV>(L, s, lc[sel], u01_32(d.z)));
-      const int coor0 = P.log ? s_coor(L.site[s.i]) : 0;
-      __syncthreads();  // every lane has read the site before it changes
-      EvResult res;
-      execute<LA, COV>(L, rtot, s, itrans, ch, res, S.sc, lane);
-      __syncthreads();  // neighbour updates by lanes 1..3 are visible to lane 0
-      err = __builtin_amdgcn_readfirstlane(res.err);  // res is complete on lane 0
-      if (lane == 0) {
-        if (P.log) {
-          const unsigned long long li = atomicAdd(&st->log_n, 1ull);
-          if (li < P.log_cap) {
-            mskg_event ev;
-            ev.iter = (int64_t)li + 1;
-            ev.site[0] = s.x; ev.site[1] = s.y; ev.site[2] = s.z;
-            ev.itrans = itrans;
-            ev.arm = res.arm;
-            ev.coor = coor0;
-            ev.rtot = rtot;
-            ev.time = st->clock + tloc;
-            P.log[li] = ev;
-          }
-        }
-        int slot = itrans <= 3 ? itrans - 1 : (itrans == 4 ? 3 : (itrans == 5 ? 4 : itrans - 1));
-        if (slot >= 0 && slot < 8) S.cnt[slot]++;
-        if (LA && L.cl && res.species && itrans <= 4) S.dcc[res.species - 1] += itrans <= 3 ? 1 : -1;
-        if (COV && itrans == 5 && res.species) S.des[res.species - 1]++;
+    const P3 s = tile_point(L.box, g, L.tile, __builtin_amdgcn_readfirstlane(lk[sel]));
+    const Rec srec = uniform_rec(load_rec(L, s.i));
+    const int cls = __builtin_amdgcn_readfirstlane((int)lc[sel]);
+    Choice ch;
+    ch.arm = -1;
+    ch.u_arm = u01_32((uint32_t)__builtin_amdgcn_readlane((int)d.w, dl));
+    const int coor0 = r_coor(srec);
+    const int itrans = __builtin_amdgcn_readfirstlane(la_swap<LA>(
+        L, pick_itrans<LA, COV>(L, TabEv<COV>{*L.tab, tabs}, coor0, r_temp(srec), cls,
+                                u01_32((uint32_t)__builtin_amdgcn_readlane((int)d.z, dl)))));
+    EvOut o;
+    execute<LA, COV>(L, tabs, rtot, s, srec, itrans, ch, o, lane);
+    err = __builtin_amdgcn_readfirstlane(o.err);
+    if (P.log && lane == 0) {
+      const unsigned long long li = atomicAdd(&st->log_n, 1ull);
+      if (li < P.log_cap) {
+        mskg_event ev;
+        ev.iter = (int64_t)li + 1;
+        ev.site[0] = s.x; ev.site[1] = s.y; ev.site[2] = s.z;
+        ev.itrans = itrans;
+        ev.arm = o.arm;
+        ev.coor = coor0;
+        ev.rtot = rtot;
+        ev.time = st->clock + tloc;
+        P.log[li] = ev;
       }
     }
+    if (lane == count_slot(itrans)) my_cnt++;
+    if (LA && o.species && itrans <= 4 && lane == o.species - 1) my_dcc += itrans <= 3 ? 1 : -1;
+    if (COV && itrans == 5 && o.species && lane == o.species - 1) my_des++;
     nev++;
     if (err) break;
-    // the touched points' new rates, one lane each, as execute() left them
-    // on chip (S.sc holds them until the next event); a point that got no
-    // new rate keeps its list entry as it is
-    const int nt = __builtin_amdgcn_readfirstlane(S.sc.ntouched);
-    int kl = -1;  // tile-local offset of touched point `lane` (-1: none / outside the tile)
-    float tr = 0.0f;
-    uint8_t tc = 0;
-    if (lane < nt) {
-      const P3 tp = S.sc.touched[lane];
-      const int ts = S.sc.tset[lane];
-      kl = ts ? tile_local(g, L.tile, tp) : -1;
-      if (kl >= 0) {
-        if (ts == 1) {
-          tr = S.sc.trate[lane];
-          tc = S.sc.tcls[lane];
-        } else {
-          tr = L.rate[tp.i];
-          tc = L.cls[tp.i];
-        }
-      }
+    // refresh the on-chip list with the touched points' new rates, which
+    // execute() left a lane each: the slot of each touched point inside the
+    // tile, one ballot of the list against its offset (list entries are
+    // distinct, so each touched point has at most one slot; a point touched
+    // twice finds the same slot), and whether an earlier touched point has
+    // the same offset
+    const int kl = o.set ? tile_local(g, L.tile, o.p) : -1;
+    float tr = o.rate;
+    int tc = o.cls;
+    if (o.set == 2 && kl >= 0) {
+      tr = L.rate[o.p.i];
+      tc = L.cls[o.p.i];
     }
-    // refresh the on-chip list: the slot of each touched point, one ballot
-    // of the list against its offset (list entries are distinct, so each
-    // touched point has at most one slot; a point touched twice finds the
-    // same slot), and whether an earlier touched point has the same offset
     int found = -1;
     bool dup = false;
     const int k_lane = lane < n ? lk[lane] : -1;  // the list's first WAVE entries, one a lane
-    for (int q = 0; q < nt; q++) {
+    for (unsigned long long tm = __ballot(kl >= 0); tm; tm &= tm - 1ull) {
+      const int q = __ffsll((long long)tm) - 1;
       const int kq = __builtin_amdgcn_readlane(kl, q);
       if (q < lane && kq == kl) dup = true;
-      if (kq < 0) continue;
       unsigned long long m = __ballot(k_lane == kq);
       int f = m ? __ffsll((long long)m) - 1 : -1;
       for (int j0 = WAVE; f < 0 && j0 < n; j0 += WAVE) {
@@ -720,26 +712,28 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
     if (kl >= 0) {
       if (found >= 0) {
         lr[found] = tr;
-        lc[found] = tc;
+        lc[found] = (uint8_t)tc;
       } else if (tc) {
         app = !dup;
       }
     }
     const unsigned long long am = __ballot(app);
-    if (app) {
-      const int slot = n + __popcll(am & ((1ull << lane) - 1ull));
-      if (slot < cap) {
-        lk[slot] = kl;
-        lr[slot] = tr;
-        lc[slot] = tc;
+    if (am) {
+      if (app) {
+        const int slot = n + __popcll(am & ((1ull << lane) - 1ull));
+        if (slot < cap) {
+          lk[slot] = kl;
+          lr[slot] = tr;
+          lc[slot] = (uint8_t)tc;
+        }
       }
+      if (n + __popcll(am) > cap) {  // the list keeps its first cap entries
+        err = ERR_CAPACITY;
+        break;
+      }
+      n += __popcll(am);
     }
-    if (n + __popcll(am) > cap) {  // the list keeps its first cap entries
-      err = ERR_CAPACITY;
-      break;
-    }
-    n += __popcll(am);
-    __syncthreads();
+    __syncthreads();  // the next event reads this one's records and list entries
   }
   if (guard >= PASS_EVENT_CAP && lane == 0) atomicAdd(&st->guard_exits, 1ull);
   // 3. write the list back (active entries only), tile totals, counters
@@ -756,17 +750,14 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
     nout += __popcll(m);
   }
   const double R = wave_sum(part);
+  if (lane < 8 && my_cnt) atomicAdd(&st->slot[t & (NSLOT - 1)].counts[lane], (unsigned long long)my_cnt);
+  if (LA && L.cl && my_dcc) atomicAdd(&st->dcc[lane], (unsigned long long)(long long)my_dcc);
+  if (COV && my_des) atomicAdd(&st->desorbed[lane], (unsigned long long)my_des);
   if (lane == 0) {
     L.tl_n[t] = nout;
     L.tl_own[t] = nout;
     L.tile_r[t] = R;
-    slot_add(st, t, R, (unsigned long long)nout, nev, S.cnt);
-    if (LA && L.cl)
-      for (int k = 0; k < 3; k++)
-        if (S.dcc[k]) atomicAdd(&st->dcc[k], (unsigned long long)S.dcc[k]);
-    if (COV)
-      for (int k = 0; k < 3; k++)
-        if (S.des[k]) atomicAdd(&st->desorbed[k], S.des[k]);
+    slot_add(st, t, R, (unsigned long long)nout, nev);
     if (nout) {
       if (g.tz < L.win[4 * colour + 2]) atomic_min_i32(&L.win[4 * colour + 2], g.tz);
       if (g.tz > L.win[4 * colour + 3]) atomic_max_i32(&L.win[4 * colour + 3], g.tz);
@@ -777,7 +768,6 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
       st->err_site[0] = p.x; st->err_site[1] = p.y; st->err_site[2] = p.z;
     }
   }
-  err = __builtin_amdgcn_readfirstlane(err);  // the same in every lane
   if (err) return err;
   __syncthreads();
   return 0;
@@ -805,12 +795,16 @@ __device__ inline int colour_tile(const Lattice &L, int colour, int zfirst, int 
 
 // One colour pass: the tiles of `colour` in the window of tile layers that
 // hold candidates, each workgroup (one wave) striding over them.  Three
-// waves per SIMD (168 VGPRs): 3072 tiles in flight on 256 CUs, against the
-// ~4096 tiles of a colour pass at the 512^3 workload.
+// waves per SIMD (168 VGPRs, no spills): 3072 tiles in flight on 256 CUs.
+// Measured on 8e6 events at 512^3 SiC: 69.1 ms; with two waves 74.9, with
+// four (128 VGPRs, spilled) 76.0.  The laser-annealing kernels hold exp and
+// erf: two waves (223 VGPRs), 55.3 ms on two exchanges of 3e4 events at
+// 264x264x384, against 60.4 with three (184 bytes a lane spilled) and 79.4
+// with four.
 template <bool LA, bool COV>
-__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3, 3))) k_pass(PassParams P) {
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_pass(PassParams P) {
   extern __shared__ unsigned char smem[];
-  __shared__ PassLds S;
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
   Lattice L = P.L;
   int32_t *lk = (int32_t *)smem;        // tile-local point offsets
@@ -819,11 +813,14 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3, 3)
   RunState *st = P.st;
   const double tau = st->tau;
   if (!(tau > 0.0) || st->err || st->stop) return;
+  L.geo = as_constant(L.geo);
+  L.tab = as_constant(L.tab);
   int zfirst;
   const int nwin = colour_tiles(L, P.ntz, P.colour, zfirst);
+  if ((int)blockIdx.x < nwin) load_tables(*L.tab, tabs, lane);
   for (int wi = blockIdx.x; wi < nwin; wi += gridDim.x) {
     const int t = colour_tile(L, P.colour, zfirst, wi);
-    if (pass_tile<LA, COV>(P, L, st, tau, t, P.colour, S, lk, lr, lc, lane)) return;
+    if (pass_tile<LA, COV>(P, L, st, tau, t, P.colour, tabs, lk, lr, lc, lane)) return;
   }
 }
 
@@ -864,9 +861,9 @@ __device__ inline void queue_layers(int zlo, int zhi, int odd, int ntz, int &fir
 constexpr long long SCHED_WAIT_TICKS = 200000000ll;
 
 template <bool LA, bool COV>
-__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3, 3))) k_sweep(PassParams P) {
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_sweep(PassParams P) {
   extern __shared__ unsigned char smem[];
-  __shared__ PassLds S;
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
   Lattice L = P.L;
   int32_t *lk = (int32_t *)smem;
@@ -878,6 +875,9 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3, 3)
   // the window as the sweep starts (L.win's first words widen during it)
   const int zlo = (int)P.sched[3], zhi = (int)P.sched[4];
   if (zlo > zhi) return;
+  L.geo = as_constant(L.geo);
+  L.tab = as_constant(L.tab);
+  load_tables(*L.tab, tabs, lane);
   int first[2], count[2];
   queue_layers(zlo, zhi, 0, P.ntz, first[0], count[0]);
   queue_layers(zlo, zhi, 1, P.ntz, first[1], count[1]);
@@ -957,7 +957,7 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3, 3)
                                                                          __HIP_MEMORY_SCOPE_AGENT));
     const int n_in = __builtin_amdgcn_readfirstlane(L.tl_n[t]);
     if (!abort && !err_now && n_in > 0) {
-      pass_tile<LA, COV>(P, L, st, tau, t, colour, S, lk, lr, lc, lane);
+      pass_tile<LA, COV>(P, L, st, tau, t, colour, tabs, lk, lr, lc, lane);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // the tile's writes before its flag
     }
     // every lane stores the same stamp
@@ -1145,30 +1145,6 @@ __global__ void __launch_bounds__(ENS_MAX) k_ens_plan(const PassParams *__restri
   }
 }
 
-// A pointer read from device memory is a generic (flat) pointer to the
-// compiler, and every access through it a flat instruction, which waits on
-// both the vector-memory and the LDS counters and takes 64-bit addresses in
-// vector registers.  Every pointer of a replica's parameters is to global
-// memory: a round trip through the global address space states that.  In
-// k_pass_ens the lattice is laundered where a wave changes replica but not
-// its first value, so the loop's merge of the two stays generic and most of
-// the tile's accesses remain flat: laundering the first value as well makes
-// them global but adds spills, and measured 2% slower on the 64-replica
-// SiGe ensemble at tile 16 (660.7 against 646.5 ms).
-template <typename T>
-__device__ inline T *as_global(T *p) {
-  // through an integer: a direct cast there and back folds away
-  __attribute__((address_space(1))) T *g = (__attribute__((address_space(1))) T *)(uintptr_t)p;
-  return (T *)g;
-}
-__device__ inline void to_global(Lattice &L) {
-  L.site = as_global(L.site); L.rate = as_global(L.rate); L.cls = as_global(L.cls);
-  L.inlist = as_global(L.inlist); L.tl_idx = as_global(L.tl_idx); L.tl_n = as_global(L.tl_n);
-  L.tl_own = as_global(L.tl_own); L.tile_r = as_global(L.tile_r); L.list_err = as_global(L.list_err);
-  L.win = as_global(L.win); L.geo = as_global(L.geo); L.tab = as_global(L.tab); L.key = as_global(L.key);
-  L.cl = as_global(L.cl);
-}
-
 // The replica whose tiles hold entry q of colour pc's queue: the last r with
 // pc[r] <= q (pc is the colour's prefix, pc[n] > q), 64 prefixes at a time.
 __device__ inline int ens_replica(const int *pc, int n, int q, int lane) {
@@ -1181,10 +1157,10 @@ __device__ inline int ens_replica(const int *pc, int n, int q, int lane) {
 }
 
 template <bool LA, bool COV>
-__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3, 3)))
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3)))
 k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
   extern __shared__ unsigned char smem[];
-  __shared__ PassLds S;
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
   const int *pc = plan + colour * (n + 1);
   const int total = __builtin_amdgcn_readfirstlane(pc[n]);
@@ -1210,6 +1186,7 @@ k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
       hi = __builtin_amdgcn_readfirstlane(pc[r + 1]);
       L = reps[r].L;
       to_global(L);
+      load_tables(*L.tab, tabs, lane);
       st = as_global(reps[r].st);
       // a replica that has failed in this sweep runs no further tiles here
       // (k_pass checks at the start of each colour pass)
@@ -1225,7 +1202,7 @@ k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
       float *lr = (float *)(lk + P.cap);
       uint8_t *lc = (uint8_t *)(lr + P.cap);
       // a wave stops its tiles of a replica whose tile failed (as k_pass's wave returns)
-      failed = __builtin_amdgcn_readfirstlane(pass_tile<LA, COV>(P, L, st, tau, t, colour, S, lk, lr, lc, lane));
+      failed = __builtin_amdgcn_readfirstlane(pass_tile<LA, COV>(P, L, st, tau, t, colour, tabs, lk, lr, lc, lane));
     }
     // the next entry: every lane adds 1 (one atomic of 64 for the wave)
     const unsigned int took = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1313,12 +1290,13 @@ __global__ void __launch_bounds__(256) k_build_slab(Lattice L, int len, int sic,
         s.kc = (uint8_t)(sp | (2 << 3));
         if (z >= t.frozen_below_z) {
           cls = CLS_EVAP;
-          r = PEv(t, sp, 2, 0, 0, 0, 0, 0);
+          r = t.pe[pe_flat(sp, 2, 0, 0, 0, 0, 0)];
         }
       } else {
         s.kc = (uint8_t)(KIND_EMPTY | (2 << 3));
         cls = CLS_ADSORB;
-        r = pd_of(t, 1, 2, 0) + pd_of(t, 2, 2, 0) + pd_of(t, 3, 2, 0) + t.pabs[0 + 6] + t.pabs[1 + 6] + t.pabs[2 + 6];
+        r = pd_of<true>(TabSrc{t}, 1, 2, 0) + pd_of<true>(TabSrc{t}, 2, 2, 0) + pd_of<true>(TabSrc{t}, 3, 2, 0) +
+            t.pabs[0 + 6] + t.pabs[1 + 6] + t.pabs[2 + 6];
       }
     }
     L.site[p] = s;
@@ -1617,20 +1595,20 @@ __device__ int scan_pick(const double *v, int n, double target, int lane, double
 constexpr int SERIAL_LDS_TILES = 4096;
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
-  __shared__ EvScratch sc;
-  __shared__ int s_tiles[MAX_TOUCHED], s_ntl, s_err;
+  __shared__ TabLds tabs;
   __shared__ double s_tsum[SERIAL_LDS_TILES], s_bsum[SERIAL_LDS_TILES / WAVE];
-  __shared__ unsigned long long s_cnt[8];
   const int lane = threadIdx.x;
   const SerialDesc D = descs[blockIdx.x];
   Lattice L = D.L;
+  to_global(L);
   L.cur_tile = -1;
-  RunState *st = D.st;
+  RunState *st = as_global(D.st);
+  load_tables(*L.tab, tabs, lane);
   if (st->err) return;
   const bool on_chip = D.ntiles <= SERIAL_LDS_TILES;
   double *tsum = on_chip ? s_tsum : D.tsum;
   double *bsum = on_chip ? s_bsum : D.bsum;
-  if (lane < 8) s_cnt[lane] = 0;
+  unsigned long long my_cnt = 0;  // lane l: events of counter l
   // initial sums
   for (int t = 0; t < D.ntiles; t++) {
     const double ts = tile_sum_compact(L, t, lane);
@@ -1691,19 +1669,19 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
     }
     if (sel < 0) sel = last_nz;
     if (sel < 0) { err = ERR_SUMS; break; }
-    const P3 s = tile_point(L.box, g, L.tile, idx[sel]);
+    const P3 s = tile_point(L.box, g, L.tile, __builtin_amdgcn_readfirstlane(idx[sel]));
     Choice ch;
     ch.arm = -1;
     ch.u_arm = u01_32(d.w);
-    const int itrans = pick_itrans<LA, COV>(L, s, L.cls[s.i], u01_32(d.z));
-    const int coor0 = s_coor(L.site[s.i]);
-    __syncthreads();
-    EvResult res;
-    execute<LA, COV>(L, R, s, itrans, ch, res, sc, lane);
-    __syncthreads();
+    const Rec srec = uniform_rec(load_rec(L, s.i));
+    const int coor0 = r_coor(srec);
+    const int itrans = __builtin_amdgcn_readfirstlane(pick_itrans<LA, COV>(
+        L, TabEv<COV>{*L.tab, tabs}, coor0, r_temp(srec), __builtin_amdgcn_readfirstlane((int)L.cls[s.i]),
+        u01_32(d.z)));
+    EvOut o;
+    execute<LA, COV>(L, tabs, R, s, srec, itrans, ch, o, lane);
     clock += dt;
     if (lane == 0) {
-      s_err = res.err;
       if (D.log) {
         const unsigned long long li = st->log_n + nev;
         if (li < D.log_cap) {
@@ -1711,44 +1689,39 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
           ev.iter = (int64_t)(events + 1);
           ev.site[0] = s.x; ev.site[1] = s.y; ev.site[2] = s.z;
           ev.itrans = itrans;
-          ev.arm = res.arm;
+          ev.arm = o.arm;
           ev.coor = coor0;
           ev.rtot = R;
           ev.time = clock;
           D.log[li] = ev;
         }
       }
-      const int slot = itrans <= 3 ? itrans - 1 : (itrans == 4 ? 3 : (itrans == 5 ? 4 : itrans - 1));
-      if (slot >= 0 && slot < 8) s_cnt[slot]++;
-      if (COV && itrans == 5 && res.species) st->desorbed[res.species - 1]++;
-      int nt = 0;
-      for (int q = 0; q < sc.ntouched; q++) {
-        if (sc.touched[q].i < 0) continue;
-        const int tq = tile_of(L, sc.touched[q]);
-        bool dup = false;
-        for (int r = 0; r < nt; r++) dup |= s_tiles[r] == tq;
-        if (!dup) s_tiles[nt++] = tq;
-      }
-      s_ntl = nt;
+      if (COV && itrans == 5 && o.species) st->desorbed[o.species - 1]++;
     }
+    if (lane == count_slot(itrans)) my_cnt++;
     __syncthreads();
     events++;
     nev++;
-    if (s_err) { err = s_err; break; }
-    const int ntl = s_ntl;
-    for (int q = 0; q < ntl; q++) {
-      const double ts = tile_sum_compact(L, s_tiles[q], lane);
-      if (lane == 0) tsum[s_tiles[q]] = ts;
+    err = __builtin_amdgcn_readfirstlane(o.err);
+    if (err) break;
+    // the tiles of the points that got a new rate, each rescanned once; then
+    // the blocks of those tiles
+    const int tq = o.set ? tile_of(L, o.p) : -1;
+    const unsigned long long tm = __ballot(o.set != 0);
+    for (unsigned long long m2 = tm; m2;) {
+      const int tt = __builtin_amdgcn_readlane(tq, __ffsll((long long)m2) - 1);
+      m2 &= ~__ballot(tq == tt);
+      const double ts = tile_sum_compact(L, tt, lane);
+      if (lane == 0) tsum[tt] = ts;
     }
     __syncthreads();
-    for (int q = 0; q < ntl; q++) {
-      const int bq = s_tiles[q] / WAVE;
-      bool dup = false;
-      for (int r = 0; r < q; r++) dup |= s_tiles[r] / WAVE == bq;
-      if (dup) continue;
-      const int tt = bq * WAVE + lane;
+    const int bq = o.set ? tq / WAVE : -1;
+    for (unsigned long long m2 = tm; m2;) {
+      const int bb = __builtin_amdgcn_readlane(bq, __ffsll((long long)m2) - 1);
+      m2 &= ~__ballot(bq == bb);
+      const int tt = bb * WAVE + lane;
       const double v = wave_sum(tt < D.ntiles ? tsum[tt] : 0.0);
-      if (lane == 0) bsum[bq] = v;
+      if (lane == 0) bsum[bb] = v;
     }
     __syncthreads();
   }
@@ -1757,9 +1730,9 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
     st->events = events;
     st->log_n += nev;
     st->stop = stop;
-    for (int q = 0; q < 8; q++) st->counts[q] += s_cnt[q];
     if (err) st->err = err;
   }
+  if (lane < 8) st->counts[lane] += my_cnt;
 }
 
 // ---- adjoint: replay with per-class accounting ---------------------------------
@@ -1796,14 +1769,19 @@ struct AdjDesc {
 __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
   extern __shared__ unsigned char smem[];
   int *cnt = (int *)smem;                 // [KEY_N] class populations
-  __shared__ EvScratch sc;
-  __shared__ int s_bad;
-  __shared__ int s_o[MAX_TOUCHED], s_nw[MAX_TOUCHED];
-  __shared__ float s_ro[MAX_TOUCHED], s_rn[MAX_TOUCHED];
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
-  const AdjDesc D = descs[blockIdx.x];
+  AdjDesc D = descs[blockIdx.x];
+  D.key_seen = as_global(D.key_seen);
+  D.rate_seen = as_global(D.rate_seen);
+  D.log = as_global(D.log);
+  D.dt = as_global(D.dt);
+  D.S = as_global(D.S);
+  D.acc = as_global(D.acc);
   Lattice L = D.L;
+  to_global(L);
   L.cur_tile = -1;
+  load_tables(*L.tab, tabs, lane);
   // the per-class integrals and change times in the segment's own device
   // memory (LDS holds the populations only, so that more waves fit a CU)
   double *const A = D.acc, *const tau = D.acc + KEY_N;
@@ -1833,56 +1811,56 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
     }
     t += dtk;
     ttot += dtk;
-    const P3 s = at(L, ev.site[0], ev.site[1], ev.site[2]);
+    const P3 s = at(L, __builtin_amdgcn_readfirstlane(ev.site[0]), __builtin_amdgcn_readfirstlane(ev.site[1]),
+                    __builtin_amdgcn_readfirstlane(ev.site[2]));
+    const int itrans = __builtin_amdgcn_readfirstlane(ev.itrans);
+    if (s.i < 0) { err = ERR_NOT_MC; break; }
+    // the site's class, key and record in one round trip
+    const int cs = L.cls[s.i], ks = __builtin_amdgcn_readfirstlane(D.key_seen[s.i]);
+    const Rec srec = uniform_rec(load_rec(L, s.i));
+    if (__builtin_amdgcn_readfirstlane(cs) == 0) err = ERR_NOT_MC;
+    else if (ks < 0) err = ERR_COVERAGE;  // a rate class the likelihood does not cover
+    else if (ks >= KEY_ADS && ks < KEY_PH && (itrans < 1 || itrans > 3)) err = ERR_NOT_MC;
+    if (err) break;
     if (lane == 0) {
-      int bad = 0;
-      const int ks = s.i >= 0 ? D.key_seen[s.i] : -1;
-      if (s.i < 0 || L.cls[s.i] == 0) bad = ERR_NOT_MC;
-      else if (ks < 0) bad = ERR_COVERAGE;  // a rate class the likelihood does not cover
-      else if (ks >= KEY_ADS && ks < KEY_PH) {
-        if (ev.itrans < 1 || ev.itrans > 3) bad = ERR_NOT_MC;
-        else atomicAdd(&D.S[KEY_N + (ev.itrans - 1) * 3 + (ks - KEY_ADS)], 1.0);
-      } else if (ks == KEY_ISO) {
-        iso_log += log((double)D.rate_seen[s.i]);
-        atomicAdd(&D.S[KEY_ISO], 1.0);
-      } else {
-        atomicAdd(&D.S[ks], 1.0);  // no return value: the wave does not wait for it
-      }
-      s_bad = bad;
+      // the selections by class: no return value, the wave does not wait
+      const int sk = ks >= KEY_ADS && ks < KEY_PH ? KEY_N + (itrans - 1) * 3 + (ks - KEY_ADS) : ks;
+      atomicAdd(&D.S[sk], 1.0);
+      if (ks == KEY_ISO) iso_log += log((double)D.rate_seen[s.i]);
     }
-    __syncthreads();
-    if (s_bad) { err = s_bad; break; }
     Choice ch;
-    ch.arm = ev.arm;
+    ch.arm = __builtin_amdgcn_readfirstlane(ev.arm);
     ch.u_arm = 0.0;
-    EvResult res;
-    execute<false, false>(L, ev.rtot, s, ev.itrans, ch, res, sc, lane);  // the likelihood excludes LA and coverage tables
+    EvOut out;
+    execute<false, false>(L, tabs, ev.rtot, s, srec, itrans, ch, out, lane);  // the likelihood excludes LA and coverage tables
     __syncthreads();
-    // the touched points' keys and rates, before and after, one lane each
-    // (a point listed twice is taken once); every class change of the event
+    // the touched points' keys and rates, before and after, a lane each (a
+    // point listed twice is taken once); every class change of the event
     // happens at time t, so the accounting below does not depend on order
-    const int nt = __builtin_amdgcn_readfirstlane(sc.ntouched);
     int o = -3, nw = -1;  // o = -3: a point an earlier lane holds (or none)
     float ro = 0.0f, rn = 0.0f;
-    if (lane < nt) {
-      const int64_t p = sc.touched[lane].i;
-      bool first = p >= 0;
-      for (int q = 0; q < lane; q++)
-        if (sc.touched[q].i == p) first = false;
-      if (first) {
-        o = D.key_seen[p];
-        nw = L.key[p];
-        ro = D.rate_seen[p];
-        rn = L.rate[p];
-        D.key_seen[p] = nw;
-        D.rate_seen[p] = rn;
-      }
-      s_o[lane] = o;
-      s_nw[lane] = nw;
-      s_ro[lane] = ro;
-      s_rn[lane] = rn;
+    if (out.set) {
+      o = D.key_seen[out.p.i];
+      nw = L.key[out.p.i];
+      ro = D.rate_seen[out.p.i];
+      rn = L.rate[out.p.i];
     }
-    int bad = __builtin_amdgcn_readfirstlane(res.err);  // res is complete on lane 0
+    if (__ballot(out.set == 2)) {  // repeated list entries
+      bool dup = false;
+      for (int q = 0; q < 4; q++) {
+        const int l = 4 * q + 1;
+        const int lo = __builtin_amdgcn_readlane((int)(uint32_t)out.p.i, l);
+        const int hi = __builtin_amdgcn_readlane((int)(out.p.i >> 32), l);
+        const int on = __builtin_amdgcn_readlane(out.set, l);
+        dup |= on && l < lane && lo == (int)(uint32_t)out.p.i && hi == (int)(out.p.i >> 32);
+      }
+      if (dup) o = -3;
+    }
+    if (out.set && o != -3) {
+      D.key_seen[out.p.i] = nw;
+      D.rate_seen[out.p.i] = rn;
+    }
+    int bad = __builtin_amdgcn_readfirstlane(out.err);
     if (!bad && __ballot(o != -3 && nw == KEY_UNSUPPORTED)) bad = ERR_COVERAGE;
     if (!bad) {
       // Every class change of the event happens at time t: a class's
@@ -1890,10 +1868,11 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
       // adds population x 0), so the earliest lane holding a class, as old
       // or new class in touched order, updates it with the population before
       // the event, and the populations then change by atomics.
-      const bool ch = o != -3 && o != nw;
-      const int co = ch && o >= 0 ? o : -1, cn = ch && nw >= 0 ? nw : -1;
+      const bool chg = o != -3 && o != nw;
+      const int co = chg && o >= 0 ? o : -1, cn = chg && nw >= 0 ? nw : -1;
       bool do_o = co >= 0, do_n = cn >= 0;
-      for (int q = 0; q < nt; q++) {
+      for (unsigned long long cm = __ballot(chg); cm; cm &= cm - 1ull) {
+        const int q = __ffsll((long long)cm) - 1;
         const int qo = __builtin_amdgcn_readlane(co, q), qn = __builtin_amdgcn_readlane(cn, q);
         if (q < lane) {
           if (qo == co || qn == co) do_o = false;
@@ -1905,20 +1884,14 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
       __syncthreads();  // every first update has read its population
       if (co >= 0) atomicAdd(&cnt[co], -1);
       if (cn >= 0) atomicAdd(&cnt[cn], 1);
-      // the isolated-atom rate sum changes in touched order (lane 0; rare)
-      const bool iso_ch = o != -3 && (o == KEY_ISO ? (double)ro : 0.0) != (nw == KEY_ISO ? (double)rn : 0.0);
-      if (__ballot(iso_ch) && lane == 0)
-        for (int q = 0; q < nt; q++) {
-          const int oq = s_o[q], nq = s_nw[q];
-          if (oq == -3) continue;
-          const double roq = oq == KEY_ISO ? (double)s_ro[q] : 0.0;
-          const double rnq = nq == KEY_ISO ? (double)s_rn[q] : 0.0;
-          if (roq != rnq) {
-            iso_int += r_iso * (t - tau_iso);
-            tau_iso = t;
-            r_iso += rnq - roq;
-          }
-        }
+      // the isolated-atom rate sum changes in touched order (rare)
+      const double roq = o == KEY_ISO ? (double)ro : 0.0, rnq = nw == KEY_ISO ? (double)rn : 0.0;
+      for (unsigned long long im = __ballot(o != -3 && roq != rnq); im; im &= im - 1ull) {
+        const int q = __ffsll((long long)im) - 1;
+        iso_int += r_iso * (t - tau_iso);
+        tau_iso = t;
+        r_iso += read_lane(rnq, q) - read_lane(roq, q);
+      }
     }
     __syncthreads();
     if (bad) { err = bad; k++; break; }

@@ -50,6 +50,7 @@ struct Lattice {
   const Tables *tab;
   int tile, ntx, nty, capg;
   int cur_tile;           // the tile whose pass is running: its list lives on chip
+  int cx, cy, cz;         // its lowest corner (when cur_tile >= 0)
   float inv_tile;         // 1 / tile
   int32_t *key;           // may be null: rate-class key of every point (likelihood accounting)
   const long long *cl;    // may be null: CountLiquid(1..3) the laser-annealing build's rates read
@@ -180,34 +181,65 @@ MSKG_HD void widen_window(const Lattice &L, int colour, int tz) {
 // A site that becomes an MC particle joins its tile's list (once).
 MSKG_HD void enlist(const Lattice &L, const P3 &p) {
   if (!L.inlist) return;
+  // the running tile keeps its list on chip and flags it on write-back
+  if (L.cur_tile >= 0 && (unsigned)(p.x - L.cx) < (unsigned)L.tile && (unsigned)(p.y - L.cy) < (unsigned)L.tile &&
+      (unsigned)(p.z - L.cz) < (unsigned)L.tile)
+    return;
+  if (L.inlist[p.i]) return;
   const int tx = tdiv(L, p.x), ty = tdiv(L, p.y), tz = tdiv(L, p.z);
   const int t = (tz * L.nty + ty) * L.ntx + tx;
-  if (t == L.cur_tile) return;  // the running tile keeps its list on chip and flags it on write-back
-  if (L.inlist[p.i]) return;
   L.inlist[p.i] = 1;
   widen_window(L, tile_colour(tx, ty, tz), tz);
   const int slot = atomic_add_i32(&L.tl_n[t], 1);
   if (slot < L.capg) L.tl_idx[(int64_t)t * L.capg + slot] = tile_pack(p.z - tz * L.tile, p.y - ty * L.tile, p.x - tx * L.tile);
   else *L.list_err = ERR_TILE_LIST;
 }
-MSKG_HD void set_rate(const Lattice &L, const P3 &p, int cls, double rate, int key = -1) {
-  if (p.i < 0) return;
-  L.rate[p.i] = cls ? (float)rate : 0.0f;
-  L.cls[p.i] = (uint8_t)cls;
-  if (L.key) L.key[p.i] = cls ? key : -1;
-  if (cls) enlist(L, p);
-}
 
 // ---- rates ---------------------------------------------------------------
-MSKG_HD double PEv(const Tables &t, int sp, int a, int b, int c, int d, int e, int f) {
-  return t.pe[(sp - 1) + 3 * (a + 4 * (b + 4 * (c + 4 * (d + 4 * (e + 4 * f)))))];
+// Where a rate evaluation takes the tables from: all of them in device
+// memory (the sweep), or an event wave's copy in LDS.
+struct TabSrc {
+  const Tables &t;
+  MSKG_HD double pe(int i) const { return t.pe[i]; }
+  MSKG_HD double pd(int i) const { return t.pd[i]; }
+  MSKG_HD double pabs(int i) const { return t.pabs[i]; }
+  MSKG_HD double pdes(int i) const { return t.pdes[i]; }
+  MSKG_HD double f2(int i) const { return t.f2[i]; }
+};
+// The tables an event reads, 2 KB of LDS a wave: a lookup is the last of an
+// event's chain of dependent reads, and from memory it cost a round trip of
+// its own.  PTransE's entries without covered neighbours are the first 192
+// of the full table; with coverage species the full table stays in memory.
+constexpr int PE_PLAIN = 192;
+struct TabLds {
+  double pe[PE_PLAIN], pd[9], pabs[12], pdes[12], f2[13];
+};
+template <bool COV>
+struct TabEv {
+  const Tables &t;
+  const TabLds &l;
+  MSKG_HD double pe(int i) const { return COV ? t.pe[i] : l.pe[i]; }
+  MSKG_HD double pd(int i) const { return l.pd[i]; }
+  MSKG_HD double pabs(int i) const { return l.pabs[i]; }
+  MSKG_HD double pdes(int i) const { return l.pdes[i]; }
+  MSKG_HD double f2(int i) const { return l.f2[i]; }
+};
+__device__ inline void load_tables(const Tables &t, TabLds &l, int lane) {
+  for (int i = lane; i < PE_PLAIN; i += 64) l.pe[i] = t.pe[i];
+  if (lane < 9) l.pd[lane] = t.pd[lane];
+  if (lane < 12) {
+    l.pabs[lane] = t.pabs[lane];
+    l.pdes[lane] = t.pdes[lane];
+  }
+  if (lane < 13) l.f2[lane] = t.f2[lane];
 }
 // The reference's kb (Get_Prob.f:70).
 #define MSKG_KB 0.00008617330350
 // LA = false compiles the laser-annealing branches out (tables with la_mode 0).
-template <bool LA = true>
-MSKG_HD double pd_of(const Tables &t, int sp, int coor, int temperature, const long long *cl = nullptr) {
-  double e = t.pd[(sp - 1) + 3 * (coor - 1)];
+template <bool LA, class Src>
+MSKG_HD double pd_of(const Src &S, int sp, int coor, int temperature, const long long *cl = nullptr) {
+  const Tables &t = S.t;
+  double e = S.pd((sp - 1) + 3 * (coor - 1));
   if (!LA || !t.la_mode) return e;
   if (t.la_variant && cl) {
     // LaserAnnealing Get_Prob.f:148-151, evaluated left to right: 0.5d0 *
@@ -223,9 +255,13 @@ MSKG_HD double pd_of(const Tables &t, int sp, int coor, int temperature, const l
   return 0.5 * t.p0 * exp(-e / (MSKG_KB * t.tm)) * (1.0 + erf((temperature - t.tflex) / t.sigma)) *
          (e != 0.0 ? 1.0 : 0.0);
 }
-template <bool LA = true>
-MSKG_HD double pe_of(const Tables &t, int sp, int a, int b, int c, int d, int e, int f, int temperature) {
-  double v = PEv(t, sp, a, b, c, d, e, f);
+MSKG_HD int pe_flat(int sp, int a, int b, int c, int d, int e, int f) {
+  return (sp - 1) + 3 * (a + 4 * (b + 4 * (c + 4 * (d + 4 * (e + 4 * f)))));
+}
+template <bool LA, class Src>
+MSKG_HD double pe_of(const Src &S, int sp, int idx, int temperature) {
+  const Tables &t = S.t;
+  double v = S.pe(idx);
   if (!LA || !t.la_mode) return v;
   const double p0 = t.la_variant ? t.la_p0[sp - 1] : t.p0;  // LaserAnnealing Get_Prob.f:144-146
   return p0 * exp(-v / (MSKG_KB * temperature)) * (v != 0.0 ? 1.0 : 0.0);
@@ -278,100 +314,62 @@ MSKG_HD double st_entry(const double *ref, int stride, int idx, const STW &w) {
   return ((double)w.wl * ref[(int64_t)w.il * stride + idx] + (double)w.wu * ref[(int64_t)w.iu * stride + idx]) /
          (double)(w.wl + w.wu);
 }
-MSKG_HD int pe_flat(int sp, int a, int b, int c, int d, int e, int f) {
-  return (sp - 1) + 3 * (a + 4 * (b + 4 * (c + 4 * (d + 4 * (e + 4 * f)))));
+// What a rate depends on besides the point's own record, packed so that the
+// lanes looking at a point's neighbours add up in one word: reciprocal
+// neighbours of species 1..3 (bits 0, 4, 8), walls (12), reciprocal covered
+// neighbours by slot (16, 20, 24), occupied second-neighbour positions (28).
+MSKG_HD uint32_t neighbour_count(int kq, bool lists) {
+  if (kq == KIND_WALL) return 1u << 12;
+  if (!lists || kq == KIND_EMPTY) return 0u;
+  return kq < KIND_WALL ? 1u << (4 * (kq - 1)) : 1u << (16 + 4 * (kq - KIND_COV0));
 }
 
-// Get_Prob, Get_Prob.f:54-331, evaluated for point p whose record is sp,
-// with the coordination and neighbour list passed explicitly (Evaporation.f:121
-// passes a stale list copy).  rtot is the total rate R used by the
-// isolated-atom rule.  No random number is drawn: the deposition species /
-// absorbed coverage is drawn when the event executes (class CLS_ADSORB).
-// Records that are newer than HBM (updated by this event on another lane):
-// reads of these points take the given record instead.  known_i /
-// known_coor: a point whose coordination the caller already holds (the
-// event's site during the neighbour updates), read by the coordination-1
-// rule of an empty site without a gather.
-struct Ovr {
-  int n;
-  int64_t idx[5];
-  Site rec[5];
-};
-MSKG_HD Site rd_o(const Lattice &L, int64_t i, const Ovr *o) {
-  if (o && i >= 0)
-    for (int k = 0; k < o->n; k++)
-      if (o->idx[k] == i) return o->rec[k];
-  return rd(L, i);
-}
-
-// The 12 second-neighbour positions of a diamond super-lattice site (the
-// fcc shell: (+-6,+-6,0) and permutations), for the optional
-// second-neighbour energy term; no reference counterpart.
-MSKG_HD P3 second_pos(const Lattice &L, const P3 &p, int k) {
-  const int a = (k & 2) ? -6 : 6, b = (k & 1) ? -6 : 6, g = k >> 2;
-  int dx = g == 2 ? 0 : a, dy = g == 0 ? b : (g == 1 ? 0 : a), dz = g == 0 ? 0 : b;
-  int x = p.x + dx, y = p.y + dy;
-  if (x >= L.box.lx) x -= L.box.lx;
-  if (x < 0) x += L.box.lx;
-  if (y >= L.box.ly) y -= L.box.ly;
-  if (y < 0) y += L.box.ly;
-  return at(L, x, y, p.z + dz);
-}
-// Index step from a point to its second-neighbour position k when neither
-// wraps nor leaves the box: (dz * plane) + (dy / 2) * hx + dx / 2 with the
-// vectors of second_pos.
-MSKG_HD int64_t second_step(const Box &b, int k) {
-  const int a = (k & 2) ? -6 : 6, c = (k & 1) ? -6 : 6, g = k >> 2;
-  const int dx = g == 2 ? 0 : a, dy = g == 0 ? c : (g == 1 ? 0 : a), dz = g == 0 ? 0 : c;
-  return (int64_t)dz * b.plane + (int64_t)(dy / 2) * b.hx + dx / 2;
-}
+// Get_Prob, Get_Prob.f:54-331, evaluated for a point at height z of this
+// kind, temperature and coordination (Evaporation.f:121 evaluates with a
+// stale list copy: the counts are those of the list the caller went by).
+// c0: the coordination of its first listed neighbour (read for an empty point
+// of coordination 1); cnt: neighbour_count summed over its list (read for an
+// atom).  rtot is the total rate R used by the isolated-atom rule.  No random
+// number is drawn: the deposition species / absorbed coverage is drawn when
+// the event executes (class CLS_ADSORB).
 // COV = false compiles the coverage-species branches out (tables without
-// coverage species and without absorption or desorption rates).  STEP: the
-// second-shell gather of interior points takes fixed index steps (fewer
-// instructions, more registers: for the event kernels, not the sweep).
-template <bool LA = true, bool COV = true, bool STEP = false>
-MSKG_HD void get_prob(const Lattice &L, double rtot, const P3 &p, const Site &sp, int coor, const NL &nn, int &cls,
-                      double &rate, int &err, const Ovr *ovr = nullptr, int *key = nullptr, int64_t known_i = -1,
-                      int known_coor = 0) {
-  const Tables &t = *L.tab;
-  int kdummy;
-  if (!key) key = &kdummy;
-  *key = -1;
-  int kind = s_kind(sp);
+// coverage species and without absorption or desorption rates).
+template <bool LA, bool COV, class Src>
+MSKG_HD void rate_of(const Src &S, const long long *cl, double rtot, int z, int kind, int temp, int coor, int c0,
+                     uint32_t cnt, int &cls, double &rate, int &err, int &key) {
+  const Tables &t = S.t;
+  key = -1;
+  cls = CLS_NONE;
+  rate = 0.0;
   int temperature = 0;
   STW w;
   const bool st = LA && t.st_n > 0;  // Get_Prob.f:77-90: tables at the site's temperature
   if (LA && (t.la_mode || st)) {
-    temperature = (int)sp.temp;
-    if (temperature == 0) { err = ERR_TEMPERATURE; cls = CLS_NONE; rate = 0.0; return; }
-    if (st && !st_weights(t, temperature, w)) { err = ERR_ST_RANGE; cls = CLS_NONE; rate = 0.0; return; }
+    temperature = temp;
+    if (temperature == 0) { err = ERR_TEMPERATURE; return; }
+    if (st && !st_weights(t, temperature, w)) { err = ERR_ST_RANGE; return; }
   }
-  if (!COV && kind >= KIND_COV0) { err = ERR_COVERAGE; cls = CLS_NONE; rate = 0.0; return; }
-  int slot = COV ? kind_cov_slot(kind) : 0;
+  if (!COV && kind >= KIND_COV0) { err = ERR_COVERAGE; return; }
+  const int slot = COV ? kind_cov_slot(kind) : 0;
   if (slot) {  // desorption, :93-123
-    if (slot > t.ncov) { err = ERR_COVERAGE; cls = CLS_NONE; rate = 0.0; return; }
+    if (slot > t.ncov) { err = ERR_COVERAGE; return; }
     if (coor <= 3) {
       cls = CLS_DESORB;
-      rate = st ? st_entry(t.st_pdes, 12, (slot - 1) + 3 * coor, w) : t.pdes[(slot - 1) + 3 * coor];
-      *key = KEY_UNSUPPORTED;
+      rate = st ? st_entry(t.st_pdes, 12, (slot - 1) + 3 * coor, w) : S.pdes((slot - 1) + 3 * coor);
+      key = KEY_UNSUPPORTED;
     }
-    else { cls = CLS_NONE; rate = 0.0; }
     return;
   }
   if (kind == KIND_EMPTY) {  // :155-214
-    if (LA && t.la_mode && t.la_variant && L.cl && (L.cl[0] < 0 || L.cl[1] < 0 || L.cl[2] < 0)) {
+    if (LA && t.la_mode && t.la_variant && cl && (cl[0] < 0 || cl[1] < 0 || cl[2] < 0)) {
       // a negative solidification rate, which a sum tree cannot hold (the
       // reference's selection goes wrong there, or UpdateTree.f:37-41 stops
       // on a rate that cancels to zero): the engine stops with an error
-      err = ERR_LIQUID; cls = CLS_NONE; rate = 0.0; return;
+      err = ERR_LIQUID;
+      return;
     }
     if (coor >= 1 && coor <= 3) {
-      bool ok = true;
-      if (coor == 1) {
-        const int64_t i0 = entry(L, nn, 0).i;
-        ok = (i0 >= 0 && i0 == known_i ? known_coor : s_coor(rd_o(L, i0, ovr))) >= 2;
-      }
-      if (ok) {
+      if (coor > 1 || c0 >= 2) {
         double pdep, pabs;
         if (st) {
           pdep = st_entry(t.st_pd, 9, 3 * (coor - 1), w) + st_entry(t.st_pd, 9, 1 + 3 * (coor - 1), w) +
@@ -380,93 +378,59 @@ MSKG_HD void get_prob(const Lattice &L, double rtot, const P3 &p, const Site &sp
                            st_entry(t.st_pabs, 12, 2 + 3 * coor, w)
                      : 0.0;
         } else {
-          pdep = pd_of<LA>(t, 1, coor, temperature, L.cl) + pd_of<LA>(t, 2, coor, temperature, L.cl) +
-                 pd_of<LA>(t, 3, coor, temperature, L.cl);
-          pabs = COV ? t.pabs[0 + 3 * coor] + t.pabs[1 + 3 * coor] + t.pabs[2 + 3 * coor] : 0.0;
+          pdep = pd_of<LA>(S, 1, coor, temperature, cl) + pd_of<LA>(S, 2, coor, temperature, cl) +
+                 pd_of<LA>(S, 3, coor, temperature, cl);
+          pabs = COV ? S.pabs(0 + 3 * coor) + S.pabs(1 + 3 * coor) + S.pabs(2 + 3 * coor) : 0.0;
         }
         cls = CLS_ADSORB;
         rate = pdep + pabs;
-        *key = (t.ncov || st) ? KEY_UNSUPPORTED : KEY_ADS + coor - 1;
+        key = (t.ncov || st) ? KEY_UNSUPPORTED : KEY_ADS + coor - 1;
       } else {
         cls = CLS_PLACEHOLDER;
         rate = (double)1.e-8f;  // REAL(4) literal, Get_Prob.f:183
-        *key = KEY_PH;
+        key = KEY_PH;
       }
-    } else {
-      cls = CLS_NONE;  // Coor 0 leaves the reference's outputs unassigned; Coor 4 is a vacancy
-      rate = 0.0;
     }
-    return;
+    return;  // Coor 0 leaves the reference's outputs unassigned; Coor 4 is a vacancy
   }
   // evaporation, :215-324
-  if (p.z < t.frozen_below_z) {  // frozen substrate (engine option, no reference counterpart)
-    cls = CLS_NONE;
-    rate = 0.0;
-    return;
-  }
-  int n_si = 0, n_c = 0, n_b = 0, n_wall = 0, covnn[3] = {0, 0, 0};
-  P3 qs[4];
-  Site sqs[4];
-  uint8_t kc2[12];
-  for (int i = 0; i < 4; i++) qs[i] = entry(L, nn, i);
-  for (int i = 0; i < 4; i++) sqs[i] = rd_o(L, qs[i].i, ovr);  // four independent gathers in flight
-  if (t.use_f2) {  // ... and the twelve second-shell kinds with them
-    // at least 6 units from every face the shell neither wraps nor leaves
-    // the box, and its indices are p's plus fixed steps
-    const bool inner = STEP && p.x >= 6 && p.x < L.box.lx - 6 && p.y >= 6 && p.y < L.box.ly - 6 && p.z >= 6 &&
-                       p.z <= L.box.lz - 6;
-    for (int k = 0; k < 12; k++) {
-      const int64_t i2 = inner ? p.i + second_step(L.box, k) : second_pos(L, p, k).i;
-      kc2[k] = i2 < 0 ? (uint8_t)0 : (ovr ? rd_o(L, i2, ovr).kc : L.site[i2].kc);
-    }
-  }
-  for (int i = 0; i < 4; i++) {
-    const P3 &q = qs[i];
-    const Site &sq = sqs[i];
-    int kq = s_kind(sq);
-    if (kind_occupied(kq)) {
-      if (kq != KIND_WALL) {
-        if (lists_point(L.box, q, sq, p)) {
-          if (kq == 1) n_si++;
-          if (kq == 2) n_c++;
-          if (kq == 3) n_b++;
-        }
-      } else {
-        n_wall++;
-      }
-    } else if (COV && kind_cov_slot(kq)) {
-      if (lists_point(L.box, q, sq, p)) {
-        int s = kind_cov_slot(kq);
-        if (s > t.ncov) { err = ERR_COVERAGE; cls = CLS_NONE; rate = 0.0; return; }
-        covnn[s - 1]++;
-      }
-    }
-  }
-  int tot = n_si + n_c + n_b + n_wall;
-  if (tot != coor) { err = ERR_COORD; cls = CLS_NONE; rate = 0.0; return; }
-  if (tot > 3) {
-    cls = CLS_NONE;
-    rate = 0.0;
-  } else if (tot == 0) {
+  if (z < t.frozen_below_z) return;  // frozen substrate (engine option, no reference counterpart)
+  const int n_si = cnt & 15, n_c = (cnt >> 4) & 15, n_b = (cnt >> 8) & 15, n_wall = (cnt >> 12) & 15;
+  const int tot = n_si + n_c + n_b + n_wall;
+  if (tot != coor) { err = ERR_COORD; return; }
+  if (tot > 3) return;
+  if (tot == 0) {
     cls = CLS_ISOLATED;
     rate = (double)100000.0f * rtot;
-    *key = KEY_ISO;
-  } else {
-    int c1 = t.ncov >= 1 ? covnn[0] : 0, c2 = t.ncov >= 2 ? covnn[1] : 0, c3 = t.ncov >= 3 ? covnn[2] : 0;
-    cls = CLS_EVAP;
-    rate = st ? st_entry(t.st_pe, 3 * 4096, pe_flat(kind, n_si + n_wall, n_c, n_b, c1, c2, c3), w)
-              : pe_of<LA>(t, kind, n_si + n_wall, n_c, n_b, c1, c2, c3, temperature);
-    int n2 = 0;
-    if (t.use_f2) {
-      for (int k = 0; k < 12; k++) {
-        const int kq = kc2[k] & 7;
-        if (kind_occupied(kq) && kq != KIND_WALL) n2++;
-      }
-      rate *= t.f2[n2];
-    }
-    *key = (t.ncov || t.la_mode || st) ? KEY_UNSUPPORTED
-                                       : (kind - 1) + 3 * (n_si + n_wall + 4 * (n_c + 4 * n_b)) + 192 * n2;
+    key = KEY_ISO;
+    return;
   }
+  const int c1 = COV ? (cnt >> 16) & 15 : 0, c2 = COV ? (cnt >> 20) & 15 : 0, c3 = COV ? (cnt >> 24) & 15 : 0;
+  const int idx = pe_flat(kind, n_si + n_wall, n_c, n_b, c1, c2, c3);
+  cls = CLS_EVAP;
+  rate = st ? st_entry(t.st_pe, 3 * 4096, idx, w) : pe_of<LA>(S, kind, idx, temperature);
+  const int n2 = t.use_f2 ? (int)(cnt >> 28) : 0;
+  if (t.use_f2) rate *= S.f2(n2);
+  key = (t.ncov || t.la_mode || st) ? KEY_UNSUPPORTED : (kind - 1) + 3 * (n_si + n_wall + 4 * (n_c + 4 * n_b)) + 192 * n2;
+}
+
+// The 12 second-neighbour positions of a diamond super-lattice site (the
+// fcc shell: (+-6,+-6,0) and permutations), for the optional
+// second-neighbour energy term; no reference counterpart.
+MSKG_HD void second_vec(int k, int &dx, int &dy, int &dz) {
+  const int a = (k & 2) ? -6 : 6, b = (k & 1) ? -6 : 6, g = k >> 2;
+  dx = g == 2 ? 0 : a;
+  dy = g == 0 ? b : (g == 1 ? 0 : a);
+  dz = g == 0 ? 0 : b;
+}
+// p shifted by a small vector, with one x/y wrap.
+MSKG_HD P3 shifted(const Lattice &L, const P3 &p, int dx, int dy, int dz) {
+  int x = p.x + dx, y = p.y + dy;
+  if (x >= L.box.lx) x -= L.box.lx;
+  if (x < 0) x += L.box.lx;
+  if (y >= L.box.ly) y -= L.box.ly;
+  if (y < 0) y += L.box.ly;
+  return at(L, x, y, p.z + dz);
 }
 
 // Where a stochastic choice of the reference comes from: the log (replay)
@@ -476,424 +440,33 @@ struct Choice {
   double u_arm;  // uniform used when the arm/zig coordination sums tie
 };
 
-constexpr int MAX_TOUCHED = 17;
-struct EvResult {
-  int arm;        // stacking choice made (-1 none)
-  int err;
-  int species;    // deposited or evaporated species (1..3), desorbed coverage slot (1..3), 0 otherwise
-};
-
-MSKG_HD bool put_list(const Lattice &L, Site &s, const P3 &p, const NL &l, EvResult &res) {
-  if (!set_list(L.box, s, p.x, p.y, p.z, l)) { res.err = ERR_GEOM; return false; }
-  return true;
-}
-
-// ---- event execution -------------------------------------------------------
-// The whole workgroup (one 64-wide wave) executes an event together: lane 0
-// updates the site itself, lanes 0..3 update its four neighbours at once.
-// The reference visits the neighbours one after the other, but each
-// neighbour's update writes only that neighbour's record and reads only
-// records the other neighbour updates do not write (two neighbours of a
-// site are never neighbours of each other), so the concurrent updates give
-// the sequential result.  When two list entries resolve to the same point
-// the neighbours are visited in order by lane 0 instead.
-struct EvScratch {
-  NL nn;            // the site's neighbour list as the update loop uses it
-  P3 pts[4];
-  int coor_old;
-  int inc[4];       // per-neighbour change of the site's own coordination
-  int err[4];
-  int unfixed[4];   // evaporation: neighbour i was unfixed (Coor 2 -> 1)
-  int found[4];     //   ... and found its reciprocal partner (NBuff) at found_pos[i]
-  int found_pos[4][3];
-  int seq;          // visit the neighbours in order on lane 0
-  int old_kind;     // evaporation: the species that left the site
-  int nvisit;       // neighbours the event visits (desorption at coordination 1: one)
-  int abort;
-  P3 sec[12];       // second-neighbour refresh: the point refreshed by lane k (i = -1: none)
-  int err2[12];
-  // every point whose rate may have changed: the site, its neighbours and
-  // (second-neighbour term) the evaporating atoms on its second-neighbour
-  // positions; complete after execute() returns
-  P3 touched[MAX_TOUCHED];
-  int ntouched;
-  // the new rate and class of touched point q as stored in HBM, when tset[q]
-  // is 1; 0: the event gave it no new rate; 2: read it from HBM (a list with
-  // repeated entries, whose points take several rates in turn)
-  float trate[MAX_TOUCHED];
-  uint8_t tcls[MAX_TOUCHED];
-  uint8_t tset[MAX_TOUCHED];
-  float secrate[12];  // the second-shell refresh of lane k + 1
-  uint8_t seccls[12];
-};
-
-// The value set_rate stores, kept on chip for touched point q.
-__device__ inline void note_rate(EvScratch &sc, int q, int cls, double rate) {
-  sc.trate[q] = cls ? (float)rate : 0.0f;
-  sc.tcls[q] = (uint8_t)cls;
-  sc.tset[q] = 1;
-}
-
-#define MSKG_SYNC() __syncthreads()
-
-__device__ inline void prefetch4(const Lattice &L, const NL &nn, P3 q[4], Site sq[4]) {
-  for (int i = 0; i < 4; i++) q[i] = entry(L, nn, i);
-  for (int i = 0; i < 4; i++) sq[i] = rd(L, q[i].i);
-}
-
-__device__ inline void resolve_neighbours(const Lattice &L, EvScratch &sc, int n) {
-  int seq = 0;
-  for (int i = 0; i < 4; i++) sc.pts[i] = entry(L, sc.nn, i);
-  for (int i = 0; i < n; i++)
-    for (int j = i + 1; j < n; j++)
-      if (sc.pts[i].i >= 0 && sc.pts[i].i == sc.pts[j].i) seq = 1;
-  sc.seq = seq;
-  for (int i = 0; i < 4; i++) {
-    sc.inc[i] = 0;
-    sc.err[i] = 0;
-    sc.unfixed[i] = 0;
-    sc.found[i] = 0;
-  }
-}
-
-__device__ inline void touched_list(const P3 &s, EvScratch &sc, int n) {
-  sc.ntouched = 0;
-  sc.touched[sc.ntouched++] = s;
-  for (int i = 0; i < n; i++) sc.touched[sc.ntouched++] = sc.pts[i];
-  for (int q = 0; q <= n; q++) sc.tset[q] = 0;
-}
-
-// Second-neighbour term: after a change of occupancy at s, the evaporating
-// atom (coordination 1..3) on second-neighbour position k of s, if any,
-// gets a fresh rate from the final state of the event.  It runs beside the
-// site's own refresh: its evaluation reads the site only for its kind (and,
-// for the rare non-bond list entry, its list), which are final by then.
-struct FinalRefresh {
-  bool active;
-  P3 p;
-  Site sp;
-  int coor;
-  NL nn;
-};
-__device__ inline void second_setup(const Lattice &L, const P3 &s, int k, EvScratch &sc, FinalRefresh &f) {
-  const P3 q = second_pos(L, s, k);
-  sc.sec[k].i = -1;
-  if (q.i < 0) return;
-  const Site sq = rd(L, q.i);
-  const int kq = s_kind(sq), cq = s_coor(sq);
-  if (!kind_occupied(kq) || kq == KIND_WALL || cq < 1 || cq > 3) return;
-  sc.sec[k] = q;
-  f.active = true;
-  f.p = q;
-  f.sp = sq;
-  f.coor = cq;
-  f.nn = list_of(L, q, sq);
-}
-
-// A rate evaluation the neighbour phase asks for: the point, its record
-// (already written back unless list_after) and the coordination and list
-// the evaluation uses.  list_after: the record is written after the
-// evaluation, with the list stored only when the point gets a rate (AddMC).
-struct RefreshReq {
-  bool need, list_after;
-  P3 p;
-  Site sp;
-  int coor;
-  NL nn;
-};
-
-// deposition.f:78-235, the update of neighbour i of the new atom at s.
-__device__ void dep_prepare(const Lattice &L, const P3 &s, int i, EvScratch &sc, int &err, RefreshReq &q) {
-  const Geometry &g = *L.geo;
-  const int lx = L.box.lx, ly = L.box.ly;
-  const P3 p = sc.pts[i];
-  Site sp = rd(L, p.i);
-  int kind = s_kind(sp), coornn = s_coor(sp);
-  NL nnn = list_of(L, p, sp);
-  bool need = false, list_after = false;
-  if (!kind_occupied(kind)) {
-    if (coornn == 0) {
-      coornn = 1;
-      s_set_coor(sp, coornn);
-      for (int j = 0; j < 4; j++) nnn.x[j] = nnn.y[j] = nnn.z[j] = 0;
-      nnn.x[0] = s.x; nnn.y[0] = s.y; nnn.z[0] = s.z;
-      need = list_after = true;
-    } else if (coornn == 1) {
-      int dx = nnn.x[0] - s.x, dy = nnn.y[0] - s.y, dz = nnn.z[0] - s.z;
-      dx = dx < 0 ? -dx : dx;
-      dx = dx < lx - dx ? dx : lx - dx;
-      dy = dy < 0 ? -dy : dy;
-      dy = dy < ly - dy ? dy : ly - dy;
-      if (dx * dx + dy * dy + dz * dz == 72) {
-        coornn = 2;
-        nnn.x[1] = s.x; nnn.y[1] = s.y; nnn.z[1] = s.z;
-        int a1[3] = {nnn.x[0], nnn.y[0], nnn.z[0]}, a2[3] = {s.x, s.y, s.z}, pc[3] = {p.x, p.y, p.z}, ns[2][3];
-        find_nn(g, lx, ly, a1, a2, pc, ns);
-        P3 qq[2];
-        Site sq[2];
-        for (int j = 2; j < 4; j++) {
-          nnn.x[j] = ns[j - 2][0]; nnn.y[j] = ns[j - 2][1]; nnn.z[j] = ns[j - 2][2];
-          qq[j - 2] = entry(L, nnn, j);
-        }
-        sq[0] = rd(L, qq[0].i);
-        sq[1] = rd(L, qq[1].i);
-        for (int j = 0; j < 2; j++) {
-          int kq = s_kind(sq[j]);
-          if (kind_occupied(kq) && s_coor(sq[j]) <= 3 && kq != KIND_WALL) {
-            if (lists_point(L.box, qq[j], sq[j], p)) coornn++;
-          }
-        }
-        s_set_coor(sp, coornn);
-        if (!set_list(L.box, sp, p.x, p.y, p.z, nnn)) { err = ERR_GEOM; return; }
-        wr(L, p.i, sp);
-        need = true;
-      }
-    } else if (coornn == 2 || coornn == 3) {
-      if (recip(nnn, s)) {
-        coornn++;
-        s_set_coor(sp, coornn);
-        wr(L, p.i, sp);
-        need = true;
-      }
-    }
-  } else if (kind != KIND_WALL) {
-    if (coornn <= 3 && recip(nnn, s)) {
-      coornn++;
-      s_set_coor(sp, coornn);
-      wr(L, p.i, sp);
-      need = true;
-      if (sc.coor_old == 1 && i >= 1) sc.inc[i] = 1;
-    }
-  } else {
-    sc.inc[i] = 1;  // wall neighbour
-  }
-  q.need = need;
-  q.list_after = list_after;
-  q.p = p;
-  q.sp = sp;
-  q.coor = coornn;
-  q.nn = nnn;
-}
-
-// The neighbours lane `lane` visits: neighbour `lane` (lanes 0..n-1), or all
-// n in order on lane 0 when two list entries are the same point.
-__device__ inline void visit_range(const EvScratch &sc, int lane, int n, int &i0, int &i1) {
-  i0 = lane;
-  i1 = lane < n ? lane + 1 : 0;
-  if (sc.seq) {
-    i0 = 0;
-    i1 = lane == 0 ? n : 0;
-  }
-}
-
-// Deposition, mcevent/deposition.f:24-74: the site takes the species and,
-// at coordination 1, its stacking (FIND_SN + IF_Arm_Choice).  Lane 0.
-__device__ void dep_site(const Lattice &L, const P3 &s, int species, const Choice &ch, EvResult &res,
-                         EvScratch &sc) {
-  const Geometry &g = *L.geo;
-  Site ss = rd(L, s.i);
-  int coor = s_coor(ss);
-  sc.coor_old = coor;
-  s_set_kind(ss, species);
-  wr(L, s.i, ss);
-  res.arm = -1;
-  NL nn_site = list_of(L, s, ss);
-  if (coor == 1) {
-    P3 c = entry(L, nn_site, 0);
-    Site scr = rd(L, c.i);
-    NL lc = list_of(L, c, scr);
-    int sn[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, j = 0;
-    for (int i = 0; i < 4; i++)
-      if (!same(lc, i, s)) {
-        if (j < 3) { sn[j][0] = lc.x[i]; sn[j][1] = lc.y[i]; sn[j][2] = lc.z[i]; }
-        j++;
-      }
-    int site[3] = {s.x, s.y, s.z}, cc[3] = {c.x, c.y, c.z}, zig[3][3], arm[3][3];
-    find_sn(g, L.box.lx, L.box.ly, site, cc, sn, zig, arm);
-    Site sa[3], sz[3];
-    for (int k = 0; k < 3; k++) {
-      sa[k] = rd(L, at(L, arm[k][0], arm[k][1], arm[k][2]).i);
-      sz[k] = rd(L, at(L, zig[k][0], zig[k][1], zig[k][2]).i);
-    }
-    int carm = 0, czig = 0;  // IF_Arm_Choice.f:35-54
-    for (int k = 0; k < 3; k++) {
-      carm += s_coor(sa[k]);
-      czig += s_coor(sz[k]);
-    }
-    int is_arm;
-    if (ch.arm >= 0) is_arm = ch.arm;
-    else if (czig > carm) is_arm = 0;
-    else if (czig == carm) is_arm = (ch.u_arm <= L.tab->ptrans_zig) ? 0 : 1;
-    else is_arm = 1;
-    res.arm = is_arm;
-    for (int k = 0; k < 3; k++) {
-      nn_site.x[k + 1] = is_arm ? arm[k][0] : zig[k][0];
-      nn_site.y[k + 1] = is_arm ? arm[k][1] : zig[k][1];
-      nn_site.z[k + 1] = is_arm ? arm[k][2] : zig[k][2];
-    }
-    if (!set_list(L.box, ss, s.x, s.y, s.z, nn_site)) sc.abort = ERR_GEOM;
-    else wr(L, s.i, ss);
-  }
-  sc.nn = nn_site;
-  resolve_neighbours(L, sc, 4);
-  touched_list(s, sc, 4);
-}
-
-// The scan of Evaporation.f:82-128 / 225-259 that unfixes a list when a site
-// drops to coordination 1: the last occupied reciprocal neighbour (NBuff).
-__device__ bool nbuff_of(const Lattice &L, const P3 &p, const NL &old, int pos[3]) {
-  P3 q[4];
-  Site sq[4];
-  prefetch4(L, old, q, sq);
-  bool f = false;
-  for (int j = 0; j < 4; j++) {
-    int kq = s_kind(sq[j]);
-    if (kind_occupied(kq) && s_coor(sq[j]) <= 3 && kq != KIND_WALL) {
-      if (lists_point(L.box, q[j], sq[j], p)) {
-        pos[0] = old.x[j]; pos[1] = old.y[j]; pos[2] = old.z[j];
-        f = true;
-      }
-    }
-  }
-  return f;
-}
-__device__ inline bool one_entry_list(const Lattice &L, Site &sp, const P3 &p, const int pos[3]) {
-  NL nl;
-  for (int j = 0; j < 4; j++) nl.x[j] = nl.y[j] = nl.z[j] = 0;
-  nl.x[0] = pos[0]; nl.y[0] = pos[1]; nl.z[0] = pos[2];
-  return set_list(L.box, sp, p.x, p.y, p.z, nl);
-}
-
-// Evaporation.f:36-208, the update of neighbour i of the atom leaving s.
-// NBuff is resolved afterwards (evap_nbuff_one) because the reference
-// carries it from one neighbour to the next.  A neighbour that keeps a rate
-// drops one coordination and asks for one rate evaluation.
-__device__ void evap_prepare(const Lattice &L, const P3 &s, int i, EvScratch &sc, int &err, RefreshReq &q) {
-  const P3 p = sc.pts[i];
-  Site sp = rd(L, p.i);
-  const int kind = s_kind(sp), coornn = s_coor(sp);
-  const NL nnn = list_of(L, p, sp);
-  if (kind == KIND_WALL) {
-    sc.inc[i] = -1;  // wall neighbour
-    return;
-  }
-  const bool occ = kind_occupied(kind);
-  if (!(occ || (coornn >= 1 && coornn <= 4)) || !recip(nnn, s)) return;
-  if (!occ && coornn == 1) {  // EraseMC + LattCoo=0, keeping the temperature bits
-    Site z = rd(L, -1);
-    z.temp = sp.temp;
-    wr(L, p.i, z);
-    set_rate(L, p, CLS_NONE, 0.0);
-    note_rate(sc, 1 + i, CLS_NONE, 0.0);
-    return;
-  }
-  if (!occ && coornn == 2) {  // unfixed: the list keeps the reciprocal partner (NBuff)
-    int pos[3] = {0, 0, 0};
-    sc.unfixed[i] = 1;
-    sc.found[i] = nbuff_of(L, p, nnn, pos) ? 1 : 0;
-    for (int k = 0; k < 3; k++) sc.found_pos[i][k] = pos[k];
-    if (!one_entry_list(L, sp, p, pos)) { err = ERR_GEOM; return; }
-  }
-  // coordination 4 -> 3 is EraseBulk/EraseVoid + AddMC; the rate of an
-  // unfixed site comes from its old list copy (Evaporation.f:121)
-  s_set_coor(sp, coornn - 1);
-  wr(L, p.i, sp);
-  q.need = true;
-  q.p = p;
-  q.sp = sp;
-  q.coor = coornn - 1;
-  q.nn = nnn;
-}
-
-// The NBuff the reference carries across the neighbours: a neighbour that
-// found no reciprocal partner gets the last one found before it (or the
-// initial (0,0,0)).  Applied neighbour by neighbour, in order; `carried`
-// is the value carried out of the loop into the site's own unfix.
-__device__ void evap_nbuff_one(const Lattice &L, EvScratch &sc, int i, int carried[3], int &err) {
-  if (!sc.unfixed[i]) return;
-  if (sc.found[i]) {
-    for (int k = 0; k < 3; k++) carried[k] = sc.found_pos[i][k];
-  } else if (carried[0] || carried[1] || carried[2]) {
-    const P3 p = sc.pts[i];
-    Site sp = rd(L, p.i);
-    if (!one_entry_list(L, sp, p, carried)) { err = ERR_GEOM; return; }
-    wr(L, p.i, sp);
-  }
-}
-
-// Evaporation, mcevent/Evaporation.f:25-35: the site empties.  Lane 0.
-__device__ inline void evap_site(const Lattice &L, const P3 &s, EvScratch &sc) {
-  Site ss = rd(L, s.i);
-  sc.coor_old = s_coor(ss);
-  sc.old_kind = s_kind(ss);
-  s_set_kind(ss, KIND_EMPTY);
-  wr(L, s.i, ss);
-  sc.nn = list_of(L, s, ss);
-  resolve_neighbours(L, sc, 4);
-  touched_list(s, sc, 4);
-}
-
-// absorption.f:25-78 / desorption.f:25-117: the site takes (absorption,
-// slot = ListCov index 1..3) or loses (slot 0) its coverage species; at
-// coordination 1 desorption visits only the first neighbour.  Lane 0.
-__device__ inline void cov_site(const Lattice &L, const P3 &s, int slot, EvScratch &sc) {
-  Site ss = rd(L, s.i);
-  sc.coor_old = s_coor(ss);
-  sc.old_kind = s_kind(ss);
-  s_set_kind(ss, slot ? KIND_COV0 + slot - 1 : KIND_EMPTY);
-  wr(L, s.i, ss);
-  sc.nn = list_of(L, s, ss);
-  sc.nvisit = (!slot && sc.coor_old == 1) ? 1 : 4;
-  resolve_neighbours(L, sc, sc.nvisit);
-  touched_list(s, sc, sc.nvisit);
-}
-
-// Their neighbour i: an atom bonded back to s gets a fresh rate
-// (absorption only for coordination <= 3, absorption.f:45-60;
-// desorption.f:45-105).
-__device__ inline void cov_prepare(const Lattice &L, const P3 &s, int i, bool absorb, EvScratch &sc, RefreshReq &q) {
-  const P3 p = sc.pts[i];
-  const Site sp = rd(L, p.i);
-  const int k = s_kind(sp);
-  if (!kind_occupied(k) || k == KIND_WALL || (absorb && s_coor(sp) > 3)) return;
-  const NL nnn = list_of(L, p, sp);
-  if (!recip(nnn, s)) return;
-  q.need = true;
-  q.p = p;
-  q.sp = sp;
-  q.coor = s_coor(sp);
-  q.nn = nnn;
-}
-
-// The reference event an MC particle of class `cls` executes.  For an
-// adsorption site this draws the species / coverage as Get_Prob.f:160-176
-// and IndexEvent_Abs (Get_Prob.f:22-52) do, with the draw taken at
-// execution instead of at rate-update time (same distribution: the class
-// is refreshed whenever the coordination changes).  Returns itrans in the
-// reference's numbering (1..3 deposit, 4 evaporate, 5 desorb, 6.. absorb).
-template <bool LA = true, bool COV = true>
-MSKG_HD int pick_itrans(const Lattice &L, const P3 &s, int cls, double u) {
-  const Tables &t = *L.tab;
+// The reference event an MC particle of class `cls`, whose record is ss,
+// executes.  For an adsorption site this draws the species / coverage as
+// Get_Prob.f:160-176 and IndexEvent_Abs (Get_Prob.f:22-52) do, with the draw
+// taken at execution instead of at rate-update time (same distribution: the
+// class is refreshed whenever the coordination changes).  Returns itrans in
+// the reference's numbering (1..3 deposit, 4 evaporate, 5 desorb, 6.. absorb).
+template <bool LA, bool COV, class Src>
+MSKG_HD int pick_itrans(const Lattice &L, const Src &S, int coor, int temp, int cls, double u) {
+  const Tables &t = S.t;
   if (cls == CLS_PLACEHOLDER) return 1;
   if (cls == CLS_EVAP || cls == CLS_ISOLATED) return 4;
   if (cls == CLS_DESORB) return 5;
-  Site ss = rd(L, s.i);
-  int coor = s_coor(ss);
-  int temperature = (LA && t.la_mode) ? (int)ss.temp : 0;
+  int temperature = (LA && t.la_mode) ? temp : 0;
   STW w;
   // InitSt 'ST': the tables at the site's temperature (its rate was evaluated
   // with them, so the temperature lies inside the references)
-  const bool st = LA && t.st_n > 0 && st_weights(t, (int)ss.temp, w);
-  auto pabs_of = [&](int i) { return st ? st_entry(t.st_pabs, 12, i + 3 * coor, w) : t.pabs[i + 3 * coor]; };
+  const bool st = LA && t.st_n > 0 && st_weights(t, temp, w);
+  auto pabs_of = [&](int i) { return st ? st_entry(t.st_pabs, 12, i + 3 * coor, w) : S.pabs(i + 3 * coor); };
   double p1, p2, p3;
   if (st) {
     p1 = st_entry(t.st_pd, 9, 3 * (coor - 1), w);
     p2 = st_entry(t.st_pd, 9, 1 + 3 * (coor - 1), w);
     p3 = st_entry(t.st_pd, 9, 2 + 3 * (coor - 1), w);
   } else {
-    p1 = pd_of<LA>(t, 1, coor, temperature, L.cl);
-    p2 = pd_of<LA>(t, 2, coor, temperature, L.cl);
-    p3 = pd_of<LA>(t, 3, coor, temperature, L.cl);
+    p1 = pd_of<LA>(S, 1, coor, temperature, L.cl);
+    p2 = pd_of<LA>(S, 2, coor, temperature, L.cl);
+    p3 = pd_of<LA>(S, 3, coor, temperature, L.cl);
   }
   double pdep = p1 + p2 + p3;
   double pabs = COV ? pabs_of(0) + pabs_of(1) + pabs_of(2) : 0.0;
@@ -914,149 +487,538 @@ MSKG_HD int pick_itrans(const Lattice &L, const P3 &s, int cls, double u) {
   return r;
 }
 
-// Execute one event of type itrans at site s.  Called by every lane of the
-// wave with the same arguments; res is complete on lane 0.  Three phases:
-// lane 0 updates the site; lanes 0..3 update its neighbours (one rate
-// evaluation each); lane 0 gives the site its final rate while, with the
-// second-neighbour term, lanes 1..12 refresh the atoms of its second shell.
-// Each phase has one rate-evaluation call site for every event type, which
-// keeps the inlined kernel small.
-template <bool LA = true, bool COV = true>
-__device__ void execute(const Lattice &L, double rtot, const P3 &s, int itrans, const Choice &ch, EvResult &res,
-                        EvScratch &sc, int lane) {
-  res.err = ERR_NONE;
-  res.arm = -1;
-  res.species = 0;
+// ---- event execution -------------------------------------------------------
+// One 64-wide wave executes an event, every lane in step: sixteen quads of
+// four lanes, each quad one point the event looks at, each lane of a quad one
+// entry of that point's neighbour list.
+//   quads 0..3    the site's four listed neighbours
+//   quads 4..15   with the second-neighbour term, the site's second shell
+// The event is then three dependent gathers (the site's record, the sixteen
+// points' records, their 64 listed neighbours' records) whatever its type,
+// and one rate evaluation for all of the points and the site itself.
+//
+// What bounds it: a wave issues one instruction every four cycles or more and
+// waits for each gather, and the waves of a pass are few and uneven, so the
+// length of one wave's instruction stream is the time of an event.  With a
+// lane a point (each lane walking its point's four neighbours and twelve
+// second neighbours in turn, 13 lanes busy) an event was about 3400
+// instructions; counts are now sums over a quad by DPP, and nothing passes
+// through LDS.  Passes before and after: 8e6 events at 512^3 SiC 92 -> 47 ms,
+// 5e5 events of SiC on 480^3 132 -> 65 ms, 2e5 of CVD on 240x240x760
+// 252 -> 144 ms, k_serial on 64 lattices of 144^3 55.6 -> 26 ms.
+//
+// The reference visits the neighbours one after the other, but each
+// neighbour's update writes only that neighbour's record and reads only
+// records the other neighbour updates do not write (two neighbours of a
+// site are never neighbours of each other), so the concurrent updates give
+// the sequential result.  When two list entries resolve to the same point
+// the neighbours are visited in order, a round each.  The site's own record
+// is written last; lanes whose gather meets the site take it from registers.
+
+// A site record as it lies in memory (struct Site), in four words.
+typedef uint4 Rec;
+__device__ inline int r_kind(const Rec &r) { return r.w & 7; }
+__device__ inline int r_coor(const Rec &r) { return (r.w >> 3) & 7; }
+__device__ inline int r_temp(const Rec &r) { return r.w >> 16; }
+__device__ inline uint32_t w_kind(uint32_t w, int k) { return (w & ~7u) | (uint32_t)k; }
+__device__ inline uint32_t w_coor(uint32_t w, int c) { return (w & ~0x38u) | (((uint32_t)c & 7u) << 3); }
+__device__ inline Rec load_rec(const Lattice &L, int64_t i) { return *(const Rec *)(L.site + i); }
+__device__ inline void store_rec(const Lattice &L, int64_t i, const Rec &r) { *(Rec *)(L.site + i) = r; }
+// Entry j's displacement, its three bytes in one word, and whether it is one.
+__device__ inline uint32_t rec_disp(const Rec &r, int j) {
+  const uint32_t lo = j < 2 ? r.x : (j == 2 ? r.y : r.z), hi = j < 2 ? r.y : r.z;
+  return __builtin_amdgcn_alignbyte(hi, lo, (4 - j) & 3) & 0xffffffu;
+}
+__device__ inline bool rec_has(const Rec &r, int j) { return (r.w >> (8 + j)) & 1; }
+// The position of a displacement from p (the absolute point (0,0,0) when it is none).
+__device__ inline P3 disp_point(const Lattice &L, const P3 &p, uint32_t d, bool has) {
+  int x = p.x + (int)(int8_t)d, y = p.y + (int)(int8_t)(d >> 8);
+  const int z = p.z + (int)(int8_t)(d >> 16);
+  if (x >= L.box.lx) x -= L.box.lx;
+  if (x < 0) x += L.box.lx;
+  if (y >= L.box.ly) y -= L.box.ly;
+  if (y < 0) y += L.box.ly;
+  return at(L, has ? x : 0, has ? y : 0, has ? z : 0);
+}
+__device__ inline P3 rec_entry(const Lattice &L, const Rec &r, const P3 &p, int j) {
+  return disp_point(L, p, rec_disp(r, j), rec_has(r, j));
+}
+// set_list for one entry: position o as a displacement from p (the point
+// (0,0,0) is no displacement); ok: it fits the record.
+__device__ inline uint32_t pack_disp(const Box &b, const P3 &p, const P3 &o, bool &has, bool &ok) {
+  has = (o.x | o.y | o.z) != 0;
+  ok = true;
+  if (!has) return 0u;
+  int dx = o.x - p.x, dy = o.y - p.y, dz = o.z - p.z;
+  if (dx > b.lx / 2) dx -= b.lx;
+  if (dx < -b.lx / 2) dx += b.lx;
+  if (dy > b.ly / 2) dy -= b.ly;
+  if (dy < -b.ly / 2) dy += b.ly;
+  ok = (unsigned)(dx + 128) < 256u && (unsigned)(dy + 128) < 256u && (unsigned)(dz + 128) < 256u;
+  return (uint32_t)(dx & 255) | ((uint32_t)(dy & 255) << 8) | ((uint32_t)(dz & 255) << 16);
+}
+// lists_point on a record in registers.
+__device__ inline bool rec_lists(const Box &b, const P3 &q, const Rec &r, const P3 &p) {
+  int wx = p.x - q.x, wy = p.y - q.y;
+  const int wz = p.z - q.z;
+  if (wx > b.lx / 2) wx -= b.lx;
+  if (wx < -b.lx / 2) wx += b.lx;
+  if (wy > b.ly / 2) wy -= b.ly;
+  if (wy < -b.ly / 2) wy += b.ly;
+  const bool in8 = (unsigned)(wx + 128) < 256u && (unsigned)(wy + 128) < 256u && (unsigned)(wz + 128) < 256u;
+  const uint32_t w = (uint32_t)(wx & 255) | ((uint32_t)(wy & 255) << 8) | ((uint32_t)(wz & 255) << 16);
+  const uint32_t v = r.w >> 8;
+  bool hit = false;
+  for (int j = 0; j < 4; j++) hit |= ((v >> j) & 1) && rec_disp(r, j) == w;
+  const bool origin = (p.x | p.y | p.z) == 0;
+  return (hit && in8) || (origin && (v & 15u) != 15u);
+}
+
+// Get_Prob of point p by one thread, from its record: the sweep.  Few of a
+// sweep's points are MC particles, so what counts here is that the branch
+// holds few registers: the second shell is taken four points at a time.
+template <bool LA, bool COV>
+__device__ inline void get_prob(const Lattice &L, double rtot, const P3 &p, const Rec &r, int &cls, double &rate,
+                                int &err, int &key) {
+  const Tables &t = *L.tab;
+  const int kind = r_kind(r), coor = r_coor(r);
+  int c0 = 0;
+  uint32_t cnt = 0;
+  if (kind == KIND_EMPTY) {
+    if (coor == 1) {
+      const int64_t i0 = rec_entry(L, r, p, 0).i;
+      c0 = i0 < 0 ? 0 : (L.site[i0].kc >> 3) & 7;
+    }
+  } else if (kind_species(kind) && p.z >= t.frozen_below_z) {
+    P3 q[4];
+    Rec sq[4];
+    for (int i = 0; i < 4; i++) q[i] = rec_entry(L, r, p, i);
+    for (int i = 0; i < 4; i++) {  // four independent gathers in flight
+      sq[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (q[i].i >= 0) sq[i] = load_rec(L, q[i].i);
+    }
+    for (int i = 0; i < 4; i++) {
+      const int kq = r_kind(sq[i]);
+      const bool lists = kq != KIND_EMPTY && kq != KIND_WALL && rec_lists(L.box, q[i], sq[i], p);
+      if (COV && lists && kind_cov_slot(kq) > t.ncov) err = ERR_COVERAGE;
+      cnt += neighbour_count(kq, lists);
+    }
+    if (t.use_f2) {
+#pragma unroll 1
+      for (int g = 0; g < 3; g++)
+        for (int k = 0; k < 4; k++) {
+          int dx, dy, dz;
+          second_vec(4 * g + k, dx, dy, dz);
+          const int64_t i2 = shifted(L, p, dx, dy, dz).i;
+          const int kq = i2 < 0 ? 0 : L.site[i2].kc & 7;
+          cnt += kind_species(kq) ? 1u << 28 : 0u;
+        }
+    }
+    if (COV && err) { cls = CLS_NONE; rate = 0.0; key = -1; return; }
+  }
+  rate_of<LA, COV>(TabSrc{t}, L.cl, rtot, p.z, kind, r_temp(r), coor, c0, cnt, cls, rate, err, key);
+}
+
+// A value of lane J of the quad; sums and ORs over the quad.  Every lane of
+// the wave must be active.
+template <int J>
+__device__ inline int quad_take(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, J * 0x55, 0xf, 0xf, false);
+}
+__device__ inline uint32_t quad_sum(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false);  // lanes 1 0 3 2
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false);  // lanes 2 3 0 1
+  return v;
+}
+__device__ inline uint32_t quad_or(uint32_t v) {
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false);
+  return v;
+}
+// The record of a quad's four entries (e, has: this lane's).
+__device__ inline void quad_list(Rec &r, uint32_t e, bool has, int j) {
+  const uint32_t e0 = quad_take<0>((int)e), e1 = quad_take<1>((int)e), e2 = quad_take<2>((int)e),
+                 e3 = quad_take<3>((int)e);
+  r.x = e0 | (e1 << 24);
+  r.y = (e1 >> 8) | (e2 << 16);
+  r.z = (e2 >> 16) | (e3 << 8);
+  r.w = (r.w & ~0xff00u) | (quad_or(has ? 1u << j : 0u) << 8);
+}
+__device__ inline Rec uniform_rec(const Rec &r) {
+  return make_uint4((uint32_t)__builtin_amdgcn_readfirstlane((int)r.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)r.y),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)r.z), (uint32_t)__builtin_amdgcn_readfirstlane((int)r.w));
+}
+
+// What an event leaves in the wave's registers: the points whose rate may
+// have changed, on lane 0 the site, on lane 4 i + 1 neighbour i, on lane
+// 17 + 4 k second-shell point k -- in lane order, the order the lists take
+// new particles in.
+struct EvOut {
+  P3 p;        // this lane's point
+  float rate;  // its new rate and class as stored, when set is 1
+  int cls;
+  int set;     // 0: no point here, or one that got no new rate; 2: read both from memory
+               // (a list with repeated entries, whose points take several rates in turn)
+  // the same in every lane
+  int arm;      // stacking choice made (-1 none)
+  int err;
+  int species;  // deposited or evaporated species (1..3), desorbed coverage slot (1..3), 0 otherwise
+};
+
+// The stacking of a deposition at coordination 1 (deposition.f:40-74,
+// FIND_SN + IF_Arm_Choice): lanes 0..2 the arm-chair and lanes 4..6 the
+// zig-zag candidates; S takes the chosen list.
+__device__ inline void ev_stacking(const Lattice &L, const P3 &s, Rec &S, const Choice &ch, EvOut &o, int lane) {
+  const int j = lane & 3;
+  const P3 c = rec_entry(L, S, s, 0);
+  Rec cr = make_uint4(0u, 0u, 0u, 0u);
+  if (c.i >= 0) cr = load_rec(L, c.i);
+  // the back bonds' ends: the first three entries of c's list that are not s
+  const P3 le = rec_entry(L, cr, c, j);
+  const unsigned m0 = (unsigned)__ballot(!(le.x == s.x && le.y == s.y && le.z == s.z)) & 15u;
+  const unsigned m1 = m0 & (m0 - 1u), m2 = m1 & (m1 - 1u);
+  const int src = __ffs((int)(j == 0 ? m0 : (j == 1 ? m1 : m2))) - 1;
+  int sn[3] = {__shfl(le.x, src & 3, 64), __shfl(le.y, src & 3, 64), __shfl(le.z, src & 3, 64)};
+  if (src < 0) sn[0] = sn[1] = sn[2] = 0;
+  const int site[3] = {s.x, s.y, s.z}, cc[3] = {c.x, c.y, c.z};
+  int cand[3];
+  find_sn_one(*L.geo, L.box.lx, L.box.ly, site, cc, sn, (lane & 4) != 0, cand);
+  const P3 cp = at(L, cand[0], cand[1], cand[2]);
+  int cco = 0;
+  if (lane < 8 && j < 3 && cp.i >= 0) cco = r_coor(load_rec(L, cp.i));
+  const int csum = (int)quad_sum((uint32_t)cco);
+  const int carm = __builtin_amdgcn_readlane(csum, 0), czig = __builtin_amdgcn_readlane(csum, 4);
+  int is_arm = 1;  // IF_Arm_Choice.f:35-54
+  if (ch.arm >= 0) is_arm = ch.arm;
+  else if (czig > carm) is_arm = 0;
+  else if (czig == carm) is_arm = (ch.u_arm <= L.tab->ptrans_zig) ? 0 : 1;
+  is_arm = __builtin_amdgcn_readfirstlane(is_arm);
+  o.arm = is_arm;
+  const int from = (is_arm ? 0 : 4) + (j > 0 ? j - 1 : 0);
+  P3 e;
+  e.x = __shfl(cand[0], from, 64);
+  e.y = __shfl(cand[1], from, 64);
+  e.z = __shfl(cand[2], from, 64);
+  if (j == 0) { e.x = c.x; e.y = c.y; e.z = c.z; }
+  bool has, ok;
+  const uint32_t d = pack_disp(L.box, s, e, has, ok);
+  if (__ballot(!ok)) o.err = ERR_GEOM;
+  quad_list(S, d, has, j);
+  S = uniform_rec(S);
+}
+
+// Execute one event of type itrans at site s, whose record is S.  Called by
+// every lane of the wave with the same arguments.
+template <bool LA, bool COV>
+__device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot, const P3 &s, Rec S, int itrans,
+                               const Choice &ch, EvOut &o, const int lane) {
+  const TabEv<COV> T{*L.tab, tabs};
+  const Tables &t = T.t;
+  const int grp = lane >> 2, j = lane & 3;
+  o.p = s;
+  o.rate = 0.0f;
+  o.cls = CLS_NONE;
+  o.set = 0;
+  o.arm = -1;
+  o.err = ERR_NONE;
+  o.species = 0;
   if (s.z > L.ztop) {  // before anything changes: the run stops with the state as it was
-    res.err = ERR_TOP;
+    o.err = ERR_TOP;
+    return;
+  }
+  if (!COV && itrans > 4) {
+    o.err = ERR_COVERAGE;
     return;
   }
   const bool dep = itrans <= 3, evap = itrans == 4, absorb = itrans >= 6;
-  if (lane < 12) {
-    sc.sec[lane].i = -1;
-    sc.err2[lane] = 0;
+  const int old_kind = r_kind(S), coor_old = r_coor(S);
+  // the site: deposition.f:24-74, Evaporation.f:25-35, absorption.f:25-78 and
+  // desorption.f:25-117 (at coordination 1 desorption visits only the first neighbour)
+  const int new_kind = dep ? itrans : (evap || itrans == 5 ? KIND_EMPTY : KIND_COV0 + itrans - 6);
+  S.w = w_kind(S.w, new_kind);
+  o.species = dep ? itrans : (evap && kind_species(old_kind) ? old_kind : 0);
+  if (COV && itrans == 5) o.species = kind_cov_slot(old_kind);  // the coverage desorbed
+  if (dep && coor_old == 1) {
+    ev_stacking(L, s, S, ch, o, lane);
+    if (o.err) return;
   }
-  if (lane == 0) {
-    sc.ntouched = 0;
-    sc.abort = 0;
-    sc.nvisit = 4;
-    if (dep) dep_site(L, s, itrans, ch, res, sc);
-    else if (evap) evap_site(L, s, sc);
-    else if (COV) cov_site(L, s, absorb ? itrans - 5 : 0, sc);
-    res.species = dep ? itrans : (evap && kind_species(sc.old_kind) ? sc.old_kind : 0);
-    if (COV && itrans == 5) res.species = kind_cov_slot(sc.old_kind);  // the coverage desorbed
-  }
-  MSKG_SYNC();
-  if (sc.abort) {
-    if (lane == 0) res.err = sc.abort;
-    return;
-  }
-  // phase 2: the neighbours
-  int nbuff[3] = {0, 0, 0};  // Evaporation.f's NBuff, carried on lane 0
+  const int nvisit = COV && itrans == 5 && coor_old == 1 ? 1 : 4;
+  // the quads' points
+  P3 p;
   {
-    int i0, i1;
-    visit_range(sc, lane, sc.nvisit, i0, i1);
+    const uint32_t e = rec_disp(S, grp & 3);
+    int dx = (int)(int8_t)e, dy = (int)(int8_t)(e >> 8), dz = (int)(int8_t)(e >> 16);
+    bool has = rec_has(S, grp & 3);
+    if (grp >= 4) {
+      second_vec(grp - 4, dx, dy, dz);
+      has = true;
+    }
+    int x = s.x + dx, y = s.y + dy;
+    const int z = s.z + dz;
+    if (x >= L.box.lx) x -= L.box.lx;
+    if (x < 0) x += L.box.lx;
+    if (y >= L.box.ly) y -= L.box.ly;
+    if (y < 0) y += L.box.ly;
+    p = at(L, has ? x : 0, has ? y : 0, has ? z : 0);
+  }
+  // repeated list entries (compared by displacement; the origin is one entry however it is listed)
+  bool seq = false;
+  {
+    const bool org = (p.x | p.y | p.z) == 0;
+    const int kd = p.i < 0 ? -1 - grp : (org ? 1 << 24 : (int)rec_disp(S, grp & 3));
+    int kk[4];
+    for (int i = 0; i < 4; i++) kk[i] = __builtin_amdgcn_readlane(kd, 4 * i);
+    for (int i = 0; i < 4; i++)
+      for (int q = i + 1; q < 4; q++) seq |= q < nvisit && kk[i] == kk[q];
+  }
+  const bool shell = t.use_f2 && (dep || evap);
+  // The rounds: all quads at once; with repeated entries a round for each
+  // neighbour and a last one for the second shell; with coverage species and
+  // a second shell the neighbours first, since a covered neighbour's new list
+  // counts for the shell.  Each round reads what the one before wrote.
+  const int lead = seq ? nvisit : (COV && shell ? 1 : 0);  // rounds before the last
+  int coor = coor_old;
+  P3 nbuff;  // Evaporation.f's NBuff, carried over the neighbours
+  nbuff.x = nbuff.y = nbuff.z = 0;
+  nbuff.i = 0;
 #pragma unroll 1
-    for (int i = i0; i < i1; i++) {
-      RefreshReq q;
-      q.need = q.list_after = false;
-      if (dep) dep_prepare(L, s, i, sc, sc.err[i], q);
-      else if (evap) evap_prepare(L, s, i, sc, sc.err[i], q);
-      else if (COV) cov_prepare(L, s, i, absorb, sc, q);
-      if (q.need) {
-        int cls = 0, key = -1;
-        double r = 0.0;
-        // the site's coordination is final only in phase 3: here it is still coor_old
-        get_prob<LA, COV, true>(L, rtot, q.p, q.sp, q.coor, q.nn, cls, r, sc.err[i], nullptr, &key, s.i,
-                                sc.coor_old);
-        bool ok = true;
-        if (q.list_after) {
-          if (cls && !set_list(L.box, q.sp, q.p.x, q.p.y, q.p.z, q.nn)) {
-            sc.err[i] = ERR_GEOM;
-            ok = false;
-          } else {
-            wr(L, q.p.i, q.sp);
+  for (int round = 0; round <= lead; round++) {
+    const bool last = round == lead;
+    const unsigned nbm = (1u << nvisit) - 1u;
+    const unsigned M = (seq ? (last ? 0u : 1u << round) : (round == 0 ? nbm : 0u)) | (last && shell ? 0xfff0u : 0u);
+    const bool act = (M >> grp) & 1u;
+    const bool nb = act && grp < 4;
+    Rec r = make_uint4(0u, 0u, 0u, 0u);
+    if ((act || (last && lead && grp < 4)) && p.i >= 0) r = load_rec(L, p.i);
+    const int kind = r_kind(r), coornn = r_coor(r);
+    const bool wall = kind == KIND_WALL, atom = kind_species(kind), empty = !atom && !wall;  // empty or covered
+    // this lane's entry of its point's list
+    P3 q = rec_entry(L, r, p, j);
+    const bool back = quad_or(q.x == s.x && q.y == s.y && q.z == s.z ? 1u : 0u) != 0u;  // the list holds the site
+    // what happens to the point
+    bool need = act && grp >= 4 && atom && coornn >= 1 && coornn <= 3;  // a second-shell atom: a fresh rate
+    bool first = false, second = false, erase = false, unfix = false;
+    int inc = 0, cn = coornn;
+    if (dep) {  // deposition.f:78-235
+      first = nb && empty && coornn == 0;
+      if (nb && wall) inc = 1;
+      if (nb && ((atom && coornn <= 3 && back) || (empty && (coornn == 2 || coornn == 3) && back))) {
+        cn = coornn + 1;
+        need = true;
+        if (atom && coor_old == 1 && grp >= 1) inc = 1;
+      }
+      if (__ballot(nb && empty && coornn == 1)) {
+        // a second fixed neighbour: the two others follow when the first is
+        // a second neighbour of the site (FIND_NN.f, a lane each)
+        const int ax = quad_take<0>(q.x), ay = quad_take<0>(q.y), az = quad_take<0>(q.z);
+        int dx = ax - s.x, dy = ay - s.y;
+        const int dz = az - s.z;
+        dx = dx < 0 ? -dx : dx;
+        dx = dx < L.box.lx - dx ? dx : L.box.lx - dx;
+        dy = dy < 0 ? -dy : dy;
+        dy = dy < L.box.ly - dy ? dy : L.box.ly - dy;
+        second = nb && empty && coornn == 1 && dx * dx + dy * dy + dz * dz == 72;
+        if (second) {
+          if (j == 1) q = s;
+          if (j >= 2) {
+            const int a1[3] = {ax, ay, az}, a2[3] = {s.x, s.y, s.z}, pc[3] = {p.x, p.y, p.z};
+            int ns[3];
+            find_nn_one(*L.geo, L.box.lx, L.box.ly, a1, a2, pc, j - 2, ns);
+            q = at(L, ns[0], ns[1], ns[2]);
           }
         }
-        if (ok) {
-          set_rate(L, q.p, cls, r, key);
-          note_rate(sc, 1 + i, cls, r);
+      }
+      if (first) {  // its list starts with the site
+        q = s;
+        if (j > 0) { q.x = q.y = q.z = 0; q.i = 0; }
+        cn = 1;
+        need = true;
+      }
+      if (second) {
+        cn = 2;
+        need = true;
+      }
+    } else if (evap) {  // Evaporation.f:36-208
+      if (nb && wall) inc = -1;
+      if (nb && !wall && (atom || coornn >= 1) && coornn <= (atom ? 7 : 4) && back) {
+        if (empty && coornn == 1) {
+          erase = true;  // EraseMC + LattCoo=0, keeping the temperature bits
+        } else {
+          unfix = empty && coornn == 2;  // the list keeps the reciprocal partner (NBuff)
+          cn = coornn - 1;  // coordination 4 -> 3 is EraseBulk/EraseVoid + AddMC
+          need = true;
         }
       }
-      if (evap && sc.seq) evap_nbuff_one(L, sc, i, nbuff, sc.err[i]);  // in order, as each neighbour is visited
+    } else if (COV) {  // an atom bonded back to the site (absorption.f:45-60, desorption.f:45-105)
+      need |= nb && atom && (!absorb || coornn <= 3) && back;
     }
-  }
-  MSKG_SYNC();
-  // phase 3: the site's final rate and the second shell
-  FinalRefresh f;
-  f.active = false;
-  Site ss;
-  bool unfix = false;
-  if (lane == 0) {
-    if (sc.seq)  // a point listed twice took several rates in turn
-      for (int q = 1; q < sc.ntouched; q++) sc.tset[q] = 2;
-    int coor = sc.coor_old;
-    for (int i = 0; i < 4; i++) {
-      if (dep || evap) coor += sc.inc[i];
-      if (sc.err[i]) res.err = sc.err[i];
+    // the listed neighbours' records (the rate of an unfixed point comes from
+    // its old list, Evaporation.f:121)
+    const bool count = need && atom && p.z >= t.frozen_below_z;
+    const bool look = count || unfix || (second && j >= 2) || (need && empty && cn == 1 && j == 0);
+    Rec er = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t k2 = 0;
+    if (look && q.i == s.i) er = S;
+    else if (look && q.i >= 0) er = load_rec(L, q.i);
+    if (t.use_f2 && count) {
+      // four second neighbours a lane in three steps; at least 6 units from
+      // every face they are at fixed index steps
+      const int a = (j & 2) ? -6 : 6, b = (j & 1) ? -6 : 6;
+      const Box &B = L.box;
+      int64_t i2[3];
+      if (p.x >= 6 && p.x < B.lx - 6 && p.y >= 6 && p.y < B.ly - 6 && p.z >= 6 && p.z <= B.lz - 6) {
+        i2[0] = p.i + (a / 2 + (b / 2) * B.hx);
+        i2[1] = p.i + (b * B.plane + a / 2);
+        i2[2] = p.i + (b * B.plane + (a / 2) * B.hx);
+      } else {
+        i2[0] = shifted(L, p, a, b, 0).i;
+        i2[1] = shifted(L, p, a, 0, b).i;
+        i2[2] = shifted(L, p, 0, a, b).i;
+      }
+      for (int k = 0; k < 3; k++) {
+        int kq = i2[k] < 0 ? 0 : L.site[i2[k]].kc & 7;
+        if (i2[k] == s.i) kq = new_kind;
+        k2 += kind_species(kq) ? 1u << 28 : 0u;
+      }
     }
-    if (evap && !sc.seq)
-      for (int i = 0; i < 4; i++) evap_nbuff_one(L, sc, i, nbuff, res.err);
-    ss = rd(L, s.i);
-    if (coor != sc.coor_old) s_set_coor(ss, coor);
-    if (evap && coor == 0) {  // EraseMC zeroes the record
-      for (int a = 0; a < 4; a++) ss.d[a][0] = ss.d[a][1] = ss.d[a][2] = 0;
-      ss.valid = 0;
-      wr(L, s.i, ss);
-      set_rate(L, s, CLS_NONE, 0.0);
-      note_rate(sc, 0, CLS_NONE, 0.0);
-    } else {
-      if (coor != sc.coor_old || evap) wr(L, s.i, ss);
-      f.active = true;
-      f.p = s;
-      f.sp = ss;
-      f.coor = coor;
-      f.nn = sc.nn;
-      unfix = evap && coor == 1;  // the site keeps one reciprocal bond (NBuff)
-    }
-  } else if (lane <= 12 && L.tab->use_f2 && (dep || evap)) {
-    second_setup(L, s, lane - 1, sc, f);
-  }
-  int cls = 0, key = -1, e = ERR_NONE;
-  double r = 0.0;
-  if (f.active) get_prob<LA, COV, true>(L, rtot, f.p, f.sp, f.coor, f.nn, cls, r, e, nullptr, &key);
-  if (unfix) {
-    int pos[3];
-    if (nbuff_of(L, s, sc.nn, pos))
-      for (int k = 0; k < 3; k++) nbuff[k] = pos[k];
-    if (!one_entry_list(L, ss, s, nbuff)) e = ERR_GEOM;
-    else wr(L, s.i, ss);
-  }
-  if (f.active) {
-    set_rate(L, f.p, cls, r, key);
-    if (lane == 0) {
-      note_rate(sc, 0, cls, r);
-    } else {
-      sc.secrate[lane - 1] = cls ? (float)r : 0.0f;
-      sc.seccls[lane - 1] = (uint8_t)cls;
-    }
-    if (e) {
-      if (lane == 0) res.err = e;
-      else sc.err2[lane - 1] = e;
-    }
-  }
-  if (L.tab->use_f2 && (dep || evap)) {
-    MSKG_SYNC();  // the second-shell refreshes are done
-    if (lane == 0)
-      for (int k = 0; k < 12; k++) {
-        if (sc.err2[k]) res.err = sc.err2[k];
-        if (sc.sec[k].i >= 0) {
-          sc.trate[sc.ntouched] = sc.secrate[k];
-          sc.tcls[sc.ntouched] = sc.seccls[k];
-          sc.tset[sc.ntouched] = 1;
-          sc.touched[sc.ntouched++] = sc.sec[k];
+    const int kq = r_kind(er);
+    const bool lists = look && kq != KIND_EMPTY && kq != KIND_WALL && rec_lists(L.box, q, er, p);
+    int err = ERR_NONE;
+    if (COV && count && lists && kind_cov_slot(kq) > t.ncov) err = ERR_COVERAGE;
+    if (COV && quad_or(err != ERR_NONE ? 1u : 0u)) err = ERR_COVERAGE;
+    uint32_t cnt = quad_sum((count ? neighbour_count(kq, lists) : 0u) + k2);
+    const bool partner = lists && kind_species(kq) && r_coor(er) <= 3;
+    const unsigned pm = quad_or(partner ? 1u << j : 0u);  // reciprocal partners by entry
+    const int c0 = quad_take<0>(r_coor(er));
+    if (second) cn += __popc(pm >> 2);
+    // the point's new record
+    Rec nr = r;
+    nr.w = w_coor(r.w, cn);
+    if (erase) nr = make_uint4(0u, 0u, 0u, r.w & 0xffff0000u);
+    if (__ballot(first || second)) {
+      bool has, ok;
+      Rec lr = nr;
+      const uint32_t d = pack_disp(L.box, p, q, has, ok);
+      const bool bad = quad_or(ok ? 0u : 1u) != 0u;
+      quad_list(lr, d, has, j);
+      if (first || second) {
+        if (bad) {
+          err = ERR_GEOM;
+          need = false;
+          nr = r;
+        } else {
+          nr = lr;
         }
       }
+    }
+    const unsigned um = (unsigned)((__ballot(unfix) >> 1) & 0x1111ull);  // unfixed neighbours, bit 4 i
+    if (um) {
+      const int jb = pm ? 31 - __clz((int)pm) : 0;  // the last partner
+      const P3 pp = rec_entry(L, r, p, jb);
+      if (unfix) {  // one entry; none for no partner, or a partner at the origin
+        const bool keep = pm && (pp.x | pp.y | pp.z) != 0;
+        nr.x = keep ? rec_disp(r, jb) : 0u;
+        nr.y = nr.z = 0u;
+        nr.w = (nr.w & ~0xff00u) | (keep ? 0x100u : 0u);
+      }
+      // NBuff over the neighbours in order: one that found no partner gets
+      // the last one found before it (or the initial (0,0,0): none)
+      for (int i = 0; i < 4; i++) {
+        if (!((um >> (4 * i)) & 1u)) continue;
+        if (__builtin_amdgcn_readlane((int)pm, 4 * i + 1)) {
+          nbuff.x = __builtin_amdgcn_readlane(pp.x, 4 * i + 1);
+          nbuff.y = __builtin_amdgcn_readlane(pp.y, 4 * i + 1);
+          nbuff.z = __builtin_amdgcn_readlane(pp.z, 4 * i + 1);
+        } else if (nbuff.x | nbuff.y | nbuff.z) {
+          bool has, ok;
+          const uint32_t d = pack_disp(L.box, p, nbuff, has, ok);
+          if (grp == i) {
+            if (!ok) err = ERR_GEOM;
+            else { nr.x = d; nr.w |= 0x100u; }
+          }
+        }
+      }
+    }
+    coor += __popcll(__ballot(inc > 0 && j == 1)) - __popcll(__ballot(inc < 0 && j == 1));
+    bool put = nb && (dep || evap) && (need || erase) && j == 1;  // this lane stores its point's record
+    bool set = (need || erase) && j == 1;
+    // what the rate evaluation below takes: the quad's point, or on lane 0
+    // the site with its final coordination and neighbours
+    int ek = kind, ecoor = cn, ec0 = c0, et = r_temp(r), ez = p.z;
+    bool eval = need;
+    int64_t wi = p.i;
+    if (last) {
+      const bool sn = lane < 16 && j == 1;  // a lane a neighbour
+      const int fk = r_kind(nr), fc = r_coor(nr);
+      const bool rem = evap && coor == 0;  // EraseMC zeroes the record
+      uint32_t scnt = 0;
+      if (dep || (evap && coor == 1)) {
+        const bool sl = sn && fk != KIND_EMPTY && fk != KIND_WALL && rec_lists(L.box, p, nr, s);
+        if (dep) {
+          const uint32_t c1 = sn ? neighbour_count(fk, sl) : 0u;
+          if (COV && __ballot(sl && kind_cov_slot(fk) > t.ncov)) { if (lane == 0) err = ERR_COVERAGE; }
+          scnt = (uint32_t)(__builtin_amdgcn_readlane((int)c1, 1) + __builtin_amdgcn_readlane((int)c1, 5) +
+                            __builtin_amdgcn_readlane((int)c1, 9) + __builtin_amdgcn_readlane((int)c1, 13));
+          if (t.use_f2) scnt += (uint32_t)__popcll(__ballot(lane >= 16 && j == 1 && atom)) << 28;
+        } else {  // the site keeps one reciprocal bond (NBuff)
+          const unsigned long long sp = __ballot(sl && kind_species(fk) && fc <= 3);
+          if (sp) {
+            const int l = 63 - __clzll((long long)sp);
+            nbuff.x = __builtin_amdgcn_readlane(p.x, l);
+            nbuff.y = __builtin_amdgcn_readlane(p.y, l);
+            nbuff.z = __builtin_amdgcn_readlane(p.z, l);
+          }
+        }
+      }
+      const uint32_t old_w = S.w;
+      S.w = w_coor(S.w, coor);
+      if (rem) S = make_uint4(0u, 0u, 0u, S.w & 0xffff0000u);
+      const int sc0 = __builtin_amdgcn_readlane(fc, 1);
+      if (lane == 0) {
+        ek = new_kind;
+        ecoor = coor;
+        ec0 = sc0;
+        cnt = scnt;
+        et = old_w >> 16;
+        ez = s.z;
+        eval = !rem && !err;
+        set = true;
+        put = true;
+        wi = s.i;
+      }
+      if (evap && coor == 1) {
+        bool has, ok;
+        const uint32_t d = pack_disp(L.box, s, nbuff, has, ok);
+        if (ok) S = make_uint4(d, 0u, 0u, (S.w & ~0xff00u) | (has ? 0x100u : 0u));
+        else if (lane == 0) err = ERR_GEOM;
+      }
+      if (lane == 0) nr = S;
+    }
+    int cls = CLS_NONE, key = -1;
+    double rate = 0.0;
+    if (eval && !err) rate_of<LA, COV>(T, L.cl, rtot, ez, ek, et, ecoor, ec0, cnt, cls, rate, err, key);
+    if (first && !cls && lane != 0) {  // AddMC stores the list with the rate only (lane 0 holds the site)
+      nr.x = r.x;
+      nr.y = r.y;
+      nr.z = r.z;
+      nr.w = (nr.w & ~0xff00u) | (r.w & 0xff00u);
+    }
+    if (put && wi >= 0) store_rec(L, wi, nr);
+    const unsigned long long em = __ballot(err != ERR_NONE);
+    if (em) o.err = __builtin_amdgcn_readlane(err, 63 - __clzll((long long)em));
+    if (set && wi >= 0) {
+      const float rf = cls ? (float)rate : 0.0f;
+      L.rate[wi] = rf;
+      L.cls[wi] = (uint8_t)cls;
+      if (L.key) L.key[wi] = cls ? key : -1;
+      const P3 sp = lane == 0 ? s : p;
+      if (cls) enlist(L, sp);
+      o.p = sp;
+      o.rate = rf;
+      o.cls = cls;
+      o.set = seq && lane != 0 && grp < 4 ? 2 : 1;
+    }
+    if (!last) __threadfence_block();  // the next round reads this one's records
   }
 }
 

@@ -102,6 +102,7 @@ struct Tables {
 struct Box {
   int lx, ly, lz, hx, hy;
   int64_t plane, npts;
+  double inv_plane, inv_hx;
 };
 
 MSKG_HD Box make_box(int lx, int ly, int lz) {
@@ -109,17 +110,29 @@ MSKG_HD Box make_box(int lx, int ly, int lz) {
   b.lx = lx; b.ly = ly; b.lz = lz; b.hx = lx / 2; b.hy = ly / 2;
   b.plane = (int64_t)b.hx * b.hy;
   b.npts = b.plane * (lz + 1);
+  b.inv_plane = 1.0 / (double)b.plane;
+  b.inv_hx = 1.0 / (double)b.hx;
   return b;
 }
 MSKG_HD bool valid_parity(int x, int y, int z) { return ((x ^ y) & 1) == 0 && ((x ^ z) & 1) == 0; }
 MSKG_HD int64_t pidx(const Box &b, int x, int y, int z) {
-  return ((int64_t)z * b.hy + (y >> 1)) * b.hx + (x >> 1);
+  // z * hy + y / 2 fits 32 bits (LenZ <= 8190, LenY < 2^20): one 32 x 32 -> 64 multiply
+  return (int64_t)((uint64_t)((uint32_t)z * (uint32_t)b.hy + (uint32_t)(y >> 1)) * (uint32_t)b.hx + (uint32_t)(x >> 1));
+}
+// a / d for 0 <= a < 2^51 by the FP64 reciprocal, which is off by at most one
+// (a 64-bit integer division is about a hundred instructions).
+MSKG_HD int64_t div_by(int64_t a, int64_t d, double inv) {
+  int64_t q = (int64_t)((double)a * inv);
+  const int64_t r = a - q * d;
+  if (r < 0) q--;
+  else if (r >= d) q++;
+  return q;
 }
 MSKG_HD void pxyz(const Box &b, int64_t p, int &x, int &y, int &z) {
-  z = (int)(p / b.plane);
-  int64_t r = p - (int64_t)z * b.plane;
-  int j = (int)(r / b.hx), i = (int)(r - (int64_t)j * b.hx);
-  int par = z & 1;
+  z = (int)div_by(p, b.plane, b.inv_plane);
+  const int64_t r = p - (int64_t)z * b.plane;
+  const int j = (int)div_by(r, b.hx, b.inv_hx), i = (int)(r - (int64_t)j * b.hx);
+  const int par = z & 1;
   x = 2 * i + par;
   y = 2 * j + par;
 }
@@ -177,11 +190,12 @@ MSKG_HD int isign_(int a, int b) { return b >= 0 ? (a < 0 ? -a : a) : (a < 0 ? a
 MSKG_HD int iabs_(int a) { return a < 0 ? -a : a; }
 MSKG_HD int nint_(double v) { return (int)round(v); }  // NINT: half away from zero
 
-// FIND_NN.f:25-77: the two remaining tetrahedral neighbours of SiteC given
-// Site1 and Site2, by rotating Site2-SiteC about unit(SiteC-Site1) by 120 and
-// 240 degrees in FP64 and rounding to the grid.
-MSKG_HD void find_nn(const Geometry &g, int lx, int ly, const int s1[3], const int s2[3], const int sc[3],
-                     int out[2][3]) {
+// FIND_NN.f:25-77: the remaining tetrahedral neighbours of SiteC given Site1
+// and Site2, by rotating Site2-SiteC about unit(SiteC-Site1) by 120 (irot 0)
+// or 240 (irot 1) degrees in FP64 and rounding to the grid.  One of the two;
+// the event kernels give each to a lane.
+MSKG_HD void find_nn_one(const Geometry &g, int lx, int ly, const int s1[3], const int s2[3], const int sc[3],
+                         int irot, int out[3]) {
   int a[3] = {s1[0], s1[1], s1[2]}, b[3] = {s2[0], s2[1], s2[2]};
   if (iabs_(sc[0] - a[0]) > lx / 2) a[0] += isign_(lx, sc[0] - a[0]);
   if (iabs_(sc[1] - a[1]) > ly / 2) a[1] += isign_(ly, sc[1] - a[1]);
@@ -191,60 +205,57 @@ MSKG_HD void find_nn(const Geometry &g, int lx, int ly, const int s1[3], const i
   for (int i = 0; i < 3; i++) ax[i] = (double)sc[i] - (double)a[i];
   double sn = sqrt(ax[0] * ax[0] + ax[1] * ax[1] + ax[2] * ax[2]);
   for (int i = 0; i < 3; i++) ax[i] = ax[i] / sn;
-  for (int irot = 0; irot < 2; irot++) {
-    const double cth = g.cth[irot], sth = g.sth[irot];
-    double R[3][3];
-    for (int i = 0; i < 3; i++) R[i][i] = ax[i] * ax[i] * (1 - cth) + cth;
-    R[1][0] = ax[0] * ax[1] * (1 - cth) - ax[2] * sth;
-    R[0][1] = ax[0] * ax[1] * (1 - cth) + ax[2] * sth;
-    R[2][0] = ax[0] * ax[2] * (1 - cth) + ax[1] * sth;
-    R[0][2] = ax[0] * ax[2] * (1 - cth) - ax[1] * sth;
-    R[2][1] = ax[1] * ax[2] * (1 - cth) - ax[0] * sth;
-    R[1][2] = ax[1] * ax[2] * (1 - cth) + ax[0] * sth;
-    for (int k = 0; k < 3; k++) {
-      double r = 0.0;
-      for (int l = 0; l < 3; l++) r = r + R[l][k] * ((double)b[l] - (double)sc[l]);
-      out[irot][k] = nint_(r) + sc[k];
-    }
-    if (out[irot][0] >= lx) out[irot][0] -= lx;
-    if (out[irot][0] < 0) out[irot][0] += lx;
-    if (out[irot][1] >= ly) out[irot][1] -= ly;
-    if (out[irot][1] < 0) out[irot][1] += ly;
+  const double cth = irot ? g.cth[1] : g.cth[0], sth = irot ? g.sth[1] : g.sth[0];
+  double R[3][3];
+  for (int i = 0; i < 3; i++) R[i][i] = ax[i] * ax[i] * (1 - cth) + cth;
+  R[1][0] = ax[0] * ax[1] * (1 - cth) - ax[2] * sth;
+  R[0][1] = ax[0] * ax[1] * (1 - cth) + ax[2] * sth;
+  R[2][0] = ax[0] * ax[2] * (1 - cth) + ax[1] * sth;
+  R[0][2] = ax[0] * ax[2] * (1 - cth) - ax[1] * sth;
+  R[2][1] = ax[1] * ax[2] * (1 - cth) - ax[0] * sth;
+  R[1][2] = ax[1] * ax[2] * (1 - cth) + ax[0] * sth;
+  for (int k = 0; k < 3; k++) {
+    double r = 0.0;
+    for (int l = 0; l < 3; l++) r = r + R[l][k] * ((double)b[l] - (double)sc[l]);
+    out[k] = nint_(r) + sc[k];
   }
+  if (out[0] >= lx) out[0] -= lx;
+  if (out[0] < 0) out[0] += lx;
+  if (out[1] >= ly) out[1] -= ly;
+  if (out[1] < 0) out[1] += ly;
+}
+MSKG_HD void find_nn(const Geometry &g, int lx, int ly, const int s1[3], const int s2[3], const int sc[3],
+                     int out[2][3]) {
+  for (int irot = 0; irot < 2; irot++) find_nn_one(g, lx, ly, s1, s2, sc, irot, out[irot]);
 }
 
-// FIND_SN.f:26-84: zig-zag (inversion through the bond centre) and
-// arm-chair (translation along the bond) candidates for the back bonds of
-// Site, whose only fixed neighbour is SiteC with further neighbours SN.
-MSKG_HD void find_sn(const Geometry &g, int lx, int ly, const int site[3], const int sc_in[3], const int sn_in[3][3],
-                     int zig[3][3], int arm[3][3]) {
-  int sc[3] = {sc_in[0], sc_in[1], sc_in[2]}, sn[3][3];
-  for (int i = 0; i < 3; i++)
-    for (int k = 0; k < 3; k++) sn[i][k] = sn_in[i][k];
+// FIND_SN.f:26-84: the zig-zag (inversion through the bond centre) or
+// arm-chair (translation along the bond) candidate for one back bond of
+// Site, whose only fixed neighbour is SiteC with the further neighbour sn_in.
+MSKG_HD void find_sn_one(const Geometry &g, int lx, int ly, const int site[3], const int sc_in[3], const int sn_in[3],
+                         bool zigzag, int out[3]) {
+  int sc[3] = {sc_in[0], sc_in[1], sc_in[2]}, sn[3] = {sn_in[0], sn_in[1], sn_in[2]};
   if (iabs_(site[0] - sc[0]) > lx / 2) sc[0] += isign_(lx, site[0] - sc[0]);
   if (iabs_(site[1] - sc[1]) > ly / 2) sc[1] += isign_(ly, site[1] - sc[1]);
-  for (int i = 0; i < 3; i++) {
-    if (iabs_(site[0] - sn[i][0]) > lx / 2) sn[i][0] += isign_(lx, site[0] - sn[i][0]);
-    if (iabs_(site[1] - sn[i][1]) > ly / 2) sn[i][1] += isign_(ly, site[1] - sn[i][1]);
-  }
+  if (iabs_(site[0] - sn[0]) > lx / 2) sn[0] += isign_(lx, site[0] - sn[0]);
+  if (iabs_(site[1] - sn[1]) > ly / 2) sn[1] += isign_(ly, site[1] - sn[1]);
   double cent[3], ax[3];
   for (int k = 0; k < 3; k++) cent[k] = 0.5 * ((double)sc[k] + (double)(float)site[k]);
   for (int k = 0; k < 3; k++) ax[k] = (double)site[k] - (double)sc[k];
   double snorm = sqrt(ax[0] * ax[0] + ax[1] * ax[1] + ax[2] * ax[2]);
   for (int k = 0; k < 3; k++) ax[k] = ax[k] / snorm;
+  for (int k = 0; k < 3; k++)
+    out[k] = nint_(zigzag ? 2 * cent[k] - (double)sn[k] : (double)sn[k] + g.arm_shift * ax[k]);
+  if (out[0] >= lx) out[0] -= lx;
+  if (out[0] < 0) out[0] += lx;
+  if (out[1] >= ly) out[1] -= ly;
+  if (out[1] < 0) out[1] += ly;
+}
+MSKG_HD void find_sn(const Geometry &g, int lx, int ly, const int site[3], const int sc_in[3], const int sn_in[3][3],
+                     int zig[3][3], int arm[3][3]) {
   for (int i = 0; i < 3; i++) {
-    for (int k = 0; k < 3; k++) {
-      zig[i][k] = nint_(2 * cent[k] - (double)sn[i][k]);
-      arm[i][k] = nint_((double)sn[i][k] + g.arm_shift * ax[k]);
-    }
-    if (zig[i][0] >= lx) zig[i][0] -= lx;
-    if (zig[i][0] < 0) zig[i][0] += lx;
-    if (zig[i][1] >= ly) zig[i][1] -= ly;
-    if (zig[i][1] < 0) zig[i][1] += ly;
-    if (arm[i][0] >= lx) arm[i][0] -= lx;
-    if (arm[i][0] < 0) arm[i][0] += lx;
-    if (arm[i][1] >= ly) arm[i][1] -= ly;
-    if (arm[i][1] < 0) arm[i][1] += ly;
+    find_sn_one(g, lx, ly, site, sc_in, sn_in[i], true, zig[i]);
+    find_sn_one(g, lx, ly, site, sc_in, sn_in[i], false, arm[i]);
   }
 }
 
