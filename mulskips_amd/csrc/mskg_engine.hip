@@ -171,11 +171,6 @@ __device__ inline double read_lane(double v, int l) {
 // the whole wave are scalar loads.  A round trip through the address space
 // states that (through an integer: a direct cast there and back folds away).
 template <typename T>
-__device__ inline T *as_global(T *p) {
-  __attribute__((address_space(1))) T *g = (__attribute__((address_space(1))) T *)(uintptr_t)p;
-  return (T *)g;
-}
-template <typename T>
 __device__ inline const T *as_constant(const T *p) {
   const __attribute__((address_space(4))) T *c = (const __attribute__((address_space(4))) T *)(uintptr_t)p;
   return (const T *)c;
@@ -187,15 +182,13 @@ __device__ inline void to_global(Lattice &L) {
   L.win = as_global(L.win); L.geo = as_constant(L.geo); L.tab = as_constant(L.tab); L.key = as_global(L.key);
   L.cl = as_global(L.cl);
 }
-__device__ inline void slot_add(RunState *st, int b, double r, unsigned long long n, unsigned long long nev) {
+__device__ inline void slot_add(RunState *st, int b, double r, unsigned long long n) {
   Slot &sl = st->slot[b & (NSLOT - 1)];
-  if (n) {
-    const unsigned long long rb = (unsigned long long)__double_as_longlong(r);
-    if (rb > sl.rmax) atomicMax(&sl.rmax, rb);
-    atomicAdd(&sl.n, n);
-    atomicAdd(&sl.tiles, 1ull);
-  }
-  if (nev) atomicAdd(&sl.events, nev);
+  if (!n) return;
+  const unsigned long long rb = (unsigned long long)__double_as_longlong(r);
+  if (rb > sl.rmax) atomicMax(&sl.rmax, rb);
+  atomicAdd(&sl.n, n);
+  atomicAdd(&sl.tiles, 1ull);
 }
 
 // The reference event's counter (RunState::counts).
@@ -426,7 +419,7 @@ __global__ void __launch_bounds__(256) k_build_lists(Lattice L, int ntiles) {
   if (lane == 0) {
     L.tl_n[t] = n;
     L.tl_own[t] = min(n, L.capg);
-    if (n) widen_window(L, tile_colour(g.tx, g.ty, g.tz), g.tz);
+    if (n) widen_window(L.win, tile_colour(g.tx, g.ty, g.tz), g.tz);
   }
 }
 
@@ -436,7 +429,7 @@ __global__ void __launch_bounds__(256) k_list_window(Lattice L, int ntiles) {
   if (t >= ntiles) return;
   if (L.tl_n[t] > 0) {
     const int tx = t % L.ntx, ty = (t / L.ntx) % L.nty, tz = t / (L.ntx * L.nty);
-    widen_window(L, tile_colour(tx, ty, tz), tz);
+    widen_window(L.win, tile_colour(tx, ty, tz), tz);
   }
 }
 
@@ -459,39 +452,33 @@ __global__ void __launch_bounds__(256) k_tile_rates(Lattice L, int ntiles, RunSt
   for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, WAVE);
   if (lane == 0) {
     L.tile_r[t] = cnt ? acc : 0.0;
-    if (cnt) slot_add(st, t, acc, (unsigned long long)cnt, 0);
+    if (cnt) slot_add(st, t, acc, (unsigned long long)cnt);
   }
 }
 
-// Sorts lk/lr/lc[lo, hi) by offset (the offsets are distinct): a bitonic
-// network across the lanes for up to 64 entries, odd-even transposition
-// rounds beyond (rare: appends from other tiles between two passes).
+// Sorts lk/lr/lc[lo, hi) by offset (the offsets are distinct): up to 64
+// entries by rank, each lane counting the smaller ones (a handful: the
+// appends from other tiles between two passes), odd-even transposition rounds
+// beyond.
 __device__ inline void sort_by_offset(int32_t *lk, float *lr, uint8_t *lc, int lo, int hi, int lane) {
   const int m = hi - lo;
   if (m <= 1) return;
   if (m <= WAVE) {
-    int key = lane < m ? lk[lo + lane] : 0x7fffffff;
-    int idx = lane;
-    for (int k = 2; k <= WAVE; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        const int ok = __shfl_xor(key, j, WAVE), oi = __shfl_xor(idx, j, WAVE);
-        const bool keep_min = ((lane & k) == 0) == ((lane & j) == 0);
-        if (keep_min ? ok < key : ok > key) {
-          key = ok;
-          idx = oi;
-        }
-      }
+    int key = 0, rank = 0;
     float r = 0.0f;
     uint8_t c = 0;
     if (lane < m) {
-      r = lr[lo + idx];
-      c = lc[lo + idx];
+      key = lk[lo + lane];
+      r = lr[lo + lane];
+      c = lc[lo + lane];
     }
+#pragma unroll 1
+    for (int q = 0; q < m; q++) rank += __builtin_amdgcn_readlane(key, q) < key ? 1 : 0;
     __syncthreads();
     if (lane < m) {
-      lk[lo + lane] = key;
-      lr[lo + lane] = r;
-      lc[lo + lane] = c;
+      lk[lo + rank] = key;
+      lr[lo + rank] = r;
+      lc[lo + rank] = c;
     }
     __syncthreads();
     return;
@@ -513,27 +500,87 @@ __device__ inline void sort_by_offset(int32_t *lk, float *lr, uint8_t *lc, int l
   }
 }
 
+// The sum of v over the wave, added as an exchange with the lane 32, 16, 8,
+// 4, 2 and 1 apart adds it (every lane the same bits): the first two steps by
+// lane swaps, the others by rotations within a row of 16, whose operands the
+// steps before made periodic.
+__device__ inline double swap_add(double v, bool rows) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  unsigned l0, l1, h0, h1;
+  if (rows) {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    l0 = l[0]; l1 = l[1]; h0 = h[0]; h1 = h[1];
+  } else {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    l0 = l[0]; l1 = l[1]; h0 = h[0]; h1 = h[1];
+  }
+  return __longlong_as_double((long long)(((unsigned long long)h0 << 32) | l0)) +
+         __longlong_as_double((long long)(((unsigned long long)h1 << 32) | l1));
+}
+__device__ inline double wave_sum_dpp(double v) {
+  v = swap_add(v, true);
+  v = swap_add(v, false);
+  v += dpp_take<0x128, 0xf>(v);  // row_ror:8
+  v += dpp_take<0x124, 0xf>(v);  // row_ror:4
+  v += dpp_take<0x122, 0xf>(v);  // row_ror:2
+  v += dpp_take<0x121, 0xf>(v);  // row_ror:1
+  return v;
+}
+
+// The parameters of a kernel whose only argument they are, in its argument segment.
+__device__ inline const PassParams *kernel_params() {
+  return as_constant((const PassParams *)__builtin_amdgcn_kernarg_segment_ptr());
+}
+// The fields an event needs of the lattice in pp; the others are read where
+// they are used.
+__device__ inline Lattice event_part(const PassParams *pp) {
+  Lattice L = pp->L;
+  to_global(L);
+  L.cold = &pp->L;
+  return L;
+}
+
 // One tile's share of a colour pass: its candidate list into LDS, rejection-
 // free KMC inside the tile for the window tau, the list back.  Returns the
 // error that ends the wave's work (0: none).  The selected site, its record
 // and the event type are kept in scalar registers: the event's addresses and
 // branches are then scalar too.
+// pp: the parameters in constant memory, read where they are needed (read_here);
+// L: the fields an event needs.  fresh: the wave's tables are to be loaded.
 template <bool LA, bool COV>
-__device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, const double tau, const int t,
-                                const int colour, const TabLds &tabs, int32_t *lk, float *lr, uint8_t *lc,
+__device__ inline int pass_tile(const PassParams *pp, Lattice &L, RunState *st, const double tau, const int t,
+                                const int colour, TabLds &tabs, const bool fresh, unsigned char *smem,
                                 const int lane) {
-  const int cap = P.cap;
+  const int cap = pp->cap;
+  int32_t *const lk = (int32_t *)smem;        // tile-local point offsets
+  float *const lr = (float *)(lk + cap);      // rates
+  uint8_t *const lc = (uint8_t *)(lr + cap);  // classes
+  TileGeom g;
+  int n = 0;
+  unsigned long long sweeps;
+  double rtot;
+  {
+  const PassParams &P = *read_here(pp);
+  int32_t *const tl_n = as_global(P.L.tl_n);
+  const int32_t *const idx = as_global(P.L.tl_idx) + (int64_t)t * P.L.capg;
+  uint8_t *const inlist = as_global(P.L.inlist);
   // The tile's first loads leave together, in one round trip: its list
   // length and own count, the first WAVE list entries (read whatever the
   // length; a lane uses its entry only below it, and the index stays in the
   // tile's list storage), and the run state the window needs.
-  const int n_in = __builtin_amdgcn_readfirstlane(L.tl_n[t]);
-  const int own = __builtin_amdgcn_readfirstlane(L.tl_own[t]);
-  const int k_first = L.tl_idx[(int64_t)t * L.capg + min(lane, L.capg - 1)];
-  const double rtot = st->rtot;
-  const unsigned long long sweeps = st->sweeps;
+  TabRegs tr;
+  if (fresh) fetch_tables(*L.tab, tr, lane);
+  const int n_raw = tl_n[t], own_raw = as_global(P.L.tl_own)[t];
+  const int k_first = idx[min(lane, P.L.capg - 1)];
+  rtot = st->rtot;
+  sweeps = st->sweeps;
+  if (fresh) put_tables(tr, tabs, lane);
+  const int n_in = __builtin_amdgcn_readfirstlane(n_raw), own = __builtin_amdgcn_readfirstlane(own_raw);
   if (n_in == 0) return 0;
-  TileGeom g = tile_geom(t, L.tile, L.ntx, L.nty, L.box.lz);
+  g = tile_geom(t, L.tile, P.L.ntx, P.L.nty, L.box.lz);
   L.cur_tile = t;
   L.cx = g.tx * L.tile;
   L.cy = g.ty * L.tile;
@@ -542,20 +589,20 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
   // 1. the tile's candidate list -> LDS, dropping entries no longer active;
   // the entries other tiles appended since the tile's last pass (an order
   // that depends on timing) are then sorted by offset
-  const int m_in = min(n_in, L.capg);
-  int n = 0, nh = 0;
+  const int m_in = min(n_in, P.L.capg);
+  int nh = 0;
   for (int j0 = 0; j0 < m_in; j0 += WAVE) {
     int j = j0 + lane;
     uint8_t c = 0;
     float r = 0.0f;
     int k = 0;
     if (j < m_in) {
-      k = j0 == 0 ? k_first : L.tl_idx[(int64_t)t * L.capg + j];
+      k = j0 == 0 ? k_first : idx[j];
       P3 p = tile_point(L.box, g, L.tile, k);
       // class and rate in one round trip (the rate is used only with a class)
       c = L.cls[p.i];
       r = L.rate[p.i];
-      if (!c) L.inlist[p.i] = 0;
+      if (!c) inlist[p.i] = 0;
     }
     unsigned long long m = __ballot(c != 0);
     int slot = n + __popcll(m & ((1ull << lane) - 1ull));
@@ -577,20 +624,24 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
   }
   __syncthreads();
   sort_by_offset(lk, lr, lc, nh, n, lane);
+  }
 
   // 2. rejection-free KMC inside the tile for the window tau
   double tloc = 0.0;
   unsigned int nev = 0;
-  unsigned int my_cnt = 0, my_des = 0;  // lane l: events of counter l, desorptions of coverage slot l + 1
+  unsigned int my_cnt = 0, my_des = 0;  // lane l + 4: events of counter l; lane l: desorptions of coverage slot l + 1
   int my_dcc = 0;                       // lane l: change of CountCrystal(l + 1) (laser-annealing build's form)
   U4 d;              // lane l: the Philox block of draw 64 b + l, b the current batch
   double wait = 0.0;  // ... and -ln of its first uniform
   int err = 0;
+  const bool logging = pp->log != nullptr;
+  pin(L.site); pin(L.rate); pin(L.cls);
   // every wave ends its pass: the window tau bounds the expected number of
   // events, and this cap bounds the worst case (a window cut short by it is
   // counted in RunState::guard_exits and reported by the run)
   int guard = 0;
   for (; guard < PASS_EVENT_CAP; guard++) {
+    pin(L.box);
     // one Philox block per event: waiting time, selection, event type and
     // stacking choice, 32 random bits each (the reference's ran3 has fewer).
     // The block depends on the draw's number only, so the wave makes 64 of
@@ -602,6 +653,7 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
       ctr.y = (uint32_t)sweeps;
       ctr.z = (uint32_t)(sweeps >> 32) ^ ((uint32_t)colour << 29);
       ctr.w = (uint32_t)(guard + lane);
+      const PassParams &P = *read_here(pp);
       d = philox4x32_10(ctr, P.key0, P.key1);
       wait = -log(u01_32(d.x));
     }
@@ -612,9 +664,6 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
     const double inc = wave_incl_scan_dpp(part);
     const double R = read_lane(inc, WAVE - 1);
     if (!(R > 0.0)) break;
-    const double dt = read_lane(wait, dl) / R;  // FP64 waiting time
-    if (tloc + dt > tau) break;
-    tloc += dt;
     const double target = u01_32((uint32_t)__builtin_amdgcn_readlane((int)d.y, dl)) * R;
     // the first lane whose inclusive prefix exceeds target (the last lane
     // with a rate when rounding leaves target at the top end), then the
@@ -646,7 +695,13 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
       if (sel < 0) break;
     }
     const P3 s = tile_point(L.box, g, L.tile, __builtin_amdgcn_readfirstlane(lk[sel]));
-    const Rec srec = uniform_rec(load_rec(L, s.i));
+    // the site's record is on its way while the waiting time is taken: the
+    // event may lie beyond the window
+    const Rec srec_v = load_rec(L, s.i);
+    const double dt = read_lane(wait, dl) / R;  // FP64 waiting time
+    if (tloc + dt > tau) break;
+    tloc += dt;
+    const Rec srec = uniform_rec(srec_v);
     const int cls = __builtin_amdgcn_readfirstlane((int)lc[sel]);
     Choice ch;
     ch.arm = -1;
@@ -658,7 +713,9 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
     EvOut o;
     execute<LA, COV>(L, tabs, rtot, s, srec, itrans, ch, o, lane);
     err = __builtin_amdgcn_readfirstlane(o.err);
-    if (P.log && lane == 0) {
+    if (logging && lane == 0) {
+      const PassParams &P = *read_here(pp);
+      mskg_event *const out = as_global(P.log);
       const unsigned long long li = atomicAdd(&st->log_n, 1ull);
       if (li < P.log_cap) {
         mskg_event ev;
@@ -669,42 +726,42 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
         ev.coor = coor0;
         ev.rtot = rtot;
         ev.time = st->clock + tloc;
-        P.log[li] = ev;
+        out[li] = ev;
       }
     }
-    if (lane == count_slot(itrans)) my_cnt++;
+    if (lane == count_slot(itrans) + 4) my_cnt++;
     if (LA && o.species && itrans <= 4 && lane == o.species - 1) my_dcc += itrans <= 3 ? 1 : -1;
     if (COV && itrans == 5 && o.species && lane == o.species - 1) my_des++;
     nev++;
     if (err) break;
     // refresh the on-chip list with the touched points' new rates, which
-    // execute() left a lane each: the slot of each touched point inside the
-    // tile, one ballot of the list against its offset (list entries are
-    // distinct, so each touched point has at most one slot; a point touched
-    // twice finds the same slot), and whether an earlier touched point has
-    // the same offset
+    // execute() left a lane each: each such lane inside the tile looks its
+    // offset up in the list, four entries a read (the offsets are distinct;
+    // what lies behind the list's end is not taken)
     const int kl = o.set ? tile_local(g, L.tile, o.p) : -1;
     float tr = o.rate;
     int tc = o.cls;
-    if (o.set == 2 && kl >= 0) {
-      tr = L.rate[o.p.i];
-      tc = L.cls[o.p.i];
-    }
     int found = -1;
+    for (int j0 = (n - 1) & ~3; j0 >= 0; j0 -= 4) {
+      const int4 v = *(const int4 *)(lk + j0);
+      found = v.w == kl ? j0 + 3 : found;
+      found = v.z == kl ? j0 + 2 : found;
+      found = v.y == kl ? j0 + 1 : found;
+      found = v.x == kl ? j0 : found;
+    }
+    if (found >= n) found = -1;
+    // repeated list entries: the rates are in memory, and a point touched
+    // twice joins the list once
     bool dup = false;
-    const int k_lane = lane < n ? lk[lane] : -1;  // the list's first WAVE entries, one a lane
-    for (unsigned long long tm = __ballot(kl >= 0); tm; tm &= tm - 1ull) {
-      const int q = __ffsll((long long)tm) - 1;
-      const int kq = __builtin_amdgcn_readlane(kl, q);
-      if (q < lane && kq == kl) dup = true;
-      unsigned long long m = __ballot(k_lane == kq);
-      int f = m ? __ffsll((long long)m) - 1 : -1;
-      for (int j0 = WAVE; f < 0 && j0 < n; j0 += WAVE) {
-        const int kj = j0 + lane < n ? lk[j0 + lane] : -1;
-        m = __ballot(kj == kq);
-        if (m) f = j0 + __ffsll((long long)m) - 1;
+    if (__ballot(o.set == 2)) {
+      if (o.set == 2 && kl >= 0) {
+        tr = L.rate[o.p.i];
+        tc = L.cls[o.p.i];
       }
-      if (lane == q) found = f;
+      for (unsigned long long tm = __ballot(kl >= 0); tm; tm &= tm - 1ull) {
+        const int q = __ffsll((long long)tm) - 1;
+        if (q < lane && __builtin_amdgcn_readlane(kl, q) == kl) dup = true;
+      }
     }
     // ... updates in place, and appends the new MC particles (first
     // occurrence of each) after the list in touched order
@@ -737,30 +794,46 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
   }
   if (guard >= PASS_EVENT_CAP && lane == 0) atomicAdd(&st->guard_exits, 1ull);
   // 3. write the list back (active entries only), tile totals, counters
+  const PassParams &P = *read_here(pp);
+  // the values the counters are compared with before an atomic (they change
+  // seldom), on their way with the list
+  Slot &sl = st->slot[t & (NSLOT - 1)];
+  int *const win = as_global(P.L.win) + 4 * colour;
+  const unsigned long long rmax = sl.rmax;
+  const int win_lo = win[2], win_hi = win[3];
+  int32_t *const idx = as_global(P.L.tl_idx) + (int64_t)t * P.L.capg;
+  uint8_t *const inlist = as_global(P.L.inlist);
   double part = 0.0;
   int nout = 0;
   for (int j0 = 0; j0 < n; j0 += WAVE) {
     int j = j0 + lane;
     bool keep = j < n && lc[j] != 0;
-    if (j < n) L.inlist[tile_point(L.box, g, L.tile, lk[j]).i] = keep ? 1 : 0;
+    if (j < n) inlist[tile_point(L.box, g, L.tile, lk[j]).i] = keep ? 1 : 0;
     if (keep && lc[j] != CLS_ISOLATED) part += (double)lr[j];
     unsigned long long m = __ballot(keep);
     int slot = nout + __popcll(m & ((1ull << lane) - 1ull));
-    if (keep) L.tl_idx[(int64_t)t * L.capg + slot] = lk[j];
+    if (keep) idx[slot] = lk[j];
     nout += __popcll(m);
   }
-  const double R = wave_sum(part);
-  if (lane < 8 && my_cnt) atomicAdd(&st->slot[t & (NSLOT - 1)].counts[lane], (unsigned long long)my_cnt);
+  const double R = wave_sum_dpp(part);
+  {
+    // the slot's sums in one atomic instruction, a lane each: n, tiles, events, counts
+    static_assert(offsetof(Slot, n) == 8 && offsetof(Slot, tiles) == 16 && offsetof(Slot, events) == 24 &&
+                  offsetof(Slot, counts) == 32, "Slot's words by lane");
+    const unsigned int v = lane == 1 ? (unsigned)nout : (lane == 2 ? (nout ? 1u : 0u) : (lane == 3 ? nev : my_cnt));
+    if (lane >= 1 && lane < 12 && v) atomicAdd(&sl.rmax + lane, (unsigned long long)v);
+  }
   if (LA && L.cl && my_dcc) atomicAdd(&st->dcc[lane], (unsigned long long)(long long)my_dcc);
   if (COV && my_des) atomicAdd(&st->desorbed[lane], (unsigned long long)my_des);
   if (lane == 0) {
-    L.tl_n[t] = nout;
-    L.tl_own[t] = nout;
-    L.tile_r[t] = R;
-    slot_add(st, t, R, (unsigned long long)nout, nev);
+    as_global(P.L.tl_n)[t] = nout;
+    as_global(P.L.tl_own)[t] = nout;
+    as_global(P.L.tile_r)[t] = R;
     if (nout) {
-      if (g.tz < L.win[4 * colour + 2]) atomic_min_i32(&L.win[4 * colour + 2], g.tz);
-      if (g.tz > L.win[4 * colour + 3]) atomic_max_i32(&L.win[4 * colour + 3], g.tz);
+      const unsigned long long rb = (unsigned long long)__double_as_longlong(R);
+      if (rb > rmax) atomicMax(&sl.rmax, rb);
+      if (g.tz < win_lo) atomic_min_i32(&win[2], g.tz);
+      if (g.tz > win_hi) atomic_max_i32(&win[3], g.tz);
     }
     if (err) {
       st->err = err;
@@ -773,12 +846,12 @@ __device__ inline int pass_tile(const PassParams &P, Lattice &L, RunState *st, c
   return 0;
 }
 
-// The tiles of `colour` in the colour's window of tile layers that hold
-// candidates (win[4c], win[4c+1], fixed during a sweep): their number, and
+// The tiles of `colour` in the colour's window of tile layers [lo, hi] that
+// hold candidates (win[4c], win[4c+1], fixed during a sweep): their number, and
 // zfirst, the lowest of those layers with the colour's layer parity.
-__device__ inline int colour_tiles(const Lattice &L, int ntz, int colour, int &zfirst) {
+__device__ inline int colour_tiles(const Lattice &L, int ntz, int colour, int lo, int hi, int &zfirst) {
   const int c2 = (colour >> 2) & 1;
-  const int zlo = max(L.win[4 * colour], 0), zhi = min(L.win[4 * colour + 1], ntz - 1);
+  const int zlo = max(lo, 0), zhi = min(hi, ntz - 1);
   zfirst = 0;
   if (zlo > zhi) return 0;  // no tile of this colour holds candidates
   zfirst = zlo + ((c2 - zlo) & 1);
@@ -795,32 +868,31 @@ __device__ inline int colour_tile(const Lattice &L, int colour, int zfirst, int 
 
 // One colour pass: the tiles of `colour` in the window of tile layers that
 // hold candidates, each workgroup (one wave) striding over them.  Three
-// waves per SIMD (168 VGPRs, no spills): 3072 tiles in flight on 256 CUs.
-// Measured on 8e6 events at 512^3 SiC: 69.1 ms; with two waves 74.9, with
-// four (128 VGPRs, spilled) 76.0.  The laser-annealing kernels hold exp and
+// waves per SIMD (157 VGPRs, no spills): 3072 tiles in flight on 256 CUs.
+// Measured on 8e6 events at 512^3 SiC (before the scalar registers were
+// relieved): 69.1 ms; with two waves 74.9, with four (128 VGPRs, spilled) 76.0.  The laser-annealing kernels hold exp and
 // erf: two waves (223 VGPRs), 55.3 ms on two exchanges of 3e4 events at
 // 264x264x384, against 60.4 with three (184 bytes a lane spilled) and 79.4
 // with four.
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_pass(PassParams P) {
-  extern __shared__ unsigned char smem[];
+  extern __shared__ __align__(16) unsigned char smem[];
   __shared__ TabLds tabs;
   const int lane = threadIdx.x;
-  Lattice L = P.L;
-  int32_t *lk = (int32_t *)smem;        // tile-local point offsets
-  float *lr = (float *)(lk + P.cap);    // rates
-  uint8_t *lc = (uint8_t *)(lr + P.cap);  // classes
-  RunState *st = P.st;
+  const PassParams *const pp = kernel_params();
+  RunState *const st = P.st;
+  // the run state and the colour's window in one round trip
   const double tau = st->tau;
-  if (!(tau > 0.0) || st->err || st->stop) return;
-  L.geo = as_constant(L.geo);
-  L.tab = as_constant(L.tab);
+  const int idle = st->err | st->stop, lo = P.L.win[4 * P.colour], hi = P.L.win[4 * P.colour + 1];
+  if (!(tau > 0.0) || idle) return;
   int zfirst;
-  const int nwin = colour_tiles(L, P.ntz, P.colour, zfirst);
-  if ((int)blockIdx.x < nwin) load_tables(*L.tab, tabs, lane);
+  const int nwin = colour_tiles(P.L, P.ntz, P.colour, lo, hi, zfirst);
+  Lattice L = event_part(pp);
+  bool fresh = true;
   for (int wi = blockIdx.x; wi < nwin; wi += gridDim.x) {
-    const int t = colour_tile(L, P.colour, zfirst, wi);
-    if (pass_tile<LA, COV>(P, L, st, tau, t, P.colour, tabs, lk, lr, lc, lane)) return;
+    const int t = colour_tile(P.L, P.colour, zfirst, wi);
+    if (pass_tile<LA, COV>(pp, L, st, tau, t, P.colour, tabs, fresh, smem, lane)) return;
+    fresh = false;
   }
 }
 
@@ -862,21 +934,17 @@ constexpr long long SCHED_WAIT_TICKS = 200000000ll;
 
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_sweep(PassParams P) {
-  extern __shared__ unsigned char smem[];
+  extern __shared__ __align__(16) unsigned char smem[];
   __shared__ TabLds tabs;
   const int lane = threadIdx.x;
-  Lattice L = P.L;
-  int32_t *lk = (int32_t *)smem;
-  float *lr = (float *)(lk + P.cap);
-  uint8_t *lc = (uint8_t *)(lr + P.cap);
+  const PassParams *const pp = kernel_params();
+  Lattice L = event_part(pp);
   RunState *st = P.st;
   const double tau = st->tau;
   if (!(tau > 0.0) || st->err || st->stop) return;
   // the window as the sweep starts (L.win's first words widen during it)
   const int zlo = (int)P.sched[3], zhi = (int)P.sched[4];
   if (zlo > zhi) return;
-  L.geo = as_constant(L.geo);
-  L.tab = as_constant(L.tab);
   load_tables(*L.tab, tabs, lane);
   int first[2], count[2];
   queue_layers(zlo, zhi, 0, P.ntz, first[0], count[0]);
@@ -957,7 +1025,7 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 
                                                                          __HIP_MEMORY_SCOPE_AGENT));
     const int n_in = __builtin_amdgcn_readfirstlane(L.tl_n[t]);
     if (!abort && !err_now && n_in > 0) {
-      pass_tile<LA, COV>(P, L, st, tau, t, colour, tabs, lk, lr, lc, lane);
+      pass_tile<LA, COV>(pp, L, st, tau, t, colour, tabs, false, smem, lane);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // the tile's writes before its flag
     }
     // every lane stores the same stamp
@@ -1123,7 +1191,7 @@ __global__ void __launch_bounds__(ENS_MAX) k_ens_plan(const PassParams *__restri
     // k_pass's condition, checked as its colour pass starts
     if (run && !st->err) {
       int zf;
-      cnt = colour_tiles(P.L, P.ntz, colour, zf);
+      cnt = colour_tiles(P.L, P.ntz, colour, P.L.win[4 * colour], P.L.win[4 * colour + 1], zf);
     }
   }
   __syncthreads();
@@ -1159,7 +1227,7 @@ __device__ inline int ens_replica(const int *pc, int n, int q, int lane) {
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3)))
 k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
-  extern __shared__ unsigned char smem[];
+  extern __shared__ __align__(16) unsigned char smem[];
   __shared__ TabLds tabs;
   const int lane = threadIdx.x;
   const int *pc = plan + colour * (n + 1);
@@ -1169,7 +1237,9 @@ k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
   // lattice and run state, the window's first layer and the window tau
   int r = -1, lo = 0, hi = 0, zfirst = 0, failed = 0;
   double tau = 0.0;
-  Lattice L = reps[0].L;
+  bool fresh = false;
+  const PassParams *pp = as_constant(reps);
+  Lattice L = event_part(pp);
   RunState *st = nullptr;
   // Every decision of this loop is wave-uniform (readfirstlane / ballot)
   // and no memory access sits under a lane-dependent branch.  A wave's
@@ -1184,25 +1254,24 @@ k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
       r = __builtin_amdgcn_readfirstlane(ens_replica(pc, n, q, lane));
       lo = __builtin_amdgcn_readfirstlane(pc[r]);
       hi = __builtin_amdgcn_readfirstlane(pc[r + 1]);
-      L = reps[r].L;
-      to_global(L);
-      load_tables(*L.tab, tabs, lane);
-      st = as_global(reps[r].st);
+      pp = as_constant(reps + r);
+      L = event_part(pp);
+      fresh = true;
+      st = as_global(pp->st);
       // a replica that has failed in this sweep runs no further tiles here
       // (k_pass checks at the start of each colour pass)
       failed = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&st->err, __ATOMIC_RELAXED,
                                                                 __HIP_MEMORY_SCOPE_AGENT));
       tau = st->tau;
-      colour_tiles(L, reps[r].ntz, colour, zfirst);
+      const int *const win = as_global(pp->L.win) + 4 * colour;
+      colour_tiles(pp->L, pp->ntz, colour, win[0], win[1], zfirst);
     }
     if (!failed) {
-      const PassParams &P = reps[r];
-      const int t = colour_tile(L, colour, zfirst, q - lo);
-      int32_t *lk = (int32_t *)smem;
-      float *lr = (float *)(lk + P.cap);
-      uint8_t *lc = (uint8_t *)(lr + P.cap);
+      const int t = colour_tile(pp->L, colour, zfirst, q - lo);
       // a wave stops its tiles of a replica whose tile failed (as k_pass's wave returns)
-      failed = __builtin_amdgcn_readfirstlane(pass_tile<LA, COV>(P, L, st, tau, t, colour, tabs, lk, lr, lc, lane));
+      failed = __builtin_amdgcn_readfirstlane(
+          pass_tile<LA, COV>(pp, L, st, tau, t, colour, tabs, fresh, smem, lane));
+      fresh = false;
     }
     // the next entry: every lane adds 1 (one atomic of 64 for the wave)
     const unsigned int took = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1601,7 +1670,7 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
   const SerialDesc D = descs[blockIdx.x];
   Lattice L = D.L;
   to_global(L);
-  L.cur_tile = -1;
+  L.cold = as_constant(&descs[blockIdx.x].L);
   RunState *st = as_global(D.st);
   load_tables(*L.tab, tabs, lane);
   if (st->err) return;
@@ -1780,7 +1849,6 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
   D.acc = as_global(D.acc);
   Lattice L = D.L;
   to_global(L);
-  L.cur_tile = -1;
   load_tables(*L.tab, tabs, lane);
   // the per-class integrals and change times in the segment's own device
   // memory (LDS holds the populations only, so that more waves fit a CU)
@@ -2460,6 +2528,8 @@ static Lattice make_lattice(mskg_engine *e) {
   L.win = e->d_win;
   L.capg = e->capg;
   L.cur_tile = -1;
+  L.cx = L.cy = L.cz = 0;
+  L.cold = nullptr;
   L.box = e->box;
   L.geo = e->d_geo;
   L.tab = e->d_tab;
@@ -3178,7 +3248,6 @@ static int refresh_range(mskg_engine *e, int64_t first, int64_t end, bool lists_
   if (rc) return rc;
   HIPCHK(e, hipMemsetAsync(e->d_err, 0, sizeof(int), e->stream));
   Lattice L = make_lattice(e);
-  L.inlist = nullptr;
   if (!lists_stay) e->lists_dirty = true;
   HIPCHK(e, hipEventRecord(e->ev0, e->stream));
   const bool la = e->tab.la_mode || e->tab.st_n;
@@ -3255,7 +3324,6 @@ int mskg_replay(mskg_engine *e, const mskg_event *log, int64_t n, int32_t clock_
     return fail_(e, MSKG_EDEVICE, "replay upload: %s", hipGetErrorString(ce));
   }
   Lattice L = make_lattice(e);
-  L.inlist = nullptr;
   e->lists_dirty = true;
   hipLaunchKernelGGL(MSKG_VARIANT(k_replay, e->tab.la_mode || e->tab.st_n, e->cov_model), dim3(1), dim3(WAVE), 0, e->stream, L, d_log, n, clock_mode, e->d_st);
   hipError_t le = hipGetLastError();
@@ -4183,7 +4251,6 @@ int mskg_adjoint_checkpointed(mskg_engine *const *engines, int32_t n, const mskg
   for (int i = 0; i < n; i++) {
     mskg_engine *e = engines[i];
     Lattice L = make_lattice(e);
-    L.inlist = nullptr;
     L.key = e->d_key;
     AdjDesc &D = descs[i];
     D.L = L;

@@ -54,6 +54,8 @@ struct Lattice {
   float inv_tile;         // 1 / tile
   int32_t *key;           // may be null: rate-class key of every point (likelihood accounting)
   const long long *cl;    // may be null: CountLiquid(1..3) the laser-annealing build's rates read
+  const Lattice *cold;    // in a kernel that keeps lists: this lattice in constant memory, for
+                          // the fields an event seldom needs (enlist); null: no lists to keep
   int ztop;               // highest z of an event's site: an event reads at most 12 and writes at
                           // most 6 planes from its site, so with only the bottom planes stored an
                           // event above this would reach past them (INT_MAX: every plane stored)
@@ -169,30 +171,75 @@ MSKG_HD int tile_colour(int tx, int ty, int tz) { return (tx & 1) | ((ty & 1) <<
 // pass visits.  A colour's window is only widened by passes of the other
 // colours (same-colour tiles never touch each other), so it is constant
 // while its own pass runs.
-MSKG_HD void widen_window(const Lattice &L, int colour, int tz) {
-  if (!L.win) return;
-  int *w = L.win + 4 * colour;
+MSKG_HD void widen_window(int *win, int colour, int tz) {
+  int *w = win + 4 * colour;
   // read first: the window rarely changes, and atomics on one word serialise
   if (tz < w[0]) atomic_min_i32(&w[0], tz);
   if (tz > w[1]) atomic_max_i32(&w[1], tz);
   if (tz < w[2]) atomic_min_i32(&w[2], tz);
   if (tz > w[3]) atomic_max_i32(&w[3], tz);
 }
+// A pointer to constant memory, read here: the compiler may not load what is
+// behind it earlier and carry it in registers.  An event's loop has more
+// values the same in every lane than scalar registers (it spilled about 80 of
+// them to vector lanes and read them back on every event).
+template <typename T>
+__device__ inline const T *read_here(const T *p) {
+  uint64_t v = (uint64_t)(uintptr_t)p;
+  asm volatile("" : "+s"(v));
+  const __attribute__((address_space(4))) T *c = (const __attribute__((address_space(4))) T *)(uintptr_t)v;
+  return (const T *)c;
+}
+template <typename T>
+__device__ inline T *as_global(T *p) {
+  __attribute__((address_space(1))) T *g = (__attribute__((address_space(1))) T *)(uintptr_t)p;
+  return (T *)g;
+}
+// A value that is the same in every lane, held in a scalar register from here
+// on: the compiler may neither load it again nor carry in registers what
+// could be computed from it before this point.
+__device__ inline void pin(int &v) {
+  v = __builtin_amdgcn_readfirstlane(v);
+  asm volatile("" : "+s"(v));
+}
+__device__ inline void pin(uint32_t &v) {
+  int i = (int)v;
+  pin(i);
+  v = (uint32_t)i;
+}
+__device__ inline void pin(int64_t &v) {
+  int lo = (int)(uint32_t)v, hi = (int)(v >> 32);
+  pin(lo);
+  pin(hi);
+  v = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+template <typename T>
+__device__ inline void pin(T *&p) {
+  int64_t v = (int64_t)(uintptr_t)p;
+  pin(v);
+  p = as_global((T *)(uintptr_t)v);
+}
+__device__ inline void pin(Box &b) {
+  pin(b.lx); pin(b.ly); pin(b.lz); pin(b.hx); pin(b.hy); pin(b.plane);
+}
 // A site that becomes an MC particle joins its tile's list (once).
-MSKG_HD void enlist(const Lattice &L, const P3 &p) {
-  if (!L.inlist) return;
+__device__ inline void enlist(const Lattice &L, const P3 &p) {
+  if (!L.cold) return;
   // the running tile keeps its list on chip and flags it on write-back
   if (L.cur_tile >= 0 && (unsigned)(p.x - L.cx) < (unsigned)L.tile && (unsigned)(p.y - L.cy) < (unsigned)L.tile &&
       (unsigned)(p.z - L.cz) < (unsigned)L.tile)
     return;
-  if (L.inlist[p.i]) return;
-  const int tx = tdiv(L, p.x), ty = tdiv(L, p.y), tz = tdiv(L, p.z);
-  const int t = (tz * L.nty + ty) * L.ntx + tx;
-  L.inlist[p.i] = 1;
-  widen_window(L, tile_colour(tx, ty, tz), tz);
-  const int slot = atomic_add_i32(&L.tl_n[t], 1);
-  if (slot < L.capg) L.tl_idx[(int64_t)t * L.capg + slot] = tile_pack(p.z - tz * L.tile, p.y - ty * L.tile, p.x - tx * L.tile);
-  else *L.list_err = ERR_TILE_LIST;
+  const Lattice &C = *read_here(L.cold);
+  uint8_t *const inlist = as_global(C.inlist);
+  if (inlist[p.i]) return;
+  inlist[p.i] = 1;
+  const int tx = tdiv(C, p.x), ty = tdiv(C, p.y), tz = tdiv(C, p.z);
+  const int t = (tz * C.nty + ty) * C.ntx + tx;
+  widen_window(as_global(C.win), tile_colour(tx, ty, tz), tz);
+  const int slot = atomic_add_i32(as_global(C.tl_n) + t, 1);
+  if (slot < C.capg)
+    as_global(C.tl_idx)[(int64_t)t * C.capg + slot] = tile_pack(p.z - tz * C.tile, p.y - ty * C.tile, p.x - tx * C.tile);
+  else *as_global(C.list_err) = ERR_TILE_LIST;
 }
 
 // ---- rates ---------------------------------------------------------------
@@ -205,6 +252,10 @@ struct TabSrc {
   MSKG_HD double pabs(int i) const { return t.pabs[i]; }
   MSKG_HD double pdes(int i) const { return t.pdes[i]; }
   MSKG_HD double f2(int i) const { return t.f2[i]; }
+  MSKG_HD double ads(int coor) const {
+    return t.pd[3 * (coor - 1)] + t.pd[1 + 3 * (coor - 1)] + t.pd[2 + 3 * (coor - 1)] +
+           (t.pabs[3 * coor] + t.pabs[1 + 3 * coor] + t.pabs[2 + 3 * coor]);
+  }
 };
 // The tables an event reads, 2 KB of LDS a wave: a lookup is the last of an
 // event's chain of dependent reads, and from memory it cost a round trip of
@@ -213,6 +264,7 @@ struct TabSrc {
 constexpr int PE_PLAIN = 192;
 struct TabLds {
   double pe[PE_PLAIN], pd[9], pabs[12], pdes[12], f2[13];
+  double ads[4];  // an adsorption site's rate by coordination (without laser annealing): PTransD + PTransAbs
 };
 template <bool COV>
 struct TabEv {
@@ -223,15 +275,33 @@ struct TabEv {
   MSKG_HD double pabs(int i) const { return l.pabs[i]; }
   MSKG_HD double pdes(int i) const { return l.pdes[i]; }
   MSKG_HD double f2(int i) const { return l.f2[i]; }
+  MSKG_HD double ads(int coor) const { return l.ads[coor]; }
 };
+// The copy in two halves, so that its loads can leave with a tile's first ones.
+struct TabRegs {
+  double pe[PE_PLAIN / 64], rest, ads;
+};
+__device__ inline void fetch_tables(const Tables &t, TabRegs &r, int lane) {
+  for (int k = 0; k < PE_PLAIN / 64; k++) r.pe[k] = t.pe[lane + 64 * k];
+  // pd (9), pabs (12), pdes (12), f2 (13): a lane each
+  const double *src = lane < 9 ? t.pd + lane : (lane < 21 ? t.pabs + (lane - 9) : (lane < 33 ? t.pdes + (lane - 21)
+                                                                                              : t.f2 + min(lane - 33, 12)));
+  r.rest = *src;
+  const int c = min(max(lane, 1), 3);
+  r.ads = TabSrc{t}.ads(c);
+}
+__device__ inline void put_tables(const TabRegs &r, TabLds &l, int lane) {
+  for (int k = 0; k < PE_PLAIN / 64; k++) l.pe[lane + 64 * k] = r.pe[k];
+  if (lane < 9) l.pd[lane] = r.rest;
+  else if (lane < 21) l.pabs[lane - 9] = r.rest;
+  else if (lane < 33) l.pdes[lane - 21] = r.rest;
+  else if (lane < 46) l.f2[lane - 33] = r.rest;
+  if (lane < 4) l.ads[lane] = r.ads;
+}
 __device__ inline void load_tables(const Tables &t, TabLds &l, int lane) {
-  for (int i = lane; i < PE_PLAIN; i += 64) l.pe[i] = t.pe[i];
-  if (lane < 9) l.pd[lane] = t.pd[lane];
-  if (lane < 12) {
-    l.pabs[lane] = t.pabs[lane];
-    l.pdes[lane] = t.pdes[lane];
-  }
-  if (lane < 13) l.f2[lane] = t.f2[lane];
+  TabRegs r;
+  fetch_tables(t, r, lane);
+  put_tables(r, l, lane);
 }
 // The reference's kb (Get_Prob.f:70).
 #define MSKG_KB 0.00008617330350
@@ -319,9 +389,8 @@ MSKG_HD double st_entry(const double *ref, int stride, int idx, const STW &w) {
 // neighbours of species 1..3 (bits 0, 4, 8), walls (12), reciprocal covered
 // neighbours by slot (16, 20, 24), occupied second-neighbour positions (28).
 MSKG_HD uint32_t neighbour_count(int kq, bool lists) {
-  if (kq == KIND_WALL) return 1u << 12;
-  if (!lists || kq == KIND_EMPTY) return 0u;
-  return kq < KIND_WALL ? 1u << (4 * (kq - 1)) : 1u << (16 + 4 * (kq - KIND_COV0));
+  // kinds 1..3, wall and covered 5..7 count at bit 4 (kind - 1)
+  return kq != KIND_EMPTY && (lists || kq == KIND_WALL) ? 1u << ((4 * kq - 4) & 31) : 0u;
 }
 
 // Get_Prob, Get_Prob.f:54-331, evaluated for a point at height z of this
@@ -370,8 +439,10 @@ MSKG_HD void rate_of(const Src &S, const long long *cl, double rtot, int z, int 
     }
     if (coor >= 1 && coor <= 3) {
       if (coor > 1 || c0 >= 2) {
-        double pdep, pabs;
-        if (st) {
+        double pdep = 0.0, pabs = 0.0;
+        if (!LA) {
+          pdep = S.ads(coor);
+        } else if (st) {
           pdep = st_entry(t.st_pd, 9, 3 * (coor - 1), w) + st_entry(t.st_pd, 9, 1 + 3 * (coor - 1), w) +
                  st_entry(t.st_pd, 9, 2 + 3 * (coor - 1), w);
           pabs = COV ? st_entry(t.st_pabs, 12, 3 * coor, w) + st_entry(t.st_pabs, 12, 1 + 3 * coor, w) +
@@ -422,6 +493,11 @@ MSKG_HD void second_vec(int k, int &dx, int &dy, int &dz) {
   dx = g == 2 ? 0 : a;
   dy = g == 0 ? b : (g == 1 ? 0 : a);
   dz = g == 0 ? 0 : b;
+}
+MSKG_HD uint32_t shell_disp(int k) {
+  int dx, dy, dz;
+  second_vec(k, dx, dy, dz);
+  return (uint32_t)(dx & 255) | ((uint32_t)(dy & 255) << 8) | ((uint32_t)(dz & 255) << 16);
 }
 // p shifted by a small vector, with one x/y wrap.
 MSKG_HD P3 shifted(const Lattice &L, const P3 &p, int dx, int dy, int dz) {
@@ -503,9 +579,9 @@ MSKG_HD int pick_itrans(const Lattice &L, const Src &S, int coor, int temp, int 
 // lane a point (each lane walking its point's four neighbours and twelve
 // second neighbours in turn, 13 lanes busy) an event was about 3400
 // instructions; counts are now sums over a quad by DPP, and nothing passes
-// through LDS.  Passes before and after: 8e6 events at 512^3 SiC 92 -> 47 ms,
-// 5e5 events of SiC on 480^3 132 -> 65 ms, 2e5 of CVD on 240x240x760
-// 252 -> 144 ms, k_serial on 64 lattices of 144^3 55.6 -> 26 ms.
+// through LDS.  Passes before and after: 8e6 events at 512^3 SiC 92 -> 42 ms,
+// 5e5 events of SiC on 480^3 132 -> 56 ms, 2e5 of CVD on 240x240x760
+// 252 -> 116 ms, k_serial on 64 lattices of 144^3 55.6 -> 25 ms.
 //
 // The reference visits the neighbours one after the other, but each
 // neighbour's update writes only that neighbour's record and reads only
@@ -516,7 +592,11 @@ MSKG_HD int pick_itrans(const Lattice &L, const Src &S, int coor, int temp, int 
 // is written last; lanes whose gather meets the site take it from registers.
 
 // A site record as it lies in memory (struct Site), in four words.
-typedef uint4 Rec;
+typedef uint32_t Rec __attribute__((ext_vector_type(4)));
+__device__ inline Rec make_rec(uint32_t x, uint32_t y, uint32_t z, uint32_t w) {
+  Rec r = {x, y, z, w};
+  return r;
+}
 __device__ inline int r_kind(const Rec &r) { return r.w & 7; }
 __device__ inline int r_coor(const Rec &r) { return (r.w >> 3) & 7; }
 __device__ inline int r_temp(const Rec &r) { return r.w >> 16; }
@@ -528,6 +608,13 @@ __device__ inline void store_rec(const Lattice &L, int64_t i, const Rec &r) { *(
 __device__ inline uint32_t rec_disp(const Rec &r, int j) {
   const uint32_t lo = j < 2 ? r.x : (j == 2 ? r.y : r.z), hi = j < 2 ? r.y : r.z;
   return __builtin_amdgcn_alignbyte(hi, lo, (4 - j) & 3) & 0xffffffu;
+}
+// The same for an entry known when compiled (scalar shifts for a record in scalar registers).
+template <int J>
+__device__ inline uint32_t rec_disp_at(const Rec &r) {
+  const uint32_t lo = J < 2 ? r.x : (J == 2 ? r.y : r.z), hi = J < 2 ? r.y : r.z;
+  const int sh = J == 0 ? 0 : (J == 1 ? 24 : (J == 2 ? 16 : 8));
+  return (uint32_t)((((uint64_t)hi << 32) | lo) >> sh) & 0xffffffu;
 }
 __device__ inline bool rec_has(const Rec &r, int j) { return (r.w >> (8 + j)) & 1; }
 // The position of a displacement from p (the absolute point (0,0,0) when it is none).
@@ -557,26 +644,30 @@ __device__ inline uint32_t pack_disp(const Box &b, const P3 &p, const P3 &o, boo
   ok = (unsigned)(dx + 128) < 256u && (unsigned)(dy + 128) < 256u && (unsigned)(dz + 128) < 256u;
   return (uint32_t)(dx & 255) | ((uint32_t)(dy & 255) << 8) | ((uint32_t)(dz & 255) << 16);
 }
-// lists_point on a record in registers.
+// The displacement back: minus each byte.
+__device__ inline uint32_t disp_back(uint32_t d) {
+  return ((0x808080u - (d & 0x7f7f7fu)) ^ (~d & 0x808080u)) & 0xffffffu;
+}
+// Does the record list the point at displacement w from it?  An entry that
+// is no displacement holds zero, which w, of another point, is not.
+__device__ inline bool rec_lists_disp(const Rec &r, uint32_t w) {
+  const uint32_t a = rec_disp_at<0>(r) ^ w, b = rec_disp_at<1>(r) ^ w, c = rec_disp_at<2>(r) ^ w,
+                 d = rec_disp_at<3>(r) ^ w;
+  return min(min(a, b), min(c, d)) == 0u;
+}
+// lists_point on a record in registers: the record r of q against the point
+// p, when the displacement between them may not fit the record or p may be
+// the origin (which entries that are no displacement stand for).
 __device__ inline bool rec_lists(const Box &b, const P3 &q, const Rec &r, const P3 &p) {
-  int wx = p.x - q.x, wy = p.y - q.y;
-  const int wz = p.z - q.z;
-  if (wx > b.lx / 2) wx -= b.lx;
-  if (wx < -b.lx / 2) wx += b.lx;
-  if (wy > b.ly / 2) wy -= b.ly;
-  if (wy < -b.ly / 2) wy += b.ly;
-  const bool in8 = (unsigned)(wx + 128) < 256u && (unsigned)(wy + 128) < 256u && (unsigned)(wz + 128) < 256u;
-  const uint32_t w = (uint32_t)(wx & 255) | ((uint32_t)(wy & 255) << 8) | ((uint32_t)(wz & 255) << 16);
-  const uint32_t v = r.w >> 8;
-  bool hit = false;
-  for (int j = 0; j < 4; j++) hit |= ((v >> j) & 1) && rec_disp(r, j) == w;
-  const bool origin = (p.x | p.y | p.z) == 0;
-  return (hit && in8) || (origin && (v & 15u) != 15u);
+  bool has, ok;
+  const uint32_t w = pack_disp(b, q, p, has, ok);
+  return has ? ok && rec_lists_disp(r, w) : ((r.w >> 8) & 15u) != 15u;
 }
 
 // Get_Prob of point p by one thread, from its record: the sweep.  Few of a
 // sweep's points are MC particles, so what counts here is that the branch
-// holds few registers: the second shell is taken four points at a time.
+// holds few registers: the neighbours are taken two at a time, the second
+// shell four.
 template <bool LA, bool COV>
 __device__ inline void get_prob(const Lattice &L, double rtot, const P3 &p, const Rec &r, int &cls, double &rate,
                                 int &err, int &key) {
@@ -590,16 +681,14 @@ __device__ inline void get_prob(const Lattice &L, double rtot, const P3 &p, cons
       c0 = i0 < 0 ? 0 : (L.site[i0].kc >> 3) & 7;
     }
   } else if (kind_species(kind) && p.z >= t.frozen_below_z) {
-    P3 q[4];
-    Rec sq[4];
-    for (int i = 0; i < 4; i++) q[i] = rec_entry(L, r, p, i);
-    for (int i = 0; i < 4; i++) {  // four independent gathers in flight
-      sq[i] = make_uint4(0u, 0u, 0u, 0u);
-      if (q[i].i >= 0) sq[i] = load_rec(L, q[i].i);
-    }
+#pragma unroll 2
     for (int i = 0; i < 4; i++) {
-      const int kq = r_kind(sq[i]);
-      const bool lists = kq != KIND_EMPTY && kq != KIND_WALL && rec_lists(L.box, q[i], sq[i], p);
+      const P3 q = rec_entry(L, r, p, i);
+      Rec sq = make_rec(0u, 0u, 0u, 0u);
+      if (q.i >= 0) sq = load_rec(L, q.i);
+      const int kq = r_kind(sq);
+      const bool lists = kq != KIND_EMPTY && kq != KIND_WALL &&
+                         (rec_has(r, i) ? rec_lists_disp(sq, disp_back(rec_disp(r, i))) : rec_lists(L.box, q, sq, p));
       if (COV && lists && kind_cov_slot(kq) > t.ncov) err = ERR_COVERAGE;
       cnt += neighbour_count(kq, lists);
     }
@@ -645,7 +734,7 @@ __device__ inline void quad_list(Rec &r, uint32_t e, bool has, int j) {
   r.w = (r.w & ~0xff00u) | (quad_or(has ? 1u << j : 0u) << 8);
 }
 __device__ inline Rec uniform_rec(const Rec &r) {
-  return make_uint4((uint32_t)__builtin_amdgcn_readfirstlane((int)r.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)r.y),
+  return make_rec((uint32_t)__builtin_amdgcn_readfirstlane((int)r.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)r.y),
                     (uint32_t)__builtin_amdgcn_readfirstlane((int)r.z), (uint32_t)__builtin_amdgcn_readfirstlane((int)r.w));
 }
 
@@ -671,7 +760,7 @@ struct EvOut {
 __device__ inline void ev_stacking(const Lattice &L, const P3 &s, Rec &S, const Choice &ch, EvOut &o, int lane) {
   const int j = lane & 3;
   const P3 c = rec_entry(L, S, s, 0);
-  Rec cr = make_uint4(0u, 0u, 0u, 0u);
+  Rec cr = make_rec(0u, 0u, 0u, 0u);
   if (c.i >= 0) cr = load_rec(L, c.i);
   // the back bonds' ends: the first three entries of c's list that are not s
   const P3 le = rec_entry(L, cr, c, j);
@@ -710,10 +799,13 @@ __device__ inline void ev_stacking(const Lattice &L, const P3 &s, Rec &S, const 
 // Execute one event of type itrans at site s, whose record is S.  Called by
 // every lane of the wave with the same arguments.
 template <bool LA, bool COV>
-__device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot, const P3 &s, Rec S, int itrans,
+__device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot, const P3 &s_in, Rec S, int itrans,
                                const Choice &ch, EvOut &o, const int lane) {
   const TabEv<COV> T{*L.tab, tabs};
   const Tables &t = T.t;
+  const P3 s = s_in;
+  const bool f2 = t.use_f2 != 0, s_origin = (s.x | s.y | s.z) == 0;
+  const int frozen = t.frozen_below_z;
   const int grp = lane >> 2, j = lane & 3;
   o.p = s;
   o.rate = 0.0f;
@@ -743,35 +835,31 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
     if (o.err) return;
   }
   const int nvisit = COV && itrans == 5 && coor_old == 1 ? 1 : 4;
-  // the quads' points
-  P3 p;
-  {
-    const uint32_t e = rec_disp(S, grp & 3);
-    int dx = (int)(int8_t)e, dy = (int)(int8_t)(e >> 8), dz = (int)(int8_t)(e >> 16);
-    bool has = rec_has(S, grp & 3);
-    if (grp >= 4) {
-      second_vec(grp - 4, dx, dy, dz);
-      has = true;
-    }
-    int x = s.x + dx, y = s.y + dy;
-    const int z = s.z + dz;
-    if (x >= L.box.lx) x -= L.box.lx;
-    if (x < 0) x += L.box.lx;
-    if (y >= L.box.ly) y -= L.box.ly;
-    if (y < 0) y += L.box.ly;
-    p = at(L, has ? x : 0, has ? y : 0, has ? z : 0);
+  // the quads' points, as displacements from the site; an entry that is no
+  // displacement is the origin
+  uint32_t pd = rec_disp(S, grp & 3);
+  bool phas = rec_has(S, grp & 3);
+  if (grp >= 4) {
+    pd = shell_disp(grp - 4);
+    phas = true;
   }
-  // repeated list entries (compared by displacement; the origin is one entry however it is listed)
-  bool seq = false;
-  {
-    const bool org = (p.x | p.y | p.z) == 0;
-    const int kd = p.i < 0 ? -1 - grp : (org ? 1 << 24 : (int)rec_disp(S, grp & 3));
-    int kk[4];
-    for (int i = 0; i < 4; i++) kk[i] = __builtin_amdgcn_readlane(kd, 4 * i);
-    for (int i = 0; i < 4; i++)
-      for (int q = i + 1; q < 4; q++) seq |= q < nvisit && kk[i] == kk[q];
+  const P3 p = disp_point(L, s, pd, phas);
+  // the site's displacement from its point
+  uint32_t to_s = disp_back(pd);
+  if (((S.w >> 8) & 15u) != 15u && !phas) {
+    bool has, ok;
+    to_s = pack_disp(L.box, p, s, has, ok);
+    if (!has || !ok) to_s = 1u << 24;  // no entry is the site
   }
-  const bool shell = t.use_f2 && (dep || evap);
+  // repeated list entries (no displacement: zero)
+  const uint32_t s0 = rec_disp_at<0>(S), s1 = rec_disp_at<1>(S), s2 = rec_disp_at<2>(S), s3 = rec_disp_at<3>(S);
+  const bool twice = nvisit == 4 && ((s0 == s1) | (s0 == s2) | (s0 == s3) | (s1 == s2) | (s1 == s3) | (s2 == s3));
+  // absorption and desorption change no neighbour's record: visits of one
+  // point give it one rate, in whatever order (a covered site of coordination
+  // 1 lists the origin three times)
+  const bool seq = twice && (dep || evap);
+  const bool shell = f2 && (dep || evap);
+  const Rec S_in = S;
   // The rounds: all quads at once; with repeated entries a round for each
   // neighbour and a last one for the second shell; with coverage species and
   // a second shell the neighbours first, since a covered neighbour's new list
@@ -784,30 +872,41 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
 #pragma unroll 1
   for (int round = 0; round <= lead; round++) {
     const bool last = round == lead;
+    // nearly always the only round: nothing of it is to be computed ahead of
+    // the loop for branches that are seldom taken (about 240 instructions)
+    P3 s = s_in;
+    Rec S = S_in;
+    pin(s.x); pin(s.y); pin(s.z); pin(s.i);
+    {
+      uint32_t a = S.x, b = S.y, c = S.z, d = S.w;
+      pin(a); pin(b); pin(c); pin(d);
+      S = make_rec(a, b, c, d);
+    }
     const unsigned nbm = (1u << nvisit) - 1u;
     const unsigned M = (seq ? (last ? 0u : 1u << round) : (round == 0 ? nbm : 0u)) | (last && shell ? 0xfff0u : 0u);
     const bool act = (M >> grp) & 1u;
     const bool nb = act && grp < 4;
-    Rec r = make_uint4(0u, 0u, 0u, 0u);
+    Rec r = make_rec(0u, 0u, 0u, 0u);
     if ((act || (last && lead && grp < 4)) && p.i >= 0) r = load_rec(L, p.i);
     const int kind = r_kind(r), coornn = r_coor(r);
     const bool wall = kind == KIND_WALL, atom = kind_species(kind), empty = !atom && !wall;  // empty or covered
     // this lane's entry of its point's list
-    P3 q = rec_entry(L, r, p, j);
-    const bool back = quad_or(q.x == s.x && q.y == s.y && q.z == s.z ? 1u : 0u) != 0u;  // the list holds the site
+    uint32_t e = rec_disp(r, j);
+    bool ehas = rec_has(r, j);
+    P3 q = disp_point(L, p, e, ehas);
+    // the list holds the site (the site at the origin: an entry that is no displacement)
+    const bool back = quad_or((ehas ? e == to_s : s_origin) ? 1u : 0u) != 0u;
     // what happens to the point
-    bool need = act && grp >= 4 && atom && coornn >= 1 && coornn <= 3;  // a second-shell atom: a fresh rate
-    bool first = false, second = false, erase = false, unfix = false;
+    bool need = act & (grp >= 4) & atom & (coornn >= 1) & (coornn <= 3);  // a second-shell atom: a fresh rate
+    bool first = false, second = false, erase = false, unfix = false, bad = false;
     int inc = 0, cn = coornn;
     if (dep) {  // deposition.f:78-235
-      first = nb && empty && coornn == 0;
-      if (nb && wall) inc = 1;
-      if (nb && ((atom && coornn <= 3 && back) || (empty && (coornn == 2 || coornn == 3) && back))) {
-        cn = coornn + 1;
-        need = true;
-        if (atom && coor_old == 1 && grp >= 1) inc = 1;
-      }
-      if (__ballot(nb && empty && coornn == 1)) {
+      const bool more = nb & back & ((atom & (coornn <= 3)) | (empty & ((coornn & 6) == 2)));
+      first = nb & empty & (coornn == 0);
+      inc = ((nb & wall) | (more & atom & (coor_old == 1) & (grp >= 1))) ? 1 : 0;
+      cn = coornn + ((more | first) ? 1 : 0);
+      need |= more | first;
+      if (__ballot(nb & empty & (coornn == 1))) {
         // a second fixed neighbour: the two others follow when the first is
         // a second neighbour of the site (FIND_NN.f, a lane each)
         const int ax = quad_take<0>(q.x), ay = quad_take<0>(q.y), az = quad_take<0>(q.z);
@@ -819,6 +918,8 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
         dy = dy < L.box.ly - dy ? dy : L.box.ly - dy;
         second = nb && empty && coornn == 1 && dx * dx + dy * dy + dz * dz == 72;
         if (second) {
+          cn = 2;
+          need = true;
           if (j == 1) q = s;
           if (j >= 2) {
             const int a1[3] = {ax, ay, az}, a2[3] = {s.x, s.y, s.z}, pc[3] = {p.x, p.y, p.z};
@@ -826,82 +927,83 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
             find_nn_one(*L.geo, L.box.lx, L.box.ly, a1, a2, pc, j - 2, ns);
             q = at(L, ns[0], ns[1], ns[2]);
           }
+          bool ok;
+          e = pack_disp(L.box, p, q, ehas, ok);
+          bad = !ok;
         }
       }
       if (first) {  // its list starts with the site
+        ehas = j == 0 && !s_origin;
+        e = ehas ? to_s & 0xffffffu : 0u;
+        bad = to_s >> 24 && !s_origin;
         q = s;
-        if (j > 0) { q.x = q.y = q.z = 0; q.i = 0; }
-        cn = 1;
-        need = true;
-      }
-      if (second) {
-        cn = 2;
-        need = true;
       }
     } else if (evap) {  // Evaporation.f:36-208
-      if (nb && wall) inc = -1;
-      if (nb && !wall && (atom || coornn >= 1) && coornn <= (atom ? 7 : 4) && back) {
-        if (empty && coornn == 1) {
-          erase = true;  // EraseMC + LattCoo=0, keeping the temperature bits
-        } else {
-          unfix = empty && coornn == 2;  // the list keeps the reciprocal partner (NBuff)
-          cn = coornn - 1;  // coordination 4 -> 3 is EraseBulk/EraseVoid + AddMC
-          need = true;
-        }
-      }
+      const bool hit = nb & back & (atom | (empty & (coornn >= 1) & (coornn <= 4)));
+      inc = (nb & wall) ? -1 : 0;
+      erase = hit & empty & (coornn == 1);  // EraseMC + LattCoo=0, keeping the temperature bits
+      need |= hit & !erase;
+      unfix = hit & empty & (coornn == 2);  // the list keeps the reciprocal partner (NBuff)
+      cn = coornn - ((hit & !erase) ? 1 : 0);  // coordination 4 -> 3 is EraseBulk/EraseVoid + AddMC
     } else if (COV) {  // an atom bonded back to the site (absorption.f:45-60, desorption.f:45-105)
-      need |= nb && atom && (!absorb || coornn <= 3) && back;
+      need |= nb & atom & (!absorb | (coornn <= 3)) & back;
     }
     // the listed neighbours' records (the rate of an unfixed point comes from
     // its old list, Evaporation.f:121)
-    const bool count = need && atom && p.z >= t.frozen_below_z;
-    const bool look = count || unfix || (second && j >= 2) || (need && empty && cn == 1 && j == 0);
-    Rec er = make_uint4(0u, 0u, 0u, 0u);
+    const bool count = need & atom & (p.z >= frozen);
+    const bool look = count | unfix | (second & (j >= 2)) | (need & empty & (cn == 1) & (j == 0));
+    Rec er = make_rec(0u, 0u, 0u, 0u);
     uint32_t k2 = 0;
-    if (look && q.i == s.i) er = S;
-    else if (look && q.i >= 0) er = load_rec(L, q.i);
-    if (t.use_f2 && count) {
+    if (look && q.i >= 0) er = load_rec(L, q.i);
+    if (f2 && count) {
       // four second neighbours a lane in three steps; at least 6 units from
       // every face they are at fixed index steps
       const int a = (j & 2) ? -6 : 6, b = (j & 1) ? -6 : 6;
       const Box &B = L.box;
-      int64_t i2[3];
-      if (p.x >= 6 && p.x < B.lx - 6 && p.y >= 6 && p.y < B.ly - 6 && p.z >= 6 && p.z <= B.lz - 6) {
-        i2[0] = p.i + (a / 2 + (b / 2) * B.hx);
-        i2[1] = p.i + (b * B.plane + a / 2);
-        i2[2] = p.i + (b * B.plane + (a / 2) * B.hx);
+      int64_t i0, i1, i2;
+      const bool inner = ((unsigned)(p.x - 6) < (unsigned)(B.lx - 12)) & ((unsigned)(p.y - 6) < (unsigned)(B.ly - 12)) &
+                         ((unsigned)(p.z - 6) <= (unsigned)(B.lz - 12));
+      if (inner) {
+        i0 = p.i + (a / 2 + (b / 2) * B.hx);
+        i1 = p.i + (b * B.plane + a / 2);
+        i2 = p.i + (b * B.plane + (a / 2) * B.hx);
       } else {
-        i2[0] = shifted(L, p, a, b, 0).i;
-        i2[1] = shifted(L, p, a, 0, b).i;
-        i2[2] = shifted(L, p, 0, a, b).i;
+        i0 = shifted(L, p, a, b, 0).i;
+        i1 = shifted(L, p, a, 0, b).i;
+        i2 = shifted(L, p, 0, a, b).i;
       }
-      for (int k = 0; k < 3; k++) {
-        int kq = i2[k] < 0 ? 0 : L.site[i2[k]].kc & 7;
-        if (i2[k] == s.i) kq = new_kind;
-        k2 += kind_species(kq) ? 1u << 28 : 0u;
-      }
+      int k0 = 0, k1 = 0, kk = 0;
+      if (i0 >= 0) k0 = L.site[i0].kc & 7;
+      if (i1 >= 0) k1 = L.site[i1].kc & 7;
+      if (i2 >= 0) kk = L.site[i2].kc & 7;
+      k0 = i0 == s.i ? new_kind : k0;
+      k1 = i1 == s.i ? new_kind : k1;
+      kk = i2 == s.i ? new_kind : kk;
+      k2 = ((uint32_t)kind_species(k0) + (uint32_t)kind_species(k1) + (uint32_t)kind_species(kk)) << 28;
     }
+    if (q.i == s.i) er = S;
     const int kq = r_kind(er);
-    const bool lists = look && kq != KIND_EMPTY && kq != KIND_WALL && rec_lists(L.box, q, er, p);
+    bool lists = rec_lists_disp(er, disp_back(e));
+    if (__ballot(look & !ehas & (kq != KIND_EMPTY)) && look && !ehas) lists = rec_lists(L.box, q, er, p);
+    lists &= look & (kq != KIND_EMPTY) & (kq != KIND_WALL);
     int err = ERR_NONE;
-    if (COV && count && lists && kind_cov_slot(kq) > t.ncov) err = ERR_COVERAGE;
-    if (COV && quad_or(err != ERR_NONE ? 1u : 0u)) err = ERR_COVERAGE;
+    if (COV) {
+      if (quad_or((count & lists & (kind_cov_slot(kq) > t.ncov)) ? 1u : 0u)) err = ERR_COVERAGE;
+    }
     uint32_t cnt = quad_sum((count ? neighbour_count(kq, lists) : 0u) + k2);
-    const bool partner = lists && kind_species(kq) && r_coor(er) <= 3;
+    const bool partner = lists & kind_species(kq) & (r_coor(er) <= 3);
     const unsigned pm = quad_or(partner ? 1u << j : 0u);  // reciprocal partners by entry
     const int c0 = quad_take<0>(r_coor(er));
     if (second) cn += __popc(pm >> 2);
     // the point's new record
     Rec nr = r;
     nr.w = w_coor(r.w, cn);
-    if (erase) nr = make_uint4(0u, 0u, 0u, r.w & 0xffff0000u);
-    if (__ballot(first || second)) {
-      bool has, ok;
+    if (erase) nr = make_rec(0u, 0u, 0u, r.w & 0xffff0000u);
+    if (__ballot(first | second)) {
       Rec lr = nr;
-      const uint32_t d = pack_disp(L.box, p, q, has, ok);
-      const bool bad = quad_or(ok ? 0u : 1u) != 0u;
-      quad_list(lr, d, has, j);
-      if (first || second) {
+      bad = quad_or(bad ? 1u : 0u) != 0u;
+      quad_list(lr, e, ehas, j);
+      if (first | second) {
         if (bad) {
           err = ERR_GEOM;
           need = false;
@@ -914,18 +1016,21 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
     const unsigned um = (unsigned)((__ballot(unfix) >> 1) & 0x1111ull);  // unfixed neighbours, bit 4 i
     if (um) {
       const int jb = pm ? 31 - __clz((int)pm) : 0;  // the last partner
-      const P3 pp = rec_entry(L, r, p, jb);
+      const uint32_t pe = rec_disp(r, jb);
       if (unfix) {  // one entry; none for no partner, or a partner at the origin
-        const bool keep = pm && (pp.x | pp.y | pp.z) != 0;
-        nr.x = keep ? rec_disp(r, jb) : 0u;
+        const bool keep = pm != 0u && rec_has(r, jb);
+        nr.x = keep ? pe : 0u;
         nr.y = nr.z = 0u;
         nr.w = (nr.w & ~0xff00u) | (keep ? 0x100u : 0u);
       }
       // NBuff over the neighbours in order: one that found no partner gets
-      // the last one found before it (or the initial (0,0,0): none)
-      for (int i = 0; i < 4; i++) {
+      // the last one found before it (or the initial (0,0,0): none).  Every
+      // neighbour with a partner needs only the last such.
+      const unsigned fm = um & (unsigned)(__ballot(pm != 0u) >> 1);
+      const P3 pp = disp_point(L, p, pe, rec_has(r, jb));
+      for (int i = fm == um ? (31 - __clz((int)um)) >> 2 : 0; i < 4; i++) {
         if (!((um >> (4 * i)) & 1u)) continue;
-        if (__builtin_amdgcn_readlane((int)pm, 4 * i + 1)) {
+        if ((fm >> (4 * i)) & 1u) {
           nbuff.x = __builtin_amdgcn_readlane(pp.x, 4 * i + 1);
           nbuff.y = __builtin_amdgcn_readlane(pp.y, 4 * i + 1);
           nbuff.z = __builtin_amdgcn_readlane(pp.z, 4 * i + 1);
@@ -953,13 +1058,14 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
       const bool rem = evap && coor == 0;  // EraseMC zeroes the record
       uint32_t scnt = 0;
       if (dep || (evap && coor == 1)) {
-        const bool sl = sn && fk != KIND_EMPTY && fk != KIND_WALL && rec_lists(L.box, p, nr, s);
+        bool sl = s_origin ? ((nr.w >> 8) & 15u) != 15u : rec_lists_disp(nr, to_s);
+        sl &= sn & (fk != KIND_EMPTY) & (fk != KIND_WALL);
         if (dep) {
           const uint32_t c1 = sn ? neighbour_count(fk, sl) : 0u;
           if (COV && __ballot(sl && kind_cov_slot(fk) > t.ncov)) { if (lane == 0) err = ERR_COVERAGE; }
           scnt = (uint32_t)(__builtin_amdgcn_readlane((int)c1, 1) + __builtin_amdgcn_readlane((int)c1, 5) +
                             __builtin_amdgcn_readlane((int)c1, 9) + __builtin_amdgcn_readlane((int)c1, 13));
-          if (t.use_f2) scnt += (uint32_t)__popcll(__ballot(lane >= 16 && j == 1 && atom)) << 28;
+          if (f2) scnt += (uint32_t)__popcll(__ballot(lane >= 16 && j == 1 && atom)) << 28;
         } else {  // the site keeps one reciprocal bond (NBuff)
           const unsigned long long sp = __ballot(sl && kind_species(fk) && fc <= 3);
           if (sp) {
@@ -972,7 +1078,7 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
       }
       const uint32_t old_w = S.w;
       S.w = w_coor(S.w, coor);
-      if (rem) S = make_uint4(0u, 0u, 0u, S.w & 0xffff0000u);
+      if (rem) S = make_rec(0u, 0u, 0u, S.w & 0xffff0000u);
       const int sc0 = __builtin_amdgcn_readlane(fc, 1);
       if (lane == 0) {
         ek = new_kind;
@@ -989,7 +1095,7 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
       if (evap && coor == 1) {
         bool has, ok;
         const uint32_t d = pack_disp(L.box, s, nbuff, has, ok);
-        if (ok) S = make_uint4(d, 0u, 0u, (S.w & ~0xff00u) | (has ? 0x100u : 0u));
+        if (ok) S = make_rec(d, 0u, 0u, (S.w & ~0xff00u) | (has ? 0x100u : 0u));
         else if (lane == 0) err = ERR_GEOM;
       }
       if (lane == 0) nr = S;
@@ -1016,7 +1122,7 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
       o.p = sp;
       o.rate = rf;
       o.cls = cls;
-      o.set = seq && lane != 0 && grp < 4 ? 2 : 1;
+      o.set = twice && lane != 0 && grp < 4 ? 2 : 1;
     }
     if (!last) __threadfence_block();  // the next round reads this one's records
   }

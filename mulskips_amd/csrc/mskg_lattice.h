@@ -140,8 +140,9 @@ MSKG_HD void pxyz(const Box &b, int64_t p, int &x, int &y, int &z) {
 // the lattice parity (the reference reads outside LattCoo for z<0; the CPU
 // oracle and this engine both read such points as zero records).
 MSKG_HD int64_t pidx_checked(const Box &b, int x, int y, int z) {
-  if (x < 0 || x >= b.lx || y < 0 || y >= b.ly || z < 0 || z > b.lz || !valid_parity(x, y, z)) return -1;
-  return pidx(b, x, y, z);
+  const bool ok = ((unsigned)x < (unsigned)b.lx) & ((unsigned)y < (unsigned)b.ly) & ((unsigned)z <= (unsigned)b.lz) &
+                  ((((x ^ y) | (x ^ z)) & 1) == 0);
+  return ok ? pidx(b, x, y, z) : -1;
 }
 
 // Absolute position of entry i of a site at (x,y,z), with the reference's
