@@ -94,6 +94,7 @@ struct RunState {
   unsigned long long desorbed[3];  // desorptions by coverage slot (CountCov)
   int final_sweep;                 // the window was shortened to end at max_time
   unsigned long long guard_exits;  // tile windows cut short by the per-window event cap
+  int ever_lo, ever_hi;            // the first / last tile layer any of the run's sweeps could visit
   // the sweep's working sums, last: the host reads and writes only the
   // fields before them (RS_HEAD bytes)
   Slot slot[NSLOT];
@@ -1111,6 +1112,8 @@ __device__ inline void sweep_end(RunState *st, int *win, const int *list_err, un
     zlo = min(zlo, win[4 * c]);
     zhi = max(zhi, win[4 * c + 1]);
   }
+  st->ever_lo = min(st->ever_lo, zlo);
+  st->ever_hi = max(st->ever_hi, zhi);
   // the dependency-scheduled sweep: a new stamp, an empty queue, the window
   sched[0]++;
   sched[1] = 0u;
@@ -2034,42 +2037,26 @@ __global__ void __launch_bounds__(256) k_key_hist(Lattice L, int *cnt, double *i
 //     are flipped to the other species; code = the species as flipped.
 //     k_wrong_mark marks those flips (bit 7 of the record's `valid` byte,
 //     which the neighbour lists leave unused) and clears the marks after.
-// Each block owns a contiguous chunk of points; k_frame_count counts,
-// the host scans, k_frame_write writes in order with a block-wide prefix
-// scan.
+// Each wave owns a contiguous segment of points: k_frame_count counts it and
+// leaves a bit a point for the points that have a record, k_frame_scan turns
+// the counts into offsets, k_frame_write writes in order.
+//
+// What bounds it: the records' bytes, read once, by the count; the write
+// reads a bit a point and the records of the few points that have one.  A
+// lattice a slab builder made and runs have changed since is read only over
+// the planes those runs could have touched (touched_planes).  With every
+// stored plane read by the count and again by the write, 65536 points a block
+// whatever the lattice, and a sizing call before each frame, a whole pass
+// (build, run, frames) took 63.6 ms at 512^3 SiC, now 52.4; Si PVD 768^2 x
+// 1536 53.0, now 50.5; 24 SiGe replicas 54.8, now 36.1; the smallest box 8.7,
+// now 8.2.
 constexpr int FRAME_THREADS = 256;
+constexpr int FRAME_GROUPS = 64;  // groups of 64 points a wave takes at a time: a lane's bits each
 enum : int { FRAME_MAIN = 0, FRAME_DEFECTS = 1 };
 template <int MODE> struct FrameShape;
 template <> struct FrameShape<FRAME_MAIN> { static constexpr int NLIST = 3, NCNT = 5; };
 template <> struct FrameShape<FRAME_DEFECTS> { static constexpr int NLIST = 2, NCNT = 2; };
 constexpr uint8_t WRONG_FLIP = 0x80;
-
-__device__ inline int frame_cat(const Lattice &L, int64_t p, const Site &sp, int *code, bool hdr[2]) {
-  int x, y, z;
-  pxyz(L.box, p, x, y, z);
-  hdr[0] = hdr[1] = false;
-  const int kind = s_kind(sp), coor = s_coor(sp);
-  if (kind == KIND_WALL || z > L.box.lz - 1) return -1;
-  const bool inner = z >= 1;
-  if (kind_species(kind)) {
-    if (coor <= 3) {
-      *code = kind;
-      hdr[0] = inner;
-      return 0;
-    }
-    if (!dia_type(x, y, z)) {
-      *code = kind;
-      return 2;
-    }
-    return -1;
-  }
-  if (kind_cov_slot(kind)) {
-    *code = -kind_cov_slot(kind);  // coverage slot, negated; the host maps it to ListCov
-    hdr[1] = inner;
-    return coor == 4 ? 1 : 0;
-  }
-  return coor == 4 ? 1 : -1;  // an empty point with coordination 4 is a vacancy
-}
 
 // Species of a record as the _w analysis sees it: the wrong-site flip swaps
 // Si (1) and C (2).
@@ -2094,34 +2081,38 @@ __device__ inline int wrong_corr(const Lattice &L, const P3 &pt, const Site &sp,
   return corr;
 }
 
-// Membership of point p in the lists of a frame, the code per list and the
-// header counts.
+// Membership of point p, whose record's last word is w, in the lists of a
+// frame, the code per list and the header counts.
 template <int MODE>
-__device__ inline void frame_point(const Lattice &L, int64_t p, const Site &sp, int sic, bool in[],
-                                   int code[], unsigned long long cnt[]) {
+__device__ inline void frame_point(const Lattice &L, int64_t p, uint32_t w, int sic, bool in[], int code[],
+                                   unsigned int cnt[]) {
+  const int kind = w & 7, coor = (w >> 3) & 7;
+  for (int k = 0; k < FrameShape<MODE>::NLIST; k++) {
+    in[k] = false;
+    code[k] = 0;
+  }
+  const bool atom = kind_species(kind), covered = kind >= KIND_COV0;
+  const bool below = p < L.box.plane * L.box.lz;  // z <= LenZ-1
   if (MODE == FRAME_MAIN) {
-    int c = 0;
-    bool hdr[2];
-    const int cat = frame_cat(L, p, sp, &c, hdr);
-    in[0] = cat == 0 || (cat == 1 && c < 0);  // a covered vacancy is also listed in the main frame
-    in[1] = cat == 1;
-    in[2] = cat == 2;
-    code[0] = code[2] = c;
-    code[1] = 0;
-    for (int k = 0; k < 3; k++) cnt[k] += in[k];
-    cnt[3] += hdr[0];
-    cnt[4] += hdr[1];
-  } else {
-    in[0] = in[1] = false;
-    code[0] = code[1] = 0;
-    const int kind = s_kind(sp), coor = s_coor(sp);
-    if (kind == KIND_WALL || coor != 4) return;
+    if (!below) return;
+    const bool inner = p >= L.box.plane;  // z >= 1
+    in[0] = covered || (atom && coor <= 3);  // a covered vacancy is also listed in the main frame
+    in[1] = coor == 4 && (covered || kind == KIND_EMPTY);
+    if (atom && coor > 3) {
+      int x, y, z;
+      pxyz(L.box, p, x, y, z);
+      in[2] = !dia_type(x, y, z);
+    }
+    code[0] = covered ? -kind_cov_slot(kind) : kind;  // the host maps a coverage slot to ListCov
+    code[2] = kind;
+    cnt[3] += in[0] && atom && inner;
+    cnt[4] += covered && inner;
+  } else if (below && coor == 4 && kind != KIND_WALL) {
     P3 pt;
     pt.i = p;
     pxyz(L.box, p, pt.x, pt.y, pt.z);
-    if (pt.z > L.box.lz - 1) return;
-    if (kind == KIND_EMPTY || kind >= KIND_COV0) {  // a vacancy: the species sum of its neighbours
-      const NL l = list_of(L, pt, sp);
+    if (!atom) {  // a vacancy: the species sum of its neighbours
+      const NL l = list_of(L, pt, L.site[p]);
       int sum = 0;
       for (int i = 0; i < 4; i++) {
         const int kq = s_kind(rd(L, entry(L, l, i).i));
@@ -2129,13 +2120,39 @@ __device__ inline void frame_point(const Lattice &L, int64_t p, const Site &sp, 
       }
       in[0] = true;
       code[0] = sum;
-    } else if (sic && kind_species(kind) && pt.z >= 1 && wrong_corr(L, pt, sp, true) == 3) {
-      in[1] = true;
+    } else if (sic && pt.z >= 1) {
+      const Site sp = L.site[p];
+      in[1] = wrong_corr(L, pt, sp, true) == 3;
       code[1] = flipped_species(sp);
     }
-    cnt[0] += in[0];
-    cnt[1] += in[1];
   }
+  for (int k = 0; k < FrameShape<MODE>::NLIST; k++) cnt[k] += in[k];
+}
+
+// The groups of 64 points from g0 (at most FRAME_GROUPS of them, below end):
+// lane g gets the bits of group g's points that are in a list; cnt counts.
+// Four records' words in flight a lane.
+template <int MODE>
+__device__ inline unsigned long long frame_bits(const Lattice &L, int64_t g0, int64_t end, int groups, int sic,
+                                                unsigned int cnt[], int lane) {
+  unsigned long long mine = 0ull;
+  for (int g = 0; g < groups && g0 + g * WAVE < end; g += 4) {
+    uint32_t w[4];
+    for (int u = 0; u < 4; u++) {
+      const int64_t p = g0 + (int64_t)(g + u) * WAVE + lane;
+      w[u] = g + u < groups && p < end ? ((const uint32_t *)(L.site + p))[3] : (uint32_t)KIND_WALL;  // no list holds a wall
+    }
+    for (int u = 0; u < 4; u++) {
+      bool in[FrameShape<MODE>::NLIST];
+      int code[FrameShape<MODE>::NLIST];
+      frame_point<MODE>(L, g0 + (int64_t)(g + u) * WAVE + lane, w[u], sic, in, code, cnt);
+      bool any = false;
+      for (int k = 0; k < FrameShape<MODE>::NLIST; k++) any |= in[k];
+      const unsigned long long m = __ballot(any);
+      if (lane == g + u) mine = m;
+    }
+  }
+  return mine;
 }
 
 // The isolated wrong atoms of the SiC analysis (WriteMolMolXYZFile.f:269-299).
@@ -2147,12 +2164,14 @@ __device__ inline void frame_point(const Lattice &L, int64_t p, const Site &sp, 
 // candidate neighbour before it in grid order flips: the candidates are few,
 // k_wrong_cand lists them with their neighbours, the host resolves that
 // order, and k_wrong_set marks (or unmarks) the flips.
-__global__ void __launch_bounds__(256) k_wrong_cand(Lattice L, int64_t cap, unsigned long long *n, int4 *out) {
-  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < L.box.npts;
+__global__ void __launch_bounds__(256) k_wrong_cand(Lattice L, int64_t first, int64_t end, int64_t cap,
+                                                    unsigned long long *n, int4 *out) {
+  for (int64_t p = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < end;
        p += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t w = ((const uint32_t *)(L.site + p))[3];
+    const int kind = w & 7;
+    if (!(kind == 1 || kind == 2) || ((w >> 3) & 7) != 4) continue;
     const Site sp = L.site[p];
-    const int kind = s_kind(sp);
-    if (!(kind == 1 || kind == 2) || s_coor(sp) != 4) continue;
     P3 pt;
     pt.i = p;
     pxyz(L.box, p, pt.x, pt.y, pt.z);
@@ -2172,122 +2191,142 @@ __global__ void __launch_bounds__(256) k_wrong_set(Lattice L, const int4 *pos, i
   }
 }
 
+// The points of a frame's kernels and how its waves share them: segment i is
+// the points [first + i * rounds * groups * 64, ...) below end, `rounds`
+// times `groups` groups of 64 points.
+struct FramePlan {
+  int64_t first, end;
+  int groups, rounds;
+  int nseg;
+  int sic;
+};
+
+// counts: [NCNT][nseg]; bits: a word a group of 64 points, null: not kept.
 template <int MODE>
-__global__ void __launch_bounds__(FRAME_THREADS) k_frame_count(Lattice L, int64_t chunk, int sic,
-                                                               unsigned long long *counts) {
-  constexpr int NL_ = FrameShape<MODE>::NLIST, NC = FrameShape<MODE>::NCNT;
-  __shared__ unsigned long long sc[NC][FRAME_THREADS / WAVE];
-  const int64_t lo = (int64_t)blockIdx.x * chunk, hi = min(lo + chunk, L.box.npts);
-  unsigned long long c[NC];
-  for (int k = 0; k < NC; k++) c[k] = 0;
-  for (int64_t p = lo + threadIdx.x; p < hi; p += FRAME_THREADS) {
-    bool in[NL_];
-    int code[NL_];
-    frame_point<MODE>(L, p, L.site[p], sic, in, code, c);
+__global__ void __launch_bounds__(FRAME_THREADS) k_frame_count(Lattice L, FramePlan F, uint32_t *counts,
+                                                               unsigned long long *bits) {
+  constexpr int NC = FrameShape<MODE>::NCNT;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int seg = blockIdx.x * (FRAME_THREADS / WAVE) + threadIdx.x / WAVE;
+  if (seg >= F.nseg) return;
+  unsigned int c[NC];
+  for (int k = 0; k < NC; k++) c[k] = 0u;
+  for (int r = 0; r < F.rounds; r++) {
+    const int64_t grp = ((int64_t)seg * F.rounds + r) * F.groups, g0 = F.first + grp * WAVE;
+    if (g0 >= F.end) break;
+    const unsigned long long mine = frame_bits<MODE>(L, g0, F.end, F.groups, F.sic, c, lane);
+    if (bits && lane < F.groups && g0 + (int64_t)lane * WAVE < F.end) bits[grp + lane] = mine;
   }
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
   for (int k = 0; k < NC; k++) {
-    unsigned long long v = c[k];
+    unsigned int v = c[k];
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-    if (lane == 0) sc[k][w] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < NC) {
-    unsigned long long v = 0;
-    for (int q = 0; q < FRAME_THREADS / WAVE; q++) v += sc[threadIdx.x][q];
-    counts[(int64_t)blockIdx.x * NC + threadIdx.x] = v;
+    if (lane == 0) counts[(int64_t)k * F.nseg + seg] = v;
   }
 }
 
+// The lanes' groups are taken a lane each: a lane reads its group's listed
+// points one after the other, once to count them by list and once to write.
 template <int MODE>
-__global__ void __launch_bounds__(FRAME_THREADS) k_frame_write(Lattice L, int64_t chunk, int sic,
+__global__ void __launch_bounds__(FRAME_THREADS) k_frame_write(Lattice L, FramePlan F, const unsigned long long *bits,
                                                                const unsigned long long *offs, int4 *out0,
                                                                int4 *out1, int4 *out2, int64_t cap0, int64_t cap1,
                                                                int64_t cap2) {
   constexpr int NL_ = FrameShape<MODE>::NLIST, NC = FrameShape<MODE>::NCNT;
-  __shared__ unsigned int wsum[NL_][FRAME_THREADS / WAVE];
-  const int64_t lo = (int64_t)blockIdx.x * chunk, hi = min(lo + chunk, L.box.npts);
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int seg = blockIdx.x * (FRAME_THREADS / WAVE) + threadIdx.x / WAVE;
+  if (seg >= F.nseg) return;
   unsigned long long base[NL_];
-  for (int k = 0; k < NL_; k++) base[k] = offs[(int64_t)blockIdx.x * NL_ + k];
+  for (int k = 0; k < NL_; k++) base[k] = offs[(int64_t)k * F.nseg + seg];
   int4 *const outs[3] = {out0, out1, out2};
   const unsigned long long caps[3] = {(unsigned long long)cap0, (unsigned long long)cap1, (unsigned long long)cap2};
-  for (int64_t p0 = lo; p0 < hi; p0 += FRAME_THREADS) {
-    const int64_t p = p0 + threadIdx.x;
+  for (int r = 0; r < F.rounds; r++) {
+    const int64_t grp = ((int64_t)seg * F.rounds + r) * F.groups, g0 = F.first + grp * WAVE;
+    if (g0 >= F.end) break;
+    unsigned long long mine = 0ull;
+    unsigned int dummy[NC];
+    for (int k = 0; k < NC; k++) dummy[k] = 0u;
+    if (!bits) mine = frame_bits<MODE>(L, g0, F.end, F.groups, F.sic, dummy, lane);
+    else if (lane < F.groups && g0 + (int64_t)lane * WAVE < F.end) mine = bits[grp + lane];
+    if (!__ballot(mine != 0ull)) continue;
+    const int64_t pl = g0 + (int64_t)lane * WAVE;
     bool in[NL_];
     int code[NL_];
-    unsigned long long cdummy[NC];
-    for (int k = 0; k < NL_; k++) in[k] = false;
-    if (p < hi) frame_point<MODE>(L, p, L.site[p], sic, in, code, cdummy);
-    int x = 0, y = 0, z = 0;
-    bool any = false;
-    for (int k = 0; k < NL_; k++) any |= in[k];
-    if (any) pxyz(L.box, p, x, y, z);
-    unsigned int rank[NL_];
-    for (int k = 0; k < NL_; k++) {
-      const unsigned long long m = __ballot(in[k]);
-      rank[k] = __popcll(m & ((1ull << lane) - 1ull));
-      if (lane == 0) wsum[k][w] = __popcll(m);
+    unsigned int n[NC];
+    for (int k = 0; k < NC; k++) n[k] = 0u;
+    for (unsigned long long m = mine; m; m &= m - 1ull) {
+      const int64_t p = pl + __ffsll((long long)m) - 1;
+      frame_point<MODE>(L, p, ((const uint32_t *)(L.site + p))[3], F.sic, in, code, n);
     }
-    __syncthreads();
+    unsigned long long at[NL_];
     for (int k = 0; k < NL_; k++) {
-      unsigned int before = 0, total = 0;
-      for (int q = 0; q < FRAME_THREADS / WAVE; q++) {
-        if (q < w) before += wsum[k][q];
-        total += wsum[k][q];
+      unsigned int inc = n[k];
+      for (int off = 1; off < WAVE; off <<= 1) {
+        const unsigned int t = __shfl_up(inc, off, WAVE);
+        if (lane >= off) inc += t;
       }
-      const unsigned long long at = base[k] + before + rank[k];
-      if (in[k] && at < caps[k]) outs[k][at] = make_int4(x, y, z, code[k]);
-      base[k] += total;
+      at[k] = base[k] + inc - n[k];
+      base[k] += __shfl(inc, WAVE - 1, WAVE);
     }
-    __syncthreads();
+    for (unsigned long long m = mine; m; m &= m - 1ull) {
+      const int64_t p = pl + __ffsll((long long)m) - 1;
+      frame_point<MODE>(L, p, ((const uint32_t *)(L.site + p))[3], F.sic, in, code, dummy);
+      int x, y, z;
+      pxyz(L.box, p, x, y, z);
+      for (int k = 0; k < NL_; k++)
+        if (in[k]) {
+          if (at[k] < caps[k]) outs[k][at[k]] = make_int4(x, y, z, code[k]);
+          at[k]++;
+        }
+    }
   }
 }
 
-// The block offsets of a frame from the block counts, on the device: one
-// block scans the counts of every list in order and writes the offsets and
-// the totals (NCNT of them).
+// The segments' offsets of a frame from their counts, and the totals (NCNT
+// of them): a block a count, which scans its segments 4096 at a time.
+constexpr int SCAN_THREADS = 1024;
 template <int MODE>
-__global__ void __launch_bounds__(256) k_frame_scan(const unsigned long long *counts, int nblk,
-                                                    unsigned long long *offs, int64_t *totals) {
-  constexpr int NL_ = FrameShape<MODE>::NLIST, NC = FrameShape<MODE>::NCNT;
-  __shared__ unsigned long long part[256];
-  for (int k = 0; k < NC; k++) {
-    // each thread sums a contiguous run of blocks, then the runs are scanned
-    const int per = (nblk + 255) / 256;
-    const int lo = min((int)threadIdx.x * per, nblk), hi = min(lo + per, nblk);
-    unsigned long long s = 0;
-    for (int b = lo; b < hi; b++) s += counts[(int64_t)b * NC + k];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned long long acc = 0;
-      for (int q = 0; q < 256; q++) {
-        const unsigned long long v = part[q];
-        part[q] = acc;
-        acc += v;
-      }
-      totals[k] = (int64_t)acc;
+__global__ void __launch_bounds__(SCAN_THREADS) k_frame_scan(const uint32_t *counts, int nseg,
+                                                             unsigned long long *offs, int64_t *totals) {
+  __shared__ unsigned long long wsum[SCAN_THREADS / WAVE];
+  const int k = blockIdx.x, lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const uint32_t *const c = counts + (int64_t)k * nseg;
+  unsigned long long *const o = k < FrameShape<MODE>::NLIST ? offs + (int64_t)k * nseg : nullptr;
+  unsigned long long base = 0ull;
+  for (int s0 = 0; s0 < nseg; s0 += 4 * SCAN_THREADS) {
+    const int i0 = s0 + 4 * (int)threadIdx.x;
+    uint32_t v[4];
+    for (int u = 0; u < 4; u++) v[u] = i0 + u < nseg ? c[i0 + u] : 0u;
+    const unsigned long long mine = (unsigned long long)v[0] + v[1] + v[2] + v[3];
+    unsigned long long inc = mine;
+    for (int off = 1; off < WAVE; off <<= 1) {
+      const unsigned long long t = __shfl_up(inc, off, WAVE);
+      if (lane >= off) inc += t;
     }
+    if (lane == WAVE - 1) wsum[w] = inc;
     __syncthreads();
-    if (k < NL_) {
-      unsigned long long acc = part[threadIdx.x];
-      for (int b = lo; b < hi; b++) {
-        offs[(int64_t)b * NL_ + k] = acc;
-        acc += counts[(int64_t)b * NC + k];
-      }
+    unsigned long long before = base, all = 0ull;
+    for (int q = 0; q < SCAN_THREADS / WAVE; q++) {
+      if (q < w) before += wsum[q];
+      all += wsum[q];
     }
+    unsigned long long at = before + inc - mine;
+    for (int u = 0; u < 4; u++) {
+      if (o && i0 + u < nseg) o[i0 + u] = at;
+      at += v[u];
+    }
+    base += all;
     __syncthreads();
   }
+  if (threadIdx.x == 0) totals[k] = (int64_t)base;
 }
 
 // Scratch of the allocation-free frame entry point (mskg_frame_device): the
-// block counts (5 per block) and offsets (3 per block) of one frame.  Every
+// counts (5 a segment, 32 bits) and offsets (3 a segment) of one frame.  Every
 // GPU the library runs on holds its own copy until the process ends; host
 // code reaches it only through the address hipGetSymbolAddress gives for the
 // device (noalloc_scratch), never through the array's name.
-constexpr int NOALLOC_FRAME_BLOCKS = 16384;
-constexpr int64_t NOALLOC_MAX_CHUNK = 1ll << 30;  // lattice points per block
+constexpr int NOALLOC_FRAME_BLOCKS = 16384;       // segments at most
+constexpr int64_t NOALLOC_MAX_CHUNK = 1ll << 30;  // lattice points a segment
 static __device__ __align__(256) unsigned long long scratch[NOALLOC_FRAME_BLOCKS * 8];
 
 // ---- census: atoms by species and covered points by coverage slot ---------
@@ -2486,6 +2525,15 @@ struct mskg_engine {
   double run_ms = 0, sweep_ms = 0;
   int64_t sweep_points = 0, sweeps_done = 0;
   bool loaded = false;
+  // The planes [slab_z0, slab_z1] that may differ from the flat slab the
+  // device builder wrote (slab: its mode; -1: some other state, of which
+  // nothing is known): its surface, and 12 planes around every tile layer
+  // that a run's sweeps could visit since.  An event's site lies in such a
+  // layer, and it writes at most 6 planes from it.
+  int slab = -1, slab_z0 = 0, slab_z1 = 0;
+  // workspaces of the frames: kept while they are small (WORK_KEEP)
+  void *d_work[2] = {nullptr, nullptr};
+  size_t work_n[2] = {0, 0};
   std::string err;
 };
 
@@ -2613,6 +2661,51 @@ static int word_kind(const mskg_engine *e, int32_t v, int *kind) {
 
 static int la_variant_off(mskg_engine *e);
 static int census(mskg_engine *e, int64_t out[6]);
+// The planes [z0, z1] outside which the state is the pristine slab: walls,
+// bulk atoms on diamond sites, empty points of coordination 0.
+static void touched_planes(const mskg_engine *e, int &z0, int &z1) {
+  z0 = e->slab < 0 ? 0 : std::max(0, e->slab_z0);
+  z1 = e->slab < 0 ? e->box.lz : std::min(e->box.lz, e->slab_z1);
+}
+// A run starts: until it has ended well, nothing is known of its state
+// (returned: what was known).  run_over puts it back, wider.
+static int run_touches(mskg_engine *e) {
+  const int slab = e->slab;
+  e->slab = -1;
+  return slab;
+}
+static void run_over(mskg_engine *e, int slab, int lo, int hi) {
+  e->slab = slab;
+  if (slab < 0 || lo > hi) return;
+  e->slab_z0 = std::min(e->slab_z0, lo * e->tile - 12);
+  e->slab_z1 = std::max(e->slab_z1, (hi + 1) * e->tile - 1 + 12);
+}
+// A workspace of at least n bytes, null when there is no memory for it; a
+// call that took one larger than WORK_KEEP gives it back at its end.
+constexpr size_t WORK_KEEP = 8u << 20;
+static void *work_take(mskg_engine *e, int k, size_t n) {
+  if (e->work_n[k] < n) {
+    hipFree(e->d_work[k]);
+    e->d_work[k] = nullptr;
+    e->work_n[k] = 0;
+    n = std::max<size_t>(n, 1 << 16);
+    if (hipMalloc(&e->d_work[k], n) != hipSuccess) {
+      (void)hipGetLastError();
+      e->d_work[k] = nullptr;
+      return nullptr;
+    }
+    e->work_n[k] = n;
+  }
+  return e->d_work[k];
+}
+static void work_done(mskg_engine *e) {
+  for (int k = 0; k < 2; k++)
+    if (e->work_n[k] > WORK_KEEP) {
+      hipFree(e->d_work[k]);
+      e->d_work[k] = nullptr;
+      e->work_n[k] = 0;
+    }
+}
 // The run state's fields before the sweep sums (slot, rpart: left as they
 // are in st).
 static int read_state(mskg_engine *e, RunState &st) {
@@ -2626,6 +2719,23 @@ static int write_state_head(mskg_engine *e, const RunState &st) {
   return MSKG_OK;
 }
 
+// The segments of a frame's kernels over the planes [z0, z1]: small enough
+// that a small lattice still fills the chip, at most max_seg of them (0: any
+// number, of FRAME_GROUPS groups at most).
+static FramePlan frame_plan(const mskg_engine *e, int z0, int z1, int sic, int max_seg) {
+  FramePlan F;
+  F.first = z0 * e->box.plane;
+  F.end = (z1 + 1) * e->box.plane;
+  F.sic = sic;
+  const int64_t ng = std::max<int64_t>(1, (F.end - F.first + WAVE - 1) / WAVE);
+  F.groups = 4;
+  while (F.groups < FRAME_GROUPS && ng / F.groups > 8192) F.groups *= 2;
+  F.rounds = 1;
+  if (max_seg) F.rounds = (int)((ng + (int64_t)F.groups * max_seg - 1) / ((int64_t)F.groups * max_seg));
+  F.nseg = (int)((ng + (int64_t)F.groups * F.rounds - 1) / ((int64_t)F.groups * F.rounds));
+  return F;
+}
+
 // The ordered record lists of one frame mode (k_frame_count / k_frame_write):
 // hosts[k] receives list k (caps[k] records), counts the NCNT totals.  A call
 // with too small capacities only sizes the lists (MSKG_ECAPACITY when it
@@ -2633,70 +2743,64 @@ static int write_state_head(mskg_engine *e, const RunState &st) {
 template <int MODE>
 static int frame_lists(mskg_engine *e, int sic, int32_t *const hosts[], const int64_t caps[], int64_t counts[]) {
   constexpr int NL_ = FrameShape<MODE>::NLIST, NC = FrameShape<MODE>::NCNT;
-  const int64_t n = e->box.npts;
-  const int nblk = (int)std::min<int64_t>(std::max<int64_t>(1, (n + 65535) / 65536), 65536);
-  const int64_t chunk = (n + nblk - 1) / nblk;
+  // outside the touched planes a slab has no record: its atoms there have
+  // coordination 4 and lie on diamond sites, its empty points coordination 0,
+  // and in the SiC slab every atom's neighbours are of the other species (an
+  // alloy's or a one-species slab's are not: every plane is read)
+  int z0 = 0, z1 = e->box.lz;
+  if (MODE == FRAME_MAIN || !sic || e->slab == 1) touched_planes(e, z0, z1);
+  const FramePlan F = frame_plan(e, z0, z1, sic, 0);
+  const int nblk = (F.nseg + FRAME_THREADS / WAVE - 1) / (FRAME_THREADS / WAVE);
   Lattice L = make_lattice(e);
-  unsigned long long *d_counts = nullptr, *d_offs = nullptr;
-  int4 *d_out[3] = {nullptr, nullptr, nullptr};
-  auto cleanup = [&]() {
-    hipFree(d_counts);
-    hipFree(d_offs);
-    for (int k = 0; k < 3; k++) hipFree(d_out[k]);
-  };
-  if (hipMalloc(&d_counts, (size_t)nblk * NC * sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&d_offs, (size_t)nblk * NL_ * sizeof(unsigned long long)) != hipSuccess) {
-    cleanup();
-    return fail_(e, MSKG_ENOMEM, "frame: no device memory for the block counts");
-  }
-  hipLaunchKernelGGL(k_frame_count<MODE>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, chunk, sic, d_counts);
-  std::vector<unsigned long long> cnt((size_t)nblk * NC), offs((size_t)nblk * NL_);
+  const size_t n_bits = (size_t)F.nseg * F.groups * 8, n_offs = (size_t)F.nseg * NL_ * 8, n_cnt = (size_t)F.nseg * NC * 4;
+  // totals, offsets, counts, then the bits (left out when there is no memory for them)
+  unsigned long long *bits = nullptr;
+  char *w = (char *)work_take(e, 0, 64 + n_offs + n_cnt + 8 + n_bits);
+  if (w) bits = (unsigned long long *)(w + 64 + n_offs + (n_cnt + 7) / 8 * 8);
+  else w = (char *)work_take(e, 0, 64 + n_offs + n_cnt);
+  if (!w) return fail_(e, MSKG_ENOMEM, "frame: no device memory for the block counts");
+  int64_t *d_tot = (int64_t *)w;
+  unsigned long long *d_offs = (unsigned long long *)(w + 64);
+  uint32_t *d_counts = (uint32_t *)(w + 64 + n_offs);
+  hipLaunchKernelGGL(k_frame_count<MODE>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, F, d_counts, bits);
+  hipLaunchKernelGGL(k_frame_scan<MODE>, dim3(NC), dim3(SCAN_THREADS), 0, e->stream, d_counts, F.nseg, d_offs, d_tot);
+  int64_t tot[NC];
   hipError_t ce = hipGetLastError();
-  if (ce == hipSuccess)
-    ce = hipMemcpyAsync(cnt.data(), d_counts, cnt.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                        e->stream);
+  if (ce == hipSuccess) ce = hipMemcpyAsync(tot, d_tot, sizeof tot, hipMemcpyDeviceToHost, e->stream);
   if (ce == hipSuccess) ce = hipStreamSynchronize(e->stream);
   if (ce != hipSuccess) {
-    cleanup();
+    work_done(e);
     return fail_(e, MSKG_EDEVICE, "frame count: %s", hipGetErrorString(ce));
   }
-  unsigned long long tot[NC];
-  for (int k = 0; k < NC; k++) tot[k] = 0;
-  for (int b = 0; b < nblk; b++)
-    for (int k = 0; k < NC; k++) {
-      if (k < NL_) offs[(size_t)b * NL_ + k] = tot[k];
-      tot[k] += cnt[(size_t)b * NC + k];
-    }
-  for (int k = 0; k < NC; k++) counts[k] = (int64_t)tot[k];
   bool fits = true, brought = false;
+  int64_t all = 0;
+  for (int k = 0; k < NC; k++) counts[k] = tot[k];
   for (int k = 0; k < NL_; k++) {
-    fits &= (int64_t)tot[k] <= caps[k];
+    fits &= tot[k] <= caps[k];
     brought |= hosts[k] && caps[k];
+    all += tot[k];
   }
   if (!fits) {
-    cleanup();
+    work_done(e);
     if (brought) return fail_(e, MSKG_ECAPACITY, "frame: the records do not fit the buffers given");
     return MSKG_OK;  // sizing call
   }
-  for (int k = 0; k < NL_; k++)
-    if (hipMalloc(&d_out[k], std::max<unsigned long long>(1, tot[k]) * sizeof(int4)) != hipSuccess) {
-      cleanup();
+  if (all) {
+    int4 *d_rec = (int4 *)work_take(e, 1, (size_t)all * sizeof(int4));
+    if (!d_rec) {
+      work_done(e);
       return fail_(e, MSKG_ENOMEM, "frame: no device memory for the records");
     }
-  ce = hipMemcpyAsync(d_offs, offs.data(), offs.size() * sizeof(unsigned long long), hipMemcpyHostToDevice,
-                      e->stream);
-  if (ce == hipSuccess) {
-    int64_t capv[3] = {0, 0, 0};
-    for (int k = 0; k < NL_; k++) capv[k] = (int64_t)tot[k];
-    hipLaunchKernelGGL(k_frame_write<MODE>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, chunk, sic, d_offs,
-                       d_out[0], d_out[1], d_out[2], capv[0], capv[1], capv[2]);
+    int4 *d_out[3] = {d_rec, d_rec + tot[0], d_rec + tot[0] + tot[1]};
+    hipLaunchKernelGGL(k_frame_write<MODE>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, F, bits, d_offs,
+                       d_out[0], d_out[1], d_out[2], tot[0], tot[1], NL_ > 2 ? tot[2] : (int64_t)0);
     ce = hipGetLastError();
+    for (int k = 0; k < NL_ && ce == hipSuccess; k++)
+      if (tot[k] && hosts[k])
+        ce = hipMemcpyAsync(hosts[k], d_out[k], tot[k] * sizeof(int4), hipMemcpyDeviceToHost, e->stream);
+    if (ce == hipSuccess) ce = hipStreamSynchronize(e->stream);
   }
-  for (int k = 0; k < NL_ && ce == hipSuccess; k++)
-    if (tot[k] && hosts[k])
-      ce = hipMemcpyAsync(hosts[k], d_out[k], tot[k] * sizeof(int4), hipMemcpyDeviceToHost, e->stream);
-  if (ce == hipSuccess) ce = hipStreamSynchronize(e->stream);
-  cleanup();
+  work_done(e);
   if (ce != hipSuccess) return fail_(e, MSKG_EDEVICE, "frame write: %s", hipGetErrorString(ce));
   return MSKG_OK;
 }
@@ -2706,7 +2810,10 @@ static int frame_lists(mskg_engine *e, int sic, int32_t *const hosts[], const in
 static int wrong_flips(mskg_engine *e, std::vector<int4> &flips) {
   flips.clear();
   Lattice L = make_lattice(e);
-  const int blocks = (int)std::min<int64_t>((e->box.npts + 255) / 256, 256 * 64);
+  int z0 = 0, z1 = e->box.lz;
+  if (e->slab == 1) touched_planes(e, z0, z1);  // every atom of the SiC slab has neighbours of the other species
+  const int64_t first = z0 * e->box.plane, end = (z1 + 1) * e->box.plane;
+  const int blocks = (int)std::min<int64_t>((end - first + 255) / 256, 256 * 64);
   int64_t cap = 1 << 16;
   for (;;) {
     unsigned long long *d_n = nullptr;
@@ -2720,7 +2827,8 @@ static int wrong_flips(mskg_engine *e, std::vector<int4> &flips) {
     std::vector<int4> c;
     hipError_t ce = hipMemsetAsync(d_n, 0, sizeof n, e->stream);
     if (ce == hipSuccess) {
-      hipLaunchKernelGGL(k_wrong_cand, dim3(blocks), dim3(256), 0, e->stream, L, cap, d_n, d_c);
+      hipLaunchKernelGGL(k_wrong_cand, dim3(blocks), dim3(256), 0, e->stream, L, first, end, cap, d_n,
+                         d_c);
       ce = hipGetLastError();
     }
     if (ce == hipSuccess) ce = hipMemcpyAsync(&n, d_n, sizeof n, hipMemcpyDeviceToHost, e->stream);
@@ -2931,6 +3039,7 @@ void mskg_destroy(mskg_engine *e) {
   hipFree(e->d_inlist); hipFree(e->d_tl_idx); hipFree(e->d_tl_n); hipFree(e->d_tl_own); hipFree(e->d_tile_r); hipFree(e->d_list_err);
   hipFree(e->d_field[0]); hipFree(e->d_field[1]); hipFree(e->d_offwall); hipFree(e->d_st_tables); hipFree(e->d_win);
   hipFree(e->d_done);
+  for (int k = 0; k < 2; k++) hipFree(e->d_work[k]);
   hipFree(e->d_geo); hipFree(e->d_tab); hipFree(e->d_st); hipFree(e->d_err); hipFree(e->d_log);
   hipFree(e->d_tsum); hipFree(e->d_bsum); hipFree(e->d_key); hipFree(e->d_key_seen); hipFree(e->d_rate_seen);
   if (e->ev0) hipEventDestroy(e->ev0);
@@ -2946,6 +3055,7 @@ int mskg_load_state(mskg_engine *e, const int32_t *latt, int32_t n_ad, const int
   if (!e || !latt) return MSKG_EINVAL;
   if (!e->d_site) return fail_(e, MSKG_EINVAL, "engine not created");
   const Box &b = e->box;
+  e->slab = -1;
   std::vector<Site> site((size_t)b.npts);
   memset(site.data(), 0, site.size() * sizeof(Site));
   std::vector<float> rate((size_t)b.npts, 0.0f);
@@ -3316,6 +3426,7 @@ int mskg_refresh_active(mskg_engine *e) {
 int mskg_replay(mskg_engine *e, const mskg_event *log, int64_t n, int32_t clock_mode) {
   if (!e || !e->loaded || (n > 0 && !log)) return fail_(e, MSKG_EINVAL, "replay: no state or no log");
   if (n == 0) return MSKG_OK;
+  e->slab = -1;  // the log's sites may lie anywhere
   mskg_event *d_log = nullptr;
   HIPCHK(e, hipMalloc(&d_log, n * sizeof(mskg_event)));
   hipError_t ce = hipMemcpyAsync(d_log, log, n * sizeof(mskg_event), hipMemcpyHostToDevice, e->stream);
@@ -3376,6 +3487,8 @@ static int run_begin(mskg_engine *e, int64_t max_events, double max_time, RunSta
     s0.events_per_pass = e->cfg.events_per_pass > 0 ? e->cfg.events_per_pass : 1.0;
     s0.max_time = max_time;
     s0.max_events = st.events + (unsigned long long)max_events;
+    s0.ever_lo = 0x7fffffff;
+    s0.ever_hi = -1;
     if (int rc2 = write_state_head(e, s0)) return rc2;
     HIPCHK(e, hipMemsetAsync((char *)e->d_st + RS_HEAD, 0, sizeof s0.slot, e->stream));
   }
@@ -3413,6 +3526,7 @@ int mskg_run(mskg_engine *e, int64_t max_events, double max_time, int64_t *event
   RunState st;
   int rc = run_begin(e, max_events, max_time, st);
   if (rc) return rc;
+  const int slab = run_touches(e);
   const unsigned long long ev_start = st.events;
   const size_t shm = (size_t)e->cap * (4 + 4 + 1) + 16;
   // one sweep = eight colour passes (or one dependency-scheduled launch) +
@@ -3470,6 +3584,7 @@ int mskg_run(mskg_engine *e, int64_t max_events, double max_time, int64_t *event
   HIPCHK(e, hipStreamSynchronize(e->stream));
   float ms = 0;
   HIPCHK(e, hipEventElapsedTime(&ms, e->ev0, e->ev1));
+  run_over(e, slab, st.ever_lo, st.ever_hi);
   e->run_ms = ms;
   e->sweeps_done = sweeps;
   if (events_done) *events_done = (int64_t)(st.events - ev_start);
@@ -3686,6 +3801,7 @@ static int build_slab(mskg_engine *e, int32_t mode, int32_t len, double fraction
     return fail_(e, MSKG_EINVAL, "slab height %d: the stored planes (stored_len_z %d) need %d more above it", len,
                  e->box.lz + 1, TOP_MARGIN + 6);
   Lattice L = make_lattice(e);
+  e->slab = -1;
   int blocks = (int)std::min<int64_t>((e->box.npts + 255) / 256, 256 * 64);
   hipLaunchKernelGGL(k_build_slab, dim3(blocks), dim3(256), 0, e->stream, L, len, mode, fraction,
                      (uint32_t)e->cfg.seed, (uint32_t)(e->cfg.seed >> 32), e->logical_lz);
@@ -3713,6 +3829,9 @@ static int build_slab(mskg_engine *e, int32_t mode, int32_t len, double fraction
   e->loaded = true;
   e->lists_dirty = true;
   e->keys_valid = false;
+  e->slab = mode;
+  e->slab_z0 = len - 3;  // the surface atoms ...
+  e->slab_z1 = len;      // ... and the empty sites above them
   return MSKG_OK;
 }
 
@@ -3728,6 +3847,7 @@ static int build_shape(mskg_engine *e, ShapeSpec S, bool walls_off_lattice) {
   S.cx = e->box.lx / 2;
   S.cy = e->box.ly / 2;
   S.cz = e->logical_lz / 2;
+  e->slab = -1;
   Lattice L = make_lattice(e);
   L.key = nullptr;
   const int blocks = (int)std::min<int64_t>((e->box.npts + 255) / 256, 256 * 64);
@@ -3867,6 +3987,7 @@ int mskg_copy_state(mskg_engine *dst, const mskg_engine *src) {
       dst->tile != src->tile)
     return fail_(dst, MSKG_EINVAL, "copy_state: engines differ in box or tile");
   const int64_t np = dst->box.npts;
+  dst->slab = -1;
   HIPCHK(dst, hipStreamSynchronize(src->stream));
   HIPCHK(dst, hipMemcpyAsync(dst->d_site, src->d_site, np * sizeof(Site), hipMemcpyDeviceToDevice, dst->stream));
   HIPCHK(dst, hipMemcpyAsync(dst->d_rate, src->d_rate, np * sizeof(float), hipMemcpyDeviceToDevice, dst->stream));
@@ -3904,6 +4025,9 @@ int mskg_copy_state(mskg_engine *dst, const mskg_engine *src) {
   if (int rc = census(dst, dst->census0)) return rc;  // the event counters restart here
   dst->loaded = true;
   dst->lists_dirty = true;
+  dst->slab = src->slab;
+  dst->slab_z0 = src->slab_z0;
+  dst->slab_z1 = src->slab_z1;
   return MSKG_OK;
 }
 
@@ -3990,6 +4114,7 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
     for (int j = 0; j < i; j++)
       if (engines[j] == e) return fail_(e0, MSKG_EINVAL, "serial run: replica %d appears twice", i);
     HIPCHK(e, hipStreamSynchronize(e->stream));
+    e->slab = -1;  // the serial run keeps no record of the layers it visits
     const int nblk = (e->ntiles + WAVE - 1) / WAVE;
     if (!e->d_tsum) {
       HIPCHK(e, hipMalloc(&e->d_tsum, e->ntiles * sizeof(double)));
@@ -4085,6 +4210,7 @@ int mskg_run_ensemble(mskg_engine *const *engines, int32_t n, const int64_t *max
   if (queue_bound > (1ll << 25)) return fail_(e0, MSKG_EINVAL, "ensemble: too many tiles per colour pass");
   std::vector<PassParams> reps(n);
   std::vector<unsigned long long> ev0(n);
+  std::vector<int> slab(n);
   for (int i = 0; i < n; i++) {
     mskg_engine *e = engines[i];
     RunState st;
@@ -4096,6 +4222,7 @@ int mskg_run_ensemble(mskg_engine *const *engines, int32_t n, const int64_t *max
     reps[i] = pass_params(e);
   }
   for (int i = 0; i < n; i++) HIPCHK(engines[i], hipStreamSynchronize(engines[i]->stream));
+  for (int i = 0; i < n; i++) slab[i] = run_touches(engines[i]);
   hipStream_t sm = e0->stream;
   PassParams *d_reps = nullptr;
   int *d_plan = nullptr;
@@ -4167,6 +4294,7 @@ int mskg_run_ensemble(mskg_engine *const *engines, int32_t n, const int64_t *max
     e->sweeps_done = sweeps;
     RunState st;
     if (int rc = read_state(e, st)) return rc;
+    run_over(e, slab[i], st.ever_lo, st.ever_hi);
     if (events_done) events_done[i] = (int64_t)(st.events - ev0[i]);
     if (kmc_time) kmc_time[i] = st.clock;
     if (stop_reason) stop_reason[i] = st.stop == STOP_AT_LIMIT || !st.stop ? MSKG_STOP_LIMIT : st.stop;
@@ -4307,6 +4435,7 @@ int mskg_adjoint_checkpointed(mskg_engine *const *engines, int32_t n, const mskg
     if (ce == hipSuccess) ce = hipMemcpyAsync(e->d_key_seen, e->d_key, np * sizeof(int32_t), hipMemcpyDeviceToDevice, sm);
     if (ce == hipSuccess) ce = hipMemcpyAsync(e->d_rate_seen, e->d_rate, np * sizeof(float), hipMemcpyDeviceToDevice, sm);
     e->lists_dirty = true;
+    e->slab = -1;
   }
   const int cblocks = (n + 255) / 256;
   std::vector<int> chk(2 * (size_t)n);
@@ -4370,20 +4499,26 @@ int mskg_frame_device(mskg_engine *e, int32_t *main_rec, int64_t cap_main, int32
   if (!e || !e->loaded || !counts) return fail_(e, MSKG_EINVAL, "frame_device: no state loaded or no counts");
   if (cap_main < 0 || cap_void < 0 || cap_noepi < 0) return fail_(e, MSKG_EINVAL, "frame_device: negative capacity");
   const int64_t n = e->box.npts;
-  const int nblk = (int)std::min<int64_t>(std::max<int64_t>(1, (n + 65535) / 65536), NOALLOC_FRAME_BLOCKS);
-  const int64_t chunk = (n + nblk - 1) / nblk;
-  if (chunk > NOALLOC_MAX_CHUNK)
+  if ((n + NOALLOC_FRAME_BLOCKS - 1) / NOALLOC_FRAME_BLOCKS > NOALLOC_MAX_CHUNK)
     return fail_(e, MSKG_EINVAL, "frame_device: %lld lattice points exceed the scratch's %d blocks of %lld points",
                  (long long)n, NOALLOC_FRAME_BLOCKS, (long long)NOALLOC_MAX_CHUNK);
   unsigned long long *sc = g_scratch[e->device];
   if (!sc) return fail_(e, MSKG_EDEVICE, "frame_device: the device's scratch is not set up");
-  unsigned long long *d_counts = sc, *d_offs = sc + (size_t)nblk * FrameShape<FRAME_MAIN>::NCNT;
+  int z0, z1;
+  touched_planes(e, z0, z1);
+  const FramePlan F = frame_plan(e, z0, z1, 0, NOALLOC_FRAME_BLOCKS);
+  const int nblk = (F.nseg + FRAME_THREADS / WAVE - 1) / (FRAME_THREADS / WAVE);
+  unsigned long long *d_offs = sc;
+  uint32_t *d_counts = (uint32_t *)(sc + (size_t)F.nseg * FrameShape<FRAME_MAIN>::NLIST);
   Lattice L = make_lattice(e);
-  hipLaunchKernelGGL(k_frame_count<FRAME_MAIN>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, chunk, 0,
-                     d_counts);
-  hipLaunchKernelGGL(k_frame_scan<FRAME_MAIN>, dim3(1), dim3(256), 0, e->stream, d_counts, nblk, d_offs, counts);
-  hipLaunchKernelGGL(k_frame_write<FRAME_MAIN>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, chunk, 0, d_offs,
-                     (int4 *)main_rec, (int4 *)void_rec, (int4 *)noepi_rec, cap_main, cap_void, cap_noepi);
+  // no bits kept between the two passes: the write reads the records again
+  hipLaunchKernelGGL(k_frame_count<FRAME_MAIN>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, F, d_counts,
+                     (unsigned long long *)nullptr);
+  hipLaunchKernelGGL(k_frame_scan<FRAME_MAIN>, dim3(FrameShape<FRAME_MAIN>::NCNT), dim3(SCAN_THREADS), 0, e->stream,
+                     d_counts, F.nseg, d_offs, counts);
+  hipLaunchKernelGGL(k_frame_write<FRAME_MAIN>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, F,
+                     (const unsigned long long *)nullptr, d_offs, (int4 *)main_rec, (int4 *)void_rec,
+                     (int4 *)noepi_rec, cap_main, cap_void, cap_noepi);
   hipError_t ce = hipGetLastError();
   if (ce == hipSuccess) ce = hipStreamSynchronize(e->stream);
   if (ce != hipSuccess) return fail_(e, MSKG_EDEVICE, "frame_device: %s", hipGetErrorString(ce));

@@ -178,22 +178,31 @@ class Engine:
         of (x, y, z, code) rows in grid order and the header counts
         (atoms of coordination <= 3, covered points; both for 1 <= z < LenZ)."""
         c = np.zeros(5, np.int64)
-        z = None
-        self._check(self.L.mskg_frame(self.h, z, 0, z, 0, z, 0, ptr(c)))
-        bufs = [np.zeros((max(int(c[k]), 1), 4), np.int32) for k in range(3)]
-        self._check(self.L.mskg_frame(self.h, ptr(bufs[0]), int(c[0]), ptr(bufs[1]), int(c[1]), ptr(bufs[2]),
-                                      int(c[2]), ptr(c)))
-        return bufs[0][:c[0]], bufs[1][:c[1]], bufs[2][:c[2]], int(c[3]), int(c[4])
+        bufs = self._records(self.L.mskg_frame, 3, c)
+        return bufs[0], bufs[1], bufs[2], int(c[3]), int(c[4])
+
+    def _records(self, call, lists, counts):
+        """A frame call's record lists.  One pass over the lattice fills
+        buffers of 4.5 monolayers' atoms a list, which a film's surface seldom
+        exceeds; the exact sizes are asked for only when it does."""
+        lx, ly, _ = self.box
+        rows = [max(lx * ly // 16, 4096)] * lists
+        for last in (False, True):
+            bufs = [np.empty((r, 4), np.int32) for r in rows]
+            rc = call(self.h, *[v for b, r in zip(bufs, rows) for v in (ptr(b), r)], ptr(counts))
+            if rc != _lib.MSKG_ECAPACITY or last:
+                break
+            rows = [max(int(n), 1) for n in counts[:lists]]
+        self._check(rc)
+        return [b[:n] for b, n in zip(bufs, counts)]
 
     def frame_defects(self):
         """The SiC defect frames' records (mskg_frame_defects): (vacancies
         with the species sum of their neighbours, wrong occupations with the
         flipped species), (x, y, z, code) rows in grid order."""
         c = np.zeros(2, np.int64)
-        self._check(self.L.mskg_frame_defects(self.h, None, 0, None, 0, ptr(c)))
-        bufs = [np.zeros((max(int(c[k]), 1), 4), np.int32) for k in range(2)]
-        self._check(self.L.mskg_frame_defects(self.h, ptr(bufs[0]), int(c[0]), ptr(bufs[1]), int(c[1]), ptr(c)))
-        return bufs[0][:c[0]], bufs[1][:c[1]]
+        bufs = self._records(self.L.mskg_frame_defects, 2, c)
+        return bufs[0], bufs[1]
 
     def track_classes(self, on=True):
         """Keep the rate-class keys current through runs (likelihood segments)."""
