@@ -34,6 +34,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/mskg.h"
@@ -2113,11 +2114,13 @@ __global__ void __launch_bounds__(256) k_key_hist(Lattice L, int *cnt, double *i
 // 1536 53.0, now 50.5; 24 SiGe replicas 54.8, now 36.1; the smallest box 8.7,
 // now 8.2.
 constexpr int FRAME_THREADS = 256;
+constexpr uint32_t NO_POINT = 0xffffffffu;  // in the place of a record's last word (whose temperature has 13 bits)
 constexpr int FRAME_GROUPS = 64;  // groups of 64 points a wave takes at a time: a lane's bits each
-enum : int { FRAME_MAIN = 0, FRAME_DEFECTS = 1 };
+enum : int { FRAME_MAIN = 0, FRAME_DEFECTS = 1, FRAME_STATE = 2 };
 template <int MODE> struct FrameShape;
 template <> struct FrameShape<FRAME_MAIN> { static constexpr int NLIST = 3, NCNT = 5; };
 template <> struct FrameShape<FRAME_DEFECTS> { static constexpr int NLIST = 2, NCNT = 2; };
+template <> struct FrameShape<FRAME_STATE> { static constexpr int NLIST = 3, NCNT = 3; };
 constexpr uint8_t WRONG_FLIP = 0x80;
 
 // Species of a record as the _w analysis sees it: the wrong-site flip swaps
@@ -2155,7 +2158,14 @@ __device__ inline void frame_point(const Lattice &L, int64_t p, uint32_t w, int 
   }
   const bool atom = kind_species(kind), covered = kind >= KIND_COV0;
   const bool below = p < L.box.plane * L.box.lz;  // z <= LenZ-1
-  if (MODE == FRAME_MAIN) {
+  if (w == NO_POINT) return;
+  if (MODE == FRAME_STATE) {
+    // the reference's lists: an atom of coordination <= 3 is an MC particle
+    // even when it has no rate (a frozen-substrate atom)
+    in[0] = (atom && coor <= 3) || L.cls[p] != 0;
+    in[1] = !in[0] && atom;
+    in[2] = !in[0] && !atom && coor == 4;
+  } else if (MODE == FRAME_MAIN) {
     if (!below) return;
     const bool inner = p >= L.box.plane;  // z >= 1
     in[0] = covered || (atom && coor <= 3);  // a covered vacancy is also listed in the main frame
@@ -2202,7 +2212,7 @@ __device__ inline unsigned long long frame_bits(const Lattice &L, int64_t g0, in
     uint32_t w[4];
     for (int u = 0; u < 4; u++) {
       const int64_t p = g0 + (int64_t)(g + u) * WAVE + lane;
-      w[u] = g + u < groups && p < end ? ((const uint32_t *)(L.site + p))[3] : (uint32_t)KIND_WALL;  // no list holds a wall
+      w[u] = g + u < groups && p < end ? ((const uint32_t *)(L.site + p))[3] : NO_POINT;
     }
     for (int u = 0; u < 4; u++) {
       bool in[FrameShape<MODE>::NLIST];
@@ -2286,21 +2296,18 @@ __global__ void __launch_bounds__(FRAME_THREADS) k_frame_count(Lattice L, FrameP
   }
 }
 
-// The lanes' groups are taken a lane each: a lane reads its group's listed
+// Calls put(list, place, point, x, y, z, code) for every record of a wave's
+// segment.  The groups are taken a lane each: a lane reads its group's listed
 // points one after the other, once to count them by list and once to write.
-template <int MODE>
-__global__ void __launch_bounds__(FRAME_THREADS) k_frame_write(Lattice L, FramePlan F, const unsigned long long *bits,
-                                                               const unsigned long long *offs, int4 *out0,
-                                                               int4 *out1, int4 *out2, int64_t cap0, int64_t cap1,
-                                                               int64_t cap2) {
+template <int MODE, class Put>
+__device__ inline void frame_put(const Lattice &L, const FramePlan &F, const unsigned long long *bits,
+                                 const unsigned long long *offs, Put put) {
   constexpr int NL_ = FrameShape<MODE>::NLIST, NC = FrameShape<MODE>::NCNT;
   const int lane = threadIdx.x & (WAVE - 1);
   const int seg = blockIdx.x * (FRAME_THREADS / WAVE) + threadIdx.x / WAVE;
   if (seg >= F.nseg) return;
   unsigned long long base[NL_];
   for (int k = 0; k < NL_; k++) base[k] = offs[(int64_t)k * F.nseg + seg];
-  int4 *const outs[3] = {out0, out1, out2};
-  const unsigned long long caps[3] = {(unsigned long long)cap0, (unsigned long long)cap1, (unsigned long long)cap2};
   for (int r = 0; r < F.rounds; r++) {
     const int64_t grp = ((int64_t)seg * F.rounds + r) * F.groups, g0 = F.first + grp * WAVE;
     if (g0 >= F.end) break;
@@ -2336,11 +2343,22 @@ __global__ void __launch_bounds__(FRAME_THREADS) k_frame_write(Lattice L, FrameP
       pxyz(L.box, p, x, y, z);
       for (int k = 0; k < NL_; k++)
         if (in[k]) {
-          if (at[k] < caps[k]) outs[k][at[k]] = make_int4(x, y, z, code[k]);
+          put(k, at[k], p, x, y, z, code[k]);
           at[k]++;
         }
     }
   }
+}
+template <int MODE>
+__global__ void __launch_bounds__(FRAME_THREADS) k_frame_write(Lattice L, FramePlan F, const unsigned long long *bits,
+                                                               const unsigned long long *offs, int4 *out0,
+                                                               int4 *out1, int4 *out2, int64_t cap0, int64_t cap1,
+                                                               int64_t cap2) {
+  int4 *const outs[3] = {out0, out1, out2};
+  const unsigned long long caps[3] = {(unsigned long long)cap0, (unsigned long long)cap1, (unsigned long long)cap2};
+  frame_put<MODE>(L, F, bits, offs, [&](int k, unsigned long long at, int64_t, int x, int y, int z, int code) {
+    if (at < caps[k]) outs[k][at] = make_int4(x, y, z, code);
+  });
 }
 
 // The segments' offsets of a frame from their counts, and the totals (NCNT
@@ -2390,6 +2408,147 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_frame_scan(const uint32_t *cou
 constexpr int NOALLOC_FRAME_BLOCKS = 16384;       // segments at most
 constexpr int64_t NOALLOC_MAX_CHUNK = 1ll << 30;  // lattice points a segment
 static __device__ __align__(256) unsigned long long scratch[NOALLOC_FRAME_BLOCKS * 8];
+
+// ---- the host's arrays: LattCoo words and particle lists ------------------------
+// The reference's lists out of the lattice (xyz, NextNXYZ; of MC particles
+// also Ind_Event and ProbTrans), and LattCoo's words in and out.  The device
+// reads and writes the records; the host copies 4 bytes a lattice point and
+// the lists, where it had copied every point's 21 bytes and gone through them
+// point by point: the whole exchange (load, 1e5 events, store) of CVD at
+// 240x240x760 took 346 ms, now 70.
+struct StateOut {
+  int32_t *xyz[3], *nn[3];
+  int32_t *event;
+  double *prob;
+};
+__global__ void __launch_bounds__(FRAME_THREADS) k_state_write(Lattice L, FramePlan F, const unsigned long long *bits,
+                                                               const unsigned long long *offs, StateOut O) {
+  frame_put<FRAME_STATE>(L, F, bits, offs, [&](int k, unsigned long long at, int64_t p, int x, int y, int z, int) {
+    int32_t *const q = O.xyz[k] + 3 * at, *const w = O.nn[k] + 12 * at;
+    q[0] = x; q[1] = y; q[2] = z;
+    const NL l = site_list(L.box, L.site[p], x, y, z);
+    for (int i = 0; i < 4; i++) {
+      w[3 * i] = l.x[i];
+      w[3 * i + 1] = l.y[i];
+      w[3 * i + 2] = l.z[i];
+    }
+    if (k == 0) {
+      const int c = L.cls[p];
+      O.event[at] = (c == CLS_EVAP || c == CLS_ISOLATED || !c) ? 4 : c == CLS_DESORB ? 5 : 1;
+      O.prob[at] = (double)L.rate[p];
+    }
+  });
+}
+
+// LattCoo's coverage indices by slot.
+struct CovList {
+  int n, index[3];
+};
+// The content of a LattCoo word; < 0: not representable.
+MSKG_HD int word_kind(const CovList &C, int32_t v) {
+  const int cov = v & 255, occ = (v >> 23) & 1, sic = (v >> 27) & 7;
+  if (cov == 113) return KIND_WALL;
+  if (cov != 0) {
+    if (occ) return -1;
+    for (int k = 0; k < C.n; k++)
+      if (C.index[k] == cov) return KIND_COV0 + k;
+    return -2;
+  }
+  if (occ) return sic < 1 || sic > 3 ? -3 : sic;
+  return sic ? -4 : KIND_EMPTY;
+}
+__global__ void __launch_bounds__(256) k_words_out(Lattice L, CovList C, int64_t first, int64_t end, int32_t *out) {
+  for (int64_t p = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < end;
+       p += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t w = ((const uint32_t *)(L.site + p))[3];
+    const int kind = w & 7;
+    uint32_t v = 0u;
+    if (kind == KIND_WALL) v = (1u << 23) | 113u;
+    else if (kind_species(kind)) v = (1u << 23) | ((uint32_t)kind << 27);
+    else if (kind >= KIND_COV0) v = (uint32_t)C.index[kind - KIND_COV0];
+    v |= ((w >> 3) & 7u) << 24;
+    v |= (w >> 16) << 9;
+    out[p - first] = (int32_t)v;
+  }
+}
+// What a piece of LattCoo (grid points g0..g0+n-1) holds that matters before
+// any of it is taken: out[0] the first lattice point that is no site state,
+// out[1] whether there are walls off the lattice.
+__global__ void __launch_bounds__(256) k_words_check(Box b, CovList C, const int32_t *latt, int64_t g0, int64_t n,
+                                                     unsigned long long *out) {
+  const int64_t face = (int64_t)b.lx * b.ly;
+  const double inv_face = 1.0 / (double)face, inv_lx = 1.0 / (double)b.lx;
+  bool walls = false;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t v = latt[i];
+    if (v == 0) continue;
+    const int64_t g = g0 + i, z = div_by(g, face, inv_face), r = g - z * face;
+    const int y = (int)div_by(r, b.lx, inv_lx), x = (int)(r - (int64_t)y * b.lx);
+    if (valid_parity(x, y, (int)z)) {
+      if (word_kind(C, v) < 0) atomicMin(&out[0], (unsigned long long)g);
+    } else {
+      walls |= (v & 255) == 113;
+    }
+  }
+  if (__ballot(walls) && (threadIdx.x & (WAVE - 1)) == 0) atomicOr(&out[1], 1ull);
+}
+// The records of the lattice points first..end-1 from their words (latt: from
+// grid point g0 on): no list, no rate.
+__global__ void __launch_bounds__(256) k_words_in(Lattice L, CovList C, const int32_t *latt, int64_t g0, int64_t first,
+                                                  int64_t end) {
+  for (int64_t p = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < end;
+       p += (int64_t)gridDim.x * blockDim.x) {
+    int x, y, z;
+    pxyz(L.box, p, x, y, z);
+    const uint32_t v = (uint32_t)latt[(int64_t)x + (int64_t)L.box.lx * ((int64_t)y + (int64_t)L.box.ly * z) - g0];
+    const uint32_t w = (uint32_t)word_kind(C, (int32_t)v) | (((v >> 24) & 7u) << 3) | (((v >> 9) & 0x1fffu) << 16);
+    store_rec(L, p, make_rec(0u, 0u, 0u, w));
+    L.rate[p] = 0.0f;
+    L.cls[p] = 0;
+  }
+}
+// The walls off the lattice of that piece, one bit per grid point (g0 and, but
+// at the grid's end, n multiples of 32): a wave 64 points at a time.
+__global__ void __launch_bounds__(256) k_words_offwall(Box b, const int32_t *latt, int64_t g0, int64_t n,
+                                                       uint32_t *bits) {
+  const int64_t face = (int64_t)b.lx * b.ly, words = (n + 31) / 32, pairs = (words + 1) / 2;
+  const double inv_face = 1.0 / (double)face, inv_lx = 1.0 / (double)b.lx;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+  for (int64_t q = wave; q < pairs; q += (int64_t)gridDim.x * (blockDim.x / WAVE)) {
+    const int64_t i = q * WAVE + lane, g = g0 + i;
+    bool wall = i < n && (latt[i] & 255) == 113;
+    if (wall) {
+      const int64_t z = div_by(g, face, inv_face), r = g - z * face;
+      const int y = (int)div_by(r, b.lx, inv_lx), x = (int)(r - (int64_t)y * b.lx);
+      wall = !valid_parity(x, y, (int)z);
+    }
+    const unsigned long long m = __ballot(wall);
+    if (lane < 2 && 2 * q + lane < words) bits[g0 / 32 + 2 * q + lane] = (uint32_t)(m >> (32 * lane));
+  }
+}
+// A listed particle: its neighbour list, and with cls >= 0 its class and rate.
+struct StateRec {
+  int64_t p;
+  uint32_t x, y, z, valid;
+  float rate;
+  int cls;
+};
+__global__ void __launch_bounds__(256) k_lists_in(Lattice L, const StateRec *rec, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const StateRec r = rec[i];
+  Rec s = load_rec(L, r.p);
+  s.x = r.x;
+  s.y = r.y;
+  s.z = r.z;
+  s.w = (s.w & ~0xff00u) | (r.valid << 8);
+  store_rec(L, r.p, s);
+  if (r.cls >= 0) {
+    L.rate[r.p] = r.rate;
+    L.cls[r.p] = (uint8_t)r.cls;
+  }
+}
 
 // ---- census: atoms by species and covered points by coverage slot ---------
 // Every deposition adds one atom of its species and every evaporation
@@ -2595,6 +2754,7 @@ struct mskg_engine {
   int slab = -1, slab_z0 = 0, slab_z1 = 0;
   bool flags_clean = false;  // no list flag outside the touched planes (d_inlist), while they are known
   // workspaces of the frames: kept while they are small (WORK_KEEP)
+  int32_t *pinned = nullptr;  // page-locked words of the host's LattCoo on their way (8 MB, on first use)
   void *d_work[2] = {nullptr, nullptr};
   size_t work_n[2] = {0, 0};
   std::string err;
@@ -2700,26 +2860,6 @@ static const char *err_name(int c) {
       return "an event site within 24 planes of the top of the stored planes (stored_len_z): store more planes";
     default: return "unknown";
   }
-}
-
-// Map one LattCoo word (defsystem.f:87-91) to a site kind.
-static int word_kind(const mskg_engine *e, int32_t v, int *kind) {
-  int cov = v & 255, occ = (v >> 23) & 1, sic = (v >> 27) & 7;
-  if (cov == 113) { *kind = KIND_WALL; return 0; }
-  if (cov != 0) {
-    if (occ) return -1;
-    for (int k = 0; k < e->ncov; k++)
-      if (e->list_cov[k] == cov) { *kind = KIND_COV0 + k; return 0; }
-    return -2;
-  }
-  if (occ) {
-    if (sic < 1 || sic > 3) return -3;
-    *kind = sic;
-    return 0;
-  }
-  if (sic) return -4;
-  *kind = KIND_EMPTY;
-  return 0;
 }
 
 static int la_variant_off(mskg_engine *e);
@@ -2865,6 +3005,141 @@ static int frame_lists(mskg_engine *e, int sic, int32_t *const hosts[], const in
   }
   work_done(e);
   if (ce != hipSuccess) return fail_(e, MSKG_EDEVICE, "frame write: %s", hipGetErrorString(ce));
+  return MSKG_OK;
+}
+
+static CovList cov_list(const mskg_engine *e) {
+  CovList C;
+  C.n = e->ncov;
+  for (int k = 0; k < 3; k++) C.index[k] = e->list_cov[k];
+  return C;
+}
+// One record a site: the neighbour list its last record gives, the class and
+// rate of its last MC record.
+static void merge_listed(std::vector<StateRec> &recs) {
+  std::unordered_map<int64_t, size_t> at;
+  std::vector<StateRec> one;
+  for (const StateRec &r : recs) {
+    const auto it = at.find(r.p);
+    if (it == at.end()) {
+      at.emplace(r.p, one.size());
+      one.push_back(r);
+      continue;
+    }
+    StateRec &o = one[it->second];
+    const float rate = o.rate;
+    const int cls = o.cls;
+    o = r;
+    if (r.cls < 0) {
+      o.cls = cls;
+      o.rate = rate;
+    }
+  }
+  recs.swap(one);
+}
+// A piece of a state's exchange: the points of whole planes, about this many.
+constexpr int64_t STATE_PIECE = 1ll << 24;
+
+// The three particle lists in grid order: tot their lengths, the first cap[k]
+// records of each to the arrays that are given.
+static int state_lists(mskg_engine *e, const int64_t cap[3], int32_t *const xyz[3], int32_t *const nn[3],
+                       int32_t *event, double *prob, int64_t tot[3]) {
+  Lattice L = make_lattice(e);
+  const int step = (int)std::max<int64_t>(1, STATE_PIECE / e->box.plane);
+  for (int z = 0; z <= e->box.lz; z += step) {
+    const FramePlan F = frame_plan(e, z, std::min(z + step - 1, e->box.lz), 0, 0);
+    const int nblk = (F.nseg + FRAME_THREADS / WAVE - 1) / (FRAME_THREADS / WAVE);
+    const size_t n_offs = (size_t)F.nseg * 3 * 8, n_cnt = ((size_t)F.nseg * 3 * 4 + 7) / 8 * 8;
+    char *w = (char *)work_take(e, 0, 64 + n_offs + n_cnt + (size_t)F.nseg * F.groups * 8);
+    if (!w) return fail_(e, MSKG_ENOMEM, "store: no device memory for the list counts");
+    int64_t *d_tot = (int64_t *)w, n[3];
+    unsigned long long *d_offs = (unsigned long long *)(w + 64), *bits = (unsigned long long *)(w + 64 + n_offs + n_cnt);
+    uint32_t *d_counts = (uint32_t *)(w + 64 + n_offs);
+    hipLaunchKernelGGL(k_frame_count<FRAME_STATE>, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, F, d_counts, bits);
+    hipLaunchKernelGGL(k_frame_scan<FRAME_STATE>, dim3(3), dim3(SCAN_THREADS), 0, e->stream, d_counts, F.nseg, d_offs,
+                       d_tot);
+    HIPCHK(e, hipGetLastError());
+    HIPCHK(e, hipMemcpyAsync(n, d_tot, sizeof n, hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(e, hipStreamSynchronize(e->stream));
+    int64_t take[3], all = n[0] + n[1] + n[2];
+    bool any = false;
+    for (int k = 0; k < 3; k++) {
+      take[k] = std::max<int64_t>(0, std::min(n[k], cap[k] - tot[k]));
+      any |= take[k] > 0 && (xyz[k] || nn[k] || (k == 0 && (event || prob)));
+    }
+    if (any) {
+      char *r = (char *)work_take(e, 1, (size_t)all * 60 + (size_t)n[0] * 12);
+      if (!r) return fail_(e, MSKG_ENOMEM, "store: no device memory for the lists");
+      StateOut O;
+      O.prob = (double *)r;
+      int32_t *q = (int32_t *)(O.prob + n[0]);
+      for (int k = 0; k < 3; k++) {
+        O.xyz[k] = q;
+        O.nn[k] = q + 3 * n[k];
+        q += 15 * n[k];
+      }
+      O.event = q;
+      hipLaunchKernelGGL(k_state_write, dim3(nblk), dim3(FRAME_THREADS), 0, e->stream, L, F, bits, d_offs, O);
+      HIPCHK(e, hipGetLastError());
+      auto out = [&](void *host, const void *dev, int64_t bytes) {
+        return host && bytes ? hipMemcpyAsync(host, dev, (size_t)bytes, hipMemcpyDeviceToHost, e->stream) : hipSuccess;
+      };
+      for (int k = 0; k < 3; k++) {
+        HIPCHK(e, out(xyz[k] ? xyz[k] + 3 * tot[k] : nullptr, O.xyz[k], take[k] * 12));
+        HIPCHK(e, out(nn[k] ? nn[k] + 12 * tot[k] : nullptr, O.nn[k], take[k] * 48));
+      }
+      HIPCHK(e, out(event ? event + tot[0] : nullptr, O.event, take[0] * 4));
+      HIPCHK(e, out(prob ? prob + tot[0] : nullptr, O.prob, take[0] * 8));
+      HIPCHK(e, hipStreamSynchronize(e->stream));
+    }
+    for (int k = 0; k < 3; k++) tot[k] += n[k];
+  }
+  return MSKG_OK;
+}
+
+// LattCoo's words at the lattice points (the others are left as the caller
+// has them).  The words come through two halves of a page-locked buffer, the
+// next on its way while the last is laid out; a word that is there already is
+// not written again (most of a box is vacuum, and so is a fresh array).
+static int state_words(mskg_engine *e, int32_t *latt) {
+  const Box &b = e->box;
+  constexpr int64_t HALF = 1 << 20;  // words
+  if (!e->pinned) HIPCHK(e, hipHostMalloc((void **)&e->pinned, 2 * HALF * 4, hipHostMallocDefault));
+  int32_t *d = (int32_t *)work_take(e, 1, 2 * HALF * 4);
+  if (!d) return fail_(e, MSKG_ENOMEM, "store: no device memory for LattCoo's words");
+  Lattice L = make_lattice(e);
+  const CovList C = cov_list(e);
+  const int64_t pieces = (b.npts + HALF - 1) / HALF;
+  auto fetch = [&](int64_t i) -> hipError_t {
+    const int64_t p0 = i * HALF, p1 = std::min(p0 + HALF, b.npts);
+    int32_t *const dst = d + (i & 1) * HALF;
+    hipLaunchKernelGGL(k_words_out, dim3((unsigned)((p1 - p0 + 255) / 256)), dim3(256), 0, e->stream, L, C, p0, p1, dst);
+    hipError_t ce = hipGetLastError();
+    if (ce == hipSuccess)
+      ce = hipMemcpyAsync(e->pinned + (i & 1) * HALF, dst, (size_t)(p1 - p0) * 4, hipMemcpyDeviceToHost, e->stream);
+    if (ce == hipSuccess) ce = hipEventRecord(i & 1 ? e->ev1 : e->ev0, e->stream);
+    return ce;
+  };
+  hipError_t ce = fetch(0);
+  for (int64_t i = 0; i < pieces && ce == hipSuccess; i++) {
+    if (i + 1 < pieces) ce = fetch(i + 1);
+    if (ce == hipSuccess) ce = hipEventSynchronize(i & 1 ? e->ev1 : e->ev0);
+    if (ce != hipSuccess) break;
+    const int32_t *src = e->pinned + (i & 1) * HALF;
+    const int64_t p1 = std::min((i + 1) * HALF, b.npts);
+    for (int64_t p = i * HALF; p < p1;) {  // row by row
+      const int64_t row = p / b.hx, end = std::min(p1, (row + 1) * b.hx);
+      const int y2 = (int)(row % b.hy), z = (int)(row / b.hy), par = z & 1;
+      int32_t *g = latt + (int64_t)b.lx * ((int64_t)(2 * y2 + par) + (int64_t)b.ly * z) + par + 2 * (p - row * b.hx);
+      for (; p < end; p++, g += 2) {
+        const int32_t v = *src++;
+        if (*g != v) *g = v;
+      }
+    }
+  }
+  const hipError_t cs = hipStreamSynchronize(e->stream);
+  if (ce == hipSuccess) ce = cs;
+  if (ce != hipSuccess) return fail_(e, MSKG_EDEVICE, "store: %s", hipGetErrorString(ce));
   return MSKG_OK;
 }
 
@@ -3103,6 +3378,7 @@ void mskg_destroy(mskg_engine *e) {
   hipFree(e->d_field[0]); hipFree(e->d_field[1]); hipFree(e->d_offwall); hipFree(e->d_st_tables); hipFree(e->d_win);
   hipFree(e->d_done);
   for (int k = 0; k < 2; k++) hipFree(e->d_work[k]);
+  if (e->pinned) hipHostFree(e->pinned);
   hipFree(e->d_geo); hipFree(e->d_tab); hipFree(e->d_st); hipFree(e->d_err); hipFree(e->d_log);
   hipFree(e->d_tsum); hipFree(e->d_bsum); hipFree(e->d_key); hipFree(e->d_key_seen); hipFree(e->d_rate_seen);
   if (e->ev0) hipEventDestroy(e->ev0);
@@ -3118,23 +3394,44 @@ int mskg_load_state(mskg_engine *e, const int32_t *latt, int32_t n_ad, const int
   if (!e || !latt) return MSKG_EINVAL;
   if (!e->d_site) return fail_(e, MSKG_EINVAL, "engine not created");
   const Box &b = e->box;
-  e->slab = -1;
-  std::vector<Site> site((size_t)b.npts);
-  memset(site.data(), 0, site.size() * sizeof(Site));
-  std::vector<float> rate((size_t)b.npts, 0.0f);
-  std::vector<uint8_t> cls((size_t)b.npts, 0);
-  for (int z = 0; z <= b.lz; z++)
-    for (int y = 0; y < b.ly; y++)
-      for (int x = (z ^ y) & 1 ? -1 : (z & 1); x < b.lx; x += 2) {
-        if (x < 0) break;  // rows with y and z of different parity hold no lattice points
-        int32_t v = latt[(int64_t)x + (int64_t)b.lx * ((int64_t)y + (int64_t)b.ly * z)];
-        int kind = 0;
-        if (word_kind(e, v, &kind))
-          return fail_(e, MSKG_ESTATE, "LattCoo(%d,%d,%d)=0x%08x is not a representable site state", x, y, z, v);
-        Site &s = site[(size_t)pidx(b, x, y, z)];
-        s.kc = (uint8_t)(kind | (((v >> 24) & 7) << 3));
-        s.temp = (uint16_t)((v >> 9) & 0x1FFF);
-      }
+  const CovList C = cov_list(e);
+  const int64_t face = (int64_t)b.lx * b.ly, grid = face * (b.lz + 1);
+  // LattCoo goes to the device whole when that takes at most WORDS_WHOLE
+  // bytes, else in pieces of planes, once to be checked and once to be taken
+  // (an even number of planes: whole words of wall bits)
+  constexpr int64_t WORDS_WHOLE = 2ll << 30;
+  int64_t planes = b.lz + 1;
+  if (grid * 4 > WORDS_WHOLE) planes = std::max<int64_t>(2, (WORDS_WHOLE / 8) / (face * 4) / 2 * 2);
+  char *w = nullptr;
+  for (;; planes = std::max<int64_t>(2, planes / 4 * 2)) {  // smaller pieces when memory is short
+    planes = std::min<int64_t>(planes, b.lz + 1);
+    if ((w = (char *)work_take(e, 1, 16 + (size_t)(planes * face) * 4))) break;
+    if (planes <= 2) return fail_(e, MSKG_ENOMEM, "load: no device memory for a piece of LattCoo");
+  }
+  struct Done {  // the workspaces go back however the call ends
+    mskg_engine *e;
+    ~Done() { work_done(e); }
+  } at_end{e};
+  (void)at_end;
+  unsigned long long *d_out = (unsigned long long *)w;
+  int32_t *d_words = (int32_t *)(w + 16);
+  const bool whole = planes == b.lz + 1;
+  unsigned long long found[2] = {~0ull, 0ull};
+  HIPCHK(e, hipMemcpyAsync(d_out, found, sizeof found, hipMemcpyHostToDevice, e->stream));
+  auto blocks_of = [](int64_t n) { return dim3((unsigned)std::min<int64_t>((n + 255) / 256, 256 * 64)); };
+  for (int64_t z = 0; z <= b.lz; z += planes) {
+    const int64_t g0 = z * face, n = std::min(planes, b.lz + 1 - z) * face;
+    HIPCHK(e, hipMemcpyAsync(d_words, latt + g0, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
+    hipLaunchKernelGGL(k_words_check, blocks_of(n), dim3(256), 0, e->stream, b, C, d_words, g0, n, d_out);
+    HIPCHK(e, hipGetLastError());
+  }
+  HIPCHK(e, hipMemcpyAsync(found, d_out, sizeof found, hipMemcpyDeviceToHost, e->stream));
+  HIPCHK(e, hipStreamSynchronize(e->stream));
+  if (found[0] != ~0ull) {
+    const int64_t g = (int64_t)found[0];
+    return fail_(e, MSKG_ESTATE, "LattCoo(%d,%d,%d)=0x%08x is not a representable site state", (int)(g % b.lx),
+                 (int)(g / b.lx % b.ly), (int)(g / face), latt[g]);
+  }
   // planes above the stored ones: vacuum or walls only, which no event reaches
   for (int z = b.lz + 1; z <= e->logical_lz; z++)
     for (int y = 0; y < b.ly; y++)
@@ -3144,24 +3441,11 @@ int mskg_load_state(mskg_engine *e, const int32_t *latt, int32_t n_ad, const int
           return fail_(e, MSKG_ESTATE, "LattCoo(%d,%d,%d)=0x%08x lies above the %d stored planes", x, y, z, v,
                        b.lz + 1);
       }
-  // walls the caller's LattCoo holds off the lattice (index 113)
-  std::vector<uint32_t> offwall;
-  for (int z = 0; z <= b.lz; z++)
-    for (int y = 0; y < b.ly; y++)
-      for (int x = 0; x < b.lx; x++) {
-        if (valid_parity(x, y, z)) continue;
-        const int64_t g = (int64_t)x + (int64_t)b.lx * ((int64_t)y + (int64_t)b.ly * z);
-        if ((latt[g] & 255) != 113) continue;
-        if (offwall.empty()) offwall.assign((size_t)((b.lx * (int64_t)b.ly * (b.lz + 1) + 31) / 32), 0u);
-        offwall[(size_t)(g >> 5)] |= 1u << (g & 31);
-      }
-  hipFree(e->d_offwall);
-  e->d_offwall = nullptr;
-  e->offwall_planes = false;
-  if (!offwall.empty()) {
-    HIPCHK(e, hipMalloc(&e->d_offwall, offwall.size() * sizeof(uint32_t)));
-    HIPCHK(e, hipMemcpy(e->d_offwall, offwall.data(), offwall.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-  }
+  // the lists: checked, and every record as the device takes it
+  std::vector<StateRec> recs;
+  recs.reserve((size_t)std::max(n_ad, 0) + std::max(n_bulk, 0) + std::max(n_void, 0));
+  std::vector<bool> listed((size_t)b.npts, false);
+  bool again = false;  // a site is listed more than once
   double rsum = 0.0;
   auto put = [&](int which, int32_t n, const int32_t *xyz, const int32_t *nn) -> int {
     for (int32_t i = 0; i < n; i++) {
@@ -3179,23 +3463,40 @@ int mskg_load_state(mskg_engine *e, const int32_t *latt, int32_t n_ad, const int
         l.y[k] = nn[12 * i + 3 * k + 1];
         l.z[k] = nn[12 * i + 3 * k + 2];
       }
-      if (!set_list(b, site[(size_t)p], s[0], s[1], s[2], l))
+      union {
+        Site site;
+        uint32_t word[4];
+      } u;
+      memset(&u, 0, sizeof u);
+      if (!set_list(b, u.site, s[0], s[1], s[2], l))
         return fail_(e, MSKG_ESTATE, "list %d record %d at (%d,%d,%d): a NextNXYZ entry is too far away", which, i,
                      s[0], s[1], s[2]);
+      StateRec r;
+      r.p = p;
+      r.x = u.word[0];
+      r.y = u.word[1];
+      r.z = u.word[2];
+      r.valid = u.site.valid;
+      r.rate = 0.0f;
+      r.cls = -1;
       if (which == 0) {
+        const int32_t v = latt[(int64_t)s[0] + (int64_t)b.lx * ((int64_t)s[1] + (int64_t)b.ly * s[2])];
         int ev = ad_event ? ad_event[i] : 1;
         double pr = ad_prob ? ad_prob[i] : 0.0;
-        int kind = s_kind(site[(size_t)p]), coor = s_coor(site[(size_t)p]);
+        int kind = word_kind(C, v), coor = (v >> 24) & 7;
         int c;
         if (ev == 4) c = (kind_species(kind) && coor == 0) ? CLS_ISOLATED : CLS_EVAP;
         else if (ev == 5) c = CLS_DESORB;
         else if (kind == KIND_EMPTY && coor == 1 && (pr == (double)1.e-8f || pr == (double)1.e-6f)) c = CLS_PLACEHOLDER;
         else c = CLS_ADSORB;
         if (!(pr > 0.0)) return fail_(e, MSKG_ESTATE, "MC record %d has a non-positive rate", i);
-        cls[(size_t)p] = (uint8_t)c;
-        rate[(size_t)p] = (float)pr;
+        r.cls = c;
+        r.rate = (float)pr;
         rsum += pr;
       }
+      again |= listed[(size_t)p];
+      listed[(size_t)p] = true;
+      recs.push_back(r);
     }
     return 0;
   };
@@ -3203,9 +3504,34 @@ int mskg_load_state(mskg_engine *e, const int32_t *latt, int32_t n_ad, const int
   if ((rc = put(0, n_ad, ad_xyz, ad_nn))) return rc;
   if ((rc = put(1, n_bulk, bulk_xyz, bulk_nn))) return rc;
   if ((rc = put(2, n_void, void_xyz, void_nn))) return rc;
-  HIPCHK(e, hipMemcpyAsync(e->d_site, site.data(), site.size() * sizeof(Site), hipMemcpyHostToDevice, e->stream));
-  HIPCHK(e, hipMemcpyAsync(e->d_rate, rate.data(), rate.size() * 4, hipMemcpyHostToDevice, e->stream));
-  HIPCHK(e, hipMemcpyAsync(e->d_cls, cls.data(), cls.size(), hipMemcpyHostToDevice, e->stream));
+  if (again) merge_listed(recs);
+  StateRec *d_recs = nullptr;
+  if (!recs.empty()) {
+    d_recs = (StateRec *)work_take(e, 0, recs.size() * sizeof(StateRec));
+    if (!d_recs) return fail_(e, MSKG_ENOMEM, "load: no device memory for the lists");
+  }
+  // from here on the state changes
+  e->slab = -1;
+  hipFree(e->d_offwall);
+  e->d_offwall = nullptr;
+  e->offwall_planes = false;
+  if (found[1]) HIPCHK(e, hipMalloc(&e->d_offwall, (size_t)((grid + 31) / 32) * sizeof(uint32_t)));
+  Lattice L = make_lattice(e);
+  for (int64_t z = 0; z <= b.lz; z += planes) {
+    const int64_t nz = std::min(planes, b.lz + 1 - z), g0 = z * face, n = nz * face;
+    if (!whole) HIPCHK(e, hipMemcpyAsync(d_words, latt + g0, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
+    hipLaunchKernelGGL(k_words_in, blocks_of(nz * b.plane), dim3(256), 0, e->stream, L, C, d_words, g0, z * b.plane,
+                       (z + nz) * b.plane);
+    if (found[1])
+      hipLaunchKernelGGL(k_words_offwall, blocks_of(n), dim3(256), 0, e->stream, b, d_words, g0, n, e->d_offwall);
+    HIPCHK(e, hipGetLastError());
+  }
+  if (d_recs) {
+    HIPCHK(e, hipMemcpyAsync(d_recs, recs.data(), recs.size() * sizeof(StateRec), hipMemcpyHostToDevice, e->stream));
+    hipLaunchKernelGGL(k_lists_in, dim3((unsigned)((recs.size() + 255) / 256)), dim3(256), 0, e->stream, L, d_recs,
+                       (int64_t)recs.size());
+    HIPCHK(e, hipGetLastError());
+  }
   RunState st;
   memset(&st, 0, sizeof st);
   st.clock = kmc_time;
@@ -3673,76 +3999,21 @@ int mskg_store_state(mskg_engine *e, int32_t *latt, int32_t cap_ad, int32_t *n_a
                      int32_t *ad_event, double *ad_prob, int32_t cap_bulk, int32_t *n_bulk, int32_t *bulk_xyz,
                      int32_t *bulk_nn, int32_t cap_void, int32_t *n_void, int32_t *void_xyz, int32_t *void_nn) {
   if (!e || !e->loaded) return fail_(e, MSKG_EINVAL, "no state loaded");
-  const Box &b = e->box;
-  std::vector<Site> site((size_t)b.npts);
-  std::vector<float> rate((size_t)b.npts);
-  std::vector<uint8_t> cls((size_t)b.npts);
-  HIPCHK(e, hipMemcpyAsync(site.data(), e->d_site, site.size() * sizeof(Site), hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(e, hipMemcpyAsync(rate.data(), e->d_rate, rate.size() * 4, hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(e, hipMemcpyAsync(cls.data(), e->d_cls, cls.size(), hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(e, hipStreamSynchronize(e->stream));
-  int32_t na = 0, nb = 0, nv = 0;
-  bool over = false;
-  for (int z = 0; z <= b.lz; z++)
-    for (int y = 0; y < b.ly; y++)
-      for (int x = 0; x < b.lx; x++) {
-        if (!valid_parity(x, y, z)) continue;  // off-lattice grid points are left as the caller has them
-        int64_t g = (int64_t)x + (int64_t)b.lx * ((int64_t)y + (int64_t)b.ly * z);
-        size_t p = (size_t)pidx(b, x, y, z);
-        const Site &s = site[p];
-        int kind = s_kind(s), coor = s_coor(s);
-        if (latt) {
-          int32_t v = 0;
-          if (kind == KIND_WALL) v = (1 << 23) | 113;
-          else if (kind_species(kind)) v = (1 << 23) | (kind << 27);
-          else if (kind >= KIND_COV0) v = e->list_cov[kind - KIND_COV0];
-          v |= coor << 24;
-          v |= (int32_t)s.temp << 9;
-          latt[g] = v;
-        }
-        int32_t xyz[3] = {x, y, z};
-        NL l = site_list(b, s, x, y, z);
-        int32_t nn[12];
-        for (int i = 0; i < 4; i++) {
-          nn[3 * i] = l.x[i];
-          nn[3 * i + 1] = l.y[i];
-          nn[3 * i + 2] = l.z[i];
-        }
-        // the reference's list membership: an atom of coordination <= 3 is an MC
-        // particle even when it has no rate (a frozen-substrate atom)
-        if (cls[p] || (kind_species(kind) && coor <= 3)) {
-          if (na < cap_ad) {
-            if (ad_xyz) memcpy(ad_xyz + 3 * na, xyz, 12);
-            if (ad_nn) memcpy(ad_nn + 12 * na, nn, 48);
-            int c = cls[p];
-            if (ad_event) ad_event[na] = (c == CLS_EVAP || c == CLS_ISOLATED || !c) ? 4 : c == CLS_DESORB ? 5 : 1;
-            if (ad_prob) ad_prob[na] = (double)rate[p];
-          } else {
-            over = true;
-          }
-          na++;
-        } else if (kind_species(kind)) {
-          if (nb < cap_bulk) {
-            if (bulk_xyz) memcpy(bulk_xyz + 3 * nb, xyz, 12);
-            if (bulk_nn) memcpy(bulk_nn + 12 * nb, nn, 48);
-          } else {
-            over = true;
-          }
-          nb++;
-        } else if ((kind == KIND_EMPTY || kind >= KIND_COV0) && coor == 4) {
-          if (nv < cap_void) {
-            if (void_xyz) memcpy(void_xyz + 3 * nv, xyz, 12);
-            if (void_nn) memcpy(void_nn + 12 * nv, nn, 48);
-          } else {
-            over = true;
-          }
-          nv++;
-        }
-      }
+  int64_t tot[3] = {0, 0, 0};
+  const int64_t cap[3] = {cap_ad, cap_bulk, cap_void};
+  int32_t *const xyz[3] = {ad_xyz, bulk_xyz, void_xyz}, *const nn[3] = {ad_nn, bulk_nn, void_nn};
+  const int rc = state_lists(e, cap, xyz, nn, ad_event, ad_prob, tot);
+  int rc2 = MSKG_OK;
+  if (!rc && latt) rc2 = state_words(e, latt);
+  work_done(e);
+  if (rc || rc2) return rc ? rc : rc2;
+  const int32_t na = (int32_t)tot[0], nb = (int32_t)tot[1], nv = (int32_t)tot[2];
   if (n_ad) *n_ad = na;
   if (n_bulk) *n_bulk = nb;
   if (n_void) *n_void = nv;
-  if (over) return fail_(e, MSKG_ECAPACITY, "list capacity too small (need %d MC, %d bulk, %d void)", na, nb, nv);
+  if (tot[0] > std::max<int64_t>(cap_ad, 0) || tot[1] > std::max<int64_t>(cap_bulk, 0) ||
+      tot[2] > std::max<int64_t>(cap_void, 0))
+    return fail_(e, MSKG_ECAPACITY, "list capacity too small (need %d MC, %d bulk, %d void)", na, nb, nv);
   return MSKG_OK;
 }
 
