@@ -250,17 +250,18 @@ int mskg_run(mskg_engine *e, int64_t max_events, double max_time,
              int64_t *events_done, double *kmc_time, int32_t *stop_reason);
 
 /* How mskg_run orders the eight colour passes of a sweep (no reference
- * counterpart; the reference's loop is serial).  MSKG_SCHEDULE_COLOURS (the
- * default): one launch per colour, each waiting for the whole previous
- * colour.  MSKG_SCHEDULE_TILES: one launch per sweep in which a tile's pass
- * starts as soon as the neighbour tiles of lower colours have finished
- * theirs (a queue of tiles in colour order, per-tile completion flags with
- * agent-scope release / acquire).  Both give the same lattice, clock and
- * counters bit for bit: a tile sees the same state, and draws the same
- * random numbers, in either order.  On MI355X the tile schedule removes the
- * idle time at the colour barriers but each acquire invalidates the L2 of
- * the waiting wave's XCD, which the other waves of that XCD then refill:
- * the barrier schedule is the faster one there. */
+ * counterpart; the reference's loop is serial).  MSKG_SCHEDULE_COLOURS: one
+ * launch per colour, each waiting for the whole previous colour.
+ * MSKG_SCHEDULE_TILES: one launch per sweep in which a tile's pass starts as
+ * soon as the neighbour tiles of lower colours have finished theirs (a queue
+ * of tiles in colour order, per-tile completion flags).  Both give the same
+ * lattice, clock and counters bit for bit: a tile sees the same state, and
+ * draws the same random numbers, in either order.  The tile schedule removes
+ * the idle time at the colour barriers.  With up to 100 tiles a colour in a
+ * tile layer it runs on one of the GPU's XCDs, whose waves share an L2; over
+ * several XCDs its acquires invalidate L2s that the other waves then refill,
+ * and the barriers are faster.  By default (nothing set) a run takes the tile
+ * schedule where it fits one XCD and the colour passes elsewhere. */
 #define MSKG_SCHEDULE_TILES 1
 #define MSKG_SCHEDULE_COLOURS 0
 int mskg_set_schedule(mskg_engine *e, int32_t schedule);

@@ -946,7 +946,18 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 
 // tile is the sweep's stamp (sched[0], advanced by k_sweep_end), stored
 // with agent-scope release after the tile's writes; a waiting wave loads it
 // at agent scope and takes an agent-scope acquire before it reads the
-// neighbours' records, so the tiles' records travel between XCDs.
+// neighbours' records, so the tiles' records travel between XCDs.  That acquire
+// drops the XCD's whole L2, which costs more than the barriers it replaces
+// (512^3 SiC: 39.8 against 75.3 M events/s).
+//
+// The same sweep on one XCD (LOCAL): the waves of one XCD, whichever the
+// first wave to start is on, take all of the queue, and the others leave.
+// They share its L2, so that a tile's writes are released when the L2 has
+// them (its stores have returned) and acquired by dropping the CU's L1 alone.
+// What bounds a sweep of a small lattice is the chain of its slowest tiles,
+// a few events of about 5 us each a colour, with a launch of 4.5 us after
+// every colour, whether it has tiles or not: a film in one tile layer has
+// tiles in four of the eight.
 
 // The tile layers of colours with layer parity `odd` that a sweep's queue
 // holds, for candidates in layers [zlo, zhi] when the sweep starts: the
@@ -959,16 +970,53 @@ __device__ inline void queue_layers(int zlo, int zhi, int odd, int ntz, int &fir
   count = first <= hi ? (hi - first) / 2 + 1 : 0;
 }
 
-// A wave waits at most this long (wall-clock ticks of 10 ns) for a
-// neighbour tile; the run then stops with ERR_SCHED instead of hanging.
-constexpr long long SCHED_WAIT_TICKS = 200000000ll;
+// A wave polls at most this often (about 1 us each; a preempted wave does not
+// poll) for its neighbour tiles; the run then stops with ERR_SCHED instead of
+// hanging.
+constexpr int SCHED_POLLS = 1 << 22;
 
-template <bool LA, bool COV>
-__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_sweep(PassParams P) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ TabLds tabs;
+// A word another CU of the same XCD has written (the L1 is passed by: the
+// coherence of a workgroup whose waves may run on several CUs).
+__device__ inline unsigned int load_xcd(const unsigned int *p) {
+  unsigned int v;
+  asm volatile("global_load_dword %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(p) : "memory");
+  return v;
+}
+template <bool LOCAL>
+__device__ inline unsigned int load_flag(const unsigned int *p) {
+  return LOCAL ? load_xcd(p) : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool LOCAL>
+__device__ inline void sweep_acquire() {
+  if (LOCAL) asm volatile("buffer_inv sc1" ::: "memory");
+  else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+}
+template <bool LOCAL>
+__device__ inline void sweep_release() {
+  if (LOCAL) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+}
+// Is this wave on the XCD that runs the sweep `stamp`?  The first wave to ask
+// settles it (sched[5]: 4 bits of XCD below 28 of the stamp), so at least one
+// wave runs, and any number of waves drains the queue.
+__device__ inline bool on_sweeps_xcd(unsigned int *word, unsigned int stamp) {
+  const unsigned int xcc = (unsigned int)__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15u;  // HW_REG_XCC_ID, bits 0..3
+  const unsigned int mine = (stamp << 4) | xcc;
+  unsigned int v = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane((int)((v ^ mine) >> 4)) != 0) {  // an earlier sweep's
+    unsigned int seen = v;
+    if (threadIdx.x == 0 && __hip_atomic_compare_exchange_strong(word, &seen, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT))
+      seen = mine;
+    v = seen;
+  }
+  return __builtin_amdgcn_readfirstlane((int)v) == (int)mine;
+}
+
+template <bool LA, bool COV, bool LOCAL>
+__device__ inline void sweep_tiles(const PassParams &P, const PassParams *const pp, TabLds &tabs, unsigned char *smem) {
   const int lane = threadIdx.x;
-  const PassParams *const pp = kernel_params();
+  if (LOCAL && !on_sweeps_xcd(P.sched + 5, P.sched[0])) return;
   Lattice L = event_part(pp);
   RunState *st = P.st;
   const double tau = st->tau;
@@ -997,7 +1045,8 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 
   for (;;) {
     // the next entry: every lane adds 1 (one atomic of 64 for the wave), so
     // the head counts entries in units of 64
-    const unsigned int took = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned int took = LOCAL ? __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                    : __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int q = __builtin_amdgcn_readfirstlane((int)(took >> 6));
     if (q >= total) break;
     // entry -> colour, tile
@@ -1031,16 +1080,15 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 
         }
       }
     }
-    const unsigned int *const flag = P.done + (dep ? n : t);  // a lane without a neighbour reads its own tile's
+    // lane 26 reads the abort flag with them; a lane without a neighbour reads its own tile's
+    const unsigned int *const flag = lane == 26 ? P.sched + 2 : P.done + (dep ? n : t);
     bool abort = false;
     if (__ballot(dep) != 0ull) {
-      const long long t0 = wall_clock64();
-      for (;;) {
-        const unsigned int f = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int polls = 0;; polls++) {
+        const unsigned int f = load_flag<LOCAL>(flag);
         if (__ballot(dep && f != stamp) == 0ull) break;
-        const unsigned int ab = __hip_atomic_load(&P.sched[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool late = wall_clock64() - t0 > SCHED_WAIT_TICKS;
-        if (__builtin_amdgcn_readfirstlane((int)ab) != 0 || late) {
+        const bool late = polls >= SCHED_POLLS;
+        if (__builtin_amdgcn_readlane((int)f, 26) != 0 || late) {
           if (late) {  // every lane stores the same values
             __hip_atomic_store(&P.sched[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             atomicCAS(&st->err, 0, ERR_SCHED);
@@ -1048,20 +1096,40 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 
           abort = true;
           break;
         }
-        __builtin_amdgcn_s_sleep(2);
+        // a waiting wave's polls delay the tiles' own loads: with more than 64 of
+        // them about 1 us between two polls (40 x 64 cycles), else 0.3 us (edge
+        // 384: 6.0 against 6.1 ms, edge 96: 4.4 against 4.4)
+        if (LOCAL && gridDim.x > 8 * 64) __builtin_amdgcn_s_sleep(40);
+        else __builtin_amdgcn_s_sleep(LOCAL ? 12 : 2);
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
-    const int err_now = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&st->err, __ATOMIC_RELAXED,
-                                                                         __HIP_MEMORY_SCOPE_AGENT));
-    const int n_in = __builtin_amdgcn_readfirstlane(L.tl_n[t]);
+    // many tiles of the queue are empty: their length (and the run's error)
+    // alone is read past the caches, and only a tile with candidates pays for
+    // the acquire
+    const int now = (int)load_flag<LOCAL>(lane == 0 ? (const unsigned int *)L.tl_n + t : (const unsigned int *)&st->err);
+    const int n_in = __builtin_amdgcn_readlane(now, 0), err_now = __builtin_amdgcn_readlane(now, 1);
     if (!abort && !err_now && n_in > 0) {
+      if (__ballot(dep) != 0ull) sweep_acquire<LOCAL>();
       pass_tile<LA, COV>(pp, L, st, tau, t, colour, tabs, false, smem, lane);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // the tile's writes before its flag
+      sweep_release<LOCAL>();  // the tile's writes before its flag
     }
     // every lane stores the same stamp
-    __hip_atomic_store(&P.done[t], stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (LOCAL) __hip_atomic_store(&P.done[t], stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else __hip_atomic_store(&P.done[t], stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+template <bool LA, bool COV>
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_sweep(PassParams P) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ TabLds tabs;
+  sweep_tiles<LA, COV, false>(P, kernel_params(), tabs, smem);
+}
+template <bool LA, bool COV>
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_sweep_xcd(PassParams P) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ TabLds tabs;
+  sweep_tiles<LA, COV, true>(P, kernel_params(), tabs, smem);
 }
 
 // The fixed-order sum of the tile totals: block b sums its chunk of tiles
@@ -2685,6 +2753,10 @@ F pick_variant(bool la, bool cov, F tt, F tf, F ft, F ff) {
 
 }  // namespace
 
+// Until a caller sets a schedule: one XCD's sweep where the rule says so
+// (xcd_waves), else the colour passes.
+constexpr int SCHEDULE_AUTO = -1;
+
 struct mskg_engine {
   mskg_config cfg;
   bool cov_model = true;  // the kernels with the coverage-species branches
@@ -2722,7 +2794,7 @@ struct mskg_engine {
   // per-tile completion stamps of the dependency-scheduled sweep, then its
   // stamp / queue / window words (PassParams::done, ::sched)
   unsigned int *d_done = nullptr;
-  int schedule = MSKG_SCHEDULE_COLOURS;
+  int schedule = SCHEDULE_AUTO;
   Geometry *d_geo = nullptr;
   Tables *d_tab = nullptr;
   RunState *d_st = nullptr;
@@ -2855,7 +2927,7 @@ static const char *err_name(int c) {
     case ERR_SUMS: return "serial selection found no event inside a positive rate sum";
     case ERR_LIQUID: return "a species' CountLiquid is negative: its solidification rate would be negative";
     case ERR_ST_RANGE: return "a site's temperature lies outside the InitSt 'ST' reference temperatures";
-    case ERR_SCHED: return "a tile waited more than 2 s for its neighbour tiles in a dependency-scheduled sweep";
+    case ERR_SCHED: return "a tile waited too long (some seconds) for its neighbour tiles in a dependency-scheduled sweep";
     case ERR_TOP:
       return "an event site within 24 planes of the top of the stored planes (stored_len_z): store more planes";
     default: return "unknown";
@@ -3920,6 +3992,23 @@ static PassParams pass_params(mskg_engine *e) {
   return P;
 }
 
+// The waves a sweep on one XCD takes, 0: the lattice is too large for it.
+// A film in one tile layer keeps a colour's tiles of that layer busy, so about
+// as many waves are wanted (a wave that finds no tile free polls memory); an
+// XCD has 128 SIMDs, and past that its waves share issue slots that seven
+// other XCDs have idle.
+// Measured against the colour passes (whole runs, edge = tiles of 24): SiC,
+// k = 4, edge 96: 4.7, 4.4 ms; 240 (CVD): 11.1, 9.0; 384: 7.0, 6.0; 480: 6.9,
+// 6.0; 528: 7.2, 6.7; the shortest windows (policy 0, k = 1, where the queue's
+// own cost counts most), edge 384: 3.9, 3.4; 480: 4.3, 4.0; 528: 4.1, 4.3.  So
+// the line lies at 480's 100 tiles a colour and layer.  With tiles of 16 it
+// is the faster one well beyond (144 a colour: 4.8, 3.9).
+constexpr int XCD_TILES = 100;
+static int xcd_waves(const mskg_engine *e) {
+  const int colour = e->ntx * e->nty / 4;
+  return colour > XCD_TILES ? 0 : (colour + 15) / 8 * 8;
+}
+
 int mskg_run(mskg_engine *e, int64_t max_events, double max_time, int64_t *events_done, double *kmc_time,
              int32_t *stop_reason) {
   RunState st;
@@ -3934,7 +4023,10 @@ int mskg_run(mskg_engine *e, int64_t max_events, double max_time, int64_t *event
     PassParams P = pass_params(e);
     const bool la = e->tab.la_mode || e->tab.st_n;
     int grid = std::max(1, std::min(e->ntiles / 8 + 1, e->pass_grid));
-    if (e->schedule == MSKG_SCHEDULE_TILES) {
+    const int local = e->schedule == MSKG_SCHEDULE_COLOURS ? 0 : xcd_waves(e);
+    if (local) {
+      grid = 8 * local;  // workgroups go to the eight XCDs in turn
+    } else if (e->schedule == MSKG_SCHEDULE_TILES) {
       // every wave the device holds at once: the waves take tiles from the
       // sweep's queue until it is empty
       int per_cu = 0, cus = 0;
@@ -3944,7 +4036,9 @@ int mskg_run(mskg_engine *e, int64_t max_events, double max_time, int64_t *event
       grid = std::max(1, per_cu * cus);
     }
     HIPCHK(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    if (e->schedule == MSKG_SCHEDULE_TILES) {
+    if (local) {
+      hipLaunchKernelGGL(MSKG_VARIANT(k_sweep_xcd, la, e->cov_model), dim3(grid), dim3(WAVE), shm, e->stream, P);
+    } else if (e->schedule == MSKG_SCHEDULE_TILES) {
       hipLaunchKernelGGL(MSKG_VARIANT(k_sweep, la, e->cov_model), dim3(grid), dim3(WAVE), shm, e->stream, P);
     } else {
       for (int c = 0; c < 8; c++) {

@@ -342,8 +342,9 @@ class Engine:
 
     def set_schedule(self, schedule):
         """Order of a sweep's colour passes (mskg_set_schedule): "colours" (a
-        barrier after each colour; the default) or "tiles" (each tile as soon
-        as its lower-colour neighbours are done).  Same results bit for bit."""
+        barrier after each colour) or "tiles" (each tile as soon as its
+        lower-colour neighbours are done).  Same results bit for bit; without
+        a call small lattices take "tiles", the others "colours"."""
         code = {"tiles": _lib.MSKG_SCHEDULE_TILES, "colours": _lib.MSKG_SCHEDULE_COLOURS}[schedule]
         self._check(self.L.mskg_set_schedule(self.h, code))
 
