@@ -16,8 +16,8 @@
 //   k_sweep        the eight colours of a sweep in one launch, each tile
 //                  starting when its lower-colour neighbours are done (same
 //                  result as eight k_pass launches, without their barriers).
-//   k_rsum         fixed-order FP64 sum of the tile rate totals;
-//   k_sweep_end    -> next tau and the clock.
+//   k_sweep_end    fixed-order FP64 sum of the tile rate totals -> next tau
+//                  and the clock.
 //   k_serial       serial BKL over a batch of lattices (one wave each).
 //   k_adjoint      log replay with per-class likelihood statistics.
 //   k_build_slab, k_frame_count / k_frame_write: device builder, frame records.
@@ -62,8 +62,8 @@ struct Slot {
   unsigned long long n, tiles, events, counts[8];
 };
 // The FP64 total rate is summed without atomics, in a fixed order: every
-// tile keeps its total (Lattice::tile_r), NPART blocks each sum a fixed
-// chunk of tiles, and k_sweep_end sums the NPART partials.  A rerun with
+// tile keeps its total (Lattice::tile_r), k_sweep_end sums NPART fixed chunks
+// of tiles and then the NPART partials.  A rerun with
 // the same seed therefore repeats the same windows.
 constexpr int NPART = 2 * NSLOT;
 
@@ -99,7 +99,6 @@ struct RunState {
   // the sweep's working sums, last: the host reads and writes only the
   // fields before them (RS_HEAD bytes)
   Slot slot[NSLOT];
-  double rpart[NPART];  // partial sums of the tile totals (k_rsum)
 };
 constexpr size_t RS_HEAD = offsetof(RunState, slot);
 
@@ -112,7 +111,7 @@ struct PassParams {
   int cap;
   uint32_t key0, key1;
   int colour;
-  int rsum_chunk;           // tiles per block of the fixed-order tile sum (k_rsum)
+  int rsum_chunk;           // tiles a chunk of the fixed-order tile sum (chunk_sum)
   // dependency-scheduled sweep: per-tile completion stamps, and sched[0]
   // the sweep's stamp, [1] queue head, [2] abort flag, [3] / [4] the first /
   // last tile layer holding candidates when the sweep starts
@@ -412,23 +411,25 @@ __global__ void __launch_bounds__(WAVE) k_replay(Lattice L, const mskg_event *lo
 // ---- synchronous sublattice -------------------------------------------------
 // Build every tile's candidate list from the classes (after a state upload,
 // a rate sweep or a replay).  One wave per tile, four of its points a lane in
-// flight.  Tiles outside the layers [zlo, zhi] hold no MC particle and no list
-// flag, which the caller knows of a slab (touched_planes): their lists are
-// empty without a look at their points.
+// flight.  Points outside the planes [zlo, zhi] are no MC particles and have no
+// list flag, which the caller knows of a slab (touched_planes): only the planes
+// [zlo, zhi] are looked at, and the lists of tiles without any are empty.
 __global__ void __launch_bounds__(256) k_build_lists(Lattice L, int ntiles, int zlo, int zhi) {
   int lane = threadIdx.x & (WAVE - 1);
   int t = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
   if (t >= ntiles) return;
   TileGeom g = tile_geom(t, L.tile, L.ntx, L.nty, L.box.lz);
   int n = 0;
-  if (g.tz >= zlo && g.tz <= zhi) {
-    for (int k0 = 0; k0 < g.npt; k0 += 4 * WAVE) {
+  {
+    const int pp = g.half * g.half;
+    const int first = max(zlo - g.z0, 0) * pp, end = min(zhi + 1 - g.z0, g.nz) * pp;
+    for (int k0 = first; k0 < end; k0 += 4 * WAVE) {
       int kp[4];
       int64_t pi[4];
       uint8_t c[4];
       for (int u = 0; u < 4; u++) {
         const int k = k0 + u * WAVE + lane;
-        const bool in = k < g.npt;
+        const bool in = k < end;
         kp[u] = tile_nth(g, in ? k : 0);
         pi[u] = tile_point(L.box, g, L.tile, kp[u]).i;
         c[u] = in ? L.cls[pi[u]] : (uint8_t)0;
@@ -1132,63 +1133,49 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 
   sweep_tiles<LA, COV, true>(P, kernel_params(), tabs, smem);
 }
 
-// The fixed-order sum of the tile totals: block b sums its chunk of tiles
-// (each thread a fixed stride, then a tree in LDS) into rpart[b].
-__device__ inline void rsum_block(const double *tile_r, int ntiles, int chunk, RunState *st, int b, double *s) {
-  const int lo = b * chunk, hi = min(lo + chunk, ntiles);
-  double acc = 0.0;
-  for (int t = lo + (int)threadIdx.x; t < hi; t += 256) acc += tile_r[t];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) s[threadIdx.x] += s[threadIdx.x + off];
-    __syncthreads();
+// The fixed-order sum of the tile totals: chunk b of `chunk` tiles into
+// part[b], in the order of 256 threads with a stride of 256 and a binary tree
+// over them, which a wave keeps with four of those threads a lane.  Only
+// chunks with a tile in the layers [zlo, zhi] are read: a tile outside the
+// windows has no list and a total of zero.
+__device__ inline double chunk_sum(const double *tile_r, int lo, int hi, int lane) {
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int t = lo + lane; t < hi; t += 4 * 256) {
+    double v[4][4];
+    for (int r = 0; r < 4; r++)
+      for (int u = 0; u < 4; u++) {
+        const int k = t + 256 * r + 64 * u;
+        v[r][u] = k < hi ? tile_r[k] : 0.0;
+      }
+    for (int r = 0; r < 4; r++)
+      for (int u = 0; u < 4; u++) acc[u] += v[r][u];
   }
-  if (threadIdx.x == 0) st->rpart[b] = s[0];
-}
-__global__ void __launch_bounds__(256) k_rsum(const double *tile_r, int ntiles, int chunk, RunState *st) {
-  __shared__ double s[256];
-  rsum_block(tile_r, ntiles, chunk, st, blockIdx.x, s);
+  double x = (acc[0] + acc[2]) + (acc[1] + acc[3]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, WAVE);
+  return x;
 }
 
-// After the eight colour passes: the clock advances by the window just used
-// (operator splitting of the master equation over the colours), the next
-// window is events_per_pass / (largest tile rate), and the reference's
-// early stop applies when at most 20 MC particles remain (main.f:307-310).
+constexpr int END_THREADS = 1024;
+constexpr int SLOT_WORDS = (int)(sizeof(Slot) / 8);
+static_assert(SLOT_WORDS == 12 && offsetof(Slot, rmax) == 0 && offsetof(Slot, counts) == 32, "a wave a word of Slot");
+static_assert(RS_HEAD % 4 == 0, "RunState's head in words");
 struct SweepEndLds {
-  double srsum[NSLOT];
-  unsigned long long srmax[NSLOT], sn[NSLOT], stl[NSLOT], sev[NSLOT], scnt[8][NSLOT];
+  double part[NPART];
+  unsigned long long sum[SLOT_WORDS];  // Slot's words: the largest rmax, the others summed
+  __align__(8) unsigned int head[RS_HEAD / 4];
+  int win[32];
+  int list_err, zlo, zhi;
+  unsigned int sched0;
 };
-__device__ inline void sweep_end(RunState *st, int *win, const int *list_err, unsigned int *sched,
-                                 SweepEndLds &E) {
-  double *srsum = E.srsum;
-  unsigned long long *srmax = E.srmax, *sn = E.sn, *stl = E.stl, *sev = E.sev;
-  unsigned long long(*scnt)[NSLOT] = E.scnt;
-  const int i = threadIdx.x;
-  Slot &sl = st->slot[i];
-  srsum[i] = st->rpart[i] + st->rpart[i + NSLOT];
-  srmax[i] = sl.rmax; sn[i] = sl.n; stl[i] = sl.tiles; sev[i] = sl.events;
-  for (int q = 0; q < 8; q++) scnt[q][i] = sl.counts[q];
-  sl.rmax = 0ull; sl.n = 0ull; sl.tiles = 0ull; sl.events = 0ull;
-  for (int q = 0; q < 8; q++) sl.counts[q] = 0ull;
-  __syncthreads();
-  for (int off = NSLOT / 2; off > 0; off >>= 1) {
-    if (i < off) {
-      srsum[i] += srsum[i + off];
-      srmax[i] = srmax[i] > srmax[i + off] ? srmax[i] : srmax[i + off];
-      sn[i] += sn[i + off];
-      stl[i] += stl[i + off];
-      sev[i] += sev[i + off];
-      for (int q = 0; q < 8; q++) scnt[q][i] += scnt[q][i + off];
-    }
-    __syncthreads();
-  }
-  if (i != 0) return;
-  const double rmax = __longlong_as_double((long long)srmax[0]);
-  const double rsum = srsum[0];
-  const long long nmc = (long long)sn[0];
-  st->events += sev[0];
-  for (int q = 0; q < 8; q++) st->counts[q] += scnt[q][0];
+// One thread's part: the state after the sweep, from its head's copy st.
+__device__ inline void sweep_end_state(const PassParams &P, SweepEndLds &E, RunState *st, const double rsum) {
+  int *const win = P.L.win;
+  unsigned int *const sched = P.sched;
+  const double rmax = __longlong_as_double((long long)E.sum[0]);
+  const long long nmc = (long long)E.sum[1];
+  st->events += E.sum[3];
+  for (int q = 0; q < 8; q++) st->counts[q] += E.sum[4 + q];
   if (st->la_variant)  // CountLiquid for the next sweep (main.f:637 of the laser-annealing build)
     for (int k = 0; k < 3; k++) {
       st->cc[k] += (long long)st->dcc[k];
@@ -1202,23 +1189,23 @@ __device__ inline void sweep_end(RunState *st, int *win, const int *list_err, un
   int zlo = 0x7fffffff, zhi = -1;
   for (int c = 0; c < 8; c++) {
     if (passes_ran) {
-      win[4 * c] = win[4 * c + 2];
-      win[4 * c + 1] = win[4 * c + 3];
+      win[4 * c] = E.win[4 * c] = E.win[4 * c + 2];
+      win[4 * c + 1] = E.win[4 * c + 1] = E.win[4 * c + 3];
       win[4 * c + 2] = 0x7fffffff;
       win[4 * c + 3] = -1;
     }
-    zlo = min(zlo, win[4 * c]);
-    zhi = max(zhi, win[4 * c + 1]);
+    zlo = min(zlo, E.win[4 * c]);
+    zhi = max(zhi, E.win[4 * c + 1]);
   }
   st->ever_lo = min(st->ever_lo, zlo);
   st->ever_hi = max(st->ever_hi, zhi);
   // the dependency-scheduled sweep: a new stamp, an empty queue, the window
-  sched[0]++;
+  sched[0] = E.sched0 + 1u;
   sched[1] = 0u;
   sched[2] = 0u;
   sched[3] = (unsigned int)zlo;
   sched[4] = (unsigned int)zhi;
-  if (*list_err && !st->err) st->err = *list_err;
+  if (E.list_err && !st->err) st->err = E.list_err;
   if (st->tau > 0.0 && !st->err && !st->stop) {
     // a window shortened to end at the time limit lands on it exactly
     st->clock = st->final_sweep ? st->max_time : st->clock + st->tau;
@@ -1230,7 +1217,7 @@ __device__ inline void sweep_end(RunState *st, int *win, const int *list_err, un
   st->n_mc = nmc;
   if (rsum > 0.0) st->rtot = rsum;
   if (st->tau_policy == 1)
-    st->tau = rsum > 0.0 ? st->events_per_pass * (double)stl[0] / rsum : 0.0;
+    st->tau = rsum > 0.0 ? st->events_per_pass * (double)E.sum[2] / rsum : 0.0;
   else
     st->tau = rmax > 0.0 ? st->events_per_pass / rmax : 0.0;
   if (!st->stop) {
@@ -1245,10 +1232,76 @@ __device__ inline void sweep_end(RunState *st, int *win, const int *list_err, un
     st->final_sweep = 1;
   }
 }
-__global__ void __launch_bounds__(NSLOT) k_sweep_end(RunState *st, int *win, const int *list_err,
-                                                     unsigned int *sched) {
+
+// After the eight colour passes: the clock advances by the window just used
+// (operator splitting of the master equation over the colours), the next
+// window is events_per_pass / (largest tile rate), and the reference's
+// early stop applies when at most 20 MC particles remain (main.f:307-310).
+//
+// One block of END_THREADS: what it needs leaves memory in two round trips --
+// a wave a word of the slots, one the windows, two the state's head; then a
+// wave a chunk of tiles -- and one thread works on the copy in LDS and writes
+// the state.  What bounds it: the launch and those round trips (the tile sums
+// had a launch of their own, and the slots a tree of barriers: 10 us a sweep,
+// 16.5 at 512^3 SiC).
+__device__ inline void sweep_end(const PassParams &P, SweepEndLds &E) {
+  int *const win = P.L.win;
+  unsigned int *const sched = P.sched;
+  const int i = threadIdx.x, lane = i & (WAVE - 1), w = i / WAVE;
+  if (i < NPART) E.part[i] = 0.0;
+  if (w < SLOT_WORDS) {
+    unsigned long long *const a = (unsigned long long *)P.st->slot + (size_t)lane * SLOT_WORDS + w;
+    static_assert(NSLOT == 2 * WAVE, "two slots a lane");
+    unsigned long long v = a[0], o = a[WAVE * SLOT_WORDS];
+    a[0] = 0ull;
+    a[WAVE * SLOT_WORDS] = 0ull;
+    for (int off = WAVE; off > 0; off >>= 1) {  // the lane's other slot first, then the other lanes
+      if (off < WAVE) o = __shfl_xor(v, off, WAVE);
+      v = w == 0 ? (v > o ? v : o) : v + o;
+    }
+    if (lane == 0) E.sum[w] = v;
+  } else if (w == SLOT_WORDS) {
+    const int v = win[lane & 31];
+    if (lane < 32) E.win[lane] = v;
+    // the windows of this sweep and of the next: tiles outside hold no rate
+    int lo = lane < 32 && !(lane & 1) ? v : 0x7fffffff, hi = lane < 32 && (lane & 1) ? v : -1;
+    for (int off = 32; off > 0; off >>= 1) {
+      lo = min(lo, __shfl_xor(lo, off, WAVE));
+      hi = max(hi, __shfl_xor(hi, off, WAVE));
+    }
+    if (lane == 0) {
+      E.zlo = max(lo, 0);
+      E.zhi = min(hi, P.ntz - 1);
+    }
+  } else if (w == SLOT_WORDS + 1) {
+    const unsigned int *const h = (const unsigned int *)P.st;
+    for (int k = lane; k < (int)(RS_HEAD / 4); k += WAVE) E.head[k] = h[k];
+  } else if (w == SLOT_WORDS + 2 && lane == 0) {
+    E.list_err = *P.L.list_err;
+    E.sched0 = sched[0];
+  }
+  __syncthreads();
+  if (E.zlo <= E.zhi) {
+    const int layer = P.L.ntx * P.L.nty, ntiles = layer * P.ntz, chunk = P.rsum_chunk;
+    const int last = min(((E.zhi + 1) * layer - 1) / chunk, NPART - 1);
+    for (int b = E.zlo * layer / chunk + w; b <= last; b += END_THREADS / WAVE) {
+      const double x = chunk_sum(P.L.tile_r, b * chunk, min(b * chunk + chunk, ntiles), lane);
+      if (lane == 0) E.part[b] = x;
+    }
+  }
+  __syncthreads();
+  if (w != 0) return;
+  double rs = (E.part[lane] + E.part[lane + NSLOT]) + (E.part[lane + WAVE] + E.part[lane + WAVE + NSLOT]);
+  for (int off = 32; off > 0; off >>= 1) rs += __shfl_down(rs, off, WAVE);
+  RunState *const st = (RunState *)E.head;  // the copy: its head only
+  if (i == 0) sweep_end_state(P, E, st, rs);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  unsigned int *const h = (unsigned int *)P.st;
+  for (int k = lane; k < (int)(RS_HEAD / 4); k += WAVE) h[k] = E.head[k];
+}
+__global__ void __launch_bounds__(END_THREADS) k_sweep_end(PassParams P) {
   __shared__ SweepEndLds E;
-  sweep_end(st, win, list_err, sched, E);
+  sweep_end(P, E);
 }
 
 // ---- the batched ensemble: one sweep over many lattices ------------------------
@@ -1380,23 +1433,15 @@ k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
   }
 }
 
-// Tile sums and the sweep's end for every replica that ran the sweep (the
-// same per-replica work as k_rsum and k_sweep_end, so the replica's window,
-// clock and stop are those it gets alone).
-__global__ void __launch_bounds__(256) k_rsum_ens(const PassParams *__restrict__ reps, int n, const int *plan) {
-  __shared__ double s[256];
-  const int r = blockIdx.y;
-  if (!plan[8 * (n + 1) + 9 + r]) return;
-  const PassParams &P = reps[r];
-  rsum_block(P.L.tile_r, P.L.ntx * P.L.nty * P.ntz, P.rsum_chunk, P.st, blockIdx.x, s);
-}
-__global__ void __launch_bounds__(NSLOT) k_sweep_end_ens(const PassParams *__restrict__ reps, int n,
-                                                         const int *plan) {
+// The sweep's end for every replica that ran the sweep (the same per-replica
+// work as k_sweep_end, so the replica's window, clock and stop are those it
+// gets alone).
+__global__ void __launch_bounds__(END_THREADS) k_sweep_end_ens(const PassParams *__restrict__ reps, int n,
+                                                               const int *plan) {
   __shared__ SweepEndLds E;
   const int r = blockIdx.x;
   if (!plan[8 * (n + 1) + 9 + r]) return;
-  const PassParams &P = reps[r];
-  sweep_end(P.st, P.L.win, P.L.list_err, P.sched, E);
+  sweep_end(reps[r], E);
 }
 
 // ---- device-side initial state ----------------------------------------------
@@ -2981,8 +3026,7 @@ static void work_done(mskg_engine *e) {
       e->work_n[k] = 0;
     }
 }
-// The run state's fields before the sweep sums (slot, rpart: left as they
-// are in st).
+// The run state's fields before the sweep sums (slot: left as it is in st).
 static int read_state(mskg_engine *e, RunState &st) {
   HIPCHK(e, hipMemcpyAsync(&st, e->d_st, RS_HEAD, hipMemcpyDeviceToHost, e->stream));
   HIPCHK(e, hipStreamSynchronize(e->stream));
@@ -3910,14 +3954,32 @@ int mskg_replay(mskg_engine *e, const mskg_event *log, int64_t n, int32_t clock_
   return MSKG_OK;
 }
 
+// The pass kernels' parameters of an engine (colour 0).
+static PassParams pass_params(mskg_engine *e) {
+  PassParams P;
+  P.L = make_lattice(e);
+  P.st = e->d_st;
+  P.log = e->d_log;
+  P.log_cap = (unsigned long long)e->log_cap;
+  P.ntz = e->ntz;
+  P.cap = e->cap;
+  P.key0 = (uint32_t)e->cfg.seed;
+  P.key1 = (uint32_t)(e->cfg.seed >> 32);
+  P.colour = 0;
+  P.rsum_chunk = e->rsum_chunk;
+  P.done = e->d_done;
+  P.sched = e->d_done + e->ntiles;
+  return P;
+}
+
 // The tile lists of the present classes.  Of a slab whose list flags were
 // cleared when it was built (flags_clean), only the touched planes hold any.
 static int build_lists(mskg_engine *e, const Lattice &L) {
   int z0 = 0, z1 = e->box.lz;
   if (e->flags_clean) touched_planes(e, z0, z1);
   HIPCHK(e, hipMemsetAsync(e->d_list_err, 0, sizeof(int), e->stream));
-  hipLaunchKernelGGL(k_build_lists, dim3((e->ntiles + 3) / 4), dim3(256), 0, e->stream, L, e->ntiles, z0 / e->tile,
-                     z1 / e->tile);
+  hipLaunchKernelGGL(k_build_lists, dim3((e->ntiles + 3) / 4), dim3(256), 0, e->stream, L, e->ntiles, z0,
+                     z1);
   HIPCHK(e, hipGetLastError());
   e->lists_dirty = false;
   return MSKG_OK;
@@ -3966,30 +4028,9 @@ static int run_begin(mskg_engine *e, int64_t max_events, double max_time, RunSta
   // tile totals of the current rates, then the first window
   hipLaunchKernelGGL(k_tile_rates, dim3(tblocks), dim3(256), 0, e->stream, L, e->ntiles, e->d_st);
   HIPCHK(e, hipGetLastError());
-  hipLaunchKernelGGL(k_rsum, dim3(NPART), dim3(256), 0, e->stream, e->d_tile_r, e->ntiles, e->rsum_chunk,
-                       e->d_st);
-  hipLaunchKernelGGL(k_sweep_end, dim3(1), dim3(NSLOT), 0, e->stream, e->d_st, e->d_win, e->d_list_err,
-                       e->d_done + e->ntiles);
+  hipLaunchKernelGGL(k_sweep_end, dim3(1), dim3(END_THREADS), 0, e->stream, pass_params(e));
   HIPCHK(e, hipGetLastError());
   return MSKG_OK;
-}
-
-// The pass kernels' parameters of an engine (colour 0).
-static PassParams pass_params(mskg_engine *e) {
-  PassParams P;
-  P.L = make_lattice(e);
-  P.st = e->d_st;
-  P.log = e->d_log;
-  P.log_cap = (unsigned long long)e->log_cap;
-  P.ntz = e->ntz;
-  P.cap = e->cap;
-  P.key0 = (uint32_t)e->cfg.seed;
-  P.key1 = (uint32_t)(e->cfg.seed >> 32);
-  P.colour = 0;
-  P.rsum_chunk = e->rsum_chunk;
-  P.done = e->d_done;
-  P.sched = e->d_done + e->ntiles;
-  return P;
 }
 
 // The waves a sweep on one XCD takes, 0: the lattice is too large for it.
@@ -4046,10 +4087,7 @@ int mskg_run(mskg_engine *e, int64_t max_events, double max_time, int64_t *event
         hipLaunchKernelGGL(MSKG_VARIANT(k_pass, la, e->cov_model), dim3(grid), dim3(WAVE), shm, e->stream, P);
       }
     }
-    hipLaunchKernelGGL(k_rsum, dim3(NPART), dim3(256), 0, e->stream, e->d_tile_r, e->ntiles, e->rsum_chunk,
-                       e->d_st);
-    hipLaunchKernelGGL(k_sweep_end, dim3(1), dim3(NSLOT), 0, e->stream, e->d_st, e->d_win, e->d_list_err,
-                       e->d_done + e->ntiles);
+    hipLaunchKernelGGL(k_sweep_end, dim3(1), dim3(END_THREADS), 0, e->stream, P);
     HIPCHK(e, hipStreamEndCapture(e->stream, &e->graph));
     HIPCHK(e, hipGraphInstantiate(&e->graph_exec, e->graph, nullptr, nullptr, 0));
   }
@@ -4730,8 +4768,7 @@ int mskg_run_ensemble(mskg_engine *const *engines, int32_t n, const int64_t *max
       if (c) hipLaunchKernelGGL(k_ens_plan, dim3(1), dim3(ENS_MAX), 0, sm, d_reps, n, d_plan, c, 0);
       hipLaunchKernelGGL(kpass, dim3(grid), dim3(WAVE), shm, sm, d_reps, n, d_plan, c);
     }
-    hipLaunchKernelGGL(k_rsum_ens, dim3(NPART, n), dim3(256), 0, sm, d_reps, n, d_plan);
-    hipLaunchKernelGGL(k_sweep_end_ens, dim3(n), dim3(NSLOT), 0, sm, d_reps, n, d_plan);
+    hipLaunchKernelGGL(k_sweep_end_ens, dim3(n), dim3(END_THREADS), 0, sm, d_reps, n, d_plan);
     hipLaunchKernelGGL(k_ens_plan, dim3(1), dim3(ENS_MAX), 0, sm, d_reps, n, d_plan, 0, 1);
     ce = hipStreamEndCapture(sm, &graph);
   }
