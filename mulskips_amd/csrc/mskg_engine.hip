@@ -101,6 +101,41 @@ struct RunState {
   Slot slot[NSLOT];
 };
 constexpr size_t RS_HEAD = offsetof(RunState, slot);
+// What the host asks of many engines' states at once.
+struct RunHead {
+  double clock, rtot;
+  unsigned long long events, log_n;
+  int err, stop, list_err;
+  int ever_lo, ever_hi;
+};
+// A run state's start: `words` words to clear (the state, or its slots alone)
+// by one small block, which takes the place of copies of 15 KB from the host.
+__device__ inline void clear_words(unsigned int *w, int words) {
+  for (int i = threadIdx.x; i < words; i += blockDim.x) w[i] = 0u;
+}
+__global__ void __launch_bounds__(256) k_state_new(RunState *st, double events_per_pass, double rtot,
+                                                   unsigned long long *atoms, int *err) {
+  clear_words((unsigned int *)st, (int)(sizeof(RunState) / 4));
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  st->events_per_pass = events_per_pass;
+  st->rtot = rtot;
+  atoms[0] = atoms[1] = 0ull;
+  *err = 0;
+}
+// The heads of n engines' states (ptr: their states, then their list errors).
+__global__ void __launch_bounds__(64) k_heads(const void *const *ptr, int n, RunHead *out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const RunState *const st = (const RunState *)ptr[i];
+  RunHead h;
+  h.clock = st->clock; h.rtot = st->rtot;
+  h.events = st->events; h.log_n = st->log_n;
+  h.err = st->err; h.stop = st->stop;
+  h.list_err = *(const int *)ptr[n + i];
+  h.ever_lo = st->ever_lo; h.ever_hi = st->ever_hi;
+  out[i] = h;
+}
 
 struct PassParams {
   Lattice L;
@@ -315,8 +350,9 @@ __device__ inline void sweep_group(const Lattice &L, double rtot, int *err, int 
 
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_rate_sweep(Lattice L, double rtot, int *err, int atoms_only) {
+k_rate_sweep(Lattice L, const double *rtot_at, int *err, int atoms_only) {
   L.tab = as_constant(L.tab);
+  const double rtot = rtot_at ? *rtot_at : 0.0;
   const int64_t n = L.box.npts;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
   for (int64_t p0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; p0 < n; p0 += stride)
@@ -328,8 +364,9 @@ k_rate_sweep(Lattice L, double rtot, int *err, int atoms_only) {
 // holds fewer than 2^31 groups).
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_rate_sweep_range(Lattice L, double rtot, int *err, int atoms_only, int64_t first, int64_t end) {
+k_rate_sweep_range(Lattice L, const double *rtot_at, int *err, int atoms_only, int64_t first, int64_t end) {
   L.tab = as_constant(L.tab);
+  const double rtot = rtot_at ? *rtot_at : 0.0;
   const int g_first = (int)(first >> 2), g_end = (int)((end + 3) >> 2);
   const int gstride = gridDim.x * blockDim.x;
   for (int g = g_first + blockIdx.x * blockDim.x + threadIdx.x; g < g_end; g += gstride)
@@ -2002,9 +2039,10 @@ struct AdjDesc {
   const mskg_event *log;
   const double *dt;
   long long n;
-  const int *cnt0;           // [KEY_N + 1] initial class populations, then the unsupported points
-  const double *iso0;        // initial sum of isolated-atom rates
-  const int *sweep_err;      // the rate sweep's error flag (the engine's)
+  int *cnt0;                 // [KEY_N + 1] initial class populations, then the unsupported points
+  double *iso0;              // initial sum of isolated-atom rates
+  int *sweep_err;            // the rate sweep's error flag (the engine's)
+  int fresh;                 // the keys are not current: a rate sweep first
   double *S;                 // [ADJ_NS]
   double *A;                 // [KEY_N]
   double *scal;              // [4]: sum dt, integral of isolated rates, sum of their log rates, events
@@ -2181,17 +2219,41 @@ __global__ void __launch_bounds__(256) k_adj_errs(const AdjDesc *descs, int n, i
   if (i < n) out[i] = descs[i].st->err;
 }
 
-// Initial class populations and isolated-rate sum of one lattice.
-__global__ void __launch_bounds__(256) k_key_hist(Lattice L, int *cnt, double *iso) {
-  const int64_t n = L.box.npts;
-  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
-    const int k = L.key[p];
-    if (k == KEY_ISO) atomicAdd(iso, (double)L.rate[p]);
-    if (k >= 0) atomicAdd(&cnt[k], 1);
-    else if (k == KEY_UNSUPPORTED) atomicAdd(&cnt[KEY_N], 1);
+// Every segment's start in one launch (block row y: segment y): the rates and
+// keys where they are not current, the class populations and isolated-rate
+// sum, and the keys and rates as first seen, four points a thread.  What
+// bounds it: the records' bytes where a sweep is needed (21 and 16 more a
+// point); a launch and two copies a segment had left most of the chip idle
+// (128 lattices of 144^3: 3.1 ms of device time and 640 calls).
+__global__ void __launch_bounds__(64) k_adj_clear(const AdjDesc *descs, int n) {
+  const int i = blockIdx.x;
+  for (int c = threadIdx.x; c < KEY_N + 1; c += blockDim.x) descs[i].cnt0[c] = 0;
+  if (threadIdx.x == 0) {
+    *descs[i].iso0 = 0.0;
+    *descs[i].sweep_err = 0;
   }
 }
-
+template <bool LA, bool COV>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_adj_start(const AdjDesc *descs) {
+  const AdjDesc &D = descs[blockIdx.y];
+  Lattice L = D.L;
+  to_global(L);
+  const double rtot = D.st->rtot;
+  const int64_t n = L.box.npts, stride = (int64_t)gridDim.x * blockDim.x * 4;
+  for (int64_t p0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; p0 < n; p0 += stride) {
+    if (D.fresh) sweep_group<LA, COV>(L, rtot, D.sweep_err, 0, p0, n);
+    for (int64_t p = p0; p < n && p < p0 + 4; p++) {
+      const int k = L.key[p];
+      const float r = L.rate[p];
+      D.key_seen[p] = k;
+      D.rate_seen[p] = r;
+      if (k == KEY_ISO) atomicAdd(D.iso0, (double)r);
+      if (k >= 0) atomicAdd(&D.cnt0[k], 1);
+      else if (k == KEY_UNSUPPORTED) atomicAdd(&D.cnt0[KEY_N], 1);
+    }
+  }
+}
 
 // ---- frame compaction (the xyz output of inpout/WriteMolMolXYZFile.f) --------
 // Ordered record lists in the reference's grid order (z, then y, then x; the
@@ -2871,7 +2933,7 @@ struct mskg_engine {
   int slab = -1, slab_z0 = 0, slab_z1 = 0;
   bool flags_clean = false;  // no list flag outside the touched planes (d_inlist), while they are known
   // workspaces of the frames: kept while they are small (WORK_KEEP)
-  int32_t *pinned = nullptr;  // page-locked words of the host's LattCoo on their way (8 MB, on first use)
+  int32_t *pinned = nullptr;  // page-locked buffer of the host's data on its way (8 MB, on first use)
   void *d_work[2] = {nullptr, nullptr};
   size_t work_n[2] = {0, 0};
   std::string err;
@@ -3055,6 +3117,75 @@ static FramePlan frame_plan(const mskg_engine *e, int z0, int z1, int sic, int m
   return F;
 }
 
+// Host pieces into device memory at dst + off (offsets increasing), through
+// the two halves of e's page-locked buffer: one copy for many small pieces,
+// the next half filled while the last is on its way.
+struct HostPiece {
+  size_t off;
+  const void *src;
+  size_t n;
+};
+constexpr int64_t PINNED_HALF = 4 << 20;  // bytes
+static hipError_t pinned_buffer(mskg_engine *e) {
+  return e->pinned ? hipSuccess : hipHostMalloc((void **)&e->pinned, 2 * PINNED_HALF, hipHostMallocDefault);
+}
+static hipError_t stage_in(mskg_engine *e, hipStream_t sm, char *dst, const std::vector<HostPiece> &pieces) {
+  hipError_t ce = pinned_buffer(e);
+  size_t begin = 0, fill = 0;  // the half holds [begin, begin + fill)
+  int half = 0;
+  bool used[2] = {false, false};
+  auto flush = [&]() {
+    if (!fill || ce != hipSuccess) return;
+    ce = hipMemcpyAsync(dst + begin, (char *)e->pinned + half * PINNED_HALF, fill, hipMemcpyHostToDevice, sm);
+    if (ce == hipSuccess) ce = hipEventRecord(half ? e->ev1 : e->ev0, sm);
+    used[half] = true;
+    half ^= 1;
+    fill = 0;
+  };
+  for (const HostPiece &p : pieces)
+    for (size_t done = 0; done < p.n && ce == hipSuccess;) {
+      const size_t off = p.off + done;
+      if (fill && off - begin >= (size_t)PINNED_HALF) flush();
+      if (!fill) {
+        begin = off;
+        if (used[half] && ce == hipSuccess) ce = hipEventSynchronize(half ? e->ev1 : e->ev0);
+      }
+      if (ce != hipSuccess) break;
+      const size_t m = std::min(p.n - done, (size_t)PINNED_HALF - (off - begin));
+      memcpy((char *)e->pinned + half * PINNED_HALF + (off - begin), (const char *)p.src + done, m);
+      fill = off - begin + m;
+      done += m;
+      if (fill == (size_t)PINNED_HALF) flush();
+    }
+  flush();
+  // the buffer is the next caller's when this returns
+  const hipError_t cs = hipStreamSynchronize(sm);
+  return ce == hipSuccess ? cs : ce;
+}
+
+// The heads of n engines' run states in one exchange, once their own streams
+// are idle (an exchange each had cost about 20 us an engine).
+static int read_heads(mskg_engine *const *engines, int n, std::vector<RunHead> &out) {
+  mskg_engine *e0 = engines[0];
+  out.resize(n);
+  std::vector<const void *> ptr(2 * (size_t)n);
+  for (int i = 0; i < n; i++) {
+    HIPCHK(engines[i], hipStreamSynchronize(engines[i]->stream));
+    ptr[i] = engines[i]->d_st;
+    ptr[n + i] = engines[i]->d_list_err;
+  }
+  char *w = (char *)work_take(e0, 0, (size_t)n * (2 * sizeof(void *) + sizeof(RunHead)));
+  if (!w) return fail_(e0, MSKG_ENOMEM, "no device memory for the states of %d engines", n);
+  const void **d_ptr = (const void **)w;
+  RunHead *d_out = (RunHead *)(w + 2 * (size_t)n * sizeof(void *));
+  HIPCHK(e0, hipMemcpyAsync(d_ptr, ptr.data(), ptr.size() * sizeof(void *), hipMemcpyHostToDevice, e0->stream));
+  hipLaunchKernelGGL(k_heads, dim3((n + 63) / 64), dim3(64), 0, e0->stream, d_ptr, n, d_out);
+  HIPCHK(e0, hipGetLastError());
+  HIPCHK(e0, hipMemcpyAsync(out.data(), d_out, (size_t)n * sizeof(RunHead), hipMemcpyDeviceToHost, e0->stream));
+  HIPCHK(e0, hipStreamSynchronize(e0->stream));
+  return MSKG_OK;
+}
+
 // The ordered record lists of one frame mode (k_frame_count / k_frame_write):
 // hosts[k] receives list k (caps[k] records), counts the NCNT totals.  A call
 // with too small capacities only sizes the lists (MSKG_ECAPACITY when it
@@ -3219,8 +3350,8 @@ static int state_lists(mskg_engine *e, const int64_t cap[3], int32_t *const xyz[
 // not written again (most of a box is vacuum, and so is a fresh array).
 static int state_words(mskg_engine *e, int32_t *latt) {
   const Box &b = e->box;
-  constexpr int64_t HALF = 1 << 20;  // words
-  if (!e->pinned) HIPCHK(e, hipHostMalloc((void **)&e->pinned, 2 * HALF * 4, hipHostMallocDefault));
+  constexpr int64_t HALF = PINNED_HALF / 4;  // words
+  HIPCHK(e, pinned_buffer(e));
   int32_t *d = (int32_t *)work_take(e, 1, 2 * HALF * 4);
   if (!d) return fail_(e, MSKG_ENOMEM, "store: no device memory for LattCoo's words");
   Lattice L = make_lattice(e);
@@ -3858,9 +3989,6 @@ int mskg_la_counts(mskg_engine *e, int64_t count[3], int64_t liquid[3]) {
 // class is zero exactly when its record makes it no MC particle, which a
 // sweep does not change), so the lists stay.
 static int refresh_range(mskg_engine *e, int64_t first, int64_t end, bool lists_stay) {
-  RunState st;
-  int rc = read_state(e, st);
-  if (rc) return rc;
   HIPCHK(e, hipMemsetAsync(e->d_err, 0, sizeof(int), e->stream));
   Lattice L = make_lattice(e);
   if (!lists_stay) e->lists_dirty = true;
@@ -3868,8 +3996,8 @@ static int refresh_range(mskg_engine *e, int64_t first, int64_t end, bool lists_
   const bool la = e->tab.la_mode || e->tab.st_n;
   if (first == 0 && end == e->box.npts) {
     const int blocks = (int)std::min<int64_t>((e->box.npts + 255) / 256, 256 * 64);
-    hipLaunchKernelGGL(MSKG_VARIANT(k_rate_sweep, la, e->cov_model), dim3(blocks), dim3(256), 0, e->stream, L, st.rtot,
-                       e->d_err, 0);
+    hipLaunchKernelGGL(MSKG_VARIANT(k_rate_sweep, la, e->cov_model), dim3(blocks), dim3(256), 0, e->stream, L,
+                       &e->d_st->rtot, e->d_err, 0);
     HIPCHK(e, hipGetLastError());
   } else if (end > first) {
     // one group of four points per thread up to 65536 blocks: the range of
@@ -3878,7 +4006,7 @@ static int refresh_range(mskg_engine *e, int64_t first, int64_t end, bool lists_
     // blocks with several groups per thread)
     const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((end - first + 1023) / 1024, 65536));
     hipLaunchKernelGGL(MSKG_VARIANT(k_rate_sweep_range, la, e->cov_model), dim3(blocks), dim3(256), 0, e->stream, L,
-                       st.rtot, e->d_err, 0, first, end);
+                       &e->d_st->rtot, e->d_err, 0, first, end);
     HIPCHK(e, hipGetLastError());
   }
   HIPCHK(e, hipEventRecord(e->ev1, e->stream));
@@ -4307,7 +4435,13 @@ static int build_slab(mskg_engine *e, int32_t mode, int32_t len, double fraction
   const int blocks = (int)std::min<int64_t>((e->box.npts + 255) / 256, 4096);
   unsigned long long *d_atoms = (unsigned long long *)work_take(e, 0, 2 * sizeof(unsigned long long));
   if (!d_atoms) return fail_(e, MSKG_ENOMEM, "slab: no device memory for the census");
-  HIPCHK(e, hipMemsetAsync(d_atoms, 0, 2 * sizeof(unsigned long long), e->stream));
+  // the total rate of the initial population seeds the isolated-atom rule
+  const double nsurf = (double)e->box.lx * e->box.ly / 36.0;  // 2 atoms per (6x6) surface cell per layer
+  const Tables &t = e->tab;
+  const double rtot = nsurf * (mode ? 0.5 * (t.pe[0 + 3 * 2] + t.pe[1 + 3 * 2]) : t.pe[0 + 3 * 2]) +
+                      nsurf * (t.pd[0 + 3] + t.pd[1 + 3] + t.pd[2 + 3]);
+  hipLaunchKernelGGL(k_state_new, dim3(1), dim3(256), 0, e->stream, e->d_st,
+                     e->cfg.events_per_pass > 0 ? e->cfg.events_per_pass : 1.0, rtot, d_atoms, e->d_err);
   hipLaunchKernelGGL(k_build_slab, dim3(blocks), dim3(256), 0, e->stream, L, len, mode, fraction,
                      (uint32_t)e->cfg.seed, (uint32_t)(e->cfg.seed >> 32), e->logical_lz, d_atoms);
   HIPCHK(e, hipGetLastError());
@@ -4319,20 +4453,10 @@ static int build_slab(mskg_engine *e, int32_t mode, int32_t len, double fraction
     // every atom of coordination 1..3 lies in the planes len-3..len-1
     const int64_t first = (len - 3) * e->box.plane, end = len * e->box.plane;
     const int sb = (int)std::max<int64_t>(1, std::min<int64_t>((end - first + 1023) / 1024, 65536));
-    HIPCHK(e, hipMemsetAsync(e->d_err, 0, sizeof(int), e->stream));
     hipLaunchKernelGGL(MSKG_VARIANT(k_rate_sweep_range, e->tab.la_mode || e->tab.st_n, e->cov_model), dim3(sb), dim3(256),
-                       0, e->stream, L, 0.0, e->d_err, 1, first, end);
+                       0, e->stream, L, (const double *)nullptr, e->d_err, 1, first, end);
     HIPCHK(e, hipGetLastError());
   }
-  // the total rate of the initial population seeds the isolated-atom rule
-  RunState st;
-  memset(&st, 0, sizeof st);
-  st.events_per_pass = e->cfg.events_per_pass > 0 ? e->cfg.events_per_pass : 1.0;
-  const double nsurf = (double)e->box.lx * e->box.ly / 36.0;  // 2 atoms per (6x6) surface cell per layer
-  const Tables &t = e->tab;
-  st.rtot = nsurf * (mode ? 0.5 * (t.pe[0 + 3 * 2] + t.pe[1 + 3 * 2]) : t.pe[0 + 3 * 2]) +
-            nsurf * (t.pd[0 + 3] + t.pd[1 + 3] + t.pd[2 + 3]);
-  HIPCHK(e, hipMemcpyAsync(e->d_st, &st, sizeof st, hipMemcpyHostToDevice, e->stream));
   unsigned long long atoms[2];
   HIPCHK(e, hipMemcpyAsync(atoms, d_atoms, sizeof atoms, hipMemcpyDeviceToHost, e->stream));
   HIPCHK(e, hipStreamSynchronize(e->stream));
@@ -4369,7 +4493,7 @@ static int build_shape(mskg_engine *e, ShapeSpec S, bool walls_off_lattice) {
   hipLaunchKernelGGL(k_shape_isolated, dim3(blocks), dim3(256), 0, e->stream, L, S);
   hipLaunchKernelGGL(k_shape_records, dim3(blocks), dim3(256), 0, e->stream, L, S, e->d_err);
   hipLaunchKernelGGL(MSKG_VARIANT(k_rate_sweep, e->tab.la_mode || e->tab.st_n, e->cov_model), dim3(blocks),
-                     dim3(256), 0, e->stream, L, 0.0, e->d_err, 0);
+                     dim3(256), 0, e->stream, L, (const double *)nullptr, e->d_err, 0);
   hipLaunchKernelGGL(k_initial_placeholders, dim3(blocks), dim3(256), 0, e->stream, L);
   HIPCHK(e, hipGetLastError());
   hipFree(e->d_offwall);
@@ -4615,7 +4739,7 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
   mskg_engine *e0 = engines[0];
   if (!e0) return MSKG_EINVAL;
   std::vector<SerialDesc> descs(n);
-  std::vector<unsigned long long> ev0(n), log0(n);
+  std::vector<unsigned long long> ev0(n);
   bool any_la = false, any_cov = false;
   for (int i = 0; i < n; i++) {
     mskg_engine *e = engines[i];
@@ -4627,7 +4751,6 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
     if (max_events[i] < 0) return fail_(e, MSKG_EINVAL, "max_events < 0");
     for (int j = 0; j < i; j++)
       if (engines[j] == e) return fail_(e0, MSKG_EINVAL, "serial run: replica %d appears twice", i);
-    HIPCHK(e, hipStreamSynchronize(e->stream));
     const int nblk = (e->ntiles + WAVE - 1) / WAVE;
     if (!e->d_tsum) {
       HIPCHK(e, hipMalloc(&e->d_tsum, e->ntiles * sizeof(double)));
@@ -4638,15 +4761,6 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
       if (int rc2 = build_lists(e, L)) return rc2;
     }
     e->slab = -1;  // the serial run keeps no record of the layers it visits
-    RunState st;
-    int rc = read_state(e, st);
-    if (rc) return rc;
-    if (st.err) return fail_(e, MSKG_ESTATE, "engine is in an error state: %s", err_name(st.err));
-    int lerr = 0;
-    HIPCHK(e, hipMemcpy(&lerr, e->d_list_err, sizeof(int), hipMemcpyDeviceToHost));
-    if (lerr) return fail_(e, MSKG_ECAPACITY, "a tile holds more MC particles than tile_capacity");
-    ev0[i] = st.events;
-    log0[i] = st.log_n;
     SerialDesc &D = descs[i];
     D.L = L;
     D.tsum = e->d_tsum;
@@ -4662,6 +4776,14 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
     D.nblk = nblk;
     D.replica = i;
   }
+  std::vector<RunHead> head;
+  if (int rc = read_heads(engines, n, head)) return rc;
+  for (int i = 0; i < n; i++) {
+    if (head[i].err)
+      return fail_(engines[i], MSKG_ESTATE, "engine is in an error state: %s", err_name(head[i].err));
+    if (head[i].list_err) return fail_(engines[i], MSKG_ECAPACITY, "a tile holds more MC particles than tile_capacity");
+    ev0[i] = head[i].events;
+  }
   SerialDesc *d_descs = nullptr;
   HIPCHK(e0, hipMalloc(&d_descs, n * sizeof(SerialDesc)));
   hipError_t ce = hipMemcpyAsync(d_descs, descs.data(), n * sizeof(SerialDesc), hipMemcpyHostToDevice, e0->stream);
@@ -4676,14 +4798,13 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
   if (ce != hipSuccess) return fail_(e0, MSKG_EDEVICE, "k_serial: %s", hipGetErrorString(ce));
   float ms = 0;
   HIPCHK(e0, hipEventElapsedTime(&ms, e0->ev0, e0->ev1));
+  if (int rc = read_heads(engines, n, head)) return rc;
   int rc_all = MSKG_OK;
   for (int i = 0; i < n; i++) {
     mskg_engine *e = engines[i];
+    const RunHead &st = head[i];
     e->run_ms = ms;
     e->lists_dirty = false;
-    RunState st;
-    int rc = read_state(e, st);
-    if (rc) return rc;
     if (events_done) events_done[i] = (int64_t)(st.events - ev0[i]);
     if (kmc_time) kmc_time[i] = st.clock;
     if (stop_reason) stop_reason[i] = st.stop;
@@ -4691,7 +4812,6 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
       rc_all = fail_(e, MSKG_ESTATE, "serial run of replica %d stopped: %s", i, err_name(st.err));
     if (e->d_log && st.log_n > (unsigned long long)e->log_cap && rc_all == MSKG_OK)
       rc_all = fail_(e, MSKG_ECAPACITY, "event log of replica %d overflowed", i);
-    (void)log0;
   }
   return rc_all;
 }
@@ -4831,8 +4951,9 @@ int mskg_adjoint_checkpointed(mskg_engine *const *engines, int32_t n, const mskg
   if (!e0) return MSKG_EINVAL;
   // every replica's state is checked and its key arrays exist before anything is queued
   std::vector<char> fresh(n);
-  std::vector<double> rtot(n);
   std::vector<int64_t> rows(n);
+  bool any_la = false, any_cov = false;
+  int64_t most = 0;
   for (int i = 0; i < n; i++) {
     mskg_engine *e = engines[i];
     if (!e || !e->loaded) return fail_(e0, MSKG_EINVAL, "adjoint: replica %d has no state loaded", i);
@@ -4848,15 +4969,18 @@ int mskg_adjoint_checkpointed(mskg_engine *const *engines, int32_t n, const mskg
           hipMalloc(&e->d_rate_seen, np * sizeof(float)) != hipSuccess)
         return fail_(e, MSKG_ENOMEM, "adjoint: no device memory for the class keys");
     }
-    RunState st;
-    if (int rc = read_state(e, st)) return rc;  // also: nothing of e's own stream is still running
-    if (st.err) return fail_(e, MSKG_ESTATE, "engine is in an error state: %s", err_name(st.err));
+    any_la |= e->tab.la_mode || e->tab.st_n;
+    any_cov |= e->cov_model;
+    most = std::max(most, np);
     // the trajectory starts from the engine's rates: a tracked engine's keys
     // are current; otherwise a sweep refreshes the rates and assigns the keys
     fresh[i] = !(e->track && e->keys_valid);
-    rtot[i] = st.rtot;
     rows[i] = every > 0 ? n_events[i] / every : 0;
   }
+  std::vector<RunHead> head;
+  if (int rc = read_heads(engines, n, head)) return rc;  // also: nothing of their own streams is still running
+  for (int i = 0; i < n; i++)
+    if (head[i].err) return fail_(engines[i], MSKG_ESTATE, "engine is in an error state: %s", err_name(head[i].err));
   // One device block for every segment, in regions of one kind each so that
   // the results come back in one copy per kind: the logs and waiting times,
   // the initial class counts (+ the unsupported points) and isolated-rate
@@ -4900,6 +5024,7 @@ int mskg_adjoint_checkpointed(mskg_engine *const *engines, int32_t n, const mskg
     D.cnt0 = d_cnt + (size_t)i * (KEY_N + 1);
     D.iso0 = d_iso + i;
     D.sweep_err = e->d_err;
+    D.fresh = fresh[i];
     D.S = (double *)(arena + o_s) + (size_t)i * ADJ_NS;
     D.A = (double *)(arena + o_a) + (size_t)i * KEY_N;
     D.scal = (double *)(arena + o_sc) + (size_t)i * 4;
@@ -4917,35 +5042,24 @@ int mskg_adjoint_checkpointed(mskg_engine *const *engines, int32_t n, const mskg
   // the copies from host memory first, while the stream is still idle (a
   // copy from pageable memory returns only when done)
   hipError_t ce = hipMemcpyAsync(d_descs, descs.data(), n * sizeof(AdjDesc), hipMemcpyHostToDevice, sm);
-  for (int i = 0; i < n && ce == hipSuccess; i++)
-    if (n_events[i] > 0) {
-      ce = hipMemcpyAsync(arena + log_off[i], logs[i], n_events[i] * sizeof(mskg_event), hipMemcpyHostToDevice, sm);
-      if (ce == hipSuccess)
-        ce = hipMemcpyAsync(arena + o_dt + dt_off[i], dts[i], n_events[i] * sizeof(double), hipMemcpyHostToDevice, sm);
-    }
-  if (ce == hipSuccess) ce = hipMemsetAsync(d_cnt, 0, cnt_b, sm);
-  if (ce == hipSuccess) ce = hipMemsetAsync(d_iso, 0, iso_b, sm);
-  // each segment's initial classes: the keys (a rate sweep if they are not
-  // current), their populations, and the keys and rates as first seen
-  for (int i = 0; i < n && ce == hipSuccess; i++) {
-    mskg_engine *e = engines[i];
-    const int64_t np = e->box.npts;
-    const int blocks = (int)std::min<int64_t>((np + 255) / 256, 256 * 64);
-    ce = hipMemsetAsync(e->d_err, 0, sizeof(int), sm);
-    if (ce == hipSuccess && fresh[i]) {
-      hipLaunchKernelGGL(MSKG_VARIANT(k_rate_sweep, e->tab.la_mode || e->tab.st_n, e->cov_model), dim3(blocks),
-                         dim3(256), 0, sm, descs[i].L, rtot[i], e->d_err, 0);
-      ce = hipGetLastError();
-    }
-    if (ce == hipSuccess) {
-      hipLaunchKernelGGL(k_key_hist, dim3(blocks), dim3(256), 0, sm, descs[i].L, d_cnt + (size_t)i * (KEY_N + 1),
-                         d_iso + i);
-      ce = hipGetLastError();
-    }
-    if (ce == hipSuccess) ce = hipMemcpyAsync(e->d_key_seen, e->d_key, np * sizeof(int32_t), hipMemcpyDeviceToDevice, sm);
-    if (ce == hipSuccess) ce = hipMemcpyAsync(e->d_rate_seen, e->d_rate, np * sizeof(float), hipMemcpyDeviceToDevice, sm);
-    e->lists_dirty = true;
-    e->slab = -1;
+  std::vector<HostPiece> logs_in;
+  for (int i = 0; i < n; i++)
+    if (n_events[i] > 0) logs_in.push_back({log_off[i], logs[i], (size_t)n_events[i] * sizeof(mskg_event)});
+  for (int i = 0; i < n; i++)
+    if (n_events[i] > 0) logs_in.push_back({o_dt + dt_off[i], dts[i], (size_t)n_events[i] * sizeof(double)});
+  if (ce == hipSuccess) ce = stage_in(e0, sm, arena, logs_in);
+  // each segment's initial classes
+  if (ce == hipSuccess) {
+    hipLaunchKernelGGL(k_adj_clear, dim3(n), dim3(64), 0, sm, d_descs, n);
+    const int blocks = (int)std::min<int64_t>((most + 1023) / 1024, 256 * 16);
+    for (int i0 = 0; i0 < n; i0 += 65535)
+      hipLaunchKernelGGL(MSKG_VARIANT(k_adj_start, any_la, any_cov), dim3(blocks, std::min(n - i0, 65535)), dim3(256), 0,
+                         sm, d_descs + i0);
+    ce = hipGetLastError();
+  }
+  for (int i = 0; i < n; i++) {
+    engines[i]->lists_dirty = true;
+    engines[i]->slab = -1;
   }
   const int cblocks = (n + 255) / 256;
   std::vector<int> chk(2 * (size_t)n);

@@ -95,6 +95,7 @@ class Engine:
             cfg.second_factor = self._arrays["second_factor"].ctypes.data
         self._cfg = cfg
         self._guard_seen = 0
+        self._log_capacity = 0
         h = C.c_void_p()
         rc = self.L.mskg_create(C.byref(cfg), C.byref(h))
         self.h = h
@@ -214,12 +215,12 @@ class Engine:
 
     def set_event_log(self, capacity):
         self._check(self.L.mskg_set_event_log(self.h, int(capacity)))
+        self._log_capacity = int(capacity)
 
     def event_log(self):
         n = C.c_int64()
-        self._check(self.L.mskg_get_event_log(self.h, None, 0, C.byref(n)))
-        log = np.zeros(max(n.value, 1), EVENT_DTYPE)
-        self._check(self.L.mskg_get_event_log(self.h, ptr(log), n.value, C.byref(n)))
+        log = np.empty(max(self._log_capacity, 1), EVENT_DTYPE)
+        self._check(self.L.mskg_get_event_log(self.h, ptr(log), self._log_capacity, C.byref(n)))
         return log[:n.value]
 
     def set_temperature(self, temp_k):
