@@ -1818,7 +1818,7 @@ struct SerialDesc {
 // Rate sum of one tile's list (every class); entries whose class fell to 0
 // leave the list.  The compaction is in place: an entry moves only to a
 // position at or before the one it was read from in the same step.
-__device__ double tile_sum_compact(const Lattice &L, int t, int lane) {
+__device__ inline double tile_sum_compact(const Lattice &L, int t, int lane) {
   const TileGeom g = tile_geom(t, L.tile, L.ntx, L.nty, L.box.lz);
   const int m = min(L.tl_n[t], L.capg);
   int32_t *idx = L.tl_idx + (int64_t)t * L.capg;
@@ -1831,9 +1831,10 @@ __device__ double tile_sum_compact(const Lattice &L, int t, int lane) {
     if (j < m) {
       k = idx[j];
       const P3 p = tile_point(L.box, g, L.tile, k);
-      const uint8_t c = L.cls[p.i];
+      const uint8_t c = L.cls[p.i];  // class and rate in one round trip
+      const float r = L.rate[p.i];
       keep = c != 0;
-      if (keep) part += (double)L.rate[p.i];
+      if (keep) part += (double)r;
       else L.inlist[p.i] = 0;
     }
     const unsigned long long msk = __ballot(keep);
@@ -1841,9 +1842,52 @@ __device__ double tile_sum_compact(const Lattice &L, int t, int lane) {
     if (keep) idx[slot] = k;
     nout += __popcll(msk);
   }
-  part = wave_sum(part);
+  part = wave_sum_dpp(part);
   if (lane == 0) L.tl_n[t] = nout;
   return part;
+}
+// The same for four tiles at once, a row of 16 lanes each (t: the row's tile,
+// -1: none): one chain of reads for all of them.  The additions are those of
+// the whole wave, whose lanes 16..63 hold zeros.  False, with nothing
+// changed, when a list is longer than a row.
+__device__ inline bool tile_sum_rows(const Lattice &L, int t, int lane, double &sum) {
+  const int rl = lane & 15;
+  const int tt = max(t, 0);
+  const int raw = L.tl_n[tt];
+  int32_t *const idx = L.tl_idx + (int64_t)tt * L.capg;
+  const int k = idx[min(rl, L.capg - 1)];  // read whatever the length, used only below it
+  const int m = t >= 0 ? min(raw, L.capg) : 0;
+  if (__ballot(m > 16)) return false;
+  double part = 0.0;
+  bool keep = false;
+  if (rl < m) {
+    const TileGeom g = tile_geom(tt, L.tile, L.ntx, L.nty, L.box.lz);
+    const P3 p = tile_point(L.box, g, L.tile, k);
+    const uint8_t c = L.cls[p.i];
+    const float r = L.rate[p.i];
+    keep = c != 0;
+    if (keep) part = (double)r;
+    else L.inlist[p.i] = 0;
+  }
+  const unsigned mask = (unsigned)(__ballot(keep) >> (lane & 48)) & 0xffffu;
+  const int slot = __popc(mask & ((1u << rl) - 1u));
+  if (keep && slot != rl) idx[slot] = k;
+  if (t >= 0 && rl == 0 && __popc(mask) != raw) L.tl_n[t] = __popc(mask);
+  part += dpp_take<0x128, 0xf>(part);  // row_ror:8
+  part += dpp_take<0x124, 0xf>(part);  // row_ror:4
+  part += dpp_take<0x122, 0xf>(part);  // row_ror:2
+  part += dpp_take<0x121, 0xf>(part);  // row_ror:1
+  sum = part;
+  return true;
+}
+// wave_incl_scan of values that lanes 16..63 hold none of, for the lanes
+// 0..15: the same additions in one row.
+__device__ inline double row_incl_scan(double v) {
+  v += dpp_take<0x111, 0xf>(v);  // row_shr:1
+  v += dpp_take<0x112, 0xf>(v);  // row_shr:2
+  v += dpp_take<0x114, 0xf>(v);  // row_shr:4
+  v += dpp_take<0x118, 0xf>(v);  // row_shr:8
+  return v;
 }
 
 // Index of the first element of v[0..n) (FP64, read from memory) whose
@@ -1856,7 +1900,7 @@ __device__ int scan_pick(const double *v, int n, double target, int lane, double
   for (int base = 0; base < n; base += WAVE) {
     const int j = base + lane;
     const double x = j < n ? v[j] : 0.0;
-    const double inc = wave_incl_scan(x, lane) + acc;
+    const double inc = (n <= 16 ? row_incl_scan(x) : wave_incl_scan(x, lane)) + acc;
     const unsigned long long nzm = __ballot(x > 0.0);
     if (nzm) {
       const int hi = 63 - __clzll((long long)nzm);
@@ -1878,6 +1922,12 @@ __device__ int scan_pick(const double *v, int n, double target, int lane, double
 // Replicas of up to SERIAL_LDS_TILES tiles keep their tile and block sums on
 // chip; larger ones use the engine's global arrays.
 constexpr int SERIAL_LDS_TILES = 4096;
+//
+// What bounds it: one wave's chain of an event's reads and instructions, about
+// 7.5 us an event, of which the event itself 3.5.  Draws and logarithms are made
+// 64 at once; the tiles an event touched are rescanned four at a time, a row
+// of 16 lanes each; lists and levels of up to 16 entries are scanned in one
+// row.  64 lattices of 144^3, 3000 events each: 27.1 ms with one after the other, now 22.6.
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
   __shared__ TabLds tabs;
@@ -1902,28 +1952,35 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
   __syncthreads();
   for (int b = 0; b < D.nblk; b++) {
     const int t = b * WAVE + lane;
-    const double v = wave_sum(t < D.ntiles ? tsum[t] : 0.0);
+    const double v = wave_sum_dpp(t < D.ntiles ? tsum[t] : 0.0);
     if (lane == 0) bsum[b] = v;
   }
   __syncthreads();
   double clock = st->clock;
   unsigned long long events = st->events, nev = 0;
   int stop = MSKG_STOP_LIMIT, err = 0;
-  U4 ctr;
-  ctr.x = 0x5e71a1u;  // the stream depends on the engine's seed only, not on its place in the batch
+  const unsigned long long log_n = st->log_n;
+  U4 draw;           // lane l: the Philox block of event 64 b + l of this call, b the current batch
+  double wait = 0.0;  // ... and -ln of its first uniform
   while ((long long)nev < D.max_events && clock < D.max_time) {
-    double part = 0.0;
-    for (int b = lane; b < D.nblk; b += WAVE) part += bsum[b];
-    const double R = wave_sum(part);
-    if (!(R > 0.0)) { stop = MSKG_STOP_NO_EVENTS; break; }
-    ctr.y = (uint32_t)events;
-    ctr.z = (uint32_t)(events >> 32);
-    ctr.w = 0;
     // one Philox block per event: waiting time, selection, event type and
     // stacking choice, 32 random bits each
-    const U4 d = philox4x32_10(ctr, D.key0, D.key1);
-    const double dt = -log(u01_32(d.x)) / R;
-    double target = u01_32(d.y) * R, below = 0.0;
+    const int dl = (int)(nev & (WAVE - 1));
+    if (dl == 0) {
+      U4 ctr;
+      ctr.x = 0x5e71a1u;  // the stream depends on the engine's seed only, not on its place in the batch
+      ctr.y = (uint32_t)(events + lane);
+      ctr.z = (uint32_t)((events + lane) >> 32);
+      ctr.w = 0;
+      draw = philox4x32_10(ctr, D.key0, D.key1);
+      wait = -log(u01_32(draw.x));
+    }
+    double part = 0.0;
+    for (int b = lane; b < D.nblk; b += WAVE) part += bsum[b];
+    const double R = wave_sum_dpp(part);
+    if (!(R > 0.0)) { stop = MSKG_STOP_NO_EVENTS; break; }
+    const double dt = read_lane(wait, dl) / R;
+    double target = u01_32((uint32_t)__builtin_amdgcn_readlane((int)draw.y, dl)) * R, below = 0.0;
     // block -> tile -> list entry
     const int b = scan_pick(bsum, D.nblk, target, lane, &below);
     if (b < 0) { stop = MSKG_STOP_NO_EVENTS; break; }
@@ -1943,11 +2000,13 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
       double v = 0.0;
       if (j < m) {
         const P3 p = tile_point(L.box, g, L.tile, idx[j]);
-        if (L.cls[p.i]) v = (double)L.rate[p.i];
+        const uint8_t c = L.cls[p.i];
+        const float r = L.rate[p.i];
+        if (c) v = (double)r;
       }
       const unsigned long long nzm = __ballot(v > 0.0);
       if (nzm) last_nz = base + 63 - __clzll((long long)nzm);
-      const double inc = wave_incl_scan(v, lane) + acc;
+      const double inc = (m <= 16 ? row_incl_scan(v) : wave_incl_scan(v, lane)) + acc;
       const unsigned long long hit = __ballot(j < m && v > 0.0 && inc > target);
       if (hit) { sel = base + __ffsll((long long)hit) - 1; break; }
       acc = __shfl(inc, WAVE - 1, WAVE);
@@ -1957,18 +2016,18 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
     const P3 s = tile_point(L.box, g, L.tile, __builtin_amdgcn_readfirstlane(idx[sel]));
     Choice ch;
     ch.arm = -1;
-    ch.u_arm = u01_32(d.w);
+    ch.u_arm = u01_32((uint32_t)__builtin_amdgcn_readlane((int)draw.w, dl));
     const Rec srec = uniform_rec(load_rec(L, s.i));
     const int coor0 = r_coor(srec);
     const int itrans = __builtin_amdgcn_readfirstlane(pick_itrans<LA, COV>(
         L, TabEv<COV>{*L.tab, tabs}, coor0, r_temp(srec), __builtin_amdgcn_readfirstlane((int)L.cls[s.i]),
-        u01_32(d.z)));
+        u01_32((uint32_t)__builtin_amdgcn_readlane((int)draw.z, dl))));
     EvOut o;
     execute<LA, COV>(L, tabs, R, s, srec, itrans, ch, o, lane);
     clock += dt;
     if (lane == 0) {
       if (D.log) {
-        const unsigned long long li = st->log_n + nev;
+        const unsigned long long li = log_n + nev;
         if (li < D.log_cap) {
           mskg_event ev;
           ev.iter = (int64_t)(events + 1);
@@ -1994,10 +2053,25 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
     const int tq = o.set ? tile_of(L, o.p) : -1;
     const unsigned long long tm = __ballot(o.set != 0);
     for (unsigned long long m2 = tm; m2;) {
-      const int tt = __builtin_amdgcn_readlane(tq, __ffsll((long long)m2) - 1);
-      m2 &= ~__ballot(tq == tt);
-      const double ts = tile_sum_compact(L, tt, lane);
-      if (lane == 0) tsum[tt] = ts;
+      int four[4];
+      for (int q = 0; q < 4; q++) {
+        four[q] = -1;
+        if (m2) {
+          four[q] = __builtin_amdgcn_readlane(tq, __ffsll((long long)m2) - 1);
+          m2 &= ~__ballot(tq == four[q]);
+        }
+      }
+      const int mine = lane < 32 ? (lane < 16 ? four[0] : four[1]) : (lane < 48 ? four[2] : four[3]);
+      double ts;
+      if (tile_sum_rows(L, mine, lane, ts)) {
+        if ((lane & 15) == 0 && mine >= 0) tsum[mine] = ts;
+      } else {
+        for (int q = 0; q < 4; q++) {
+          if (four[q] < 0) continue;
+          ts = tile_sum_compact(L, four[q], lane);
+          if (lane == 0) tsum[four[q]] = ts;
+        }
+      }
     }
     __syncthreads();
     const int bq = o.set ? tq / WAVE : -1;
@@ -2005,7 +2079,7 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
       const int bb = __builtin_amdgcn_readlane(bq, __ffsll((long long)m2) - 1);
       m2 &= ~__ballot(bq == bb);
       const int tt = bb * WAVE + lane;
-      const double v = wave_sum(tt < D.ntiles ? tsum[tt] : 0.0);
+      const double v = wave_sum_dpp(tt < D.ntiles ? tsum[tt] : 0.0);
       if (lane == 0) bsum[bb] = v;
     }
     __syncthreads();
