@@ -154,6 +154,16 @@ struct PassParams {
   unsigned int *sched;
 };
 
+// Between the lanes of a workgroup of one wave: what one has written the
+// others read from here on.  The hardware takes a wave's LDS and its vector
+// memory instructions in order, so nothing is waited for; a workgroup barrier
+// waits until every store has returned, a round trip on every event (whole
+// passes with it and without: CVD 95.0, 93.7 ms; 512^3 SiC 48.2, 47.6).
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ inline double wave_sum(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
@@ -400,7 +410,7 @@ __global__ void __launch_bounds__(WAVE) k_replay(Lattice L, const mskg_event *lo
   L.geo = as_constant(L.geo);
   L.tab = as_constant(L.tab);
   load_tables(*L.tab, tabs, lane);
-  __syncthreads();
+  wave_sync();
   double clock = st->clock;
   int bad = 0;
   P3 s;
@@ -432,7 +442,7 @@ __global__ void __launch_bounds__(WAVE) k_replay(Lattice L, const mskg_event *lo
         for (int q = 0; q < 3; q++) st->cl[q] = st->cinit[q] - st->cc[q];
       }
     }
-    __syncthreads();  // the next event reads this one's records, rates and counts
+    wave_sync();  // the next event reads this one's records, rates and counts
   }
   if (lane != 0) return;
   if (bad) {
@@ -543,13 +553,13 @@ __device__ inline void sort_by_offset(int32_t *lk, float *lr, uint8_t *lc, int l
     }
 #pragma unroll 1
     for (int q = 0; q < m; q++) rank += __builtin_amdgcn_readlane(key, q) < key ? 1 : 0;
-    __syncthreads();
+    wave_sync();
     if (lane < m) {
       lk[lo + rank] = key;
       lr[lo + rank] = r;
       lc[lo + rank] = c;
     }
-    __syncthreads();
+    wave_sync();
     return;
   }
   for (int round = 0; round < m; round++) {
@@ -565,7 +575,7 @@ __device__ inline void sort_by_offset(int32_t *lk, float *lr, uint8_t *lc, int l
         lc[i] = lc[i + 1];
         lc[i + 1] = tc;
       }
-    __syncthreads();
+    wave_sync();
   }
 }
 
@@ -691,7 +701,7 @@ __device__ inline int pass_tile(const PassParams *pp, Lattice &L, RunState *st, 
     }
     return ERR_CAPACITY;
   }
-  __syncthreads();
+  wave_sync();
   sort_by_offset(lk, lr, lc, nh, n, lane);
   }
 
@@ -859,7 +869,7 @@ __device__ inline int pass_tile(const PassParams *pp, Lattice &L, RunState *st, 
       }
       n += __popcll(am);
     }
-    __syncthreads();  // the next event reads this one's records and list entries
+    wave_sync();  // the next event reads this one's records and list entries
   }
   if (guard >= PASS_EVENT_CAP && lane == 0) atomicAdd(&st->guard_exits, 1ull);
   // 3. write the list back (active entries only), tile totals, counters
@@ -911,7 +921,7 @@ __device__ inline int pass_tile(const PassParams *pp, Lattice &L, RunState *st, 
     }
   }
   if (err) return err;
-  __syncthreads();
+  wave_sync();
   return 0;
 }
 
@@ -1949,13 +1959,13 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
     const double ts = tile_sum_compact(L, t, lane);
     if (lane == 0) tsum[t] = ts;
   }
-  __syncthreads();
+  wave_sync();
   for (int b = 0; b < D.nblk; b++) {
     const int t = b * WAVE + lane;
     const double v = wave_sum_dpp(t < D.ntiles ? tsum[t] : 0.0);
     if (lane == 0) bsum[b] = v;
   }
-  __syncthreads();
+  wave_sync();
   double clock = st->clock;
   unsigned long long events = st->events, nev = 0;
   int stop = MSKG_STOP_LIMIT, err = 0;
@@ -2043,7 +2053,7 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
       if (COV && itrans == 5 && o.species) st->desorbed[o.species - 1]++;
     }
     if (lane == count_slot(itrans)) my_cnt++;
-    __syncthreads();
+    wave_sync();
     events++;
     nev++;
     err = __builtin_amdgcn_readfirstlane(o.err);
@@ -2073,7 +2083,7 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
         }
       }
     }
-    __syncthreads();
+    wave_sync();
     const int bq = o.set ? tq / WAVE : -1;
     for (unsigned long long m2 = tm; m2;) {
       const int bb = __builtin_amdgcn_readlane(bq, __ffsll((long long)m2) - 1);
@@ -2082,7 +2092,7 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
       const double v = wave_sum_dpp(tt < D.ntiles ? tsum[tt] : 0.0);
       if (lane == 0) bsum[bb] = v;
     }
-    __syncthreads();
+    wave_sync();
   }
   if (lane == 0) {
     st->clock = clock;
@@ -2150,7 +2160,7 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
     cnt[c] = D.cnt0[c];
   }
   for (int c = lane; c < ADJ_NS; c += WAVE) D.S[c] = 0.0;
-  __syncthreads();
+  wave_sync();
   double t = 0.0, ttot = 0.0, r_iso = *D.iso0, tau_iso = 0.0, iso_int = 0.0, iso_log = 0.0;
   int err = 0;
   long long k = 0;
@@ -2192,7 +2202,7 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
     ch.u_arm = 0.0;
     EvOut out;
     execute<false, false>(L, tabs, ev.rtot, s, srec, itrans, ch, out, lane);  // the likelihood excludes LA and coverage tables
-    __syncthreads();
+    wave_sync();
     // the touched points' keys and rates, before and after, a lane each (a
     // point listed twice is taken once); every class change of the event
     // happens at time t, so the accounting below does not depend on order
@@ -2240,7 +2250,7 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
       }
       if (do_o) { A[co] += cnt[co] * (t - tau[co]); tau[co] = t; }
       if (do_n) { A[cn] += cnt[cn] * (t - tau[cn]); tau[cn] = t; }
-      __syncthreads();  // every first update has read its population
+      wave_sync();  // every first update has read its population
       if (co >= 0) atomicAdd(&cnt[co], -1);
       if (cn >= 0) atomicAdd(&cnt[cn], 1);
       // the isolated-atom rate sum changes in touched order (rare)
@@ -2252,7 +2262,7 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
         r_iso += read_lane(rnq, q) - read_lane(roq, q);
       }
     }
-    __syncthreads();
+    wave_sync();
     if (bad) { err = bad; k++; break; }
     if (D.hist && (k + 1) % D.every == 0) {  // checkpoint: the class populations after event k
       int32_t *row = D.hist + ((k + 1) / D.every - 1) * KEY_N;
@@ -2266,7 +2276,7 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
       iso_int += r_iso * (t - tau_iso);
       tau_iso = 0.0;
       t = 0.0;
-      __syncthreads();
+      wave_sync();
     }
   }
   for (int c = lane; c < KEY_N; c += WAVE) D.A[c] = A[c] + cnt[c] * (t - tau[c]);
