@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(WAVE) k_replay(Lattice L, const mskg_event *lo
   const int lane = threadIdx.x;
   L.geo = as_constant(L.geo);
   L.tab = as_constant(L.tab);
-  load_tables(*L.tab, tabs, lane);
+  load_tables<LA>(*L.tab, tabs, lane);
   wave_sync();
   double clock = st->clock;
   int bad = 0;
@@ -651,12 +651,12 @@ __device__ inline int pass_tile(const PassParams *pp, Lattice &L, RunState *st, 
   // length; a lane uses its entry only below it, and the index stays in the
   // tile's list storage), and the run state the window needs.
   TabRegs tr;
-  if (fresh) fetch_tables(*L.tab, tr, lane);
+  if (fresh) fetch_tables<LA>(*L.tab, tr, lane);
   const int n_raw = tl_n[t], own_raw = as_global(P.L.tl_own)[t];
   const int k_first = idx[min(lane, P.L.capg - 1)];
   rtot = st->rtot;
   sweeps = st->sweeps;
-  if (fresh) put_tables(tr, tabs, lane);
+  if (fresh) put_tables<LA>(tr, tabs, lane);
   const int n_in = __builtin_amdgcn_readfirstlane(n_raw), own = __builtin_amdgcn_readfirstlane(own_raw);
   if (n_in == 0) return 0;
   g = tile_geom(t, L.tile, P.L.ntx, P.L.nty, L.box.lz);
@@ -1072,7 +1072,7 @@ __device__ inline void sweep_tiles(const PassParams &P, const PassParams *const 
   // the window as the sweep starts (L.win's first words widen during it)
   const int zlo = (int)P.sched[3], zhi = (int)P.sched[4];
   if (zlo > zhi) return;
-  load_tables(*L.tab, tabs, lane);
+  load_tables<LA>(*L.tab, tabs, lane);
   int first[2], count[2];
   queue_layers(zlo, zhi, 0, P.ntz, first[0], count[0]);
   queue_layers(zlo, zhi, 1, P.ntz, first[1], count[1]);
@@ -1572,7 +1572,9 @@ __global__ void __launch_bounds__(256) k_build_slab(Lattice L, int len, int sic,
       } else {
         s.kc = (uint8_t)(KIND_EMPTY | (2 << 3));
         cls = CLS_ADSORB;
-        r = pd_of<true>(TabSrc{t}, 1, 2, 0) + pd_of<true>(TabSrc{t}, 2, 2, 0) + pd_of<true>(TabSrc{t}, 3, 2, 0) +
+        double pd[3];
+        pd_of<true>(TabSrc{t}, 2, 0, nullptr, pd);
+        r = pd[0] + pd[1] + pd[2] +
             t.pabs[0 + 6] + t.pabs[1 + 6] + t.pabs[2 + 6];
       }
       if (z <= len - 1) mine[sp - 1]++;
@@ -1948,7 +1950,7 @@ __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
   to_global(L);
   L.cold = as_constant(&descs[blockIdx.x].L);
   RunState *st = as_global(D.st);
-  load_tables(*L.tab, tabs, lane);
+  load_tables<LA>(*L.tab, tabs, lane);
   if (st->err) return;
   const bool on_chip = D.ntiles <= SERIAL_LDS_TILES;
   double *tsum = on_chip ? s_tsum : D.tsum;
@@ -2150,7 +2152,7 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
   D.acc = as_global(D.acc);
   Lattice L = D.L;
   to_global(L);
-  load_tables(*L.tab, tabs, lane);
+  load_tables<false>(*L.tab, tabs, lane);
   // the per-class integrals and change times in the segment's own device
   // memory (LDS holds the populations only, so that more waves fit a CU)
   double *const A = D.acc, *const tau = D.acc + KEY_N;

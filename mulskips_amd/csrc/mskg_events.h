@@ -243,6 +243,8 @@ __device__ inline void enlist(const Lattice &L, const P3 &p) {
 }
 
 // ---- rates ---------------------------------------------------------------
+// The reference's kb (Get_Prob.f:70).
+#define MSKG_KB 0.00008617330350
 // Where a rate evaluation takes the tables from: all of them in device
 // memory (the sweep), or an event wave's copy in LDS.
 struct TabSrc {
@@ -252,6 +254,11 @@ struct TabSrc {
   MSKG_HD double pabs(int i) const { return t.pabs[i]; }
   MSKG_HD double pdes(int i) const { return t.pdes[i]; }
   MSKG_HD double f2(int i) const { return t.f2[i]; }
+  // the Boltzmann factor of laser-annealing deposition entry i (species i % 3)
+  // at the species' melting temperature
+  MSKG_HD double ex(int i, bool variant) const {
+    return exp(-t.pd[i] / (MSKG_KB * (variant ? t.la_tm[i % 3] : t.tm)));
+  }
   MSKG_HD double ads(int coor) const {
     return t.pd[3 * (coor - 1)] + t.pd[1 + 3 * (coor - 1)] + t.pd[2 + 3 * (coor - 1)] +
            (t.pabs[3 * coor] + t.pabs[1 + 3 * coor] + t.pabs[2 + 3 * coor]);
@@ -265,6 +272,7 @@ constexpr int PE_PLAIN = 192;
 struct TabLds {
   double pe[PE_PLAIN], pd[9], pabs[12], pdes[12], f2[13];
   double ads[4];  // an adsorption site's rate by coordination (without laser annealing): PTransD + PTransAbs
+  double ex[9];   // laser annealing: TabSrc::ex, nine exponentials a wave instead of three a rate
 };
 template <bool COV>
 struct TabEv {
@@ -276,11 +284,13 @@ struct TabEv {
   MSKG_HD double pdes(int i) const { return l.pdes[i]; }
   MSKG_HD double f2(int i) const { return l.f2[i]; }
   MSKG_HD double ads(int coor) const { return l.ads[coor]; }
+  MSKG_HD double ex(int i, bool) const { return l.ex[i]; }
 };
 // The copy in two halves, so that its loads can leave with a tile's first ones.
 struct TabRegs {
-  double pe[PE_PLAIN / 64], rest, ads;
+  double pe[PE_PLAIN / 64], rest, ads, ex;
 };
+template <bool LA>
 __device__ inline void fetch_tables(const Tables &t, TabRegs &r, int lane) {
   for (int k = 0; k < PE_PLAIN / 64; k++) r.pe[k] = t.pe[lane + 64 * k];
   // pd (9), pabs (12), pdes (12), f2 (13): a lane each
@@ -289,7 +299,9 @@ __device__ inline void fetch_tables(const Tables &t, TabRegs &r, int lane) {
   r.rest = *src;
   const int c = min(max(lane, 1), 3);
   r.ads = TabSrc{t}.ads(c);
+  if (LA) r.ex = t.la_mode ? TabSrc{t}.ex(min(lane, 8), t.la_variant != 0) : 0.0;
 }
+template <bool LA>
 __device__ inline void put_tables(const TabRegs &r, TabLds &l, int lane) {
   for (int k = 0; k < PE_PLAIN / 64; k++) l.pe[lane + 64 * k] = r.pe[k];
   if (lane < 9) l.pd[lane] = r.rest;
@@ -297,33 +309,39 @@ __device__ inline void put_tables(const TabRegs &r, TabLds &l, int lane) {
   else if (lane < 33) l.pdes[lane - 21] = r.rest;
   else if (lane < 46) l.f2[lane - 33] = r.rest;
   if (lane < 4) l.ads[lane] = r.ads;
+  if (LA && lane < 9) l.ex[lane] = r.ex;
 }
+template <bool LA>
 __device__ inline void load_tables(const Tables &t, TabLds &l, int lane) {
   TabRegs r;
-  fetch_tables(t, r, lane);
-  put_tables(r, l, lane);
+  fetch_tables<LA>(t, r, lane);
+  put_tables<LA>(r, l, lane);
 }
-// The reference's kb (Get_Prob.f:70).
-#define MSKG_KB 0.00008617330350
+// The deposition rates of the three species at a site of coordination coor.
 // LA = false compiles the laser-annealing branches out (tables with la_mode 0).
 template <bool LA, class Src>
-MSKG_HD double pd_of(const Src &S, int sp, int coor, int temperature, const long long *cl = nullptr) {
+MSKG_HD void pd_of(const Src &S, int coor, int temperature, const long long *cl, double p[3]) {
   const Tables &t = S.t;
-  double e = S.pd((sp - 1) + 3 * (coor - 1));
-  if (!LA || !t.la_mode) return e;
+  double e[3];
+  for (int k = 0; k < 3; k++) p[k] = e[k] = S.pd(k + 3 * (coor - 1));
+  if (!LA || !t.la_mode) return;
   if (t.la_variant && cl) {
     // LaserAnnealing Get_Prob.f:148-151, evaluated left to right: 0.5d0 *
     // P0(k) * FLOAT(CountLiquid(k)) / SUM(CountLiquid) * EXP(..) * (1 + ERF(..)),
     // FLOAT the REAL(4) conversion.  With no liquid left (the reference
     // divides by zero) solidification stops.
     const long long sum = cl[0] + cl[1] + cl[2];
-    if (sum <= 0 || sp > t.ncrystal) return 0.0;  // PD(k,:) is set for k <= NCrystal only
-    return 0.5 * t.la_p0[sp - 1] * (double)(float)(int)cl[sp - 1] / (double)sum *
-           exp(-e / (MSKG_KB * t.la_tm[sp - 1])) * (1.0 + erf((temperature - t.la_tflex[sp - 1]) / t.la_sigma[sp - 1])) *
-           (e != 0.0 ? 1.0 : 0.0);
+    for (int k = 0; k < 3; k++)
+      p[k] = sum <= 0 || k >= t.ncrystal ? 0.0  // PD(k,:) is set for k <= NCrystal only
+                                         : 0.5 * t.la_p0[k] * (double)(float)(int)cl[k] / (double)sum *
+                                               S.ex(k + 3 * (coor - 1), true) *
+                                               (1.0 + erf((temperature - t.la_tflex[k]) / t.la_sigma[k])) *
+                                               (e[k] != 0.0 ? 1.0 : 0.0);
+    return;
   }
-  return 0.5 * t.p0 * exp(-e / (MSKG_KB * t.tm)) * (1.0 + erf((temperature - t.tflex) / t.sigma)) *
-         (e != 0.0 ? 1.0 : 0.0);
+  const double step = 1.0 + erf((temperature - t.tflex) / t.sigma);
+  for (int k = 0; k < 3; k++)
+    p[k] = 0.5 * t.p0 * S.ex(k + 3 * (coor - 1), false) * step * (e[k] != 0.0 ? 1.0 : 0.0);
 }
 MSKG_HD int pe_flat(int sp, int a, int b, int c, int d, int e, int f) {
   return (sp - 1) + 3 * (a + 4 * (b + 4 * (c + 4 * (d + 4 * (e + 4 * f)))));
@@ -449,8 +467,9 @@ MSKG_HD void rate_of(const Src &S, const long long *cl, double rtot, int z, int 
                            st_entry(t.st_pabs, 12, 2 + 3 * coor, w)
                      : 0.0;
         } else {
-          pdep = pd_of<LA>(S, 1, coor, temperature, cl) + pd_of<LA>(S, 2, coor, temperature, cl) +
-                 pd_of<LA>(S, 3, coor, temperature, cl);
+          double p[3];
+          pd_of<LA>(S, coor, temperature, cl, p);
+          pdep = p[0] + p[1] + p[2];
           pabs = COV ? S.pabs(0 + 3 * coor) + S.pabs(1 + 3 * coor) + S.pabs(2 + 3 * coor) : 0.0;
         }
         cls = CLS_ADSORB;
@@ -540,9 +559,11 @@ MSKG_HD int pick_itrans(const Lattice &L, const Src &S, int coor, int temp, int 
     p2 = st_entry(t.st_pd, 9, 1 + 3 * (coor - 1), w);
     p3 = st_entry(t.st_pd, 9, 2 + 3 * (coor - 1), w);
   } else {
-    p1 = pd_of<LA>(S, 1, coor, temperature, L.cl);
-    p2 = pd_of<LA>(S, 2, coor, temperature, L.cl);
-    p3 = pd_of<LA>(S, 3, coor, temperature, L.cl);
+    double p[3];
+    pd_of<LA>(S, coor, temperature, L.cl, p);
+    p1 = p[0];
+    p2 = p[1];
+    p3 = p[2];
   }
   double pdep = p1 + p2 + p3;
   double pabs = COV ? pabs_of(0) + pabs_of(1) + pabs_of(2) : 0.0;
