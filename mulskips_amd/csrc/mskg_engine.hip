@@ -837,6 +837,9 @@ __device__ inline int pass_tile(const PassParams *pp, Lattice &L, RunState *st, 
         tr = L.rate[o.p.i];
         tc = L.cls[o.p.i];
       }
+      // the loads are waited for here, in this seldom taken branch: where it
+      // joins the others they would make every event wait for its stores
+      asm volatile("" : "+v"(tr), "+v"(tc));
       for (unsigned long long tm = __ballot(kl >= 0); tm; tm &= tm - 1ull) {
         const int q = __ffsll((long long)tm) - 1;
         if (q < lane && __builtin_amdgcn_readlane(kl, q) == kl) dup = true;

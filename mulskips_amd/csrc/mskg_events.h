@@ -1000,13 +1000,12 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
         i1 = shifted(L, p, a, 0, b).i;
         i2 = shifted(L, p, 0, a, b).i;
       }
-      int k0 = 0, k1 = 0, kk = 0;
-      if (i0 >= 0) k0 = L.site[i0].kc & 7;
-      if (i1 >= 0) k1 = L.site[i1].kc & 7;
-      if (i2 >= 0) kk = L.site[i2].kc & 7;
-      k0 = i0 == s.i ? new_kind : k0;
-      k1 = i1 == s.i ? new_kind : k1;
-      kk = i2 == s.i ? new_kind : kk;
+      // every lane loads all three (outside the box: point 0, not used): a load
+      // under a condition of its own is waited for before the next leaves
+      const int r0 = L.site[i0 < 0 ? 0 : i0].kc, r1 = L.site[i1 < 0 ? 0 : i1].kc, r2 = L.site[i2 < 0 ? 0 : i2].kc;
+      const int k0 = i0 == s.i ? new_kind : (i0 < 0 ? 0 : r0 & 7);
+      const int k1 = i1 == s.i ? new_kind : (i1 < 0 ? 0 : r1 & 7);
+      const int kk = i2 == s.i ? new_kind : (i2 < 0 ? 0 : r2 & 7);
       k2 = ((uint32_t)kind_species(k0) + (uint32_t)kind_species(k1) + (uint32_t)kind_species(kk)) << 28;
     }
     if (q.i == s.i) er = S;
