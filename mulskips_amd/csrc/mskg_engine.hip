@@ -405,7 +405,7 @@ __global__ void __launch_bounds__(256) k_site_rates(Lattice L, int64_t n, const 
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) k_replay(Lattice L, const mskg_event *log, int64_t n, int clock_mode,
                                                  RunState *st) {
-  __shared__ typename TabsOf<LA>::type tabs;
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
   L.geo = as_constant(L.geo);
   L.tab = as_constant(L.tab);
@@ -959,7 +959,7 @@ __device__ inline int colour_tile(const Lattice &L, int colour, int zfirst, int 
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_pass(PassParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ typename TabsOf<LA>::type tabs;
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
   const PassParams *const pp = kernel_params();
   RunState *const st = P.st;
@@ -1173,13 +1173,13 @@ __device__ inline void sweep_tiles(const PassParams &P, const PassParams *const 
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_sweep(PassParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ typename TabsOf<LA>::type tabs;
+  __shared__ TabLds tabs;
   sweep_tiles<LA, COV, false>(P, kernel_params(), tabs, smem);
 }
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_sweep_xcd(PassParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ typename TabsOf<LA>::type tabs;
+  __shared__ TabLds tabs;
   sweep_tiles<LA, COV, true>(P, kernel_params(), tabs, smem);
 }
 
@@ -1432,7 +1432,7 @@ template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3)))
 k_pass_ens(const PassParams *__restrict__ reps, int n, int *plan, int colour) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ typename TabsOf<LA>::type tabs;
+  __shared__ TabLds tabs;
   const int lane = threadIdx.x;
   const int *pc = plan + colour * (n + 1);
   const int total = __builtin_amdgcn_readfirstlane(pc[n]);
@@ -1945,7 +1945,7 @@ constexpr int SERIAL_LDS_TILES = 4096;
 // row.  64 lattices of 144^3, 3000 events each: 27.1 ms with one after the other, now 22.6.
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) k_serial(const SerialDesc *descs) {
-  __shared__ typename TabsOf<LA>::type tabs;
+  __shared__ TabLds tabs;
   __shared__ double s_tsum[SERIAL_LDS_TILES], s_bsum[SERIAL_LDS_TILES / WAVE];
   const int lane = threadIdx.x;
   const SerialDesc D = descs[blockIdx.x];
