@@ -460,11 +460,24 @@ __global__ void __launch_bounds__(WAVE) k_replay(Lattice L, const mskg_event *lo
 // a rate sweep or a replay).  One wave per tile, four of its points a lane in
 // flight.  Points outside the planes [zlo, zhi] are no MC particles and have no
 // list flag, which the caller knows of a slab (touched_planes): only the planes
-// [zlo, zhi] are looked at, and the lists of tiles without any are empty.
-__global__ void __launch_bounds__(256) k_build_lists(Lattice L, int ntiles, int zlo, int zhi) {
+// [zlo, zhi] are looked at, by the first `full` blocks, which take the tiles
+// from t0 on that hold such planes; a thread of the others empties the list of
+// a tile outside (a wave each for those cost 80 us at 83000 tiles).
+// zeroed: no list flag is set anywhere, and none needs clearing (a store for
+// every eight points of a tile's row, otherwise).
+__global__ void __launch_bounds__(256) k_build_lists(Lattice L, int ntiles, int zlo, int zhi, int t0, int t1,
+                                                     int full, int zeroed) {
   int lane = threadIdx.x & (WAVE - 1);
-  int t = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-  if (t >= ntiles) return;
+  if ((int)blockIdx.x >= full) {
+    int q = ((int)blockIdx.x - full) * 256 + (int)threadIdx.x;
+    if (q >= t0) q += t1 - t0;
+    if (q >= ntiles) return;
+    L.tl_n[q] = 0;
+    L.tl_own[q] = 0;
+    return;
+  }
+  int t = t0 + blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+  if (t >= t1) return;
   TileGeom g = tile_geom(t, L.tile, L.ntx, L.nty, L.box.lz);
   int n = 0;
   {
@@ -484,7 +497,7 @@ __global__ void __launch_bounds__(256) k_build_lists(Lattice L, int ntiles, int 
       }
       for (int u = 0; u < 4; u++) {
         const bool on = c[u] != 0;
-        if (pi[u] >= 0) L.inlist[pi[u]] = on ? 1 : 0;
+        if (pi[u] >= 0 && (on || !zeroed)) L.inlist[pi[u]] = on ? 1 : 0;
         const unsigned long long m = __ballot(on);
         const int slot = n + __popcll(m & ((1ull << lane) - 1ull));
         if (on) {
@@ -498,27 +511,66 @@ __global__ void __launch_bounds__(256) k_build_lists(Lattice L, int ntiles, int 
   if (lane == 0) {
     L.tl_n[t] = n;
     L.tl_own[t] = min(n, L.capg);
-    if (n) widen_window(L.win, tile_colour(g.tx, g.ty, g.tz), g.tz);
   }
 }
 
-// Window of tile layers from lists that are already built.
-__global__ void __launch_bounds__(256) k_list_window(Lattice L, int ntiles) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ntiles) return;
-  if (L.tl_n[t] > 0) {
-    const int tx = t % L.ntx, ty = (t / L.ntx) % L.nty, tz = t / (L.ntx * L.nty);
-    widen_window(L.win, tile_colour(tx, ty, tz), tz);
-  }
+// Windows of tile layers from the lists: a block a layer (from layer l0 on),
+// which finds the colours that hold any and widens their windows once.  (Every
+// tile had widened its colour's itself: all of them at once, against windows
+// still empty, 100 us of atomics on one word at 18000 tiles.)
+__global__ void __launch_bounds__(1024) k_list_window(Lattice L, int l0) {
+  __shared__ unsigned int found;
+  const int tz = l0 + blockIdx.x, layer = L.ntx * L.nty;
+  if (threadIdx.x == 0) found = 0u;
+  __syncthreads();
+  unsigned int mine = 0u;
+  for (int i = threadIdx.x; i < layer; i += blockDim.x)
+    if (L.tl_n[tz * layer + i] > 0) mine |= 1u << tile_colour(i % L.ntx, i / L.ntx, tz);
+  for (int off = 32; off > 0; off >>= 1) mine |= __shfl_xor(mine, off, WAVE);
+  if ((threadIdx.x & (WAVE - 1)) == 0 && mine) atomicOr(&found, mine);
+  __syncthreads();
+  if (threadIdx.x < 8 && ((found >> threadIdx.x) & 1u)) widen_window(L.win, threadIdx.x, tz);
 }
 
-// Rate total (without isolated atoms) and population of every tile's list.
-__global__ void __launch_bounds__(256) k_tile_rates(Lattice L, int ntiles, RunState *st) {
+// A run's start, by one block: empty windows, empty slots, the run's limits and
+// a zero window tau in the state (k_sweep_end then sets the first).
+__global__ void __launch_bounds__(256) k_run_start(RunState *st, int *win, int *list_err, int lists, int tau_policy,
+                                                   double events_per_pass, double max_time,
+                                                   unsigned long long max_events) {
+  const int i = threadIdx.x;
+  if (i < 32) win[i] = i & 1 ? -1 : 0x7fffffff;
+  if (i == 32 && lists) *list_err = 0;
+  clear_words((unsigned int *)st->slot, (int)(sizeof st->slot / 4));
+  if (i != 0) return;
+  st->tau = 0.0;
+  st->stop = 0;
+  st->final_sweep = 0;
+  st->tau_policy = tau_policy;
+  st->events_per_pass = events_per_pass;
+  st->max_time = max_time;
+  st->max_events = st->events + max_events;
+  st->ever_lo = 0x7fffffff;
+  st->ever_hi = -1;
+}
+
+// Rate total (without isolated atoms) and population of every tile's list; the
+// tiles outside [t0, t1) have none (k_build_lists).
+__global__ void __launch_bounds__(256) k_tile_rates(Lattice L, int ntiles, RunState *st, int t0, int t1, int full) {
   int lane = threadIdx.x & (WAVE - 1);
-  int t = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-  if (t >= ntiles) return;
-  TileGeom g = tile_geom(t, L.tile, L.ntx, L.nty, L.box.lz);
+  if ((int)blockIdx.x >= full) {
+    int q = ((int)blockIdx.x - full) * 256 + (int)threadIdx.x;
+    if (q >= t0) q += t1 - t0;
+    if (q < ntiles) L.tile_r[q] = 0.0;
+    return;
+  }
+  int t = t0 + blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+  if (t >= t1) return;
   const int m = min(L.tl_n[t], L.capg);
+  if (m <= 0) {  // most tiles of a box
+    if (lane == 0) L.tile_r[t] = 0.0;
+    return;
+  }
+  TileGeom g = tile_geom(t, L.tile, L.ntx, L.nty, L.box.lz);
   double acc = 0.0;
   int cnt = 0;
   for (int j = lane; j < m; j += WAVE) {
@@ -3020,6 +3072,7 @@ struct mskg_engine {
   // that a run's sweeps could visit since.  An event's site lies in such a
   // layer, and it writes at most 6 planes from it.
   int slab = -1, slab_z0 = 0, slab_z1 = 0;
+  bool flags_zero = false;   // no list flag is set at all: a slab was built, and no lists since
   bool flags_clean = false;  // no list flag outside the touched planes (d_inlist), while they are known
   // workspaces of the frames: kept while they are small (WORK_KEEP)
   int32_t *pinned = nullptr;  // page-locked buffer of the host's data on its way (8 MB, on first use)
@@ -4191,12 +4244,34 @@ static PassParams pass_params(mskg_engine *e) {
 
 // The tile lists of the present classes.  Of a slab whose list flags were
 // cleared when it was built (flags_clean), only the touched planes hold any.
+struct TouchedTiles {
+  int z0, z1;      // planes
+  int t0, t1;      // tiles of their layers
+  int full, rest;  // blocks: a wave a tile for those, a thread a tile for the others
+};
+static TouchedTiles touched_tiles(const mskg_engine *e) {
+  TouchedTiles T;
+  T.z0 = 0;
+  T.z1 = e->box.lz;
+  if (e->flags_clean) touched_planes(e, T.z0, T.z1);
+  const int layer = e->ntx * e->nty;
+  T.t0 = T.z0 / e->tile * layer;
+  T.t1 = (T.z1 / e->tile + 1) * layer;
+  T.full = (T.t1 - T.t0 + 3) / 4;
+  T.rest = (e->ntiles - (T.t1 - T.t0) + 255) / 256;
+  return T;
+}
+static void list_windows(mskg_engine *e, const Lattice &L) {
+  const TouchedTiles T = touched_tiles(e);
+  const int l0 = T.z0 / e->tile, layers = T.z1 / e->tile - l0 + 1;
+  hipLaunchKernelGGL(k_list_window, dim3(layers), dim3(1024), 0, e->stream, L, l0);
+}
 static int build_lists(mskg_engine *e, const Lattice &L) {
-  int z0 = 0, z1 = e->box.lz;
-  if (e->flags_clean) touched_planes(e, z0, z1);
-  HIPCHK(e, hipMemsetAsync(e->d_list_err, 0, sizeof(int), e->stream));
-  hipLaunchKernelGGL(k_build_lists, dim3((e->ntiles + 3) / 4), dim3(256), 0, e->stream, L, e->ntiles, z0,
-                     z1);
+  const TouchedTiles T = touched_tiles(e);
+  hipLaunchKernelGGL(k_build_lists, dim3(T.full + T.rest), dim3(256), 0, e->stream, L, e->ntiles, T.z0, T.z1, T.t0, T.t1,
+                     T.full, e->flags_zero ? 1 : 0);
+  e->flags_zero = false;
+  list_windows(e, L);
   HIPCHK(e, hipGetLastError());
   e->lists_dirty = false;
   return MSKG_OK;
@@ -4213,37 +4288,20 @@ static int run_begin(mskg_engine *e, int64_t max_events, double max_time, RunSta
   int rc = read_state(e, st);
   if (rc) return rc;
   if (st.err) return fail_(e, MSKG_ESTATE, "engine is in an error state: %s", err_name(st.err));
-  const int tblocks = (e->ntiles + 3) / 4;
-  {
-    static int w0[32];
-    for (int c = 0; c < 8; c++) {
-      w0[4 * c] = w0[4 * c + 2] = 0x7fffffff;
-      w0[4 * c + 1] = w0[4 * c + 3] = -1;
-    }
-    HIPCHK(e, hipMemcpyAsync(e->d_win, w0, sizeof w0, hipMemcpyHostToDevice, e->stream));
-  }
+  hipLaunchKernelGGL(k_run_start, dim3(1), dim3(256), 0, e->stream, e->d_st, e->d_win, e->d_list_err,
+                     e->lists_dirty ? 1 : 0, (int)e->cfg.tau_policy,
+                     e->cfg.events_per_pass > 0 ? e->cfg.events_per_pass : 1.0, max_time,
+                     (unsigned long long)max_events);
   if (e->lists_dirty) {
     if (int rc2 = build_lists(e, L)) return rc2;
   } else {
-    hipLaunchKernelGGL(k_list_window, dim3(tblocks), dim3(256), 0, e->stream, L, e->ntiles);
-    HIPCHK(e, hipGetLastError());
-  }
-  {
-    RunState s0 = st;
-    s0.tau = 0.0;  // k_sweep_end with tau = 0 only sets the next window
-    s0.stop = 0;
-    s0.final_sweep = 0;
-    s0.tau_policy = e->cfg.tau_policy;
-    s0.events_per_pass = e->cfg.events_per_pass > 0 ? e->cfg.events_per_pass : 1.0;
-    s0.max_time = max_time;
-    s0.max_events = st.events + (unsigned long long)max_events;
-    s0.ever_lo = 0x7fffffff;
-    s0.ever_hi = -1;
-    if (int rc2 = write_state_head(e, s0)) return rc2;
-    HIPCHK(e, hipMemsetAsync((char *)e->d_st + RS_HEAD, 0, sizeof s0.slot, e->stream));
+    list_windows(e, L);
   }
   // tile totals of the current rates, then the first window
-  hipLaunchKernelGGL(k_tile_rates, dim3(tblocks), dim3(256), 0, e->stream, L, e->ntiles, e->d_st);
+  // (the touched tiles hold every list, also of a run before this one)
+  const TouchedTiles T = touched_tiles(e);
+  hipLaunchKernelGGL(k_tile_rates, dim3(T.full + T.rest), dim3(256), 0, e->stream, L, e->ntiles, e->d_st, T.t0, T.t1,
+                     T.full);
   HIPCHK(e, hipGetLastError());
   hipLaunchKernelGGL(k_sweep_end, dim3(1), dim3(END_THREADS), 0, e->stream, pass_params(e));
   HIPCHK(e, hipGetLastError());
@@ -4554,7 +4612,7 @@ static int build_slab(mskg_engine *e, int32_t mode, int32_t len, double fraction
   e->loaded = true;
   e->lists_dirty = true;
   e->keys_valid = false;
-  e->flags_clean = true;
+  e->flags_clean = e->flags_zero = true;
   e->slab = mode;
   e->slab_z0 = len - 3;  // the surface atoms ...
   e->slab_z1 = len;      // ... and the empty sites above them
@@ -4714,7 +4772,7 @@ int mskg_copy_state(mskg_engine *dst, const mskg_engine *src) {
     return fail_(dst, MSKG_EINVAL, "copy_state: engines differ in box or tile");
   const int64_t np = dst->box.npts;
   dst->slab = -1;
-  dst->flags_clean = false;
+  dst->flags_clean = dst->flags_zero = false;
   HIPCHK(dst, hipStreamSynchronize(src->stream));
   HIPCHK(dst, hipMemcpyAsync(dst->d_site, src->d_site, np * sizeof(Site), hipMemcpyDeviceToDevice, dst->stream));
   HIPCHK(dst, hipMemcpyAsync(dst->d_rate, src->d_rate, np * sizeof(float), hipMemcpyDeviceToDevice, dst->stream));
@@ -4847,6 +4905,7 @@ int mskg_run_serial(mskg_engine *const *engines, int32_t n, const int64_t *max_e
     }
     Lattice L = make_lattice(e);
     if (e->lists_dirty) {
+      HIPCHK(e, hipMemsetAsync(e->d_list_err, 0, sizeof(int), e->stream));
       if (int rc2 = build_lists(e, L)) return rc2;
     }
     e->slab = -1;  // the serial run keeps no record of the layers it visits
