@@ -1840,25 +1840,31 @@ __global__ void __launch_bounds__(256) k_initial_placeholders(Lattice L) {
 }
 
 // Walls on the grid points off the stored lattice, one bit per grid point
-// (what the phase maps report): a wave takes 64 consecutive grid points at a
-// time, a lane a point, and its vote is two words -- consecutive lanes read
-// consecutive geometry ids, and a position costs two divisions by the FP64
-// reciprocals (a thread a word of 32 points took six 64-bit remainders a
-// point: 519 us at 768x768x384).
+// (what the phase maps report): a lane takes four consecutive grid points (of
+// one row: LenX is a multiple of 12), eight lanes a word.  A position costs
+// two divisions by the FP64 reciprocals for four points, and a lane's reads of
+// their geometry ids are in flight together (a thread a word of 32 points took
+// six 64-bit remainders a point, a wave 64 points at a time one read at a
+// time: 519 and 612 us at 768x768x384).
 __global__ void __launch_bounds__(256) k_shape_offwall(Lattice L, ShapeSpec S, uint32_t *bits, int64_t words) {
   const int lx = L.box.lx, ly = L.box.ly;
-  const int64_t face = (int64_t)lx * ly, pairs = (words + 1) / 2;
+  const int64_t face = (int64_t)lx * ly, lanes = words * 8;
   const double inv_face = 1.0 / (double)face, inv_lx = 1.0 / (double)lx;
-  const int lane = threadIdx.x & (WAVE - 1);
-  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-  for (int64_t q = wave; q < pairs; q += (int64_t)gridDim.x * (blockDim.x / WAVE)) {
-    const int64_t g = q * WAVE + lane;
-    const int64_t z = div_by(g, face, inv_face), r = g - z * face;
-    const int y = (int)div_by(r, lx, inv_lx), x = (int)(r - (int64_t)y * lx);
-    const bool wall = z <= L.box.lz && !valid_parity(x, y, (int)z) &&
-                      shape_content(S, x, y, (int)z, lx, ly, 0) == KIND_WALL;
-    const unsigned long long m = __ballot(wall);
-    if (lane < 2 && 2 * q + lane < words) bits[2 * q + lane] = (uint32_t)(m >> (32 * lane));
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t rounds = (lanes + stride - 1) / stride;  // the same for every lane: all of a word's take part
+  for (int64_t r = 0; r < rounds; r++) {
+    const int64_t q = r * stride + (int64_t)blockIdx.x * blockDim.x + threadIdx.x, g = 4 * q;
+    const int64_t z = div_by(g, face, inv_face), f = g - z * face;
+    const int y = (int)div_by(f, lx, inv_lx), x = (int)(f - (int64_t)y * lx);
+    uint32_t m = 0;
+    if (q < lanes && z <= L.box.lz)
+      for (int k = 0; k < 4; k++)
+        if (!valid_parity(x + k, y, (int)z) && shape_content(S, x + k, y, (int)z, lx, ly, 0) == KIND_WALL) m |= 1u << k;
+    m <<= 4 * (threadIdx.x & 7);
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xb1, 0xf, 0xf, false);   // lanes 1 0 3 2
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4e, 0xf, 0xf, false);   // lanes 2 3 0 1
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, false);  // row_half_mirror: the other four
+    if (q < lanes && (threadIdx.x & 7) == 0) bits[q >> 3] = m;
   }
 }
 
@@ -4649,7 +4655,7 @@ static int build_shape(mskg_engine *e, ShapeSpec S, bool walls_off_lattice) {
   if (walls_off_lattice) {
     const int64_t words = (e->box.lx * (int64_t)e->box.ly * (e->box.lz + 1) + 31) / 32;
     HIPCHK(e, hipMalloc(&e->d_offwall, words * sizeof(uint32_t)));
-    const int wb = (int)std::min<int64_t>(((words + 1) / 2 + 3) / 4, 256 * 64);
+    const int wb = (int)std::min<int64_t>((words * 8 + 255) / 256, 256 * 64);
     hipLaunchKernelGGL(k_shape_offwall, dim3(wb), dim3(256), 0, e->stream, L, S, e->d_offwall, words);
     HIPCHK(e, hipGetLastError());
   }
