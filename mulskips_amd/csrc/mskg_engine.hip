@@ -15,12 +15,16 @@
 //                  LDS, FP64 partial sums and Philox-4x32-10 draws.
 //   k_sweep        the eight colours of a sweep in one launch, each tile
 //                  starting when its lower-colour neighbours are done (same
-//                  result as eight k_pass launches, without their barriers).
+//                  result as eight k_pass launches, without their barriers);
+//   k_sweep_xcd    the same on one XCD, for small lattices.
 //   k_sweep_end    fixed-order FP64 sum of the tile rate totals -> next tau
 //                  and the clock.
 //   k_serial       serial BKL over a batch of lattices (one wave each).
 //   k_adjoint      log replay with per-class likelihood statistics.
-//   k_build_slab, k_frame_count / k_frame_write: device builder, frame records.
+//   k_build_slab, k_frame_count / k_frame_scan / k_frame_write: device builder,
+//                  frame records.
+//   k_words_in / k_words_out / k_lists_in / k_state_write: LattCoo and the
+//                  particle lists in and out.
 // The event kernels are templates on the rate model (laser annealing,
 // coverage species), chosen at launch from the tables.
 #include <hip/hip_runtime.h>
@@ -1004,10 +1008,11 @@ __device__ inline int colour_tile(const Lattice &L, int colour, int zfirst, int 
 // hold candidates, each workgroup (one wave) striding over them.  Three
 // waves per SIMD (157 VGPRs, no spills): 3072 tiles in flight on 256 CUs.
 // Measured on 8e6 events at 512^3 SiC (before the scalar registers were
-// relieved): 69.1 ms; with two waves 74.9, with four (128 VGPRs, spilled) 76.0.  The laser-annealing kernels hold exp and
-// erf: two waves (223 VGPRs), 55.3 ms on two exchanges of 3e4 events at
-// 264x264x384, against 60.4 with three (184 bytes a lane spilled) and 79.4
-// with four.
+// relieved): 69.1 ms; with two waves 74.9, with four (128 VGPRs, spilled) 76.0.
+// The laser-annealing kernels hold exp and erf: two waves (223 VGPRs), 55.3 ms
+// on two exchanges of 3e4 events at 264x264x384, against 60.4 with three (184
+// bytes a lane spilled) and 79.4 with four (before the exponentials of the
+// deposition rates went to the tables).
 template <bool LA, bool COV>
 __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 2 : 3, LA ? 2 : 3))) k_pass(PassParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -2420,7 +2425,7 @@ k_adj_start(const AdjDesc *descs) {
 //     first neighbours of the other species (Si around C, C around Si), read
 //     while the isolated wrong atoms -- bulk atoms with no such neighbour --
 //     are flipped to the other species; code = the species as flipped.
-//     k_wrong_mark marks those flips (bit 7 of the record's `valid` byte,
+//     k_wrong_set marks those flips (bit 7 of the record's `valid` byte,
 //     which the neighbour lists leave unused) and clears the marks after.
 // Each wave owns a contiguous segment of points: k_frame_count counts it and
 // leaves a bit a point for the points that have a record, k_frame_scan turns
@@ -4248,8 +4253,8 @@ static PassParams pass_params(mskg_engine *e) {
   return P;
 }
 
-// The tile lists of the present classes.  Of a slab whose list flags were
-// cleared when it was built (flags_clean), only the touched planes hold any.
+// The planes and tiles that may hold list entries: of a slab whose list flags
+// were cleared when it was built (flags_clean), the touched planes.
 struct TouchedTiles {
   int z0, z1;      // planes
   int t0, t1;      // tiles of their layers
@@ -4267,11 +4272,13 @@ static TouchedTiles touched_tiles(const mskg_engine *e) {
   T.rest = (e->ntiles - (T.t1 - T.t0) + 255) / 256;
   return T;
 }
+// The windows of tile layers of the present lists.
 static void list_windows(mskg_engine *e, const Lattice &L) {
   const TouchedTiles T = touched_tiles(e);
   const int l0 = T.z0 / e->tile, layers = T.z1 / e->tile - l0 + 1;
   hipLaunchKernelGGL(k_list_window, dim3(layers), dim3(1024), 0, e->stream, L, l0);
 }
+// The tile lists of the present classes, and their windows.
 static int build_lists(mskg_engine *e, const Lattice &L) {
   const TouchedTiles T = touched_tiles(e);
   hipLaunchKernelGGL(k_build_lists, dim3(T.full + T.rest), dim3(256), 0, e->stream, L, e->ntiles, T.z0, T.z1, T.t0, T.t1,
