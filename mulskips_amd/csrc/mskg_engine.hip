@@ -1566,6 +1566,20 @@ __device__ inline int dia_type(int x, int y, int z) {
 __constant__ int c_jump_dia[8][3] = {{3, 3, 3}, {3, -3, -3}, {-3, -3, 3}, {-3, 3, -3},
                                      {3, 3, -3}, {3, -3, 3}, {-3, -3, -3}, {-3, 3, 3}};
 
+// A block's threads' atoms of species 1 and 2 into atoms[].
+__device__ inline void count_atoms(const unsigned int mine[2], unsigned long long *atoms) {
+  __shared__ unsigned int sum[2];
+  if (threadIdx.x < 2) sum[threadIdx.x] = 0u;
+  __syncthreads();
+  for (int k = 0; k < 2; k++) {
+    unsigned int v = mine[k];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
+    if ((threadIdx.x & (WAVE - 1)) == 0 && v) atomicAdd(&sum[k], v);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2 && sum[threadIdx.x]) atomicAdd(&atoms[threadIdx.x], (unsigned long long)sum[threadIdx.x]);
+}
+
 // The flat (001) slab of SetSi.f:25-220 (sic=0: Si on both sublattices,
 // wall layers z=0..5 and LenZ-6..LenZ-1) or SetSiC3C.f:25-198 (sic=1: Si on
 // A, C on B, no walls): bulk below len-3, the top atomic layer as MC
@@ -1644,16 +1658,7 @@ __global__ void __launch_bounds__(256) k_build_slab(Lattice L, int len, int sic,
     L.cls[p] = (uint8_t)cls;
     L.inlist[p] = 0;
   }
-  __shared__ unsigned int sum[2];
-  if (threadIdx.x < 2) sum[threadIdx.x] = 0u;
-  __syncthreads();
-  for (int k = 0; k < 2; k++) {
-    unsigned int v = mine[k];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-    if ((threadIdx.x & (WAVE - 1)) == 0 && v) atomicAdd(&sum[k], v);
-  }
-  __syncthreads();
-  if (threadIdx.x < 2 && sum[threadIdx.x]) atomicAdd(&atoms[threadIdx.x], (unsigned long long)sum[threadIdx.x]);
+  count_atoms(mine, atoms);
 }
 
 // ---- the shaped initial states (main.f:224-294) ----------------------------------
@@ -1802,13 +1807,17 @@ __global__ void __launch_bounds__(256) k_shape_isolated(Lattice L, ShapeSpec S) 
 // its atoms (with walls = 1; every occupied neighbour otherwise); an empty
 // site of coordination 1 keeps only that neighbour, in entry 1.  Atoms and
 // empty sites of coordination >= 1 get their list; walls and the empty
-// sites of coordination 0 keep a bare record.
-__global__ void __launch_bounds__(256) k_shape_records(Lattice L, ShapeSpec S, int *err) {
+// sites of coordination 0 keep a bare record.  The atoms are final here and
+// counted on the way (a census read every record once more: 218 us at
+// 768x768x384).
+__global__ void __launch_bounds__(256) k_shape_records(Lattice L, ShapeSpec S, int *err, unsigned long long *atoms) {
   const int64_t n = L.box.npts;
+  unsigned int mine[2] = {0u, 0u};
   for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
     Site s = L.site[p];
     const int kind = s_kind(s);
     if (kind == KIND_WALL) continue;
+    if (kind_species(kind)) mine[kind - 1]++;  // the builders place species 1 and 2
     int x, y, z;
     pxyz(L.box, p, x, y, z);
     const int t = dia_type(x, y, z);
@@ -1834,6 +1843,7 @@ __global__ void __launch_bounds__(256) k_shape_records(Lattice L, ShapeSpec S, i
     if (!set_list(L.box, s, x, y, z, l)) atomicExch(err, ERR_GEOM);
     L.site[p] = s;
   }
+  count_atoms(mine, atoms);
 }
 
 // The placeholder deposition rate of an initial state is Get_Prob_Ini's
@@ -4648,26 +4658,35 @@ static int build_shape(mskg_engine *e, ShapeSpec S, bool walls_off_lattice) {
   Lattice L = make_lattice(e);
   L.key = nullptr;
   const int blocks = (int)std::min<int64_t>((e->box.npts + 255) / 256, 256 * 64);
+  unsigned long long *d_atoms = (unsigned long long *)work_take(e, 0, 2 * sizeof(unsigned long long));
+  if (!d_atoms) return fail_(e, MSKG_ENOMEM, "builder: no device memory for the census");
+  HIPCHK(e, hipMemsetAsync(d_atoms, 0, 2 * sizeof(unsigned long long), e->stream));
   HIPCHK(e, hipMemsetAsync(e->d_err, 0, sizeof(int), e->stream));
   hipLaunchKernelGGL(k_shape_place, dim3(blocks), dim3(256), 0, e->stream, L, S);
   hipLaunchKernelGGL(k_shape_isolated, dim3(blocks), dim3(256), 0, e->stream, L, S);
-  hipLaunchKernelGGL(k_shape_records, dim3(blocks), dim3(256), 0, e->stream, L, S, e->d_err);
+  hipLaunchKernelGGL(k_shape_records, dim3(blocks), dim3(256), 0, e->stream, L, S, e->d_err,
+                     d_atoms);
   hipLaunchKernelGGL(MSKG_VARIANT(k_rate_sweep, e->tab.la_mode || e->tab.st_n, e->cov_model), dim3(blocks),
                      dim3(256), 0, e->stream, L, (const double *)nullptr, e->d_err, 0);
   hipLaunchKernelGGL(k_initial_placeholders, dim3(blocks), dim3(256), 0, e->stream, L);
   HIPCHK(e, hipGetLastError());
-  hipFree(e->d_offwall);
-  e->d_offwall = nullptr;
+  if (!walls_off_lattice) {
+    hipFree(e->d_offwall);
+    e->d_offwall = nullptr;
+  }
   e->offwall_planes = false;
   if (walls_off_lattice) {
     const int64_t words = (e->box.lx * (int64_t)e->box.ly * (e->box.lz + 1) + 31) / 32;
-    HIPCHK(e, hipMalloc(&e->d_offwall, words * sizeof(uint32_t)));
+    if (!e->d_offwall) HIPCHK(e, hipMalloc(&e->d_offwall, words * sizeof(uint32_t)));
     const int wb = (int)std::min<int64_t>((words * 8 + 255) / 256, 256 * 64);
     hipLaunchKernelGGL(k_shape_offwall, dim3(wb), dim3(256), 0, e->stream, L, S, e->d_offwall, words);
     HIPCHK(e, hipGetLastError());
   }
   int err = 0;
   HIPCHK(e, hipMemcpyAsync(&err, e->d_err, sizeof(int), hipMemcpyDeviceToHost, e->stream));
+  unsigned long long atoms[2];
+  HIPCHK(e, hipMemcpyAsync(atoms, d_atoms, sizeof atoms, hipMemcpyDeviceToHost, e->stream));
+  // the new run state only now: the rates above go by the liquid counts of the state before
   RunState st;
   memset(&st, 0, sizeof st);
   st.events_per_pass = e->cfg.events_per_pass > 0 ? e->cfg.events_per_pass : 1.0;
@@ -4681,7 +4700,7 @@ static int build_shape(mskg_engine *e, ShapeSpec S, bool walls_off_lattice) {
     return fail_(e, MSKG_ESTATE, "shaped builder: %s", err_name(err));
   }
   if (int rc_la = la_variant_off(e)) return rc_la;
-  if (int rc_c = census(e, e->census0)) return rc_c;
+  for (int k = 0; k < 6; k++) e->census0[k] = k < 2 ? (int64_t)atoms[k] : 0;
   return MSKG_OK;
 }
 
