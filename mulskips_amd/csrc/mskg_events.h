@@ -985,9 +985,7 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
       const int a = (j & 2) ? -6 : 6, b = (j & 1) ? -6 : 6;
       const Box &B = L.box;
       int64_t i0, i1, i2;
-      const bool inner = ((unsigned)(p.x - 6) < (unsigned)(B.lx - 12)) & ((unsigned)(p.y - 6) < (unsigned)(B.ly - 12)) &
-                         ((unsigned)(p.z - 6) <= (unsigned)(B.lz - 12));
-      if (inner) {
+      if (shell_inside(B, p.x, p.y, p.z)) {
         i0 = p.i + (a / 2 + (b / 2) * B.hx);
         i1 = p.i + (b * B.plane + a / 2);
         i2 = p.i + (b * B.plane + (a / 2) * B.hx);

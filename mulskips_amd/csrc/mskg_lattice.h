@@ -145,6 +145,14 @@ MSKG_HD int64_t pidx_checked(const Box &b, int x, int y, int z) {
   return ok ? pidx(b, x, y, z) : -1;
 }
 
+// Is (x, y, z) at least 6 units from every face, so that the twelve points of
+// its second shell, (+-6, +-6, 0) and permutations, neither wrap nor leave the
+// box?  z with signed limits: LenZ may be less than 12.
+MSKG_HD bool shell_inside(const Box &b, int x, int y, int z) {
+  return ((unsigned)(x - 6) < (unsigned)(b.lx - 12)) & ((unsigned)(y - 6) < (unsigned)(b.ly - 12)) &
+         (z >= 6) & (z <= b.lz - 6);
+}
+
 // Absolute position of entry i of a site at (x,y,z), with the reference's
 // single x/y wrap of every neighbour-producing routine.
 MSKG_HD void entry_pos(const Box &b, const Site &s, int x, int y, int z, int i, int &ox, int &oy, int &oz) {
