@@ -2501,7 +2501,7 @@ __device__ inline void frame_point(const Lattice &L, int64_t p, uint32_t w, int 
     // even when it has no rate (a frozen-substrate atom)
     in[0] = (atom && coor <= 3) || L.cls[p] != 0;
     in[1] = !in[0] && atom;
-    in[2] = !in[0] && !atom && coor == 4;
+    in[2] = !in[0] && !atom && kind != KIND_WALL && coor == 4;
   } else if (MODE == FRAME_MAIN) {
     if (!below) return;
     const bool inner = p >= L.box.plane;  // z >= 1
