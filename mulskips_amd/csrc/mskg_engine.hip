@@ -1078,10 +1078,17 @@ __device__ inline void queue_layers(int zlo, int zhi, int odd, int ntz, int &fir
   count = first <= hi ? (hi - first) / 2 + 1 : 0;
 }
 
-// A wave polls at most this often (about 1 us each; a preempted wave does not
-// poll) for its neighbour tiles; the run then stops with ERR_SCHED instead of
-// hanging.
-constexpr int SCHED_POLLS = 1 << 22;
+// A wave polls at most this often for its neighbour tiles (a preempted wave does
+// not poll); the run then stops with ERR_SCHED instead of hanging.  The longest
+// wait of a correct run is the chain of the seven colours below a tile's, each
+// tile with PASS_EVENT_CAP events in its window.  An event takes 5 us in a short
+// list, 38 in one of 1460 entries and about 80 in one of 3400 (laser annealing,
+// whose events are the slowest; a list holds at most 6144), and a poll 0.5 us at
+// least: 512 polls an event are 256 us or more, two minutes in all.  (With 2^22
+// polls, 2.2 s, a laser-annealing run of 48-wide tiles whose windows reach the
+// cap stopped with the error, where the colour passes finish.)
+constexpr int EVENT_POLLS = 512;
+constexpr int SCHED_POLLS = 7 * PASS_EVENT_CAP * EVENT_POLLS;
 
 // A word another CU of the same XCD has written (the L1 is passed by: the
 // coherence of a workgroup whose waves may run on several CUs).
@@ -3197,7 +3204,7 @@ static const char *err_name(int c) {
     case ERR_SUMS: return "serial selection found no event inside a positive rate sum";
     case ERR_LIQUID: return "a species' CountLiquid is negative: its solidification rate would be negative";
     case ERR_ST_RANGE: return "a site's temperature lies outside the InitSt 'ST' reference temperatures";
-    case ERR_SCHED: return "a tile waited too long (some seconds) for its neighbour tiles in a dependency-scheduled sweep";
+    case ERR_SCHED: return "a tile waited too long (some minutes) for its neighbour tiles in a dependency-scheduled sweep";
     case ERR_TOP:
       return "an event site within 24 planes of the top of the stored planes (stored_len_z): store more planes";
     default: return "unknown";
