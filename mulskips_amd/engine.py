@@ -15,6 +15,7 @@ import numpy as np
 from . import _lib
 from ._lib import Config, EVENT_DTYPE, MSKG_FIELD_PLANES, MSKG_FIELD_SOCKET, ptr
 
+LOG_ROWS = 4096  # events a first call brings of a log (192 KB)
 CLASS_NAMES = {0: "none", 1: "adsorb", 2: "placeholder", 4: "evaporate", 5: "desorb", 6: "isolated"}
 
 
@@ -95,7 +96,6 @@ class Engine:
             cfg.second_factor = self._arrays["second_factor"].ctypes.data
         self._cfg = cfg
         self._guard_seen = 0
-        self._log_capacity = 0
         h = C.c_void_p()
         rc = self.L.mskg_create(C.byref(cfg), C.byref(h))
         self.h = h
@@ -215,12 +215,17 @@ class Engine:
 
     def set_event_log(self, capacity):
         self._check(self.L.mskg_set_event_log(self.h, int(capacity)))
-        self._log_capacity = int(capacity)
 
     def event_log(self):
+        """The events logged so far.  One call brings a short log; a longer
+        one is asked for again with an array of its own length, so that the
+        host's memory follows the events, not the log's capacity."""
         n = C.c_int64()
-        log = np.empty(max(self._log_capacity, 1), EVENT_DTYPE)
-        self._check(self.L.mskg_get_event_log(self.h, ptr(log), self._log_capacity, C.byref(n)))
+        log = np.empty(LOG_ROWS, EVENT_DTYPE)
+        self._check(self.L.mskg_get_event_log(self.h, ptr(log), len(log), C.byref(n)))
+        if n.value > len(log):
+            log = np.empty(n.value, EVENT_DTYPE)
+            self._check(self.L.mskg_get_event_log(self.h, ptr(log), len(log), C.byref(n)))
         return log[:n.value]
 
     def set_temperature(self, temp_k):
