@@ -3102,8 +3102,7 @@ struct mskg_engine {
   int slab = -1, slab_z0 = 0, slab_z1 = 0;
   bool flags_zero = false;   // no list flag is set at all: a slab was built, and no lists since
   bool flags_clean = false;  // no list flag outside the touched planes (d_inlist), while they are known
-  // workspaces of the frames: kept while they are small (WORK_KEEP)
-  int32_t *pinned = nullptr;  // page-locked buffer of the host's data on its way (8 MB, on first use)
+  // workspaces of the frames and of the exchange: kept while they are small (work_keep)
   void *d_work[2] = {nullptr, nullptr};
   size_t work_n[2] = {0, 0};
   std::string err;
@@ -3233,8 +3232,13 @@ static void run_over(mskg_engine *e, int slab, int lo, int hi) {
   e->slab_z1 = std::max(e->slab_z1, (hi + 1) * e->tile - 1 + 12);
 }
 // A workspace of at least n bytes, null when there is no memory for it; a
-// call that took one larger than WORK_KEEP gives it back at its end.
-constexpr size_t WORK_KEEP = 8u << 20;
+// call that took one larger than work_keep gives it back at its end.  What is
+// kept follows the lattice (a sixteenth of its records, rates and classes, 8 MB
+// at most): a scan over hundreds of small lattices keeps little beside them.
+static size_t work_keep(const mskg_engine *e) {
+  const int64_t lattice = e->box.npts * (int64_t)(sizeof(Site) + sizeof(float) + 1);
+  return (size_t)std::min<int64_t>(8 << 20, std::max<int64_t>(lattice / 16, 1 << 16));
+}
 static void *work_take(mskg_engine *e, int k, size_t n) {
   if (e->work_n[k] < n) {
     hipFree(e->d_work[k]);
@@ -3252,7 +3256,7 @@ static void *work_take(mskg_engine *e, int k, size_t n) {
 }
 static void work_done(mskg_engine *e) {
   for (int k = 0; k < 2; k++)
-    if (e->work_n[k] > WORK_KEEP) {
+    if (e->work_n[k] > work_keep(e)) {
       hipFree(e->d_work[k]);
       e->d_work[k] = nullptr;
       e->work_n[k] = 0;
@@ -3287,26 +3291,77 @@ static FramePlan frame_plan(const mskg_engine *e, int z0, int z1, int sic, int m
   return F;
 }
 
+// Page-locked buffers of two halves for the host's data on its way, taken by a
+// call and given back at its end (nothing of the call's is in flight then).
+// The process keeps up to PINNED_IDLE that no call holds, for whichever engine
+// and thread is next, until its last engine is destroyed: an allocation of one
+// costs milliseconds, and a buffer an engine is memory that a scan over
+// hundreds of engines does not get back.
+constexpr int64_t PINNED_HALF = 4 << 20;  // bytes
+constexpr int PINNED_IDLE = 2;
+static std::mutex g_pinned_mu;  // guards the three below
+static char *g_pinned_idle[PINNED_IDLE];
+static int g_pinned_n = 0;
+static int g_engines = 0;  // engines alive
+struct Pinned {
+  char *buf = nullptr;
+  hipError_t take() {
+    {
+      std::lock_guard<std::mutex> lock(g_pinned_mu);
+      if (g_pinned_n > 0) {
+        buf = g_pinned_idle[--g_pinned_n];
+        return hipSuccess;
+      }
+    }
+    const hipError_t ce = hipHostMalloc((void **)&buf, 2 * PINNED_HALF, hipHostMallocPortable);
+    if (ce != hipSuccess) buf = nullptr;
+    return ce;
+  }
+  char *half(int64_t i) const { return buf + (i & 1) * PINNED_HALF; }
+  ~Pinned() {
+    if (!buf) return;
+    {
+      std::lock_guard<std::mutex> lock(g_pinned_mu);
+      if (g_engines > 0 && g_pinned_n < PINNED_IDLE) {
+        g_pinned_idle[g_pinned_n++] = buf;
+        return;
+      }
+    }
+    (void)hipHostFree(buf);
+  }
+};
+static void engine_born() {
+  std::lock_guard<std::mutex> lock(g_pinned_mu);
+  g_engines++;
+}
+static void engine_gone() {
+  char *idle[PINNED_IDLE];
+  int n = 0;
+  {
+    std::lock_guard<std::mutex> lock(g_pinned_mu);
+    if (--g_engines == 0)
+      while (g_pinned_n > 0) idle[n++] = g_pinned_idle[--g_pinned_n];
+  }
+  while (n > 0) (void)hipHostFree(idle[--n]);
+}
+
 // Host pieces into device memory at dst + off (offsets increasing), through
-// the two halves of e's page-locked buffer: one copy for many small pieces,
-// the next half filled while the last is on its way.
+// the two halves of a page-locked buffer: one copy for many small pieces, the
+// next half filled while the last is on its way.
 struct HostPiece {
   size_t off;
   const void *src;
   size_t n;
 };
-constexpr int64_t PINNED_HALF = 4 << 20;  // bytes
-static hipError_t pinned_buffer(mskg_engine *e) {
-  return e->pinned ? hipSuccess : hipHostMalloc((void **)&e->pinned, 2 * PINNED_HALF, hipHostMallocDefault);
-}
 static hipError_t stage_in(mskg_engine *e, hipStream_t sm, char *dst, const std::vector<HostPiece> &pieces) {
-  hipError_t ce = pinned_buffer(e);
+  Pinned pin;
+  hipError_t ce = pin.take();
   size_t begin = 0, fill = 0;  // the half holds [begin, begin + fill)
   int half = 0;
   bool used[2] = {false, false};
   auto flush = [&]() {
     if (!fill || ce != hipSuccess) return;
-    ce = hipMemcpyAsync(dst + begin, (char *)e->pinned + half * PINNED_HALF, fill, hipMemcpyHostToDevice, sm);
+    ce = hipMemcpyAsync(dst + begin, pin.half(half), fill, hipMemcpyHostToDevice, sm);
     if (ce == hipSuccess) ce = hipEventRecord(half ? e->ev1 : e->ev0, sm);
     used[half] = true;
     half ^= 1;
@@ -3322,7 +3377,7 @@ static hipError_t stage_in(mskg_engine *e, hipStream_t sm, char *dst, const std:
       }
       if (ce != hipSuccess) break;
       const size_t m = std::min(p.n - done, (size_t)PINNED_HALF - (off - begin));
-      memcpy((char *)e->pinned + half * PINNED_HALF + (off - begin), (const char *)p.src + done, m);
+      memcpy(pin.half(half) + (off - begin), (const char *)p.src + done, m);
       fill = off - begin + m;
       done += m;
       if (fill == (size_t)PINNED_HALF) flush();
@@ -3520,8 +3575,9 @@ static int state_lists(mskg_engine *e, const int64_t cap[3], int32_t *const xyz[
 // not written again (most of a box is vacuum, and so is a fresh array).
 static int state_words(mskg_engine *e, int32_t *latt) {
   const Box &b = e->box;
-  constexpr int64_t HALF = PINNED_HALF / 4;  // words
-  HIPCHK(e, pinned_buffer(e));
+  const int64_t HALF = std::min<int64_t>(PINNED_HALF / 4, b.npts);  // words
+  Pinned pin;
+  HIPCHK(e, pin.take());
   int32_t *d = (int32_t *)work_take(e, 1, 2 * HALF * 4);
   if (!d) return fail_(e, MSKG_ENOMEM, "store: no device memory for LattCoo's words");
   Lattice L = make_lattice(e);
@@ -3533,7 +3589,7 @@ static int state_words(mskg_engine *e, int32_t *latt) {
     hipLaunchKernelGGL(k_words_out, dim3((unsigned)((p1 - p0 + 255) / 256)), dim3(256), 0, e->stream, L, C, p0, p1, dst);
     hipError_t ce = hipGetLastError();
     if (ce == hipSuccess)
-      ce = hipMemcpyAsync(e->pinned + (i & 1) * HALF, dst, (size_t)(p1 - p0) * 4, hipMemcpyDeviceToHost, e->stream);
+      ce = hipMemcpyAsync(pin.half(i), dst, (size_t)(p1 - p0) * 4, hipMemcpyDeviceToHost, e->stream);
     if (ce == hipSuccess) ce = hipEventRecord(i & 1 ? e->ev1 : e->ev0, e->stream);
     return ce;
   };
@@ -3542,7 +3598,7 @@ static int state_words(mskg_engine *e, int32_t *latt) {
     if (i + 1 < pieces) ce = fetch(i + 1);
     if (ce == hipSuccess) ce = hipEventSynchronize(i & 1 ? e->ev1 : e->ev0);
     if (ce != hipSuccess) break;
-    const int32_t *src = e->pinned + (i & 1) * HALF;
+    const int32_t *src = (const int32_t *)pin.half(i);
     const int64_t p1 = std::min((i + 1) * HALF, b.npts);
     for (int64_t p = i * HALF; p < p1;) {  // row by row
       const int64_t row = p / b.hx, end = std::min(p1, (row + 1) * b.hx);
@@ -3668,6 +3724,7 @@ int mskg_create(const mskg_config *cfg, mskg_engine **out) {
   *out = nullptr;
   mskg_engine *e = new (std::nothrow) mskg_engine();
   if (!e) return MSKG_ENOMEM;
+  engine_born();
   *out = e;
   e->cfg = *cfg;
   if (cfg->len_x <= 0 || cfg->len_y <= 0 || cfg->len_z <= 0 || cfg->len_x % 12 || cfg->len_y % 12)
@@ -3795,13 +3852,13 @@ void mskg_destroy(mskg_engine *e) {
   hipFree(e->d_field[0]); hipFree(e->d_field[1]); hipFree(e->d_offwall); hipFree(e->d_st_tables); hipFree(e->d_win);
   hipFree(e->d_done);
   for (int k = 0; k < 2; k++) hipFree(e->d_work[k]);
-  if (e->pinned) hipHostFree(e->pinned);
   hipFree(e->d_geo); hipFree(e->d_tab); hipFree(e->d_st); hipFree(e->d_err); hipFree(e->d_log);
   hipFree(e->d_tsum); hipFree(e->d_bsum); hipFree(e->d_key); hipFree(e->d_key_seen); hipFree(e->d_rate_seen);
   if (e->ev0) hipEventDestroy(e->ev0);
   if (e->ev1) hipEventDestroy(e->ev1);
   if (e->stream) hipStreamDestroy(e->stream);
   delete e;
+  engine_gone();
 }
 
 int mskg_load_state(mskg_engine *e, const int32_t *latt, int32_t n_ad, const int32_t *ad_xyz, const int32_t *ad_nn,
