@@ -1054,14 +1054,18 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(LA ? 
 // tile is the sweep's stamp (sched[0], advanced by k_sweep_end), stored
 // with agent-scope release after the tile's writes; a waiting wave loads it
 // at agent scope and takes an agent-scope acquire before it reads the
-// neighbours' records, so the tiles' records travel between XCDs.  That acquire
-// drops the XCD's whole L2, which costs more than the barriers it replaces
-// (512^3 SiC: 39.8 against 75.3 M events/s).
+// neighbours' records, so the tiles' records travel between XCDs.  The release
+// writes the XCD's L2 back and the acquire invalidates it for all of its waves,
+// which costs more than the barriers they replace (512^3 SiC: 39.8 against 75.3
+// M events/s).
 //
 // The same sweep on one XCD (LOCAL): the waves of one XCD, whichever the
 // first wave to start is on, take all of the queue, and the others leave.
-// They share its L2, so that a tile's writes are released when the L2 has
-// them (its stores have returned) and acquired by dropping the CU's L1 alone.
+// They share its L2, so that a tile's writes are released when the L2 has them
+// (its stores have returned), without the write-back.  The acquire is the same
+// agent-scope invalidate (a workgroup's would do for the L1, but outside
+// threadgroup-split mode its loads and invalidates leave other CUs' writes
+// unseen); a few dozen waves can afford its refetches.
 // What bounds a sweep of a small lattice is the chain of its slowest tiles,
 // a few events of about 5 us each a colour, with a launch of 4.5 us after
 // every colour, whether it has tiles or not: a film in one tile layer has
@@ -1090,8 +1094,8 @@ __device__ inline void queue_layers(int zlo, int zhi, int odd, int ntz, int &fir
 constexpr int EVENT_POLLS = 512;
 constexpr int SCHED_POLLS = 7 * PASS_EVENT_CAP * EVENT_POLLS;
 
-// A word another CU of the same XCD has written (the L1 is passed by: the
-// coherence of a workgroup whose waves may run on several CUs).
+// A word another CU of the same XCD has written, read at agent scope (past the
+// L1), the load and its wait in one block.
 __device__ inline unsigned int load_xcd(const unsigned int *p) {
   unsigned int v;
   asm volatile("global_load_dword %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(p) : "memory");
@@ -1160,8 +1164,7 @@ __device__ inline void sweep_tiles(const PassParams &P, const PassParams *const 
   for (;;) {
     // the next entry: every lane adds 1 (one atomic of 64 for the wave), so
     // the head counts entries in units of 64
-    const unsigned int took = LOCAL ? __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                    : __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned int took = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int q = __builtin_amdgcn_readfirstlane((int)(took >> 6));
     if (q >= total) break;
     // entry -> colour, tile
@@ -1229,8 +1232,7 @@ __device__ inline void sweep_tiles(const PassParams &P, const PassParams *const 
       sweep_release<LOCAL>();  // the tile's writes before its flag
     }
     // every lane stores the same stamp
-    if (LOCAL) __hip_atomic_store(&P.done[t], stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else __hip_atomic_store(&P.done[t], stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&P.done[t], stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -4400,12 +4402,17 @@ static int run_begin(mskg_engine *e, int64_t max_events, double max_time, RunSta
 // as many waves are wanted (a wave that finds no tile free polls memory); an
 // XCD has 128 SIMDs, and past that its waves share issue slots that seven
 // other XCDs have idle.
-// Measured against the colour passes (whole runs, edge = tiles of 24): SiC,
-// k = 4, edge 96: 4.7, 4.4 ms; 240 (CVD): 11.1, 9.0; 384: 7.0, 6.0; 480: 6.9,
-// 6.0; 528: 7.2, 6.7; the shortest windows (policy 0, k = 1, where the queue's
-// own cost counts most), edge 384: 3.9, 3.4; 480: 4.3, 4.0; 528: 4.1, 4.3.  So
-// the line lies at 480's 100 tiles a colour and layer.  With tiles of 16 it
-// is the faster one well beyond (144 a colour: 4.8, 3.9).
+// Where the line lies: a sweep's time over the colour passes', SiC, Si, CVD and
+// laser annealing in tiles of 16 to 48, films in one tile layer and in two, with
+// 64, 81 and 100 tiles a colour and layer.  Windows of four events a tile
+// (policy 1): 0.70-0.91, 0.66-0.89 (one of 1.11), 0.70-0.90; of one: 0.69-0.90,
+// 0.64-1.00, 0.69-0.96; the shortest (policy 0, k = 1, where the queue's own
+// cost, an entry a tile with events or without, counts most) in tiles of 32
+// and more: 0.72-0.81, 0.75-0.96, 0.77-1.06, in smaller ones: 0.73-1.03 (mean
+// 0.86), 0.78-1.12 (0.93), 0.83-1.27 (1.02).  So 100 is the break-even of the
+// shortest windows in small tiles.  Above it longer windows and tiles of 16
+// would still gain (121 tiles of 24, k = 4: 7.2, 6.7 ms a run; 144 of 16: 4.8,
+// 3.9): the rule does not look at either.
 constexpr int XCD_TILES = 100;
 static int xcd_waves(const mskg_engine *e) {
   const int colour = e->ntx * e->nty / 4;
