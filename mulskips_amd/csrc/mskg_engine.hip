@@ -3055,7 +3055,6 @@ struct mskg_engine {
   int32_t *d_tl_n = nullptr;
   int32_t *d_tl_own = nullptr;
   double *d_tile_r = nullptr;
-  int32_t *d_tile_n = nullptr;
   int32_t *d_field[2] = {nullptr, nullptr};  // grid-sized maps of the laser-annealing coupling (on first use)
   // walls on grid points off the diamond super-lattice (the reference's
   // builders fill whole wall regions), which only the phase maps report:

@@ -93,17 +93,7 @@ MSKG_HD Site rd(const Lattice &L, int64_t i) {
   }
   return L.site[i];
 }
-MSKG_HD void wr(const Lattice &L, int64_t i, const Site &s) {
-  if (i >= 0) L.site[i] = s;
-}
 MSKG_HD NL list_of(const Lattice &L, const P3 &p, const Site &s) { return site_list(L.box, s, p.x, p.y, p.z); }
-MSKG_HD bool same(const NL &l, int j, const P3 &a) { return l.x[j] == a.x && l.y[j] == a.y && l.z[j] == a.z; }
-// The reference's Recipr loops: does list l contain the position a?
-MSKG_HD bool recip(const NL &l, const P3 &a) {
-  for (int j = 0; j < 4; j++)
-    if (same(l, j, a)) return true;
-  return false;
-}
 
 // x / tile for 0 <= x < 2^20: the FP32 quotient is off by at most one.
 MSKG_HD int tdiv(const Lattice &L, int x) {
@@ -120,10 +110,6 @@ MSKG_HD int tile_of(const Lattice &L, const P3 &p) {
 // (x / 2) in tile-local coordinates (tile edge <= 254), so that decoding
 // needs no division; offsets sort like the points' (z, y, x) order.
 MSKG_HD int tile_pack(int zl, int yl, int xl) { return (zl << 14) | ((yl >> 1) << 7) | (xl >> 1); }
-MSKG_HD int tile_offset(const Lattice &L, const P3 &p) {
-  const int tx = tdiv(L, p.x), ty = tdiv(L, p.y), tz = tdiv(L, p.z);
-  return tile_pack(p.z - tz * L.tile, p.y - ty * L.tile, p.x - tx * L.tile);
-}
 MSKG_HD int atomic_add_i32(int32_t *a, int v) {
 #ifdef __HIP_DEVICE_COMPILE__
   return atomicAdd(a, v);
@@ -146,25 +132,6 @@ MSKG_HD void atomic_max_i32(int *a, int v) {
 #else
   if (v > *a) *a = v;
 #endif
-}
-// Does the record sq of point q list position p?  The reference's Recipr
-// loops (list_of(q) contains p), evaluated on the stored displacements: a
-// valid entry holds p - q wrapped as set_list wraps it (no displacement is
-// near half a box edge), an unused entry stands for the origin.
-MSKG_HD bool lists_point(const Box &b, const P3 &q, const Site &sq, const P3 &p) {
-  int wx = p.x - q.x, wy = p.y - q.y;
-  const int wz = p.z - q.z;
-  if (wx > b.lx / 2) wx -= b.lx;
-  if (wx < -b.lx / 2) wx += b.lx;
-  if (wy > b.ly / 2) wy -= b.ly;
-  if (wy < -b.ly / 2) wy += b.ly;
-  const bool origin = p.x == 0 && p.y == 0 && p.z == 0;
-  bool hit = false;
-  for (int j = 0; j < 4; j++) {
-    if ((sq.valid >> j) & 1) hit |= sq.d[j][0] == wx && sq.d[j][1] == wy && sq.d[j][2] == wz;
-    else hit |= origin;
-  }
-  return hit;
 }
 MSKG_HD int tile_colour(int tx, int ty, int tz) { return (tx & 1) | ((ty & 1) << 1) | ((tz & 1) << 2); }
 // A tile layer that holds candidates joins the window of layers its colour's
@@ -679,9 +646,11 @@ __device__ inline bool rec_lists_disp(const Rec &r, uint32_t w) {
                  d = rec_disp_at<3>(r) ^ w;
   return min(min(a, b), min(c, d)) == 0u;
 }
-// lists_point on a record in registers: the record r of q against the point
-// p, when the displacement between them may not fit the record or p may be
-// the origin (which entries that are no displacement stand for).
+// Does the record r of point q list position p?  The reference's Recipr loops
+// (q's list contains p) on the stored displacements: a valid entry holds p - q
+// wrapped as set_list wraps it, an entry that is no displacement stands for the
+// origin.  For a displacement that may not fit the record or a p that may be
+// the origin; rec_lists_disp does for the others.
 __device__ inline bool rec_lists(const Box &b, const P3 &q, const Rec &r, const P3 &p) {
   bool has, ok;
   const uint32_t w = pack_disp(b, q, p, has, ok);

@@ -56,7 +56,6 @@ struct NL {
 
 MSKG_HD int s_kind(const Site &s) { return s.kc & 7; }
 MSKG_HD int s_coor(const Site &s) { return (s.kc >> 3) & 7; }
-MSKG_HD void s_set_kind(Site &s, int k) { s.kc = (uint8_t)((s.kc & ~7) | k); }
 MSKG_HD void s_set_coor(Site &s, int c) { s.kc = (uint8_t)((s.kc & 7) | (c << 3)); }
 MSKG_HD bool kind_occupied(int k) { return k >= 1 && k <= 4; }  // species or wall: Occ bit set
 MSKG_HD bool kind_species(int k) { return k >= 1 && k <= 3; }
