@@ -639,8 +639,9 @@ __device__ inline uint32_t pack_disp(const Box &b, const P3 &p, const P3 &o, boo
 __device__ inline uint32_t disp_back(uint32_t d) {
   return ((0x808080u - (d & 0x7f7f7fu)) ^ (~d & 0x808080u)) & 0xffffffu;
 }
-// Does the record list the point at displacement w from it?  An entry that
-// is no displacement holds zero, which w, of another point, is not.
+// Does the record list the point at displacement w from it, which is not the
+// origin?  An entry that is no displacement holds zero, which w, of another
+// point, is not; it stands for the origin, which rec_lists looks for.
 __device__ inline bool rec_lists_disp(const Rec &r, uint32_t w) {
   const uint32_t a = rec_disp_at<0>(r) ^ w, b = rec_disp_at<1>(r) ^ w, c = rec_disp_at<2>(r) ^ w,
                  d = rec_disp_at<3>(r) ^ w;
@@ -674,6 +675,7 @@ __device__ inline void get_prob(const Lattice &L, double rtot, const P3 &p, cons
       c0 = i0 < 0 ? 0 : (L.site[i0].kc >> 3) & 7;
     }
   } else if (kind_species(kind) && p.z >= t.frozen_below_z) {
+    const bool origin = (p.x | p.y | p.z) == 0;
 #pragma unroll 2
     for (int i = 0; i < 4; i++) {
       const P3 q = rec_entry(L, r, p, i);
@@ -681,7 +683,8 @@ __device__ inline void get_prob(const Lattice &L, double rtot, const P3 &p, cons
       if (q.i >= 0) sq = load_rec(L, q.i);
       const int kq = r_kind(sq);
       const bool lists = kq != KIND_EMPTY && kq != KIND_WALL &&
-                         (rec_has(r, i) ? rec_lists_disp(sq, disp_back(rec_disp(r, i))) : rec_lists(L.box, q, sq, p));
+                         (rec_has(r, i) && !origin ? rec_lists_disp(sq, disp_back(rec_disp(r, i)))
+                                                   : rec_lists(L.box, q, sq, p));
       if (COV && lists && kind_cov_slot(kq) > t.ncov) err = ERR_COVERAGE;
       cnt += neighbour_count(kq, lists);
     }
@@ -974,7 +977,9 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
     if (q.i == s.i) er = S;
     const int kq = r_kind(er);
     bool lists = rec_lists_disp(er, disp_back(e));
-    if (__ballot(look & !ehas & (kq != KIND_EMPTY)) && look && !ehas) lists = rec_lists(L.box, q, er, p);
+    // ... for a neighbour or a point at the origin by the form its position has in a list
+    const bool origin = !ehas | ((p.x | p.y | p.z) == 0);
+    if (__ballot(look & origin & (kq != KIND_EMPTY)) && look && origin) lists = rec_lists(L.box, q, er, p);
     lists &= look & (kq != KIND_EMPTY) & (kq != KIND_WALL);
     int err = ERR_NONE;
     if (COV) {
