@@ -2301,10 +2301,10 @@ __global__ void __launch_bounds__(WAVE) k_adjoint(const AdjDesc *descs) {
       ro = D.rate_seen[out.p.i];
       rn = L.rate[out.p.i];
     }
-    if (__ballot(out.set == 2)) {  // repeated list entries
+    if (__ballot(out.set == 2)) {  // repeated list entries, or the site among them
       bool dup = false;
-      for (int q = 0; q < 4; q++) {
-        const int l = 4 * q + 1;
+      for (int q = -1; q < 4; q++) {
+        const int l = q < 0 ? 0 : 4 * q + 1;
         const int lo = __builtin_amdgcn_readlane((int)(uint32_t)out.p.i, l);
         const int hi = __builtin_amdgcn_readlane((int)(out.p.i >> 32), l);
         const int on = __builtin_amdgcn_readlane(out.set, l);

@@ -580,7 +580,8 @@ MSKG_HD int pick_itrans(const Lattice &L, const Src &S, int coor, int temp, int 
 // site are never neighbours of each other), so the concurrent updates give
 // the sequential result.  When two list entries resolve to the same point
 // the neighbours are visited in order, a round each.  The site's own record
-// is written last; lanes whose gather meets the site take it from registers.
+// is written last, and before each round that has another after it; lanes
+// whose gather meets the site take it from registers.
 
 // A site record as it lies in memory (struct Site), in four words.
 typedef uint32_t Rec __attribute__((ext_vector_type(4)));
@@ -675,7 +676,7 @@ __device__ inline void get_prob(const Lattice &L, double rtot, const P3 &p, cons
       c0 = i0 < 0 ? 0 : (L.site[i0].kc >> 3) & 7;
     }
   } else if (kind_species(kind) && p.z >= t.frozen_below_z) {
-    const bool origin = (p.x | p.y | p.z) == 0;
+    const bool origin = p.i == 0;
 #pragma unroll 2
     for (int i = 0; i < 4; i++) {
       const P3 q = rec_entry(L, r, p, i);
@@ -847,15 +848,19 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
     to_s = pack_disp(L.box, p, s, has, ok);
     if (!has || !ok) to_s = 1u << 24;  // no entry is the site
   }
-  // repeated list entries (no displacement: zero)
+  // repeated list entries (no displacement: zero), or a zero one, which may be
+  // the site itself: an atom deposited on an unfixed site whose one neighbour is
+  // the origin, with no list there, takes the site for its zig-zag candidates,
+  // and the origin lists itself with an entry that is no displacement
   const uint32_t s0 = rec_disp_at<0>(S), s1 = rec_disp_at<1>(S), s2 = rec_disp_at<2>(S), s3 = rec_disp_at<3>(S);
-  const bool twice = nvisit == 4 && ((s0 == s1) | (s0 == s2) | (s0 == s3) | (s1 == s2) | (s1 == s3) | (s2 == s3));
+  const bool twice = nvisit == 4 && ((s0 == s1) | (s0 == s2) | (s0 == s3) | (s1 == s2) | (s1 == s3) | (s2 == s3) |
+                                     (min(min(s0, s1), min(s2, s3)) == 0u));
   // absorption and desorption change no neighbour's record: visits of one
   // point give it one rate, in whatever order (a covered site of coordination
   // 1 lists the origin three times)
   const bool seq = twice && (dep || evap);
   const bool shell = f2 && (dep || evap);
-  const Rec S_in = S;
+  Rec S_in = S;
   // The rounds: all quads at once; with repeated entries a round for each
   // neighbour and a last one for the second shell; with coverage species and
   // a second shell the neighbours first, since a covered neighbour's new list
@@ -877,6 +882,10 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
       uint32_t a = S.x, b = S.y, c = S.z, d = S.w;
       pin(a); pin(b); pin(c); pin(d);
       S = make_rec(a, b, c, d);
+    }
+    if (!last) {
+      if (lane == 0) store_rec(L, s.i, S);
+      __threadfence_block();
     }
     const unsigned nbm = (1u << nvisit) - 1u;
     const unsigned M = (seq ? (last ? 0u : 1u << round) : (round == 0 ? nbm : 0u)) | (last && shell ? 0xfff0u : 0u);
@@ -978,7 +987,7 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
     const int kq = r_kind(er);
     bool lists = rec_lists_disp(er, disp_back(e));
     // ... for a neighbour or a point at the origin by the form its position has in a list
-    const bool origin = !ehas | ((p.x | p.y | p.z) == 0);
+    const bool origin = !ehas | (p.i == 0);
     if (__ballot(look & origin & (kq != KIND_EMPTY)) && look && origin) lists = rec_lists(L.box, q, er, p);
     lists &= look & (kq != KIND_EMPTY) & (kq != KIND_WALL);
     int err = ERR_NONE;
@@ -1072,7 +1081,7 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
         }
       }
       const uint32_t old_w = S.w;
-      S.w = w_coor(S.w, coor);
+      if (!dep || coor != coor_old) S.w = w_coor(S.w, coor);  // deposition.f:236 writes a changed one only
       if (rem) S = make_rec(0u, 0u, 0u, S.w & 0xffff0000u);
       const int sc0 = __builtin_amdgcn_readlane(fc, 1);
       if (lane == 0) {
@@ -1119,7 +1128,10 @@ __device__ inline void execute(const Lattice &L, const TabLds &tabs, double rtot
       o.cls = cls;
       o.set = twice && lane != 0 && grp < 4 ? 2 : 1;
     }
-    if (!last) __threadfence_block();  // the next round reads this one's records
+    if (!last) {  // the next round reads this one's records, the site's too where it lists itself
+      __threadfence_block();
+      S_in = uniform_rec(load_rec(L, s.i));
+    }
   }
 }
 
