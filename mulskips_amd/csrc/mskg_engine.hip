@@ -310,7 +310,7 @@ __device__ inline bool sweep_mc(uint32_t w, int atoms_only, bool &keep) {
 // Four consecutive points from p0, or the points p0..n-1 at the end.  One
 // instance of Get_Prob: the group's MC particles are taken in turn and their
 // records read again (from the cache), so that the stream itself holds few
-// registers -- 62 with 8 waves per SIMD, against 128 and 4 with Get_Prob
+// registers -- 44 with 7 waves per SIMD, against 128 and 4 with Get_Prob
 // inlined for each of the four records.
 template <bool LA, bool COV>
 __device__ inline void sweep_group(const Lattice &L, double rtot, int *err, int atoms_only, int64_t p0, int64_t n) {
