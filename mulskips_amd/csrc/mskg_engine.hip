@@ -3234,11 +3234,12 @@ static void run_over(mskg_engine *e, int slab, int lo, int hi) {
 }
 // A workspace of at least n bytes, null when there is no memory for it; a
 // call that took one larger than work_keep gives it back at its end.  What is
-// kept follows the lattice (a sixteenth of its records, rates and classes, 8 MB
-// at most): a scan over hundreds of small lattices keeps little beside them.
+// kept follows the lattice (a fifth of its records, rates and classes, which is
+// what the words of a small one take on their way out; 8 MB at most): a scan over
+// hundreds of small lattices keeps little beside them.
 static size_t work_keep(const mskg_engine *e) {
   const int64_t lattice = e->box.npts * (int64_t)(sizeof(Site) + sizeof(float) + 1);
-  return (size_t)std::min<int64_t>(8 << 20, std::max<int64_t>(lattice / 16, 1 << 16));
+  return (size_t)std::min<int64_t>(8 << 20, std::max<int64_t>(lattice / 5, 1 << 16));
 }
 static void *work_take(mskg_engine *e, int k, size_t n) {
   if (e->work_n[k] < n) {
@@ -3576,10 +3577,10 @@ static int state_lists(mskg_engine *e, const int64_t cap[3], int32_t *const xyz[
 // not written again (most of a box is vacuum, and so is a fresh array).
 static int state_words(mskg_engine *e, int32_t *latt) {
   const Box &b = e->box;
-  const int64_t HALF = std::min<int64_t>(PINNED_HALF / 4, b.npts);  // words
+  constexpr int64_t HALF = PINNED_HALF / 4;  // words
   Pinned pin;
   HIPCHK(e, pin.take());
-  int32_t *d = (int32_t *)work_take(e, 1, 2 * HALF * 4);
+  int32_t *d = (int32_t *)work_take(e, 1, b.npts <= HALF ? b.npts * 4 : 2 * HALF * 4);  // one piece, or two in turn
   if (!d) return fail_(e, MSKG_ENOMEM, "store: no device memory for LattCoo's words");
   Lattice L = make_lattice(e);
   const CovList C = cov_list(e);
